@@ -2705,86 +2705,34 @@ __global__ __launch_bounds__(256) void conv3x3_dw_stream_kernel(float* __restric
     }
 }
 
-// dW[g][q] += sum over the S partial vectors of group g (a weight copy), in a fixed order: eight threads per
-// entry add a contiguous eighth each in ascending order, then the eight sums are added in ascending order.
-__global__ __launch_bounds__(256) void small_dw_reduce_kernel(float* __restrict__ dW, const float* __restrict__ P, int S,
-                                                              int Q) {
-    __shared__ float part[8][32];
+// dW[g][q] += sum over the S partial vectors of group g (a weight copy), in a fixed order: 32 threads per entry add a
+// contiguous 32nd each in ascending order, then the 32 sums are added in ascending order. The sums are a few KB: what
+// counts is the number of trips to memory, so a thread's loads are requested eight at a time (eight threads per entry,
+// each waiting for one load after the other: 256 partials of 27 entries, ten groups: 10 -> 4.7 us).
+__global__ __launch_bounds__(1024) void small_dw_reduce_kernel(float* __restrict__ dW, const float* __restrict__ P, int S,
+                                                               int Q) {
+    __shared__ float part[32][33];
     const int k = threadIdx.x >> 5, tl = threadIdx.x & 31;
     const int q = blockIdx.x * 32 + tl, g = blockIdx.y;
     const bool live = q < Q;
-    const float* src = P + (long)g * S * Q + q;
-    const int per = (S + 7) / 8, s0 = k * per, s1 = (s0 + per) < S ? (s0 + per) : S;
+    const float* src = P + (long)g * S * Q + (live ? q : 0);
+    const int per = (S + 31) / 32, s0 = k * per, s1 = (s0 + per) < S ? (s0 + per) : S;
     float sum = 0.f;
-    if (live)
-        for (int s = s0; s < s1; s++) sum += src[(long)s * Q];
+    int s = s0;
+    for (; s + 8 <= s1; s += 8) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = src[(long)(s + u) * Q];
+#pragma unroll
+        for (int u = 0; u < 8; u++) sum += v[u];
+    }
+    for (; s < s1; s++) sum += src[(long)s * Q];
     part[k][tl] = sum;
     __syncthreads();
     if (k != 0 || !live) return;
 #pragma unroll
-    for (int j = 1; j < 8; j++) sum += part[j][tl];
+    for (int j = 1; j < 32; j++) sum += part[j][tl];
     dW[(long)g * Q + q] += sum;
-}
-
-// Gradient of the per-pixel, per-channel bias the reference's Conv2d adds to the matmul result ([1,1,HW,O]):
-//   dbias[p][o] += sum over n of dz[n][o][p]   (dz in NCHW),
-// i.e. Col2ImgNode::backward (a transpose of the whole gradient) followed by AddNode::backward (a sum over the
-// batch) without the transposed copy. A workgroup owns 64 pixels x 32 channels: it starts from the values
-// already in dbias and adds the images in ascending order (the order of the two-step chain), reading dz
-// along pixels and writing dbias along channels; the tile is turned in LDS on the way in and on the way out.
-// MASK: dz is not given but made here, dz[n][o][p] = y[n][o][p] > 0 ? dy[n][o][p] : 0 (the gradient through the ReLU
-// that follows the convolution, ReLUNode::backward), written out for the other gradient kernels and summed on the way.
-template <bool MASK>
-__global__ __launch_bounds__(256) void conv_bias_grad_kernel(float* __restrict__ dbias, const float* __restrict__ dz, int N,
-                                                             int O, long HW, float* __restrict__ dz_out,
-                                                             const float* __restrict__ y) {
-    __shared__ float tile[64][33];                               // [pixel][channel]
-    const long p0 = (long)blockIdx.x * 64;
-    const int o0 = blockIdx.y * 32;
-    {   // in: rows of dbias (channels contiguous)
-        const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-#pragma unroll
-        for (int r = 0; r < 64; r += 8) {
-            const long p = p0 + ty + r;
-            const int o = o0 + tx;
-            tile[ty + r][tx] = (p < HW && o < O) ? dbias[p * O + o] : 0.f;
-        }
-    }
-    __syncthreads();
-    const int px = threadIdx.x & 63, oy = threadIdx.x >> 6;      // this thread's pixel, and channels oy, oy + 4, ...
-    const long p = p0 + px;
-    float acc[8];
-#pragma unroll
-    for (int r = 0; r < 8; r++) acc[r] = tile[px][oy + r * 4];
-    if (p < HW)
-        for (int n = 0; n < N; n++) {
-#pragma unroll
-            for (int r = 0; r < 8; r++) {
-                const int o = o0 + oy + r * 4;
-                if (o < O) {
-                    const long at = ((long)n * O + o) * HW + p;
-                    float g = dz[at];
-                    if (MASK) {
-                        g = y[at] > 0.f ? g : 0.f;
-                        dz_out[at] = g;
-                    }
-                    acc[r] += g;
-                }
-            }
-        }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 8; r++) tile[px][oy + r * 4] = acc[r];
-    __syncthreads();
-    {   // out: rows of dbias again
-        const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-#pragma unroll
-        for (int r = 0; r < 64; r += 8) {
-            const long pp = p0 + ty + r;
-            const int o = o0 + tx;
-            if (pp < HW && o < O) dbias[pp * O + o] = tile[ty + r][tx];
-        }
-    }
 }
 
 // Weights of the data-gradient convolution: the gradient with respect to x of a stride-1 convolution is
@@ -3419,75 +3367,118 @@ extern "C" int nzhip_conv2d_backward_data(float* dx, const float* dy, const floa
 
 namespace nzhip {
 
-// The same tile with 16-byte accesses (HW a multiple of 4, 16-byte aligned tensors): a thread owns four adjacent pixels
-// of channels oc and oc + 16, every element still one chain over ascending n (the same sums, bit for bit); two images'
-// loads are in flight at a time.
-template <bool MASK>
-__global__ __launch_bounds__(256) void conv_bias_grad_vec_kernel(float* __restrict__ dbias, const float* __restrict__ dz, int N,
-                                                                 int O, long HW, float* __restrict__ dz_out,
-                                                                 const float* __restrict__ y) {
-    __shared__ float tile[64][33];                               // [pixel][channel]
-    const long p0 = (long)blockIdx.x * 64;
-    const int o0 = blockIdx.y * 32;
-    {
-        const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+// Gradient of the per-pixel, per-channel bias the reference's Conv2d adds to the matmul result ([1,1,HW,O]):
+//   dbias[p][o] += sum over n of dz[n][o][p]   (dz in NCHW),
+// i.e. Col2ImgNode::backward (a transpose of the whole gradient) followed by AddNode::backward (a sum over the
+// batch) without the transposed copy. Every element is one chain: the value already in dbias, then the images in
+// ascending order (the order of the two-step chain, bit for bit).
+// MASK: dz is not given but made here, dz[n][o][p] = y[n][o][p] > 0 ? dy[n][o][p] : 0 (the gradient through the ReLU
+// that follows the convolution, ReLUNode::backward), written out for the other gradient kernels and summed on the way.
+//
+// A workgroup owns 256 V / TO pixels x TO channels, a thread V adjacent pixels of one channel; with more than one channel
+// the tile of dbias is turned in LDS on the way in and on the way out, with one channel dbias and dz have the same layout
+// and LDS is not used. Bound by memory: the loads of eight images are requested before the first is added. (A fixed tile
+// of 64 pixels x 32 channels left 31 of 32 threads idle for one channel and gave a 14 x 14 layer 32 workgroups:
+// 10 x 1 x 1024 x 1024 54 -> 9.6 us (4.8 TB/s), masked 72 -> 22; 16 x 256 x 14 x 14 masked 17 -> 5.5, 16 x 128 x 28 x 28 masked 23 -> 7.5.)
+template <bool MASK, int V, int TO>
+__global__ __launch_bounds__(256) void conv_bias_grad_kernel(float* __restrict__ dbias, const float* __restrict__ dz, int N,
+                                                             int O, long HW, float* __restrict__ dz_out,
+                                                             const float* __restrict__ y) {
+    constexpr int TP = 256 * V / TO, PT = TP / V;                // pixels of the tile; threads along them
+    constexpr int U = 8;                                         // images in flight
+    __shared__ float tile[TO > 1 ? TP : 1][TO + 1];              // [pixel][channel]
+    const long p0 = (long)blockIdx.x * TP;
+    const int o0 = blockIdx.y * TO;
+    const int px = (threadIdx.x % PT) * V, oc = threadIdx.x / PT;
+    const long p = p0 + px;
+    const bool live = p < HW && o0 + oc < O;                     // V == 4: HW % 4 == 0, the four pixels are inside together
+    auto turn = [&](auto&& element) {                            // channels fastest, as dbias lies
+        constexpr int ROWS = 256 / TO;
+        const int tx = threadIdx.x % TO, ty = threadIdx.x / TO;
 #pragma unroll
-        for (int r = 0; r < 64; r += 8) {
-            const long p = p0 + ty + r;
-            const int o = o0 + tx;
-            tile[ty + r][tx] = (p < HW && o < O) ? dbias[p * O + o] : 0.f;
+        for (int r = 0; r < TP; r += ROWS) {
+            const long pp = p0 + ty + r;
+            if (pp < HW && o0 + tx < O) element(dbias[pp * O + o0 + tx], tile[ty + r][tx]);
         }
+    };
+    auto load = [&](const float* src, float (&v)[V]) {
+        if constexpr (V == 4) {
+            const floatx4 q = *reinterpret_cast<const floatx4*>(src);
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = q[e];
+        } else {
+            v[0] = *src;
+        }
+    };
+    auto store = [&](float* dst, const float (&v)[V]) {
+        if constexpr (V == 4) *reinterpret_cast<floatx4*>(dst) = floatx4{v[0], v[1], v[2], v[3]};
+        else *dst = v[0];
+    };
+    float acc[V];
+    if constexpr (TO > 1) {
+        turn([](float& d, float& t) { t = d; });
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < V; e++) acc[e] = tile[px + e][oc];
+    } else if (live) {
+        load(dbias + p, acc);
     }
-    __syncthreads();
-    const int pq = threadIdx.x & 15, oc = threadIdx.x >> 4;      // pixels 4 pq .. 4 pq + 3, channels oc and oc + 16
-    const long p = p0 + 4 * pq;
-    float acc[2][4];
+    if (live) {
+        const long image = (long)O * HW, at0 = (long)(o0 + oc) * HW + p;
+        auto some = [&](const int n0, auto count) {
+            constexpr int C = decltype(count)::value;
+            float g[C][V], yy[MASK ? C : 1][V];
 #pragma unroll
-    for (int h = 0; h < 2; h++)
+            for (int u = 0; u < C; u++) {
+                load(dz + (long)(n0 + u) * image + at0, g[u]);
+                if constexpr (MASK) load(y + (long)(n0 + u) * image + at0, yy[u]);
+            }
 #pragma unroll
-        for (int e = 0; e < 4; e++) acc[h][e] = tile[4 * pq + e][oc + 16 * h];
-    if (p < HW) {                                                // HW % 4 == 0: the four pixels are inside together
-        const bool live[2] = {o0 + oc < O, o0 + oc + 16 < O};
-        const long plane = HW, image = (long)O * HW;
-        const long at0 = (long)(o0 + oc) * plane + p;
-        auto step = [&](const int n) {
+            for (int u = 0; u < C; u++) {
+                if constexpr (MASK) {
 #pragma unroll
-            for (int h = 0; h < 2; h++)
-                if (live[h]) {
-                    const long at = (long)n * image + at0 + (long)h * 16 * plane;
-                    floatx4 g = *reinterpret_cast<const floatx4*>(dz + at);
-                    if (MASK) {
-                        const floatx4 yy = *reinterpret_cast<const floatx4*>(y + at);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) g[e] = yy[e] > 0.f ? g[e] : 0.f;
-                        *reinterpret_cast<floatx4*>(dz_out + at) = g;
-                    }
-#pragma unroll
-                    for (int e = 0; e < 4; e++) acc[h][e] += g[e];
+                    for (int e = 0; e < V; e++) g[u][e] = yy[u][e] > 0.f ? g[u][e] : 0.f;
+                    store(dz_out + (long)(n0 + u) * image + at0, g[u]);
                 }
+#pragma unroll
+                for (int e = 0; e < V; e++) acc[e] += g[u][e];
+            }
         };
         int n = 0;
-        for (; n + 2 <= N; n += 2) {
-            step(n);
-            step(n + 1);
-        }
-        if (n < N) step(n);
+        for (; n + U <= N; n += U) some(n, std::integral_constant<int, U>{});
+        for (; n + 2 <= N; n += 2) some(n, std::integral_constant<int, 2>{});
+        if (n < N) some(n, std::integral_constant<int, 1>{});
     }
-    __syncthreads();
+    if constexpr (TO > 1) {
+        __syncthreads();
 #pragma unroll
-    for (int h = 0; h < 2; h++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) tile[4 * pq + e][oc + 16 * h] = acc[h][e];
-    __syncthreads();
-    {
-        const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-#pragma unroll
-        for (int r = 0; r < 64; r += 8) {
-            const long pp = p0 + ty + r;
-            const int o = o0 + tx;
-            if (pp < HW && o < O) dbias[pp * O + o] = tile[ty + r][tx];
-        }
+        for (int e = 0; e < V; e++) tile[px + e][oc] = acc[e];
+        __syncthreads();
+        turn([](float& d, float& t) { d = t; });
+    } else if (live) {
+        store(dbias + p, acc);
     }
+}
+
+// Which tile: one channel needs no turning; up to four channels take a tile of four; beyond that 32 x 32 elements with
+// 16-byte accesses when that still gives every compute unit two workgroups, else 32 pixels x 8 channels, a pixel a thread,
+// for four times the workgroups.
+template <bool MASK>
+static int conv_bias_grad_launch(float* dbias, const float* dz, size_t N, size_t O, size_t HW, float* dz_out, const float* y,
+                                 hipStream_t s) {
+    const bool vec = HW % 4 == 0 && ((reinterpret_cast<uintptr_t>(dz) | reinterpret_cast<uintptr_t>(dz_out) | reinterpret_cast<uintptr_t>(y) |
+                                      (O == 1 ? reinterpret_cast<uintptr_t>(dbias) : 0)) & 15) == 0;
+    const bool many = HW * O >= (size_t)device_cu_count() * 2 * 1024;
+    auto go = [&](auto kernel, size_t tp, size_t to) {
+        const size_t gx = (HW + tp - 1) / tp, gy = (O + to - 1) / to;
+        if (gx > 0x7fffffffull || gy > 65535) return set_error(NZHIP_E_UNSUPPORTED, "conv bias gradient: extent too large");
+        hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, dbias, dz, (int)N, (int)O, (long)HW, dz_out, y);
+        hipError_t e = hipGetLastError();
+        return e == hipSuccess ? NZHIP_OK : set_hip_error(e, "conv_bias_grad kernel launch");
+    };
+    if (O == 1) return vec && many ? go(conv_bias_grad_kernel<MASK, 4, 1>, 1024, 1) : go(conv_bias_grad_kernel<MASK, 1, 1>, 256, 1);
+    if (O <= 4) return vec && many ? go(conv_bias_grad_kernel<MASK, 4, 4>, 256, 4) : go(conv_bias_grad_kernel<MASK, 1, 4>, 64, 4);
+    return vec && many ? go(conv_bias_grad_kernel<MASK, 4, 32>, 32, 32) : go(conv_bias_grad_kernel<MASK, 1, 8>, 32, 8);
 }
 
 }  // namespace nzhip
@@ -3498,15 +3489,8 @@ __global__ __launch_bounds__(256) void conv_bias_grad_vec_kernel(float* __restri
 extern "C" int nzhip_conv2d_backward_bias(float* dbias, const float* dz, size_t N, size_t O, size_t HW, void* stream) {
     if (!dbias || !dz) return set_error(NZHIP_E_INVALID, "nzhip_conv2d_backward_bias: null pointer");
     if (N == 0 || O == 0 || HW == 0) return NZHIP_OK;
-    if (N > 0x7fffffff || O > 0x7fffffff || (O + 31) / 32 > 65535 || (HW + 63) / 64 > 0x7fffffffull)
-        return set_error(NZHIP_E_UNSUPPORTED, "nzhip_conv2d_backward_bias: extent too large");
-    dim3 grid((unsigned)((HW + 63) / 64), (unsigned)((O + 31) / 32));
-    const bool vec = HW % 4 == 0 && (reinterpret_cast<uintptr_t>(dz) & 15) == 0;
-    hipLaunchKernelGGL(vec ? conv_bias_grad_vec_kernel<false> : conv_bias_grad_kernel<false>, grid, dim3(256), 0,
-                       reinterpret_cast<hipStream_t>(stream), dbias, dz, (int)N, (int)O, (long)HW, static_cast<float*>(nullptr),
-                       static_cast<const float*>(nullptr));
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? NZHIP_OK : set_hip_error(e, "conv_bias_grad kernel launch");
+    if (N > 0x7fffffff || O > 0x7fffffff) return set_error(NZHIP_E_UNSUPPORTED, "nzhip_conv2d_backward_bias: extent too large");
+    return conv_bias_grad_launch<false>(dbias, dz, N, O, HW, nullptr, nullptr, reinterpret_cast<hipStream_t>(stream));
 }
 
 /* The same with the ReLU gradient in front (Conv2d followed by ReLU): dz[n][o][p] = y[n][o][p] > 0 ? dy[n][o][p] : 0
@@ -3516,14 +3500,8 @@ extern "C" int nzhip_conv2d_backward_relu_bias(float* dz, float* dbias, const fl
                                                size_t HW, void* stream) {
     if (!dz || !dbias || !y || !dy) return set_error(NZHIP_E_INVALID, "nzhip_conv2d_backward_relu_bias: null pointer");
     if (N == 0 || O == 0 || HW == 0) return NZHIP_OK;
-    if (N > 0x7fffffff || O > 0x7fffffff || (O + 31) / 32 > 65535 || (HW + 63) / 64 > 0x7fffffffull)
-        return set_error(NZHIP_E_UNSUPPORTED, "nzhip_conv2d_backward_relu_bias: extent too large");
-    dim3 grid((unsigned)((HW + 63) / 64), (unsigned)((O + 31) / 32));
-    const bool vec = HW % 4 == 0 && ((reinterpret_cast<uintptr_t>(dz) | reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(dy)) & 15) == 0;
-    hipLaunchKernelGGL(vec ? conv_bias_grad_vec_kernel<true> : conv_bias_grad_kernel<true>, grid, dim3(256), 0,
-                       reinterpret_cast<hipStream_t>(stream), dbias, dy, (int)N, (int)O, (long)HW, dz, y);
-    hipError_t e = hipGetLastError();
-    return e == hipSuccess ? NZHIP_OK : set_hip_error(e, "conv_bias_grad (masked) kernel launch");
+    if (N > 0x7fffffff || O > 0x7fffffff) return set_error(NZHIP_E_UNSUPPORTED, "nzhip_conv2d_backward_relu_bias: extent too large");
+    return conv_bias_grad_launch<true>(dbias, dy, N, O, HW, dz, y, reinterpret_cast<hipStream_t>(stream));
 }
 
 // dw[i] += P[0][i] + P[1][i] + ... (ascending, then added to dw once): the per-image products of the 1x1 weight gradient
@@ -4126,7 +4104,7 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
         if (rc == NZHIP_OK) {
             const bool shared = w_batch == 1;
             const int S = (int)(shared ? per_image * N : per_image), groups = shared ? 1 : (int)N;
-            hipLaunchKernelGGL(small_dw_reduce_kernel, dim3((unsigned)((Q + 31) / 32), (unsigned)groups), dim3(256), 0, s, dw,
+            hipLaunchKernelGGL(small_dw_reduce_kernel, dim3((unsigned)((Q + 31) / 32), (unsigned)groups), dim3(1024), 0, s, dw,
                                partial, S, (int)Q);
             e = hipGetLastError();
             if (e != hipSuccess) rc = set_hip_error(e, "small_dw_reduce kernel launch");

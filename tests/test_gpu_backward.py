@@ -525,6 +525,27 @@ def test_conv2d_backward_relu_bias_equals_relu_backward_then_bias(nz, oracle, N,
     assert np.array_equal(host(dz), dz_want) and np.array_equal(host(db), db_want)
 
 
+@pytest.mark.parametrize("N,O,H,W", [(11, 1, 512, 1028), (3, 1, 37, 41), (9, 3, 420, 420), (10, 33, 128, 130), (17, 34, 9, 14), (8, 4, 5, 13)])
+def test_conv2d_bias_gradients_on_every_tile_shape(nz, oracle, N, O, H, W):
+    """One, up to four and more channels, with and without 16-byte accesses, image counts around the eight in flight, edges in
+    both directions: one chain per element, so bit for bit."""
+    rng = np.random.default_rng(N + O + H + W)
+    y = np.maximum(rng.standard_normal((N, O, H, W), dtype=np.float32), 0)
+    dy = rng.standard_normal((N, O, H, W), dtype=np.float32)
+    base = rng.standard_normal((1, 1, H * W, O), dtype=np.float32)
+    dz_want = np.where(y > 0, dy, np.float32(0))
+    for masked, dz in ((False, dy), (True, dz_want)):
+        want = base.copy()
+        for n in range(N):
+            want += dz[n].reshape(O, H * W).T[None, None]
+        db = dev(base)
+        if masked:
+            assert np.array_equal(host(nz.conv2d_backward_relu_bias(db, dev(y), dev(dy))), dz_want)
+        else:
+            nz.conv2d_backward_bias(db, dev(dy))
+        assert np.array_equal(host(db), want), masked
+
+
 def test_conv2d_backward_weights_rejects_what_it_does_not_cover(nz):
     from neuzephyr_amd.capi import NzHipError
     with pytest.raises(NzHipError) as e:      # stride 5
