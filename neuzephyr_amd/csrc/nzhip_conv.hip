@@ -64,6 +64,15 @@ __device__ __forceinline__ void xcd_contiguous_block_z_fastest(int& bx, int& by,
     by = (int)(unit / (gz * gx));
 }
 
+// Where the weight of (input channel c, tap, output channel o) of the convolution a kernel runs lies in w_ref.
+// mirror == 0: w_ref is that convolution's own parameter, [(c, tap)][o]. mirror != 0: the kernel runs the data gradient
+// of a convolution whose parameter w_ref is ([(c_f, tap_f)][o_f] with C output and O input channels in the kernel's
+// terms): its weights are w'[(o_f, tap)][c_f] = w[(c_f, taps - 1 - tap)][o_f], read in place, so that no mirrored
+// copy has to be written first.
+__device__ __forceinline__ long weight_source_index(int c, int tap, int o, int C, int O, int taps, int mirror) {
+    return mirror ? ((long)o * taps + (taps - 1 - tap)) * C + c : ((long)c * taps + tap) * O + o;
+}
+
 // O_T: output channels per thread; C_T: compile-time input-channel count (0 = runtime loop);
 // VEC: W % 4 == 0 and 16-byte aligned tensors, so every lane's 4 pixels are inside the row and
 // move as one 16-byte access.
@@ -72,13 +81,14 @@ __global__ __launch_bounds__(256) void conv3x3_direct_kernel(float* __restrict__
                                                              const float* __restrict__ w_ref,
                                                              const float* __restrict__ bias, int C_rt, int H, int W,
                                                              int O, long w_batch_stride, long bias_sp, long bias_sc,
-                                                             int relu) {
+                                                             int relu, int mirror) {
     __shared__ _Float16 wsm[DC_MAX_C * 9 * DC_MAX_O];
     const int C = C_T ? C_T : C_rt;
     int bx, by, b;
     xcd_contiguous_block(bx, by, b);
     const float* wb = w_ref + (long)b * w_batch_stride;
-    for (int i = threadIdx.x; i < C * 9 * O; i += 256) wsm[i] = (_Float16)wb[i];     // [q][o], RNE
+    for (int i = threadIdx.x; i < C * 9 * O; i += 256)                               // [q][o], RNE
+        wsm[i] = (_Float16)wb[mirror ? weight_source_index(i / (9 * O), i / O % 9, i % O, C, O, 9, 1) : i];
     __syncthreads();
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -219,15 +229,34 @@ __device__ __forceinline__ float from_lane_above(float v) {
                                                                  0x130 /* wave_shl:1 */, 0xf, 0xf, false));
 }
 
+// A lane's quad of a row whose 16-byte pieces are not aligned, cut by the end of the row or past it: one 16-byte access at a
+// 4-byte aligned address, moved left into the row (W >= 4) where the quad does not fit, and turned back in registers. `back`
+// is how far it was moved; elements past the end of the row come out as some element of the row.
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load_ragged_quad(const float* row, int at, int back, float (&v)[4]) {
+    const floatx4 q = *reinterpret_cast<const floatx4u*>(row + at);
+    const float a = back & 1 ? q[1] : q[0], b = back & 1 ? q[2] : q[1], c = back & 1 ? q[3] : q[2];
+    v[0] = back & 2 ? c : a;
+    v[1] = back & 2 ? q[3] : b;
+    v[2] = c;
+    v[3] = q[3];
+}
+
 // PIX_BIAS: 0 none or per channel; 1 per pixel with any strides; 2 per pixel in the layout of the
 // reference's Bias node ([pixel][channel], 16-byte aligned), where a lane's 4 pixels x O_T channels are one
 // contiguous run fetched with 16-byte loads.
-template <int O_T, int C_T, int PIX_BIAS>
+// VEC: rows of whole, aligned 16-byte pieces. Otherwise (rows of 1023) the same walk with 16-byte accesses at 4-byte aligned
+// addresses, which the memory path takes at nearly the aligned rate: 10 x 3 x 1000 x 1023 -> 1 42 us against 39 for 1024
+// columns. (83 us on the four-row blocks of the direct kernel, which re-reads half its rows element by element; 72 us with
+// this kernel's quads as four 4-byte accesses each.) The quad cut by the end of the row is moved left into it and turned back.
+// mirror: the weights are those of the convolution whose data gradient this is (weight_source_index).
+template <int O_T, int C_T, int PIX_BIAS, bool VEC>
 __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__ y, const float* __restrict__ x,
                                                              const float* __restrict__ w_ref,
                                                              const float* __restrict__ bias, int H, int W,
                                                              long w_batch_stride, long bias_sp, long bias_sc,
-                                                             int relu) {
+                                                             int relu, int mirror) {
+    static_assert(VEC || PIX_BIAS != 2 || O_T == 1, "runs of bias for several channels need aligned rows");
     __shared__ float wsm[C_T * 9 * O_T];
     int bx, by, b;
     xcd_contiguous_block(bx, by, b);
@@ -235,7 +264,8 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
     static_assert(C_T * 9 * O_T <= 128, "one weight per thread");
     // requested now, parked in LDS after the first input rows have been requested (the rows then do not
     // queue up behind the round trip of the weights)
-    const float w_mine = threadIdx.x < C_T * 9 * O_T ? wb[threadIdx.x] : 0.f;
+    const int w_i = threadIdx.x < C_T * 9 * O_T ? threadIdx.x : 0;
+    const float w_mine = wb[mirror ? weight_source_index(w_i / (9 * O_T), w_i / O_T % 9, w_i % O_T, C_T, O_T, 9, 1) : w_i];
     auto park_weights = [&]() {
         if (threadIdx.x < C_T * 9 * O_T) wsm[threadIdx.x] = round_f16(w_mine);   // [q][o]
         __syncthreads();
@@ -251,7 +281,11 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
     // Lanes past the last column stay in the walk (the barrier in park_weights() must not sit in a branch that
     // only some lanes of a wave take): they work on the image's last quad of columns and store nothing.
     const bool active = (bx * 64 + lane) * 4 < W;
-    const int w0 = active ? (bx * 64 + lane) * 4 : W - 4;
+    const int w0 = active ? (bx * 64 + lane) * 4 : (W - 1) / 4 * 4;
+    bool col[4];                                                 // the lane's columns inside the row
+#pragma unroll
+    for (int e = 0; e < 4; e++) col[e] = VEC || w0 + e < W;
+    const int w_at = w0 + 4 <= W ? w0 : W - 4;
     const float* xb = x + (long)b * C_T * H * W;
     float* yb = y + (long)b * O_T * H * W;
     const long plane = (long)H * W;
@@ -286,7 +320,12 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
             // the bias of the output row a step completes travels with that step's input row, so its
             // wait never drains the rows requested after it
             const int hb = (t >= 2 && t < T) ? out_row(t) : h0;
-            if (PIX_BIAS == 2) {
+            if constexpr (PIX_BIAS == 2 && !VEC) {
+                float v[4];
+                load_ragged_quad(bias + (long)hb * W, w_at, w0 - w_at, v);
+#pragma unroll
+                for (int e = 0; e < 4; e++) bdst[0][e] = v[e];
+            } else if constexpr (PIX_BIAS == 2) {
                 const floatx4* run = reinterpret_cast<const floatx4*>(bias + ((long)hb * W + w0) * O_T);
 #pragma unroll
                 for (int k = 0; k < O_T; k++) {
@@ -298,16 +337,23 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
 #pragma unroll
                 for (int o = 0; o < O_T; o++)
 #pragma unroll
-                    for (int e = 0; e < 4; e++) bdst[o][e] = bias[((long)hb * W + w0 + e) * bias_sp + (long)o * bias_sc];
+                    for (int e = 0; e < 4; e++) bdst[o][e] = bias[((long)hb * W + (col[e] ? w0 + e : w0)) * bias_sp + (long)o * bias_sc];
             }
         }
 #pragma unroll
         for (int c = 0; c < C_T; c++) {
-            const floatx4 q = *reinterpret_cast<const floatx4*>(row + c * plane + w0);
-            dst[c][0] = q[0];
-            dst[c][1] = q[1];
-            dst[c][2] = q[2];
-            dst[c][3] = q[3];
+            if constexpr (VEC) {
+                const floatx4 q = *reinterpret_cast<const floatx4*>(row + c * plane + w0);
+                dst[c][0] = q[0];
+                dst[c][1] = q[1];
+                dst[c][2] = q[2];
+                dst[c][3] = q[3];
+            } else {
+                float v[4];
+                load_ragged_quad(row + c * plane, w_at, w0 - w_at, v);
+#pragma unroll
+                for (int e = 0; e < 4; e++) dst[c][e] = v[e];
+            }
             dst[c][4] = row[c * plane + wx];
         }
     };
@@ -334,7 +380,7 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
                     // load and the wave waits for every row as soon as it has asked for it.
                     float v = raw[u][c][e];
                     asm volatile("" : "+v"(v));
-                    r5[e] = in_img ? round_f16(v) : 0.f;
+                    r5[e] = in_img && (e == 4 || col[e == 4 ? 0 : e]) ? round_f16(v) : 0.f;
                 }
                 const float below = from_lane_below(r5[3]), above = from_lane_above(r5[0]);
                 win[wu][c][0] = has_l ? (lane == 0 ? r5[4] : below) : 0.f;
@@ -383,7 +429,18 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
                     if (relu) a = a > 0.f ? a : 0.f;
                     ov[e] = a;
                 }
-                if (active) *reinterpret_cast<floatx4*>(yb + ((long)o * H + ho) * W + w0) = ov;
+                float* dst = yb + ((long)o * H + ho) * W + w0;
+                if constexpr (VEC) {
+                    if (active) *reinterpret_cast<floatx4*>(dst) = ov;
+                } else {
+                    if (active && col[3]) {
+                        *reinterpret_cast<floatx4u*>(dst) = ov;
+                    } else if (active) {
+#pragma unroll
+                        for (int e = 0; e < 3; e++)
+                            if (col[e]) dst[e] = ov[e];
+                    }
+                }
             }
         }
     }
@@ -397,27 +454,27 @@ static bool conv_direct_applicable(size_t C, size_t O, size_t K_h, size_t K_w, s
 }
 
 static int conv_direct(float* y, const float* x, const float* w_ref, const float* bias, size_t N, size_t C, size_t H,
-                       size_t W, size_t O, size_t w_batch, int64_t bias_sp, int64_t bias_sc, int act, hipStream_t s) {
+                       size_t W, size_t O, size_t w_batch, int64_t bias_sp, int64_t bias_sc, int act, bool w_mirror, hipStream_t s) {
     if (N > 65535) return set_error(NZHIP_E_UNSUPPORTED, "nzhip_conv2d_forward: batch above 65535");
     const int vec = (W % 4 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0) && ((reinterpret_cast<uintptr_t>(y) & 15) == 0);
     dim3 grid((unsigned)((W + 255) / 256), (unsigned)((H + 4 * DC_ROWS - 1) / (4 * DC_ROWS)), (unsigned)N);
     const long wbs = w_batch > 1 ? (long)(C * 9 * O) : 0;
-    if (vec && C <= 4 && O <= 2 && H >= 8) {
+    if (C <= 4 && O <= 2 && H >= 8 && W >= 4) {
         dim3 sgrid((unsigned)((W + 255) / 256), (unsigned)((H + 4 * ST_ROWS - 1) / (4 * ST_ROWS)), (unsigned)N);
         const bool pixb = bias && bias_sp != 0;
         // the reference's Bias node: [pixel][channel], so the bias of a lane's 4 pixels is one aligned run
-        const bool pixrun = pixb && bias_sp == (int64_t)O && bias_sc == 1 && (reinterpret_cast<uintptr_t>(bias) & 15) == 0;
+        const bool pixlayout = pixb && bias_sp == (int64_t)O && bias_sc == 1, pixrun = pixlayout && (reinterpret_cast<uintptr_t>(bias) & 15) == 0;
+#define NZHIP_STK(OT, CT, PB, V)                                                                                      \
+    hipLaunchKernelGGL((conv3x3_stream_kernel<OT, CT, PB, V>), sgrid, dim3(256), 0, s, y, x, w_ref, bias, (int)H, (int)W, wbs, \
+                       (long)bias_sp, (long)bias_sc, act == NZHIP_ACT_RELU, w_mirror ? 1 : 0)
 #define NZHIP_ST(OT, CT)                                                                                             \
     do {                                                                                                             \
-        if (pixrun)                                                                                                  \
-            hipLaunchKernelGGL((conv3x3_stream_kernel<OT, CT, 2>), sgrid, dim3(256), 0, s, y, x, w_ref, bias, (int)H,  \
-                               (int)W, wbs, (long)bias_sp, (long)bias_sc, act == NZHIP_ACT_RELU);                   \
-        else if (pixb)                                                                                               \
-            hipLaunchKernelGGL((conv3x3_stream_kernel<OT, CT, 1>), sgrid, dim3(256), 0, s, y, x, w_ref, bias, (int)H,  \
-                               (int)W, wbs, (long)bias_sp, (long)bias_sc, act == NZHIP_ACT_RELU);                   \
-        else                                                                                                         \
-            hipLaunchKernelGGL((conv3x3_stream_kernel<OT, CT, 0>), sgrid, dim3(256), 0, s, y, x, w_ref, bias, (int)H,  \
-                               (int)W, wbs, (long)bias_sp, (long)bias_sc, act == NZHIP_ACT_RELU);                   \
+        if (vec && pixrun) NZHIP_STK(OT, CT, 2, true);                                                                \
+        else if (vec && pixb) NZHIP_STK(OT, CT, 1, true);                                                             \
+        else if (vec) NZHIP_STK(OT, CT, 0, true);                                                                     \
+        else if (OT == 1 && pixlayout) NZHIP_STK(OT, CT, OT == 1 ? 2 : 1, false);                                     \
+        else if (pixb) NZHIP_STK(OT, CT, 1, false);                                                                   \
+        else NZHIP_STK(OT, CT, 0, false);                                                                             \
     } while (0)
         switch ((int)(O * 10 + C)) {
             case 11: NZHIP_ST(1, 1); break;
@@ -430,12 +487,13 @@ static int conv_direct(float* y, const float* x, const float* w_ref, const float
             default: NZHIP_ST(2, 4); break;
         }
 #undef NZHIP_ST
+#undef NZHIP_STK
         hipError_t e = hipGetLastError();
         return e == hipSuccess ? NZHIP_OK : set_hip_error(e, "conv3x3_stream_kernel launch");
     }
 #define NZHIP_DC(OT, CT, V)                                                                                     \
     hipLaunchKernelGGL((conv3x3_direct_kernel<OT, CT, V>), grid, dim3(256), 0, s, y, x, w_ref, bias, (int)C, (int)H, \
-                       (int)W, (int)O, wbs, (long)bias_sp, (long)bias_sc, act == NZHIP_ACT_RELU)
+                       (int)W, (int)O, wbs, (long)bias_sp, (long)bias_sc, act == NZHIP_ACT_RELU, w_mirror ? 1 : 0)
 #define NZHIP_DC_O(CT, V)            \
     switch (O) {                     \
         case 1: NZHIP_DC(1, CT, V); break; \
@@ -493,14 +551,6 @@ struct IgemmGeom {
     static constexpr int PASSES = (UNITS + 255) / 256;
 };
 
-// Where the weight of (input channel c, tap, output channel o) of the convolution a kernel runs lies in w_ref.
-// mirror == 0: w_ref is that convolution's own parameter, [(c, tap)][o]. mirror != 0: the kernel runs the data gradient
-// of a convolution whose parameter w_ref is ([(c_f, tap_f)][o_f] with C output and O input channels in the kernel's
-// terms): its weights are w'[(o_f, tap)][c_f] = w[(c_f, taps - 1 - tap)][o_f], read in place, so that no mirrored
-// copy has to be written first.
-__device__ __forceinline__ long weight_source_index(int c, int tap, int o, int C, int O, int taps, int mirror) {
-    return mirror ? ((long)o * taps + (taps - 1 - tap)) * C + c : ((long)c * taps + tap) * O + o;
-}
 // The 16 input channels of chunk `chunk` at (tap, output channel o), rounded: h[0] holds channels 0..7, h[1] 8..15
 // (zeros past C or O). The pre-passes below give one thread one (row, tap) of a slab, adjacent threads adjacent output
 // channels: with a convolution's own parameter each of the 16 reads is contiguous across the wave; with a mirrored one
@@ -2389,9 +2439,8 @@ struct ConvDwArgs {
     int n_images;
 };
 
-// VEC: W is a multiple of 8 and x, dy are 16-byte aligned (two 16-byte loads per group of 8 pixels); otherwise
-// every pixel is loaded and bounds-checked on its own.
-template <bool VEC>
+// W is a multiple of 8 and x, dy are 16-byte aligned: two 16-byte loads per group of 8 pixels, a group is wholly inside or
+// outside the image.
 __global__ __launch_bounds__(256) void conv_dw_kernel(const ConvDwArgs p) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     char* xs = lds;                       // [slot 3][shift 3][channel 32] rows of DW_PITCH bytes
@@ -2426,24 +2475,18 @@ __global__ __launch_bounds__(256) void conv_dw_kernel(const ConvDwArgs p) {
         for (int u = 0; u < 2; u++) {
             const int c = u * 16 + (tid >> 4);
             const int w = w0 + g * 8;
-            const bool ok = c < nch && h >= 0 && h < p.H && w < p.W;       // VEC: a group is wholly inside or outside
+            const bool ok = c < nch && h >= 0 && h < p.H && w < p.W; 
             const float* src = ximg + (long)c * plane + (long)h * p.W + w;
 #pragma unroll
             for (int e = 0; e < 8; e++) xr[u][e] = 0.f;
             xl[u] = 0.f;
             xrt[u] = 0.f;
             if (ok) {
-                if (VEC) {
-                    const floatx4 a = *reinterpret_cast<const floatx4*>(src), b = *reinterpret_cast<const floatx4*>(src + 4);
+                const floatx4 a = *reinterpret_cast<const floatx4*>(src), b = *reinterpret_cast<const floatx4*>(src + 4);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        xr[u][e] = a[e];
-                        xr[u][4 + e] = b[e];
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; e++)
-                        if (w + e < p.W) xr[u][e] = src[e];
+                for (int e = 0; e < 4; e++) {
+                    xr[u][e] = a[e];
+                    xr[u][4 + e] = b[e];
                 }
                 if (g == 0 && w > 0) xl[u] = src[-1];
                 if (g == 15 && w + 8 < p.W) xrt[u] = src[8];
@@ -2460,17 +2503,11 @@ __global__ __launch_bounds__(256) void conv_dw_kernel(const ConvDwArgs p) {
 #pragma unroll
             for (int e = 0; e < 8; e++) zr[i][e] = 0.f;
             if (ok) {
-                if (VEC) {
-                    const floatx4 a = *reinterpret_cast<const floatx4*>(src), b = *reinterpret_cast<const floatx4*>(src + 4);
+                const floatx4 a = *reinterpret_cast<const floatx4*>(src), b = *reinterpret_cast<const floatx4*>(src + 4);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        zr[i][e] = a[e];
-                        zr[i][4 + e] = b[e];
-                    }
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; e++)
-                        if (w + e < p.W) zr[i][e] = src[e];
+                for (int e = 0; e < 4; e++) {
+                    zr[i][e] = a[e];
+                    zr[i][4 + e] = b[e];
                 }
             }
         }
@@ -2623,77 +2660,122 @@ __global__ __launch_bounds__(256) void conv_dw_reduce_few_kernel(float* __restri
 //     acc[(c, r, s)][o] += f16(x[c][h + r - 1][w + s - 1]) * f16(dy[o][h][w]).
 // A wave adds its lanes in a fixed tree and writes one partial vector per strip; small_dw_reduce_kernel
 // adds the strips (and, for shared weights, the images) in ascending order.
-template <int O_T, int C_T>
+//
+// As in the forward kernel every row of x and dy is requested three rows before it is used (a row asked for and used in the same
+// step left the wave waiting for memory once a row: 10 x 3 x 1024 x 1024, 168 MB, 49.5 -> 46.8 us), odd strips walk upwards so
+// that neighbours meet at the rows they share, and VEC says whether rows are whole, aligned 16-byte pieces (otherwise
+// load_ragged_quad: 10 x 3 x 500 x 655 21 us, 30 with four 4-byte loads per quad; such rows used to go to the gather kernel,
+// which multiplied mostly padding).
+template <int O_T, int C_T, bool VEC>
 __global__ __launch_bounds__(256) void conv3x3_dw_stream_kernel(float* __restrict__ partial, const float* __restrict__ x,
                                                                 const float* __restrict__ dy, int H, int W) {
-    constexpr int Q = C_T * 9 * O_T;
+    constexpr int Q = C_T * 9 * O_T, AHEAD = 3;
     int bx, by, b;
     xcd_contiguous_block(bx, by, b);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int w0 = (bx * 64 + lane) * 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int strip = by * 4 + wave, n_strips = gridDim.y * 4;
     const int h0 = strip * ST_ROWS;
     float acc[Q];
 #pragma unroll
     for (int q = 0; q < Q; q++) acc[q] = 0.f;
     if (h0 < H) {                                                // uniform over the wave
-        const bool col_ok = w0 < W;                              // W % 4 == 0: a lane's quad is all in or all out
-        const int wq = col_ok ? w0 : 0;
-        const bool has_l = col_ok && w0 > 0, has_r = col_ok && w0 + 4 < W;
-        const int wx = lane == 0 ? (has_l ? w0 - 1 : wq) : (lane == 63 && has_r ? w0 + 4 : wq);
+        const bool inside = (bx * 64 + lane) * 4 < W;
+        const int w0 = inside ? (bx * 64 + lane) * 4 : (W - 1) / 4 * 4;     // lanes past the row re-read its end and add nothing
+        bool col[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) col[e] = inside && (VEC || w0 + e < W);
+        const int w_at = w0 + 4 <= W ? w0 : W - 4;
+        const bool has_l = w0 > 0, has_r = w0 + 4 < W;
+        const int wx = lane == 0 ? (has_l ? w0 - 1 : w0) : (lane == 63 && has_r ? w0 + 4 : w0);
         const float* xb = x + (long)b * C_T * H * W;
         const float* gb = dy + (long)b * O_T * H * W;
         const long plane = (long)H * W;
         const int rows = (H - h0) < ST_ROWS ? (H - h0) : ST_ROWS;
         const int T = rows + 2;
-        float win[3][C_T][6];
-        for (int t0 = 0; t0 < T; t0 += 3) {
+        auto walk = [&](auto upwards) {
+            constexpr bool UP = decltype(upwards)::value;
+            const int row_first = UP ? h0 + rows : h0 - 1, row_step = UP ? -1 : 1;
+            auto out_row = [&](int t) { return UP ? h0 + rows + 1 - t : h0 + t - 2; };   // whose window step t >= 2 completes
+            auto row_in_image = [&](int t) { const int hi = row_first + t * row_step; return t < T && hi >= 0 && hi < H; };
+            float win[3][C_T][6];                                // rounded rows t-2, t-1, t (t % 3)
+            float raw[AHEAD][C_T][5], graw[AHEAD][O_T][4];       // rows in flight
+            auto quad = [&](const float* row, float (&v)[4]) {
+                if constexpr (VEC) {
+                    const floatx4 q = *reinterpret_cast<const floatx4*>(row + w0);
 #pragma unroll
-            for (int u = 0; u < 3; u++) {
-                const int t = t0 + u;
-                if (t >= T) break;
-                const int hi = h0 - 1 + t;
-                const bool in_img = hi >= 0 && hi < H;
-                const float* row = xb + (long)(in_img ? hi : 0) * W;
+                    for (int e = 0; e < 4; e++) v[e] = q[e];
+                } else {
+                    load_ragged_quad(row, w_at, w0 - w_at, v);
+                }
+            };
+            auto request = [&](int t, float (&xr)[C_T][5], float (&gr)[O_T][4]) {
+                const float* row = xb + (long)(row_in_image(t) ? row_first + t * row_step : 0) * W;
+                const long ho = t >= 2 && t < T ? out_row(t) : h0;
 #pragma unroll
                 for (int c = 0; c < C_T; c++) {
-                    const floatx4 qv = *reinterpret_cast<const floatx4*>(row + c * plane + wq);
-                    const float ex = row[c * plane + wx];
-                    float r5[5];
+                    float v[4];
+                    quad(row + c * plane, v);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) r5[e] = (in_img && col_ok) ? round_f16(qv[e]) : 0.f;
-                    r5[4] = in_img ? round_f16(ex) : 0.f;
-                    const float below = from_lane_below(r5[3]), above = from_lane_above(r5[0]);
-                    win[u][c][0] = has_l ? (lane == 0 ? r5[4] : below) : 0.f;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) win[u][c][1 + e] = r5[e];
-                    win[u][c][5] = has_r ? (lane == 63 ? r5[4] : above) : 0.f;
-                }
-                if (t < 2) continue;
-                const int ho = h0 + t - 2;                       // rows t-2, t-1, t are the window of output row ho
-                float g[O_T][4];
-#pragma unroll
-                for (int o = 0; o < O_T; o++) {
-                    const floatx4 gv = *reinterpret_cast<const floatx4*>(gb + (long)o * plane + (long)ho * W + wq);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) g[o][e] = col_ok ? round_f16(gv[e]) : 0.f;
+                    for (int e = 0; e < 4; e++) xr[c][e] = v[e];
+                    xr[c][4] = row[c * plane + wx];
                 }
 #pragma unroll
-                for (int c = 0; c < C_T; c++)
+                for (int o = 0; o < O_T; o++) quad(gb + (long)o * plane + ho * W, gr[o]);
+            };
 #pragma unroll
-                    for (int r = 0; r < 3; r++) {
-                        const int slot = (u + 1 + r) % 3;        // step t-2+r lives in slot (t-2+r) % 3, and t % 3 == u
+            for (int t = 0; t < AHEAD; t++) request(t, raw[t], graw[t]);
+            for (int t0 = 0; t0 < T; t0 += AHEAD) {
 #pragma unroll
-                        for (int s2 = 0; s2 < 3; s2++)
+                for (int u = 0; u < AHEAD; u++) {
+                    const int t = t0 + u;
+                    const bool in_img = row_in_image(t);         // (no way out of the middle of the loop: it would make every wait drain)
+                    float g[O_T][4];
 #pragma unroll
-                            for (int o = 0; o < O_T; o++)
+                    for (int c = 0; c < C_T; c++) {
+                        float r5[5];
 #pragma unroll
-                                for (int e = 0; e < 4; e++)
-                                    acc[((c * 3 + r) * 3 + s2) * O_T + o] =
-                                        __builtin_fmaf(win[slot][c][e + s2], g[o][e], acc[((c * 3 + r) * 3 + s2) * O_T + o]);
+                        for (int e = 0; e < 5; e++) {
+                            float v = raw[u][c][e];
+                            asm volatile("" : "+v"(v));          // the wait for the row belongs here, not at its request
+                            r5[e] = in_img && (e == 4 || col[e == 4 ? 0 : e]) ? round_f16(v) : 0.f;
+                        }
+                        const float below = from_lane_below(r5[3]), above = from_lane_above(r5[0]);
+                        win[u][c][0] = has_l ? (lane == 0 ? r5[4] : below) : 0.f;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) win[u][c][1 + e] = r5[e];
+                        win[u][c][5] = has_r ? (lane == 63 ? r5[4] : above) : 0.f;
                     }
+#pragma unroll
+                    for (int o = 0; o < O_T; o++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            g[o][e] = col[e] ? round_f16(graw[u][o][e]) : 0.f;
+                            asm volatile("" : "+v"(g[o][e]));    // rounded before the registers are asked for the next row
+                        }
+                    __builtin_amdgcn_sched_barrier(0);           // the old rows are consumed: their registers take the new ones
+                    request(t + AHEAD, raw[u], graw[u]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (t >= 2 && t < T) {
+#pragma unroll
+                        for (int c = 0; c < C_T; c++)
+#pragma unroll
+                            for (int r = 0; r < 3; r++) {
+                                const int slot = UP ? (u + 3 - r) % 3 : (u + 1 + r) % 3;     // the x row under filter row r
+#pragma unroll
+                                for (int s2 = 0; s2 < 3; s2++)
+#pragma unroll
+                                    for (int o = 0; o < O_T; o++)
+#pragma unroll
+                                        for (int e = 0; e < 4; e++)
+                                            acc[((c * 3 + r) * 3 + s2) * O_T + o] =
+                                                __builtin_fmaf(win[slot][c][e + s2], g[o][e], acc[((c * 3 + r) * 3 + s2) * O_T + o]);
+                            }
+                    }
+                }
             }
-        }
+        };
+        if (strip & 1) walk(std::true_type{});
+        else walk(std::false_type{});
     }
     float* dst = partial + (((long)b * n_strips + strip) * gridDim.x + bx) * Q;
 #pragma unroll
@@ -2944,8 +3026,8 @@ static ConvRoute conv_forward_route(const float* x, size_t N, size_t C, size_t H
 
 // w_mirror: w_ref is the parameter of the convolution whose DATA GRADIENT this call computes ([(c_f, tap)][o_f] with
 // c_f running over this call's O channels and o_f over its C), to be used with channels swapped and taps mirrored.
-// The implicit-GEMM routes read it that way while they build their fp16 weight image; the routes that take the
-// weights as they lie (column matrix, direct kernels) get a mirrored copy first.
+// The implicit-GEMM routes read it that way while they build their fp16 weight image, the direct kernels while they fetch
+// their few weights; the column-matrix route, which takes the weights as they lie, gets a mirrored copy first.
 static int conv2d_forward_impl(float* y, const float* x, const float* w_ref, const float* bias, size_t N, size_t C,
                                size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad,
                                size_t w_batch, int64_t bias_stride_pixel, int64_t bias_stride_channel,
@@ -3048,12 +3130,12 @@ static int conv2d_forward_impl(float* y, const float* x, const float* w_ref, con
     const bool fixed_geometry = route == CONV_ROUTE_FIXED, any_geometry = route == CONV_ROUTE_ANY;
     if (bias_stride_image != 0 && !fixed_geometry && !any_geometry)
         return set_error(NZHIP_E_UNSUPPORTED, "conv2d: a per-image bias needs an implicit-GEMM route");
+    if (route == CONV_ROUTE_DIRECT)
+        return conv_direct(y, x, w_ref, bias, N, C, H, W, O, w_batch, bias_stride_pixel, bias_stride_channel,
+                           activation, w_mirror, s);
     if (w_mirror && !fixed_geometry && !any_geometry)
         return conv2d_forward_mirrored_copy(y, x, w_ref, bias, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, bias_stride_pixel,
                                             bias_stride_channel, bias_stride_image, activation, stream);
-    if (route == CONV_ROUTE_DIRECT)
-        return conv_direct(y, x, w_ref, bias, N, C, H, W, O, w_batch, bias_stride_pixel, bias_stride_channel,
-                           activation, s);
     if (fixed_geometry || any_geometry) {
         // The reference's bias parameter is pixel-major ([1,1,H_out*W_out,O], src/Model.cu:252-256), while the kernels'
         // lanes are adjacent pixels: read as it lies, every bias load touches 64 lines 4 O bytes apart. One pass turns it
@@ -4060,7 +4142,7 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
     const bool prefer_gather = dw_env ? dw_env[0] == 'g' : (W <= 64 && C >= 128);
     const bool own3x3 = K_h == 3 && K_w == 3 && stride == 1 && pad == 1 &&
                         ((W % 8 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15) == 0 && !prefer_gather) ||
-                         (C <= 4 && O <= 2));
+                         (C <= 4 && O <= 2 && W >= 4));
     if (!own3x3) {
         // any other geometry: the gather kernel (up to 128 taps, stride up to 4, extents that fit its index arithmetic)
         const bool fits = K_h * K_w <= (size_t)DWG_ROWS && stride <= 4 && pad < 0x10000 && H < 0x3fffffff && W < 0x3fffffff &&
@@ -4076,10 +4158,10 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
     }
     if (H == 0 || W == 0 || H > 0x3fffffff || W > 0x3fffffff || C > 0x3fffffff || O > 0x3fffffff || N > 65535)
         return set_error(NZHIP_E_UNSUPPORTED, "nzhip_conv2d_backward_weights: extents beyond the fused kernels (use the column-matrix chain)");
-    const bool vec = W % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(dy) & 15) == 0;
     if (N == 0 || C == 0 || O == 0) return NZHIP_OK;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (C <= 4 && O <= 2 && W % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(dy) & 15) == 0) {
+    if (C <= 4 && O <= 2) {
+        const bool pieces = W % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15) == 0;
         // a handful of channels: stream x and dy once, C*9*O running sums per lane
         dim3 grid((unsigned)((W + 255) / 256), (unsigned)((H + 4 * ST_ROWS - 1) / (4 * ST_ROWS)), (unsigned)N);
         const size_t Q = C * 9 * O, per_image = (size_t)grid.x * grid.y * 4;
@@ -4087,7 +4169,8 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
         float* partial = nullptr;
         if (int rc = workspace_alloc(reinterpret_cast<void**>(&partial), per_image * N * Q * sizeof(float), s)) return rc;
 #define NZHIP_DWS(OT, CT)                                                                                            \
-    hipLaunchKernelGGL((conv3x3_dw_stream_kernel<OT, CT>), grid, dim3(256), 0, s, partial, x, dy, (int)H, (int)W)
+    hipLaunchKernelGGL((pieces ? conv3x3_dw_stream_kernel<OT, CT, true> : conv3x3_dw_stream_kernel<OT, CT, false>), grid, dim3(256), 0, s, \
+                       partial, x, dy, (int)H, (int)W)
         switch ((int)(O * 10 + C)) {
             case 11: NZHIP_DWS(1, 1); break;
             case 12: NZHIP_DWS(1, 2); break;
@@ -4132,11 +4215,10 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
     a.C = (int)C; a.H = (int)H; a.W = (int)W; a.O = (int)O;
     a.bands = bands; a.band_rows = band_rows; a.n_images = (int)N;
     const int lds_bytes = DW_XS_BYTES + DW_ZS_BYTES;
-    auto kfn = vec ? conv_dw_kernel<true> : conv_dw_kernel<false>;
-    int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kfn), lds_bytes, "hipFuncSetAttribute(conv_dw)");
+    int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(conv_dw_kernel), lds_bytes, "hipFuncSetAttribute(conv_dw)");
     if (rc == NZHIP_OK) {
         dim3 grid((unsigned)(N * bands), (unsigned)chunks, (unsigned)otiles);
-        hipLaunchKernelGGL(kfn, grid, dim3(256), lds_bytes, s, a);
+        hipLaunchKernelGGL(conv_dw_kernel, grid, dim3(256), lds_bytes, s, a);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) rc = set_hip_error(e, "conv_dw kernel launch");
     }

@@ -380,3 +380,36 @@ def test_config4b_conv_memory_bound_single_channel_out(nz, oracle):
     got = host(nz.conv2d_forward(dev(x), dev(oracle.weights_oihw_to_ref(w)), dev(bias), 3, 3, 1, 1, bias_strides=(0, 1), relu=True))
     truth = oracle.conv2d_direct_f64(x, w, bias, 1, 1, relu=True)
     check_tolerance(oracle, got, truth, "CB")
+
+
+@pytest.mark.parametrize("O,C,bias", [(1, 3, "pixel"), (2, 4, "channel"), (1, 1, "none"), (2, 1, "pixel")])
+@pytest.mark.parametrize("H,W", [(8, 5), (17, 254), (33, 255), (16, 257), (66, 259), (19, 512), (9, 1)])
+def test_thin_layers_on_rows_of_any_width_forward_and_gradients(nz, H, W, O, C, bias):
+    """The row-streaming kernels (up to four channels in, two out) on rows that are and are not whole 16-byte pieces, quads cut by
+    the end of the row, one and several 256-column blocks, whole and partial 16-row strips walked both ways, mirrored weights:
+    integers, so exact whatever the order of the sums."""
+    import torch
+    import torch.nn.functional as F
+    N = 3
+    g = torch.Generator().manual_seed(H * 1000 + W + 10 * O + C)
+    draw = lambda *s: torch.randint(-4, 5, s, generator=g).double()
+    x, dy = draw(N, C, H, W), draw(N, O, H, W)
+    w = draw(N, 1, C * 9, O)
+    b = {"pixel": draw(1, 1, H * W, O), "channel": draw(O), "none": None}[bias]
+    strides = (O, 1) if bias == "pixel" else (0, 1)
+    up = lambda t: None if t is None else t.float().cuda()
+    y = nz.conv2d_forward(up(x), up(w), up(b), 3, 3, 1, 1, bias_strides=strides, relu=True)
+    dx = nz.conv2d_backward_data(torch.full((N, C, H, W), float("nan"), device="cuda"), up(dy), up(w), 3, 3, 1, 1, accumulate=False)
+    dw = nz.conv2d_backward_weights(torch.zeros(N, 1, C * 9, O, device="cuda"), up(x), up(dy), 3, 3, 1, 1)
+    for n in range(N):
+        wt = w[n, 0].view(C, 3, 3, O).permute(3, 0, 1, 2).contiguous().requires_grad_(True)
+        xt = x[n:n + 1].clone().requires_grad_(True)
+        z = F.conv2d(xt, wt, None, 1, 1)
+        gx, gw = torch.autograd.grad(z, (xt, wt), dy[n:n + 1])
+        if bias == "pixel":
+            z = z + b.view(H, W, O).permute(2, 0, 1)[None]
+        elif bias == "channel":
+            z = z + b.view(1, O, 1, 1)
+        assert torch.equal(y[n].double().cpu(), z.detach().relu()[0])
+        assert torch.equal(dx[n].double().cpu(), gx[0])
+        assert torch.equal(dw[n, 0].view(C, 3, 3, O).permute(3, 0, 1, 2).double().cpu(), gw)
