@@ -150,9 +150,14 @@ def shape4(s) -> C.Array:
 # Torch-facing helpers. torch is used for device memory and streams only.
 # --------------------------------------------------------------------------------------------
 def _stream_handle(stream=None) -> int:
+    """The hipStream_t a call goes to. For the current stream the handle is asked for directly: building the Stream object around
+    it costs 2.7 us, a third of a small call (relu_backward of 256 elements: 8.4 -> 6.0 us on the host)."""
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
+    if stream is not None:
+        return int(stream.cuda_stream)
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dev(t):
