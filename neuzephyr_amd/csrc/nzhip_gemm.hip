@@ -8,11 +8,13 @@
 //   * v_mfma_f32_32x32x16_f16 with fp32 accumulators;
 //   * two LDS stages (one barrier per k tile), rows padded by 16 B so that the
 //     128-bit fragment reads and the staging writes hit distinct banks;
-//   * edges are predicated (zero fill on load, masked store) -- no padded copies;
+//   * no padded copies: at the edges accesses are moved into the operands, the last k tile's missing
+//     elements are zeroed on the way into LDS, stores are masked;
 //   * batch (n,c), broadcast strides, bias and ReLU are handled in-kernel.
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>
+#include <type_traits>
 
 #include "nzhip_internal.h"
 
@@ -40,7 +42,6 @@ struct GemmKernelArgs {
     int tiles_m, tiles_n;
     int group_m;                      // tile rows per rasterisation group
     int k_total;                      // > 0: member j of the inner batch contracts min(K, k_total - j*K) (split-k chunks)
-    int c_vec;                        // 16-byte stores to C are legal (alignment, ldc and N multiples of 4)
 };
 
 // Physical LDS row of logical tile row r. A wave owns TR = 32*FR logical rows; its MFMA
@@ -55,10 +56,42 @@ __device__ __forceinline__ int phys_row(int r) {
 
 // ---- operand staging: global fp32 -> registers -> fp16 in LDS ----------------------------
 // KCONTIG: the operand is stored with k contiguous (A row-major MxK, or B given as NxK).
-// FULL: the tile lies wholly inside the operand and K is a multiple of BK, so no predicate is
-// evaluated. Otherwise loads are predicated WITHOUT branches: an out-of-range lane reads the
-// operand's first element (always mapped) and the value is replaced by zero afterwards.
-template <int BR, int BK, int NT, int TR, int FR, int ROWB, bool VEC, bool FULL>
+// EDGE INTERIOR: the tile lies wholly inside the operand and K is a multiple of BK. Otherwise nothing is predicated where the operand
+// is LOADED -- a value that depends on a load where it is issued makes the wave wait for it there -- but every access is moved
+// into the operand: a row past the end is the last row (its products land in rows or columns of C that are not stored), a
+// 16-byte piece cut by the end of the contiguous extent starts earlier. Where the registers are CONVERTED, one uniform test
+// per k tile finds the last one, whose missing k are zeroed, and one per tile the pieces that have to be turned back.
+// 16-byte accesses need no more than the 4-byte alignment of their elements: rows of 777 or 513 floats stream at the rate of
+// rows of 776 or 512 (1000 x 777 x 513: @A us; element by element it was 33, through zero-padded copies of the operands 21).
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
+
+// element e of a piece that was moved back by `back` elements; what lies beyond the extent comes out as some element of it
+__device__ __forceinline__ floatx4 turn_back(const floatx4 q, int back) {
+    const float a = back & 1 ? q[1] : q[0], b = back & 1 ? q[2] : q[1], c = back & 1 ? q[3] : q[2];
+    return floatx4{back & 2 ? c : a, back & 2 ? q[3] : b, c, q[3]};
+}
+// How the accesses of an instance are kept inside the operands. INTERIOR: they are. PIECES: rows and 16-byte pieces are moved.
+// ELEMENTS: some contiguous extent is below 4, so pieces are made of single elements (an instance of its own: the choice made
+// in the kernel, at every load, cost the loads their place in the order the waits rely on, 1040 x 1280 x 1968 35 -> 55 us).
+enum Edge { INTERIOR, PIECES, ELEMENTS };
+
+// the piece at offset `at` of a row of `extent` contiguous elements, moved into the row
+template <int EDGE>
+__device__ __forceinline__ floatx4 load_piece(const float* row, int at, int extent) {
+    if constexpr (EDGE == PIECES) {
+        return *reinterpret_cast<const floatx4u*>(row + (at + 4 <= extent ? at : extent - 4));
+    } else {
+        floatx4 v;
+#pragma unroll
+        for (int e = 0; e < 4; e++) v[e] = row[at + e < extent ? at + e : extent - 1];
+        return v;
+    }
+}
+template <int EDGE>
+__device__ __forceinline__ int moved_back(int at, int extent) { return EDGE == PIECES && at + 4 > extent ? at + 4 - extent : 0; }
+
+template <int BR, int BK, int NT, int TR, int FR, int ROWB, int EDGE>
 struct StageKContig {
     static constexpr int F4_PER_ROW = BK / 4;
     static constexpr int ROWS_PER_PASS = NT / F4_PER_ROW;
@@ -73,29 +106,23 @@ struct StageKContig {
 #pragma unroll
         for (int p = 0; p < PASSES; p++) {
             const int gr = row_base + r0 + p * ROWS_PER_PASS;
-            const float* src = X + (long)gr * ldx + gk;
-            if constexpr (FULL) {
-                regs[p] = *reinterpret_cast<const floatx4*>(src);
-            } else if constexpr (VEC) {
-                const bool ok = gr < R && gk < K;
-                const floatx4 v = *reinterpret_cast<const floatx4*>(ok ? src : X);
-                const floatx4 z = {0.f, 0.f, 0.f, 0.f};
-                regs[p] = ok ? v : z;
-            } else {
-                floatx4 v;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const bool ok = gr < R && gk + e < K;
-                    const float x = *(ok ? src + e : X);
-                    v[e] = ok ? x : 0.f;
-                }
-                regs[p] = v;
-            }
+            if constexpr (EDGE == INTERIOR) regs[p] = *reinterpret_cast<const floatx4*>(X + (long)gr * ldx + gk);
+            else regs[p] = load_piece<EDGE>(X + (long)(gr < R ? gr : R - 1) * ldx, gk, K);
         }
     }
 
-    __device__ __forceinline__ void store(char* lds, int tid) const {
+    // k_base, K as in load(): the last k tile's missing elements become zero
+    __device__ __forceinline__ void store(char* lds, int tid, int, int, int k_base, int K) {
         const int k4 = tid % F4_PER_ROW, r0 = tid / F4_PER_ROW;
+        if (EDGE != INTERIOR && k_base + BK > K) {
+            const int gk = k_base + k4 * 4, back = moved_back<EDGE>(gk, K);
+#pragma unroll
+            for (int p = 0; p < PASSES; p++) {
+                const floatx4 v = turn_back(regs[p], back);
+#pragma unroll
+                for (int e = 0; e < 4; e++) regs[p][e] = gk + e < K ? v[e] : 0.f;
+            }
+        }
 #pragma unroll
         for (int p = 0; p < PASSES; p++) {
             const int r = r0 + p * ROWS_PER_PASS;
@@ -112,7 +139,7 @@ struct StageKContig {
 // RCONTIG: the operand is stored with the tile dimension contiguous (B row-major KxN, or
 // A given as KxM). Each thread takes 4 neighbouring tile rows over KPT consecutive k and
 // transposes them in registers, so LDS still holds k-contiguous rows.
-template <int BR, int BK, int NT, int TR, int FR, int ROWB, bool VEC, bool FULL>
+template <int BR, int BK, int NT, int TR, int FR, int ROWB, int EDGE>
 struct StageRContig {
     static constexpr int F4_PER_KROW = BR / 4;
     static constexpr int KGROUPS = NT / F4_PER_KROW;
@@ -128,29 +155,24 @@ struct StageRContig {
 #pragma unroll
         for (int q = 0; q < KPT; q++) {
             const int gk = k_base + kg * KPT + q;
-            const float* src = X + (long)gk * ldx + gr;
-            if constexpr (FULL) {
-                regs[q] = *reinterpret_cast<const floatx4*>(src);
-            } else if constexpr (VEC) {
-                const bool ok = gk < K && gr < R;
-                const floatx4 v = *reinterpret_cast<const floatx4*>(ok ? src : X);
-                const floatx4 z = {0.f, 0.f, 0.f, 0.f};
-                regs[q] = ok ? v : z;
-            } else {
-                floatx4 v;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const bool ok = gk < K && gr + e < R;
-                    const float x = *(ok ? src + e : X);
-                    v[e] = ok ? x : 0.f;
-                }
-                regs[q] = v;
-            }
+            if constexpr (EDGE == INTERIOR) regs[q] = *reinterpret_cast<const floatx4*>(X + (long)gk * ldx + gr);
+            else regs[q] = load_piece<EDGE>(X + (long)(gk < K ? gk : K - 1) * ldx, gr, R);
         }
     }
 
-    __device__ __forceinline__ void store(char* lds, int tid) const {
+    __device__ __forceinline__ void store(char* lds, int tid, int row_base, int R, int k_base, int K) {
         const int r4 = tid % F4_PER_KROW, kg = tid / F4_PER_KROW;
+        if (EDGE != INTERIOR && row_base + BR > R) {
+            const int back = moved_back<EDGE>(row_base + r4 * 4, R);
+#pragma unroll
+            for (int q = 0; q < KPT; q++) regs[q] = turn_back(regs[q], back);
+        }
+        if (EDGE != INTERIOR && k_base + BK > K) {
+#pragma unroll
+            for (int q = 0; q < KPT; q++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) regs[q][e] = k_base + kg * KPT + q < K ? regs[q][e] : 0.f;
+        }
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             char* dst = lds + phys_row<TR, FR>(r4 * 4 + e) * ROWB + kg * KPT * 2;
@@ -174,21 +196,20 @@ struct StageRContig {
     }
 };
 
-template <bool RCONTIG, int BR, int BK, int NT, int TR, int FR, int ROWB, bool VEC, bool FULL>
+template <bool RCONTIG, int BR, int BK, int NT, int TR, int FR, int ROWB, int EDGE>
 struct StageSelect {
-    using type = StageKContig<BR, BK, NT, TR, FR, ROWB, VEC, FULL>;
+    using type = StageKContig<BR, BK, NT, TR, FR, ROWB, EDGE>;
 };
-template <int BR, int BK, int NT, int TR, int FR, int ROWB, bool VEC, bool FULL>
-struct StageSelect<true, BR, BK, NT, TR, FR, ROWB, VEC, FULL> {
-    using type = StageRContig<BR, BK, NT, TR, FR, ROWB, VEC, FULL>;
+template <int BR, int BK, int NT, int TR, int FR, int ROWB, int EDGE>
+struct StageSelect<true, BR, BK, NT, TR, FR, ROWB, EDGE> {
+    using type = StageRContig<BR, BK, NT, TR, FR, ROWB, EDGE>;
 };
 
 // ---- the kernel ----------------------------------------------------------------------------
 // BM x BN x BK workgroup tile, WM x WN waves, each wave a (BM/WM) x (BN/WN) tile of 32x32 MFMA
-// blocks.  A_TRANS: A given as KxM.  B_TRANS: B given as NxK.  VEC: 16-byte global accesses
-// are legal for both operands (alignment and extents checked on the host).  FULL: M, N and K
-// are multiples of BM, BN and BK (implies VEC), so loads and stores carry no predicates.
-template <int BM, int BN, int BK, int WM, int WN, bool A_TRANS, bool B_TRANS, bool VEC, bool FULL>
+// blocks.  A_TRANS: A given as KxM.  B_TRANS: B given as NxK.  EDGE: INTERIOR when M, N and K are
+// multiples of BM, BN and BK and every row is 16-byte aligned, so no access is moved or tested.
+template <int BM, int BN, int BK, int WM, int WN, bool A_TRANS, bool B_TRANS, int EDGE>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKernelArgs p) {
     constexpr int NT = WM * WN * 64;
     constexpr int TM = BM / WM, TN = BN / WN;
@@ -234,8 +255,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
     const float* __restrict__ B = p.B + bi * p.b_sn + bj * p.b_sc;
     float* __restrict__ C = p.C + bi * p.c_sn + bj * p.c_sc;
 
-    using StageA = typename StageSelect<A_TRANS, BM, BK, NT, TM, FM, ROWB, VEC, FULL>::type;
-    using StageB = typename StageSelect<!B_TRANS, BN, BK, NT, TN, FN, ROWB, VEC, FULL>::type;
+    using StageA = typename StageSelect<A_TRANS, BM, BK, NT, TM, FM, ROWB, EDGE>::type;
+    using StageB = typename StageSelect<!B_TRANS, BN, BK, NT, TN, FN, ROWB, EDGE>::type;
     // With 128 or fewer accumulator registers per lane (128x128 tiles, or 256x256 tiles on eight waves)
     // there is room for a second staging set per operand: the tile two k steps ahead is requested
     // while the current one is multiplied, so a request has two MFMA phases to land before it is
@@ -266,6 +287,12 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
         ra.load(A, p.lda, m0, p.M, kc * BK, K, tid);
         rb.load(B, p.ldb, n0, p.N, kc * BK, K, tid);
     };
+    // convert tile kt (or, past the end, the repeat of the last one) into an LDS stage
+    auto convert = [&](StageA& ra, StageB& rb, int kt, char* st) {
+        const int kb = (kt < nk ? kt : nk - 1) * BK;
+        ra.store(st, tid, m0, p.M, kb, K);
+        rb.store(st + A_BYTES, tid, n0, p.N, kb, K);
+    };
     auto multiply = [&](const char* cur) {
         const char* la = cur + ((wm * FM) * 32 + li) * ROWB + lh * 16;
         const char* lb = cur + A_BYTES + ((wn * FN) * 32 + li) * ROWB + lh * 16;
@@ -290,14 +317,12 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
         auto step = [&](int kt, char* cur, char* nxt, StageA& ra, StageB& rb, StageA& qa, StageB& qb) {
             request(ra, rb, kt + 2);
             if (kt < nk) multiply(cur);
-            qa.store(nxt, tid);                               // tile kt + 1 (a repeat of the last tile past the end)
-            qb.store(nxt + A_BYTES, tid);
+            convert(qa, qb, kt + 1, nxt);
             lds_barrier();
         };
         request(sa0, sb0, 0);
         request(sa1, sb1, 1);
-        sa0.store(lds, tid);
-        sb0.store(lds + A_BYTES, tid);
+        convert(sa0, sb0, 0, lds);
         lds_barrier();
         char* st0 = lds;
         char* st1 = lds + STAGE_BYTES;
@@ -311,8 +336,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
     } else {
         sa0.load(A, p.lda, m0, p.M, 0, K, tid);
         sb0.load(B, p.ldb, n0, p.N, 0, K, tid);
-        sa0.store(lds, tid);
-        sb0.store(lds + A_BYTES, tid);
+        convert(sa0, sb0, 0, lds);
         __syncthreads();
         for (int kt = 0; kt < nk; kt++) {
             char* cur = lds + (kt & 1) * STAGE_BYTES;
@@ -323,10 +347,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
                 sb0.load(B, p.ldb, n0, p.N, (kt + 1) * BK, K, tid);
             }
             multiply(cur);
-            if (more) {
-                sa0.store(nxt, tid);
-                sb0.store(nxt + A_BYTES, tid);
-            }
+            if (more) convert(sa0, sb0, kt + 1, nxt);
             __syncthreads();
         }
     }
@@ -336,7 +357,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
     // the bias does not vary along rows) so the stores never wait on one load each.
     const float* bias = p.bias ? p.bias + bi * p.bias_sn + bj * p.bias_sc : nullptr;
     const int gn = n0 + wn * TN + li * FN;                // first of this lane's FN columns
-    const bool vec_store = FULL || (VEC && p.c_vec && (FN == 2 || FN == 4) && (gn + FN <= p.N));
+    const bool vec_store = EDGE == INTERIOR || gn + FN <= p.N;               // (4-byte alignment is enough)
     float bcol[FN];
     const bool bias_rowless = bias && p.bias_sm == 0;
 #pragma unroll
@@ -344,10 +365,9 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
     // A bias that varies along rows (a bias matrix, C itself when a gradient is accumulated in place) is requested half
     // a block (8 rows) ahead of the stores that need it: a load issued after stores is not counted as returned before
     // those stores are acknowledged, so requesting a block after storing the one before made every block wait for
-    // its predecessor. 16- or 8-byte loads when the bias rows are contiguous and aligned like the rows of C.
+    // its predecessor. 16- or 8-byte loads when the bias rows are contiguous.
     const bool bias_rows = bias && !bias_rowless;
-    const bool bias_vec = bias_rows && (FN == 2 || FN == 4) && p.bias_sk == 1 && (p.bias_sm & (FN - 1)) == 0 &&
-                          (reinterpret_cast<uintptr_t>(bias) & (FN * 4 - 1)) == 0 && gn + FN <= p.N;
+    const bool bias_vec = bias_rows && (FN == 2 || FN == 4) && p.bias_sk == 1 && gn + FN <= p.N;
     float bvs[2][8][FN];
     auto bias_request = [&](float (&bv)[8][FN], const int i, const int h) {
 #pragma unroll
@@ -357,11 +377,11 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
             const float* bp = bias + (long)(gm < p.M ? gm : 0) * p.bias_sm;
             if (bias_vec) {
                 if constexpr (FN == 4) {
-                    const floatx4 v = *reinterpret_cast<const floatx4*>(bp + gn);
+                    const floatx4 v = *reinterpret_cast<const floatx4u*>(bp + gn);
 #pragma unroll
                     for (int e = 0; e < 4; e++) bv[r8][e] = v[e];
                 } else if constexpr (FN == 2) {
-                    const floatx2 v = *reinterpret_cast<const floatx2*>(bp + gn);
+                    const floatx2 v = *reinterpret_cast<const floatx2u*>(bp + gn);
                     bv[r8][0] = v[0];
                     bv[r8][1] = v[1];
                 }
@@ -380,7 +400,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
                 bias_request(bvs[(i * 2 + (r >> 3) + 1) & 1], (i * 2 + (r >> 3) + 1) >> 1, (i * 2 + (r >> 3) + 1) & 1);
             const int im = (r >> 2) * 8 + lh * 4 + (r & 3);
             const int gm = m0 + wm * TM + im * FM + i;
-            if (!FULL && gm >= p.M) continue;
+            if (EDGE != INTERIOR && gm >= p.M) continue;
             float v[FN];
 #pragma unroll
             for (int j = 0; j < FN; j++) {
@@ -392,10 +412,10 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
             if (vec_store) {
                 if constexpr (FN == 4) {
                     floatx4 o = {v[0], v[1], v[2], v[3]};
-                    *reinterpret_cast<floatx4*>(dst) = o;
+                    *reinterpret_cast<floatx4u*>(dst) = o;
                 } else if constexpr (FN == 2) {
                     floatx2 o = {v[0], v[1]};
-                    *reinterpret_cast<floatx2*>(dst) = o;
+                    *reinterpret_cast<floatx2u*>(dst) = o;
                 } else {
                     dst[0] = v[0];
                 }
@@ -410,88 +430,66 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
 
 // ---- host-side selection -------------------------------------------------------------------
 template <int BM, int BN, int BK, int WM, int WN>
-static int launch_cfg(const GemmKernelArgs& a, bool a_trans, bool b_trans, bool vec, int batch, hipStream_t s) {
-    const bool full = vec && a.c_vec && a.M % BM == 0 && a.N % BN == 0 && a.K % BK == 0 && (a.k_total <= 0 || a.k_total % a.K == 0);
+static int launch_cfg(const GemmKernelArgs& a, bool a_trans, bool b_trans, bool aligned, int batch, hipStream_t s) {
+    const bool full = aligned && a.M % BM == 0 && a.N % BN == 0 && a.K % BK == 0 && (a.k_total <= 0 || a.k_total % a.K == 0);
     constexpr int ROWB = BK * 2 + 16;
     constexpr size_t lds_bytes = 2 * (size_t)(BM + BN) * ROWB;
     dim3 grid((unsigned)((int64_t)a.tiles_m * a.tiles_n * batch), 1, 1), block(WM * WN * 64, 1, 1);
-#define NZHIP_LAUNCH(AT, BT, V, F)                                                                       \
-    do {                                                                                                 \
-        auto kfn = gemm_f16mfma_kernel<BM, BN, BK, WM, WN, AT, BT, V, F>;                                \
-        if (int lrc = ensure_dynamic_lds(reinterpret_cast<const void*>(kfn), (int)lds_bytes,             \
-                                         "hipFuncSetAttribute(gemm)"))                                   \
-            return lrc;                                                                                  \
-        hipLaunchKernelGGL(kfn, grid, block, lds_bytes, s, a);                                           \
-    } while (0)
-    if (full) {
-        if (!a_trans && !b_trans) NZHIP_LAUNCH(false, false, true, true);
-        else if (!a_trans && b_trans) NZHIP_LAUNCH(false, true, true, true);
-        else if (a_trans && !b_trans) NZHIP_LAUNCH(true, false, true, true);
-        else NZHIP_LAUNCH(true, true, true, true);
-    } else if (vec) {
-        if (!a_trans && !b_trans) NZHIP_LAUNCH(false, false, true, false);
-        else if (!a_trans && b_trans) NZHIP_LAUNCH(false, true, true, false);
-        else if (a_trans && !b_trans) NZHIP_LAUNCH(true, false, true, false);
-        else NZHIP_LAUNCH(true, true, true, false);
-    } else {
-        if (!a_trans && !b_trans) NZHIP_LAUNCH(false, false, false, false);
-        else if (!a_trans && b_trans) NZHIP_LAUNCH(false, true, false, false);
-        else if (a_trans && !b_trans) NZHIP_LAUNCH(true, false, false, false);
-        else NZHIP_LAUNCH(true, true, false, false);
-    }
-#undef NZHIP_LAUNCH
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return set_hip_error(e, "gemm kernel launch");
-    return NZHIP_OK;
+    auto launch = [&](auto kfn) {
+        if (int lrc = ensure_dynamic_lds(reinterpret_cast<const void*>(kfn), (int)lds_bytes, "hipFuncSetAttribute(gemm)")) return lrc;
+        hipLaunchKernelGGL(kfn, grid, block, lds_bytes, s, a);
+        hipError_t e = hipGetLastError();
+        return e == hipSuccess ? NZHIP_OK : set_hip_error(e, "gemm kernel launch");
+    };
+    auto pick = [&](auto edge) {
+        constexpr int E = decltype(edge)::value;
+        if (!a_trans && !b_trans) return launch(gemm_f16mfma_kernel<BM, BN, BK, WM, WN, false, false, E>);
+        if (!a_trans && b_trans) return launch(gemm_f16mfma_kernel<BM, BN, BK, WM, WN, false, true, E>);
+        if (a_trans && !b_trans) return launch(gemm_f16mfma_kernel<BM, BN, BK, WM, WN, true, false, E>);
+        return launch(gemm_f16mfma_kernel<BM, BN, BK, WM, WN, true, true, E>);
+    };
+    if (full) return pick(std::integral_constant<int, INTERIOR>{});
+    // the shortest contiguous extent, the last chunk of a split contraction included
+    const int last_k = a.k_total > 0 ? a.k_total - (a.batch_c - 1) * a.K : a.K, k_min = last_k < a.K ? last_k : a.K;
+    const bool pieces = (a_trans ? a.M : k_min) >= 4 && (b_trans ? k_min : a.N) >= 4;
+    return pieces ? pick(std::integral_constant<int, PIECES>{}) : pick(std::integral_constant<int, ELEMENTS>{});
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// 16-byte accesses are legal when every row start is 16-byte aligned and the contiguous extent is
-// a multiple of 4, for every batch member: the operands decide which kernel instance loads them,
-// C only whether the epilogue may use vector stores.
-bool gemm_operand_vec_legal(const float* X, int64_t ld, int64_t contig, int64_t stride_n, int64_t stride_c) {
-    auto ok4 = [](int64_t v) { return (v & 3) == 0; };
-    return aligned16(X) && ok4(ld) && ok4(contig) && ok4(stride_n) && ok4(stride_c);
-}
-
-// padded: bit 0 / bit 1 = the rows of A / B are readable up to the next multiple of 4 elements and hold
-// zeros there (the library's own padded copies), so their contiguous extent need not be a multiple of 4
-bool gemm_operands_vec_legal(const nzhip_gemm_desc& d, int padded) {
+// Every row of A, B and C starts on 16 bytes and is a multiple of 4 elements long, for every batch member.
+bool gemm_vec_legal(const nzhip_gemm_desc& d) {
+    auto rows = [](const float* X, int64_t ld, int64_t contiguous, int64_t stride_n, int64_t stride_c) {
+        return aligned16(X) && ((ld | contiguous | stride_n | stride_c) & 3) == 0;
+    };
     const bool a_trans = d.a_layout == NZHIP_LAYOUT_TRANS, b_trans = d.b_layout == NZHIP_LAYOUT_TRANS;
-    return gemm_operand_vec_legal(d.A, d.lda, (padded & 1) ? 0 : (a_trans ? d.M : d.K), d.a_stride_n, d.a_stride_c) &&
-           gemm_operand_vec_legal(d.B, d.ldb, (padded & 2) ? 0 : (b_trans ? d.K : d.N), d.b_stride_n, d.b_stride_c);
+    return rows(d.A, d.lda, a_trans ? d.M : d.K, d.a_stride_n, d.a_stride_c) &&
+           rows(d.B, d.ldb, b_trans ? d.K : d.N, d.b_stride_n, d.b_stride_c) && rows(d.C, d.ldc, d.N, d.c_stride_n, d.c_stride_c);
 }
-
-bool gemm_c_vec_legal(const nzhip_gemm_desc& d) {
-    return gemm_operand_vec_legal(d.C, d.ldc, d.N, d.c_stride_n, d.c_stride_c);
-}
-
-bool gemm_vec_legal(const nzhip_gemm_desc& d) { return gemm_operands_vec_legal(d, 0) && gemm_c_vec_legal(d); }
 
 // ---- tile and split choice for products that do not fill the device -------------------------------
 // The fused kernel's k loop is bound by the rate at which one CU takes fp32 tiles in through its L1
-// (about 50 GB/s per CU with 16-byte loads, 36 GB/s when they carry predicates, 9 GB/s element by element), so the time of a launch is
+// (about 50 GB/s per CU, 45 in the instance that keeps its accesses inside ragged operands), so the time of a launch is
 // the bytes the busiest CU streams: rounds of workgroups x (tile rows + tile columns, as far as the
 // operands reach) x chunk length x 4 bytes. 64 x 64 tiles stream twice the bytes of 128 x 128 tiles in total but put four times
 // as many CUs to work (1024^3: 23.6 us -> 14.2 us); a split contraction adds a pass over the partial sums.
 struct FusedCostInput {
     int64_t M, N, K, members;       // members: batch_n * batch_c of the product as given
     double cus;
-    bool vec, c_vec;
+    bool aligned;
 };
 
 static double fused_cost_us(const FusedCostInput& q, int tile, int64_t parts, int64_t Kc) {
     const int64_t tiles = ((q.M + tile - 1) / tile) * ((q.N + tile - 1) / tile) * q.members * parts;
     const double rounds = (double)((tiles + (int64_t)q.cus - 1) / (int64_t)q.cus);
-    const bool full = q.vec && q.c_vec && q.M % tile == 0 && q.N % tile == 0 && Kc % 32 == 0 && q.K % 32 == 0;   // unpredicated instance
+    const bool full = q.aligned && q.M % tile == 0 && q.N % tile == 0 && Kc % 32 == 0 && q.K % 32 == 0;   // unpredicated instance
     // rows past the operand's extent are predicated off, not loaded: a narrow operand costs what it has
     const double rows = (double)(q.M < tile ? q.M : tile) + (double)(q.N < tile ? q.N : tile);
     // two or more workgroups on a CU overlap their waits: the CU takes in up to 1.3 x what one workgroup draws
     // (16 x 8192 x 8192: 50 us in eight chunks, two workgroups per CU, against 57 us in four)
     const double per_cu = (double)tiles / q.cus;
     const double overlap = per_cu >= 2.0 ? 1.3 : per_cu > 1.0 ? 1.0 + 0.3 * (per_cu - 1.0) : 1.0;
-    const double stream = rounds * rows * (double)Kc * 4.0 / ((full ? 50e3 : q.vec ? 36e3 : 9e3) * overlap);   // bytes / (bytes per us)
+    const double stream = rounds * rows * (double)Kc * 4.0 / ((full ? 50e3 : 45e3) * overlap);   // bytes / (bytes per us)
     const double out = (double)q.M * q.N * q.members * 4.0;
     const double reduce = parts > 1 ? 6.0 + (double)(parts + 1) * out / 3e6 : 0.0;
     // what a workgroup spends outside its k loop (first requests, predicated epilogue): 17 x 33 x 15 takes 10 us with a
@@ -500,12 +498,12 @@ static double fused_cost_us(const FusedCostInput& q, int tile, int64_t parts, in
     return 3.0 + ends + stream + reduce;
 }
 
-static FusedCostInput fused_cost_input(const nzhip_gemm_desc& d, int padded) {
-    return {d.M, d.N, d.K, d.batch_n * d.batch_c, (double)device_cu_count(), gemm_operands_vec_legal(d, padded), gemm_c_vec_legal(d)};
+static FusedCostInput fused_cost_input(const nzhip_gemm_desc& d) {
+    return {d.M, d.N, d.K, d.batch_n * d.batch_c, (double)device_cu_count(), gemm_vec_legal(d)};
 }
 
-GemmPlan gemm_fused_plan(const nzhip_gemm_desc& d, int padded) {
-    const FusedCostInput q = fused_cost_input(d, padded);
+GemmPlan gemm_fused_plan(const nzhip_gemm_desc& d) {
+    const FusedCostInput q = fused_cost_input(d);
     GemmPlan best = {128, 1, d.K, 0.0};
     double best_cost = fused_cost_us(q, 128, 1, d.K);
     auto consider = [&](int tile, int64_t parts, int64_t Kc) {
@@ -516,7 +514,7 @@ GemmPlan gemm_fused_plan(const nzhip_gemm_desc& d, int padded) {
     // a batch over n alone (batch_c == 1) can be split as well: the chunks take the c dimension of the launch
     if (d.batch_c == 1 && d.batch_n <= 65535 && d.K >= 512) {
         const bool narrow = d.M <= 64 || d.N <= 64;                // padded tiles: the k loop is shorter per byte
-        const int64_t min_chunk = q.vec && !narrow ? 512 : 128;
+        const int64_t min_chunk = !narrow ? 512 : 128;
         for (int64_t S = 2; S <= 1024 && S <= d.K / min_chunk; S += (S < 8 ? 1 : S / 4)) {   // about 25 candidates
             const int64_t Kc = ((d.K + S - 1) / S + 31) / 32 * 32;              // chunk length, whole 32-wide k tiles
             const int64_t parts = (d.K + Kc - 1) / Kc;                           // the last one may be shorter
@@ -529,13 +527,13 @@ GemmPlan gemm_fused_plan(const nzhip_gemm_desc& d, int padded) {
     return best;
 }
 
-bool gemm_small_tile(const nzhip_gemm_desc& d, int padded) {
+bool gemm_small_tile(const nzhip_gemm_desc& d) {
     // called with the descriptor of the launch itself (split chunks are its inner batch)
-    const FusedCostInput q = fused_cost_input(d, padded);
+    const FusedCostInput q = fused_cost_input(d);
     return fused_cost_us(q, 64, 1, d.K) < 0.97 * fused_cost_us(q, 128, 1, d.K);
 }
 
-int gemm_mfma_dispatch(const nzhip_gemm_desc& d, hipStream_t stream, int force_tile, int64_t k_total, int padded) {
+int gemm_mfma_dispatch(const nzhip_gemm_desc& d, hipStream_t stream, int force_tile, int64_t k_total) {
     GemmKernelArgs a;
     a.A = d.A;
     a.B = d.B;
@@ -563,18 +561,17 @@ int gemm_mfma_dispatch(const nzhip_gemm_desc& d, hipStream_t stream, int force_t
     a.k_total = (int)k_total;
 
     const bool a_trans = d.a_layout == NZHIP_LAYOUT_TRANS, b_trans = d.b_layout == NZHIP_LAYOUT_TRANS;
-    const bool vec = gemm_operands_vec_legal(d, padded);
-    a.c_vec = gemm_c_vec_legal(d);
+    const bool vec = gemm_vec_legal(d);
     const int64_t batch = d.batch_n * d.batch_c;
 
     // Tile choice: 256x256 tiles need enough of them to fill the 256 CUs and pay only in their
     // unpredicated instance (5000x1000x5000: 379 us with predicated 256x256 tiles, 156 us with
     // 128x128 tiles).
     const int64_t t256 = ((d.M + 255) / 256) * ((d.N + 255) / 256) * batch;
-    const bool whole256 = vec && a.c_vec && d.M % 256 == 0 && d.N % 256 == 0 && d.K % 32 == 0 && (k_total <= 0 || k_total % d.K == 0);
+    const bool whole256 = vec && d.M % 256 == 0 && d.N % 256 == 0 && d.K % 32 == 0 && (k_total <= 0 || k_total % d.K == 0);
     static const char* tile_env = getenv("NZHIP_GEMM_TILE");         // 128 | 256: benchmarking only
     if (!force_tile && tile_env && (atoi(tile_env) == 128 || atoi(tile_env) == 256)) force_tile = atoi(tile_env);
-    int tile = force_tile ? force_tile : (t256 >= 192 && whole256 ? 256 : gemm_small_tile(d, padded) ? 64 : 128);
+    int tile = force_tile ? force_tile : (t256 >= 192 && whole256 ? 256 : gemm_small_tile(d) ? 64 : 128);
     const int bm = tile, bn = tile;
     a.tiles_m = (int)((d.M + bm - 1) / bm);
     a.tiles_n = (int)((d.N + bn - 1) / bn);
@@ -592,7 +589,7 @@ int gemm_mfma_dispatch(const nzhip_gemm_desc& d, hipStream_t stream, int force_t
     if (tile == 64) {
         // whole tiles: 64-wide k steps halve the number of barriers (1024^3: 14.2 -> 13.0 us); with predicates
         // the wider step only adds padding (1000 x 777 x 513: 22.0 -> 23.2 us)
-        const bool whole = vec && a.c_vec && d.M % 64 == 0 && d.N % 64 == 0 && d.K % 64 == 0 && (k_total <= 0 || k_total % d.K == 0);
+        const bool whole = vec && d.M % 64 == 0 && d.N % 64 == 0 && d.K % 64 == 0 && (k_total <= 0 || k_total % d.K == 0);
         if (whole) return launch_cfg<64, 64, 64, 2, 2>(a, a_trans, b_trans, vec, (int)batch, stream);
         return launch_cfg<64, 64, 32, 2, 2>(a, a_trans, b_trans, vec, (int)batch, stream);
     }

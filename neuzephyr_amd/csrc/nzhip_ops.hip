@@ -416,71 +416,11 @@ __global__ __launch_bounds__(256) void splitk_reduce_wide_kernel(nzhip_gemm_desc
 }
 
 
-// ---- operands that do not allow 16-byte loads ----------------------------------------------------
-// Rows that start off a 16-byte boundary or whose contiguous extent is not a multiple of 4 (1000 x 777 x 513)
-// make the fused kernel load element by element, which more than halves the rate at which a CU takes
-// tiles in. For a product big enough to notice, such an operand is first copied into a workspace with the
-// same layout and rows padded with zeros to a multiple of 4 elements (one launch for both operands).
-struct RepackOperand {
-    const float* src;
-    float* dst;
-    long rows, cols, ld_src, ld_dst;          // rows == 0: nothing to do
-};
-
-__global__ __launch_bounds__(256) void repack_pair_kernel(const RepackOperand a, const RepackOperand b) {
-    const RepackOperand& q = blockIdx.y ? b : a;
-    const long per_row = q.ld_dst / 4, total = q.rows * per_row;
-    for (long idx = (long)blockIdx.x * 256 + threadIdx.x; idx < total; idx += (long)gridDim.x * 256) {
-        const long r = idx / per_row, c = (idx - r * per_row) * 4;
-        const float* src = q.src + r * q.ld_src + c;
-        floatx4 v;
-#pragma unroll
-        for (int e = 0; e < 4; e++) v[e] = c + e < q.cols ? src[e] : 0.f;
-        *reinterpret_cast<floatx4*>(q.dst + r * q.ld_dst + c) = v;
-    }
-}
-
 }  // namespace nzhip
 
 using namespace nzhip;
 
-static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s, int padded = 0);
-
-// Returns NZHIP_OK and sets *done when the product was computed from padded copies; leaves *done false when
-// the copies would not pay (or the workspace is not to be had) and the caller goes on with the operands as given.
-static int gemm_try_repacked(const nzhip_gemm_desc& d, hipStream_t s, bool* done) {
-    *done = false;
-    if (d.batch_n * d.batch_c != 1) return NZHIP_OK;
-    const bool a_trans = d.a_layout == NZHIP_LAYOUT_TRANS, b_trans = d.b_layout == NZHIP_LAYOUT_TRANS;
-    const int64_t a_rows = a_trans ? d.K : d.M, a_cols = a_trans ? d.M : d.K;
-    const int64_t b_rows = b_trans ? d.N : d.K, b_cols = b_trans ? d.K : d.N;
-    const bool a_ok = gemm_operand_vec_legal(d.A, d.lda, a_cols, 0, 0), b_ok = gemm_operand_vec_legal(d.B, d.ldb, b_cols, 0, 0);
-    if (a_ok && b_ok) return NZHIP_OK;
-    const int64_t a_ld = (a_cols + 3) / 4 * 4, b_ld = (b_cols + 3) / 4 * 4;
-    const size_t a_bytes = a_ok ? 0 : (size_t)a_rows * a_ld * sizeof(float), b_bytes = b_ok ? 0 : (size_t)b_rows * b_ld * sizeof(float);
-    nzhip_gemm_desc g = d;
-    const int padded = (a_ok ? 0 : 1) | (b_ok ? 0 : 2);
-    // stand-in addresses for the cost estimate: only alignment and leading dimensions matter to it
-    if (!a_ok) { g.A = nullptr; g.lda = a_ld; }
-    if (!b_ok) { g.B = nullptr; g.ldb = b_ld; }
-    const double copy_us = 5.0 + 2.0 * (double)(a_bytes + b_bytes) / 3e6;      // launch and latency of the copy kernel, then its traffic
-    if (gemm_fused_plan(g, padded).cost_us + copy_us >= 0.9 * gemm_fused_plan(d).cost_us) return NZHIP_OK;   // two plans, ~50 estimates each
-    const size_t a_off = (a_bytes + 255) & ~(size_t)255;
-    char* ws = nullptr;
-    if (workspace_alloc(reinterpret_cast<void**>(&ws), a_off + b_bytes, s) != NZHIP_OK) return NZHIP_OK;   // no room: as given
-    RepackOperand ra = {d.A, reinterpret_cast<float*>(ws), a_ok ? 0 : a_rows, a_cols, d.lda, a_ld};
-    RepackOperand rb = {d.B, reinterpret_cast<float*>(ws + a_off), b_ok ? 0 : b_rows, b_cols, d.ldb, b_ld};
-    if (!a_ok) g.A = ra.dst;
-    if (!b_ok) g.B = rb.dst;
-    const long units = std::max(ra.rows * (ra.ld_dst / 4), rb.rows * (rb.ld_dst / 4));
-    const unsigned blocks = (unsigned)std::min<long>((units + 255) / 256, 4096);
-    hipLaunchKernelGGL(repack_pair_kernel, dim3(blocks, 2), dim3(256), 0, s, ra, rb);
-    int rc = check_launch("repack_pair_kernel");
-    if (rc == NZHIP_OK) rc = gemm_routed(g, s, padded);
-    const int rc2 = workspace_free(ws, s);
-    *done = true;
-    return rc ? rc : rc2;
-}
+static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s);
 
 extern "C" {
 
@@ -493,16 +433,8 @@ int nzhip_gemm(const nzhip_gemm_desc* desc, void* stream) {
 
 }  // extern "C"
 
-namespace nzhip {
-int gemm_padded_rows(const nzhip_gemm_desc& d, int padded, hipStream_t stream) {
-    if (int rc = validate_gemm(d)) return rc;
-    if (d.M == 0 || d.N == 0) return NZHIP_OK;
-    return gemm_routed(d, stream, padded);
-}
-}  // namespace nzhip
-
 // The route choice behind nzhip_gemm, for a validated descriptor with M, N > 0.
-static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s, int padded) {
+static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s) {
     if (d.K == 0) {
         dim3 grid((unsigned)((d.M * d.N + 255) / 256), (unsigned)(d.batch_n * d.batch_c));
         hipLaunchKernelGGL(fill_bias_act_kernel, grid, dim3(256), 0, s, d);
@@ -521,19 +453,11 @@ static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s, int padded) {
     const bool allow_coop = !(coop_env && atoi(coop_env) == 0);
     if (!force_fused && allow_coop && gemm_h16_coop_applicable(d)) return gemm_h16_coop_dispatch(d, s);
     if (!force_fused && (force_h16 || gemm_h16_applicable(d))) return gemm_h16_dispatch(d, s);
-    {
-        static const char* repack_env = getenv("NZHIP_REPACK");          // 0: never copy operands (benchmarking only)
-        bool done = false;
-        if (!padded && !(repack_env && atoi(repack_env) == 0)) {
-            const int rc = gemm_try_repacked(d, s, &done);
-            if (done || rc) return rc;
-        }
-    }
-    GemmPlan plan = gemm_fused_plan(d, padded);
+    GemmPlan plan = gemm_fused_plan(d);
     static const char* trace_env = getenv("NZHIP_TRACE");               // 1: one line per product on stderr (debugging only)
     if (trace_env && atoi(trace_env))
-        fprintf(stderr, "nzhip_gemm %ld x %ld x %ld batch %ld x %ld%s: fused kernel, %d^2 tiles, %ld chunk(s) of %ld, model %.1f us\n",
-                (long)d.M, (long)d.K, (long)d.N, (long)d.batch_n, (long)d.batch_c, padded ? " (padded copies)" : "", plan.tile,
+        fprintf(stderr, "nzhip_gemm %ld x %ld x %ld batch %ld x %ld: fused kernel, %d^2 tiles, %ld chunk(s) of %ld, model %.1f us\n",
+                (long)d.M, (long)d.K, (long)d.N, (long)d.batch_n, (long)d.batch_c, plan.tile,
                 (long)plan.parts, (long)plan.Kc, plan.cost_us);
     static const char* sk_env = getenv("NZHIP_SPLITK");                  // benchmarking only: number of chunks
     if (sk_env && atoi(sk_env) >= 1 && d.batch_c == 1 && d.batch_n <= 65535) {
@@ -555,7 +479,7 @@ static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s, int padded) {
         g.b_stride_c = d.b_layout == NZHIP_LAYOUT_ROW ? Kc * d.ldb : Kc;
         g.c_stride_c = d.M * d.N;
         g.bias = nullptr; g.activation = NZHIP_ACT_NONE;
-        int rc = gemm_mfma_dispatch(g, s, plan.tile, d.K, padded);
+        int rc = gemm_mfma_dispatch(g, s, plan.tile, d.K);
         if (rc == NZHIP_OK) {
             if (parts >= 64 && d.M * d.N <= 4096) {                     // a handful of outputs: one wave each
                 const long groups = (d.M * d.N + 3) / 4;
@@ -572,7 +496,7 @@ static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s, int padded) {
         const int rc2 = workspace_free(P, s);
         return rc ? rc : rc2;
     }
-    return gemm_mfma_dispatch(d, s, 0, 0, padded);
+    return gemm_mfma_dispatch(d, s, 0, 0);
 }
 
 extern "C" {

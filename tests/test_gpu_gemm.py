@@ -410,6 +410,26 @@ def _embedded_cases():
     return cases
 
 
+@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("a_trans,b_trans", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,K,N", [(3, 70, 66), (65, 3, 130), (66, 35, 2), (4, 4, 4), (67, 33, 65), (131, 36, 129), (5, 2, 3)])
+def test_fused_kernel_at_the_ends_of_its_operands(nz, M, K, N, a_trans, b_trans, tile):
+    """Extents below one 16-byte piece, of exactly one, and pieces cut by every edge, behind NaN guards on both sides: accesses are
+    moved into the operand, so nothing outside it may reach a sum."""
+    import torch
+    g = torch.Generator().manual_seed(M * 10007 + K * 101 + N)
+    A, B = torch.randint(-4, 5, (M, K), generator=g).double(), torch.randint(-4, 5, (K, N), generator=g).double()
+
+    def guarded(X, off):
+        buf = torch.full((X.numel() + 16,), float("nan"), device="cuda")
+        v = buf[off:off + X.numel()].view(X.shape)
+        v.copy_(X)
+        return v
+    got = nz.gemm(guarded(A.t().contiguous() if a_trans else A, 5), guarded(B.t().contiguous() if b_trans else B, 7),
+                  a_trans=a_trans, b_trans=b_trans, force_tile=tile)
+    assert torch.equal(got.double().cpu(), A @ B)
+
+
 @pytest.mark.parametrize("M,K,N,a_trans,b_trans,slack,offset,bias_form,seed", _embedded_cases())
 def test_embedded_operands_random_sweep(nz, M, K, N, a_trans, b_trans, slack, offset, bias_form, seed):
     # random shapes, layouts, leading dimensions and base offsets through the default route choice (streaming,
