@@ -62,7 +62,7 @@ __device__ __forceinline__ int phys_row(int r) {
 // 16-byte piece cut by the end of the contiguous extent starts earlier. Where the registers are CONVERTED, one uniform test
 // per k tile finds the last one, whose missing k are zeroed, and one per tile the pieces that have to be turned back.
 // 16-byte accesses need no more than the 4-byte alignment of their elements: rows of 777 or 513 floats stream at the rate of
-// rows of 776 or 512 (1000 x 777 x 513: @A us; element by element it was 33, through zero-padded copies of the operands 21).
+// rows of 776 or 512 (1000 x 777 x 513: 14.9 us; element by element it was 33, through zero-padded copies of the operands 21).
 typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
 
@@ -483,13 +483,19 @@ static double fused_cost_us(const FusedCostInput& q, int tile, int64_t parts, in
     const int64_t tiles = ((q.M + tile - 1) / tile) * ((q.N + tile - 1) / tile) * q.members * parts;
     const double rounds = (double)((tiles + (int64_t)q.cus - 1) / (int64_t)q.cus);
     const bool full = q.aligned && q.M % tile == 0 && q.N % tile == 0 && Kc % 32 == 0 && q.K % 32 == 0;   // unpredicated instance
-    // rows past the operand's extent are predicated off, not loaded: a narrow operand costs what it has
+    // rows past the operand's extent are repeats of its last row, served by L1: a narrow operand costs what it has
     const double rows = (double)(q.M < tile ? q.M : tile) + (double)(q.N < tile ? q.N : tile);
     // two or more workgroups on a CU overlap their waits: the CU takes in up to 1.3 x what one workgroup draws
     // (16 x 8192 x 8192: 50 us in eight chunks, two workgroups per CU, against 57 us in four)
     const double per_cu = (double)tiles / q.cus;
     const double overlap = per_cu >= 2.0 ? 1.3 : per_cu > 1.0 ? 1.0 + 0.3 * (per_cu - 1.0) : 1.0;
-    const double stream = rounds * rows * (double)Kc * 4.0 / ((full ? 50e3 : 45e3) * overlap);   // bytes / (bytes per us)
+    // One tile of results: all there is to choose is the number of chunks, and these want more of them than the rate says
+    // (10 x 260100 x 16: 452 chunks 14.8 us, 233 chunks, the choice at 45, 16.7; 10 x 259081 x 16 450 and 232, 14.6 and 16.6;
+    // 4 x 80772 x 16 level from 181 to 505). The lower rates also keep the grouping of sums of that length, whose last bits
+    // decide roundings to fp16 further down a network.
+    const bool one_tile = q.M <= 64 && q.N <= 64;
+    const double rate = full ? 50e3 : !one_tile ? 45e3 : q.aligned ? 36e3 : 9e3;                            // bytes per us
+    const double stream = rounds * rows * (double)Kc * 4.0 / (rate * overlap);
     const double out = (double)q.M * q.N * q.members * 4.0;
     const double reduce = parts > 1 ? 6.0 + (double)(parts + 1) * out / 3e6 : 0.0;
     // what a workgroup spends outside its k loop (first requests, predicated epilogue): 17 x 33 x 15 takes 10 us with a
