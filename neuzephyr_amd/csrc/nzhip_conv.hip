@@ -264,8 +264,9 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
     static_assert(C_T * 9 * O_T <= 128, "one weight per thread");
     // requested now, parked in LDS after the first input rows have been requested (the rows then do not
     // queue up behind the round trip of the weights)
-    const int w_i = threadIdx.x < C_T * 9 * O_T ? threadIdx.x : 0;
-    const float w_mine = wb[mirror ? weight_source_index(w_i / (9 * O_T), w_i / O_T % 9, w_i % O_T, C_T, O_T, 9, 1) : w_i];
+    long w_i = threadIdx.x;
+    if (mirror) w_i = weight_source_index(threadIdx.x / (9 * O_T), threadIdx.x / O_T % 9, threadIdx.x % O_T, C_T, O_T, 9, 1);
+    const float w_mine = threadIdx.x < C_T * 9 * O_T ? wb[w_i] : 0.f;
     auto park_weights = [&]() {
         if (threadIdx.x < C_T * 9 * O_T) wsm[threadIdx.x] = round_f16(w_mine);   // [q][o]
         __syncthreads();
