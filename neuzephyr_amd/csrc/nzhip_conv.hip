@@ -2653,11 +2653,18 @@ __global__ __launch_bounds__(256) void conv_dw_reduce_few_kernel(float* __restri
 // As in the forward kernel every row of x and dy is requested three rows before it is used (a row asked for and used in the same
 // step left the wave waiting for memory once a row: 10 x 3 x 1024 x 1024, 168 MB, 49.5 -> 46.8 us), odd strips walk upwards so
 // that neighbours meet at the rows they share, and VEC says whether rows are whole, aligned 16-byte pieces (otherwise
-// load_ragged_quad: 10 x 3 x 500 x 655 21 us, 30 with four 4-byte loads per quad; such rows used to go to the gather kernel,
-// which multiplied mostly padding).
-template <int O_T, int C_T, bool VEC>
+// load_ragged_quad: 10 x 3 x 500 x 655 21 us, 30 with four 4-byte loads per quad).
+//
+// A column past the end of the row has a zero gradient, but that alone does not keep it out of the sums: its neighbour is the
+// row's last pixel, and 0 x Inf (70000 is one once rounded) is a NaN in taps that this pixel has no part in. Its factors are
+// zeros as well: a lane past the row has no left neighbour, and in the quad that the end of the row cuts the first column past
+// it, at filter column 0, is the only one that meets a pixel. That column is REM = W % 4, a template parameter, so that one
+// register per row and channel holds the masked factor: with all three possible columns kept (176 registers for three
+// channels, two waves per SIMD instead of three) 10 x 3 x 1000 x 1023 took 43.8 us, with one (158) 37.9, as without the masks.
+template <int O_T, int C_T, bool VEC, int REM>
 __global__ __launch_bounds__(256) void conv3x3_dw_stream_kernel(float* __restrict__ partial, const float* __restrict__ x,
                                                                 const float* __restrict__ dy, int H, int W) {
+    static_assert(REM >= 0 && REM < 4 && (!VEC || REM == 0), "aligned rows end with a whole quad");
     constexpr int Q = C_T * 9 * O_T, AHEAD = 3;
     int bx, by, b;
     xcd_contiguous_block(bx, by, b);
@@ -2672,9 +2679,9 @@ __global__ __launch_bounds__(256) void conv3x3_dw_stream_kernel(float* __restric
         const int w0 = inside ? (bx * 64 + lane) * 4 : (W - 1) / 4 * 4;     // lanes past the row re-read its end and add nothing
         bool col[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) col[e] = inside && (VEC || w0 + e < W);
+        for (int e = 0; e < 4; e++) col[e] = inside && (REM == 0 || e < REM || w0 + 4 <= W);
         const int w_at = w0 + 4 <= W ? w0 : W - 4;
-        const bool has_l = w0 > 0, has_r = w0 + 4 < W;
+        const bool has_l = inside && w0 > 0, has_r = inside && w0 + 4 < W;
         const int wx = lane == 0 ? (has_l ? w0 - 1 : w0) : (lane == 63 && has_r ? w0 + 4 : w0);
         const float* xb = x + (long)b * C_T * H * W;
         const float* gb = dy + (long)b * O_T * H * W;
@@ -2687,6 +2694,7 @@ __global__ __launch_bounds__(256) void conv3x3_dw_stream_kernel(float* __restric
             auto out_row = [&](int t) { return UP ? h0 + rows + 1 - t : h0 + t - 2; };   // whose window step t >= 2 completes
             auto row_in_image = [&](int t) { const int hi = row_first + t * row_step; return t < T && hi >= 0 && hi < H; };
             float win[3][C_T][6];                                // rounded rows t-2, t-1, t (t % 3)
+            float left[3][C_T];                                  // column REM as the factor at filter column 0
             float raw[AHEAD][C_T][5], graw[AHEAD][O_T][4];       // rows in flight
             auto quad = [&](const float* row, float (&v)[4]) {
                 if constexpr (VEC) {
@@ -2733,6 +2741,7 @@ __global__ __launch_bounds__(256) void conv3x3_dw_stream_kernel(float* __restric
 #pragma unroll
                         for (int e = 0; e < 4; e++) win[u][c][1 + e] = r5[e];
                         win[u][c][5] = has_r ? (lane == 63 ? r5[4] : above) : 0.f;
+                        if constexpr (REM != 0) left[u][c] = col[REM] ? win[u][c][REM] : 0.f;
                     }
 #pragma unroll
                     for (int o = 0; o < O_T; o++)
@@ -2756,8 +2765,8 @@ __global__ __launch_bounds__(256) void conv3x3_dw_stream_kernel(float* __restric
                                     for (int o = 0; o < O_T; o++)
 #pragma unroll
                                         for (int e = 0; e < 4; e++)
-                                            acc[((c * 3 + r) * 3 + s2) * O_T + o] =
-                                                __builtin_fmaf(win[slot][c][e + s2], g[o][e], acc[((c * 3 + r) * 3 + s2) * O_T + o]);
+                                            acc[((c * 3 + r) * 3 + s2) * O_T + o] = __builtin_fmaf(REM != 0 && s2 == 0 && e == REM ? left[slot][c] : win[slot][c][e + s2], g[o][e],
+                                                                                                   acc[((c * 3 + r) * 3 + s2) * O_T + o]);
                             }
                     }
                 }
@@ -4124,8 +4133,12 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
         float* partial = nullptr;
         if (int rc = workspace_alloc(reinterpret_cast<void**>(&partial), per_image * N * Q * sizeof(float), s)) return rc;
 #define NZHIP_DWS(OT, CT)                                                                                            \
-    hipLaunchKernelGGL((pieces ? conv3x3_dw_stream_kernel<OT, CT, true> : conv3x3_dw_stream_kernel<OT, CT, false>), grid, dim3(256), 0, s, \
-                       partial, x, dy, (int)H, (int)W)
+    hipLaunchKernelGGL((pieces ? conv3x3_dw_stream_kernel<OT, CT, true, 0>                                               \
+                        : W % 4 == 0 ? conv3x3_dw_stream_kernel<OT, CT, false, 0>                                        \
+                        : W % 4 == 1 ? conv3x3_dw_stream_kernel<OT, CT, false, 1>                                        \
+                        : W % 4 == 2 ? conv3x3_dw_stream_kernel<OT, CT, false, 2>                                        \
+                                     : conv3x3_dw_stream_kernel<OT, CT, false, 3>),                                      \
+                       grid, dim3(256), 0, s, partial, x, dy, (int)H, (int)W)
         switch ((int)(O * 10 + C)) {
             case 11: NZHIP_DWS(1, 1); break;
             case 12: NZHIP_DWS(1, 2); break;

@@ -546,6 +546,28 @@ def test_conv2d_bias_gradients_on_every_tile_shape(nz, oracle, N, O, H, W):
         assert np.array_equal(host(db), want), masked
 
 
+@pytest.mark.parametrize("special", [70000.0, float("inf"), float("nan")])
+@pytest.mark.parametrize("C,O", [(1, 1), (3, 1), (4, 2)])
+@pytest.mark.parametrize("W,offset", [(5, 0), (6, 0), (28, 0), (28, 1), (30, 0), (31, 0), (255, 0), (256, 0), (257, 0), (260, 0), (260, 1)])
+def test_thin_weight_gradient_keeps_a_pixel_out_of_taps_it_has_no_part_in(nz, W, offset, C, O, special):
+    """A pixel that is no finite fp16 value at an edge of its row is a factor of some taps of its channel and of no others: those
+    match the definition exactly (integers), with lanes and columns past the row present (W % 256 != 0, W % 4 != 0) and not, rows on and off 16-byte boundaries."""
+    import torch
+    N, H = 2, 18
+    g = torch.Generator().manual_seed(W * 100 + 10 * C + O)
+    x = torch.randint(-4, 5, (N, C, H, W), generator=g).float()
+    dy = torch.randint(1, 5, (N, O, H, W), generator=g).float()
+    x[0, C - 1, 7, W - 1] = special
+    x[1, 0, 0, 0] = special
+    x_dev = torch.empty(x.numel() + 4, device="cuda")[offset:offset + x.numel()].view(x.shape).copy_(x)
+    dw = nz.conv2d_backward_weights(torch.zeros(N, 1, C * 9, O, device="cuda"), x_dev, dy.cuda(), 3, 3, 1, 1).cpu()
+    xr = torch.nn.functional.pad(x.half().double(), (1, 1, 1, 1))          # 70000 rounds to Inf
+    want = torch.stack([torch.stack([(xr[:, c, None, r:r + H, s:s + W] * dy.double()).sum((2, 3)) for r in range(3) for s in range(3)], 1)
+                        for c in range(C)], 1).view(N, C * 9, O)
+    assert torch.isfinite(want).any() and not torch.isfinite(want).all()
+    assert torch.equal(torch.nan_to_num(dw[:, 0].double(), 1e30, 2e30, -2e30), torch.nan_to_num(want, 1e30, 2e30, -2e30))
+
+
 def test_conv2d_backward_weights_rejects_what_it_does_not_cover(nz):
     from neuzephyr_amd.capi import NzHipError
     with pytest.raises(NzHipError) as e:      # stride 5
