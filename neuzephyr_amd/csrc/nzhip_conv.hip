@@ -4,6 +4,7 @@
 
 #include <type_traits>
 
+#include <algorithm>
 #include <cstdlib>
 
 #include "nzhip_internal.h"
@@ -3444,8 +3445,9 @@ __global__ __launch_bounds__(256) void conv_bias_grad_kernel(float* __restrict__
     constexpr int TP = 256 * V / TO, PT = TP / V;                // pixels of the tile; threads along them
     constexpr int U = 8;                                         // images in flight
     __shared__ float tile[TO > 1 ? TP : 1][TO + 1];              // [pixel][channel]
-    const long p0 = (long)blockIdx.x * TP;
+    const long p0 = ((long)blockIdx.z * gridDim.x + blockIdx.x) * TP;
     const int o0 = blockIdx.y * TO;
+    if (p0 >= HW) return;
     const int px = (threadIdx.x % PT) * V, oc = threadIdx.x / PT;
     const long p = p0 + px;
     const bool live = p < HW && o0 + oc < O;                     // V == 4: HW % 4 == 0, the four pixels are inside together
@@ -3527,9 +3529,13 @@ static int conv_bias_grad_launch(float* dbias, const float* dz, size_t N, size_t
                                       (O == 1 ? reinterpret_cast<uintptr_t>(dbias) : 0)) & 15) == 0;
     const bool many = HW * O >= (size_t)device_cu_count() * 2 * 1024;
     auto go = [&](auto kernel, size_t tp, size_t to) {
-        const size_t gx = (HW + tp - 1) / tp, gy = (O + to - 1) / to;
-        if (gx > 0x7fffffffull || gy > 65535) return set_error(NZHIP_E_UNSUPPORTED, "conv bias gradient: extent too large");
-        hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, s, dbias, dz, (int)N, (int)O, (long)HW, dz_out, y);
+        // A launch counts its threads in 32 bits along each direction and drops what is above without an error: tiles beyond
+        // 2^22 along the pixels (images of 1.3e8 pixels and more) go on along z.
+        const size_t tiles = (HW + tp - 1) / tp, gx = std::min<size_t>(tiles, (size_t)1 << 22), gz = (tiles + gx - 1) / gx;
+        const size_t gy = (O + to - 1) / to;
+        if (gz > 65535 || gy > 65535) return set_error(NZHIP_E_UNSUPPORTED, "conv bias gradient: extent too large");
+        hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)gy, (unsigned)gz), dim3(256), 0, s, dbias, dz, (int)N, (int)O, (long)HW,
+                           dz_out, y);
         hipError_t e = hipGetLastError();
         return e == hipSuccess ? NZHIP_OK : set_hip_error(e, "conv_bias_grad kernel launch");
     };

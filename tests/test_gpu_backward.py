@@ -546,6 +546,17 @@ def test_conv2d_bias_gradients_on_every_tile_shape(nz, oracle, N, O, H, W):
         assert np.array_equal(host(db), want), masked
 
 
+def test_conv2d_bias_gradient_of_an_image_beyond_32_bit_thread_counts(nz):
+    """537 million pixels and five channels: more than 2^32 threads along the pixels, which one grid dimension does not hold."""
+    import torch
+    O, HW = 5, (1 << 29) + 130301
+    dz = torch.empty(1, O, 1, HW, device="cuda").uniform_(-1, 1, generator=torch.Generator(device="cuda").manual_seed(3))
+    db = torch.zeros(1, 1, HW, O, device="cuda")
+    nz.conv2d_backward_bias(db, dz)
+    for p in range(0, HW, 1 << 27):
+        assert torch.equal(db[0, 0, p:p + (1 << 27)].t(), dz[0, :, 0, p:p + (1 << 27)])
+
+
 @pytest.mark.parametrize("special", [70000.0, float("inf"), float("nan")])
 @pytest.mark.parametrize("C,O", [(1, 1), (3, 1), (4, 2)])
 @pytest.mark.parametrize("W,offset", [(5, 0), (6, 0), (28, 0), (28, 1), (30, 0), (31, 0), (255, 0), (256, 0), (257, 0), (260, 0), (260, 1)])
