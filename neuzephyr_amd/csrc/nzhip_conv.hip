@@ -3441,13 +3441,13 @@ namespace nzhip {
 template <bool MASK, int V, int TO>
 __global__ __launch_bounds__(256) void conv_bias_grad_kernel(float* __restrict__ dbias, const float* __restrict__ dz, int N,
                                                              int O, long HW, float* __restrict__ dz_out,
-                                                             const float* __restrict__ y) {
+                                                             const float* __restrict__ y, int pixel_folds) {
     constexpr int TP = 256 * V / TO, PT = TP / V;                // pixels of the tile; threads along them
     constexpr int U = 8;                                         // images in flight
     __shared__ float tile[TO > 1 ? TP : 1][TO + 1];              // [pixel][channel]
-    const long p0 = ((long)blockIdx.z * gridDim.x + blockIdx.x) * TP;
-    const int o0 = blockIdx.y * TO;
-    if (p0 >= HW) return;
+    const long p0 = ((long)(blockIdx.z % pixel_folds) * gridDim.x + blockIdx.x) * TP;
+    const long o0 = ((long)(blockIdx.z / pixel_folds) * gridDim.y + blockIdx.y) * TO;
+    if (p0 >= HW || o0 >= O) return;
     const int px = (threadIdx.x % PT) * V, oc = threadIdx.x / PT;
     const long p = p0 + px;
     const bool live = p < HW && o0 + oc < O;                     // V == 4: HW % 4 == 0, the four pixels are inside together
@@ -3530,12 +3530,12 @@ static int conv_bias_grad_launch(float* dbias, const float* dz, size_t N, size_t
     const bool many = HW * O >= (size_t)device_cu_count() * 2 * 1024;
     auto go = [&](auto kernel, size_t tp, size_t to) {
         // A launch counts its threads in 32 bits along each direction and drops what is above without an error: tiles beyond
-        // 2^22 along the pixels (images of 1.3e8 pixels and more) go on along z.
-        const size_t tiles = (HW + tp - 1) / tp, gx = std::min<size_t>(tiles, (size_t)1 << 22), gz = (tiles + gx - 1) / gx;
-        const size_t gy = (O + to - 1) / to;
-        if (gz > 65535 || gy > 65535) return set_error(NZHIP_E_UNSUPPORTED, "conv bias gradient: extent too large");
-        hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)gy, (unsigned)gz), dim3(256), 0, s, dbias, dz, (int)N, (int)O, (long)HW,
-                           dz_out, y);
+        // 2^22 along the pixels (images of 1.3e8 pixels and more) go on along z, and so do those beyond 65535 along the channels.
+        const size_t tx = (HW + tp - 1) / tp, gx = std::min<size_t>(tx, (size_t)1 << 22), zx = (tx + gx - 1) / gx;
+        const size_t ty = (O + to - 1) / to, gy = std::min<size_t>(ty, 65535), zy = (ty + gy - 1) / gy;
+        if (zx * zy > 65535) return set_error(NZHIP_E_UNSUPPORTED, "conv bias gradient: extent too large");
+        hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)gy, (unsigned)(zx * zy)), dim3(256), 0, s, dbias, dz, (int)N, (int)O,
+                           (long)HW, dz_out, y, (int)zx);
         hipError_t e = hipGetLastError();
         return e == hipSuccess ? NZHIP_OK : set_hip_error(e, "conv_bias_grad kernel launch");
     };

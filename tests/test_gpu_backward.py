@@ -546,6 +546,21 @@ def test_conv2d_bias_gradients_on_every_tile_shape(nz, oracle, N, O, H, W):
         assert np.array_equal(host(db), want), masked
 
 
+@pytest.mark.parametrize("O,HW", [(524281, 3), (1100000, 1), (2097121, 2), (600000, 4)])
+def test_conv2d_bias_gradients_of_more_channels_than_one_grid_dimension_holds(nz, O, HW):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(O)
+    y, dy = (torch.empty(2, O, 1, HW, device="cuda").uniform_(-1, 1, generator=g) for _ in range(2))
+    dz = torch.where(y > 0, dy, torch.zeros_like(dy))
+    for masked in (False, True):
+        db = torch.zeros(1, 1, HW, O, device="cuda")
+        if masked:
+            assert torch.equal(nz.conv2d_backward_relu_bias(db, y, dy), dz)
+        else:
+            nz.conv2d_backward_bias(db, dz)
+        assert torch.equal(db[0, 0], (dz[0, :, 0] + dz[1, :, 0]).t())
+
+
 def test_conv2d_bias_gradient_of_an_image_beyond_32_bit_thread_counts(nz):
     """537 million pixels and five channels: more than 2^32 threads along the pixels, which one grid dimension does not hold."""
     import torch
