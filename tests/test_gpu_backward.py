@@ -525,7 +525,8 @@ def test_conv2d_backward_relu_bias_equals_relu_backward_then_bias(nz, oracle, N,
     assert np.array_equal(host(dz), dz_want) and np.array_equal(host(db), db_want)
 
 
-@pytest.mark.parametrize("N,O,H,W", [(11, 1, 512, 1028), (3, 1, 37, 41), (9, 3, 420, 420), (10, 33, 128, 130), (17, 34, 9, 14), (8, 4, 5, 13)])
+@pytest.mark.parametrize("N,O,H,W", [(11, 1, 512, 1028), (2, 1, 513, 1028), (3, 1, 37, 41), (9, 3, 420, 420), (10, 33, 128, 130),
+                                     (3, 33, 130, 130), (17, 34, 9, 14), (8, 4, 5, 13)])
 def test_conv2d_bias_gradients_on_every_tile_shape(nz, oracle, N, O, H, W):
     """One, up to four and more channels, with and without 16-byte accesses, image counts around the eight in flight, edges in
     both directions: one chain per element, so bit for bit."""
