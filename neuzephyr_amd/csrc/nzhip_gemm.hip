@@ -13,6 +13,7 @@
 //   * batch (n,c), broadcast strides, bias and ReLU are handled in-kernel.
 #include <hip/hip_runtime.h>
 
+#include <cstdio>
 #include <cstdlib>
 #include <type_traits>
 
@@ -76,7 +77,8 @@ __device__ __forceinline__ floatx4 turn_back(const floatx4 q, int back) {
 // in the kernel, at every load, cost the loads their place in the order the waits rely on, 1040 x 1280 x 1968 35 -> 55 us).
 enum Edge { INTERIOR, PIECES, ELEMENTS };
 
-// the piece at offset `at` of a row of `extent` contiguous elements, moved into the row
+// the piece at offset `at` of a row of `extent` contiguous elements, moved into the row (or, where `extent` is the end of a chunk
+// of fewer than 4, into the row's chunk before it)
 template <int EDGE>
 __device__ __forceinline__ floatx4 load_piece(const float* row, int at, int extent) {
     if constexpr (EDGE == PIECES) {
@@ -429,6 +431,11 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
 }
 
 // ---- host-side selection -------------------------------------------------------------------
+bool gemm_trace() {
+    static const char* env = getenv("NZHIP_TRACE");                  // 1: two lines per product on stderr (debugging only)
+    return env && atoi(env);
+}
+
 template <int BM, int BN, int BK, int WM, int WN>
 static int launch_cfg(const GemmKernelArgs& a, bool a_trans, bool b_trans, bool aligned, int batch, hipStream_t s) {
     const bool full = aligned && a.M % BM == 0 && a.N % BN == 0 && a.K % BK == 0 && (a.k_total <= 0 || a.k_total % a.K == 0);
@@ -449,9 +456,14 @@ static int launch_cfg(const GemmKernelArgs& a, bool a_trans, bool b_trans, bool 
         return launch(gemm_f16mfma_kernel<BM, BN, BK, WM, WN, true, true, E>);
     };
     if (full) return pick(std::integral_constant<int, INTERIOR>{});
-    // the shortest contiguous extent, the last chunk of a split contraction included
-    const int last_k = a.k_total > 0 ? a.k_total - (a.batch_c - 1) * a.K : a.K, k_min = last_k < a.K ? last_k : a.K;
-    const bool pieces = (a_trans ? a.M : k_min) >= 4 && (b_trans ? k_min : a.N) >= 4;
+    // By pieces where no contiguous extent is below 4. Along k that is the whole contraction, also of a split one: however few
+    // elements its last chunk has, those before it in the row are the previous chunk's, so a piece moved left out of the chunk
+    // is still inside the operand, and what it brings along is zeroed like anything past the end. (Judged by the last chunk
+    // alone, one left-over element put all chunks on single elements: 10 x 40001 x 16 in 51 chunks 23.4 us, by pieces 14.2;
+    // 32 x 4962 x 1024 18.6 and 11.5, 1024 x 1154 x 32 11.5 and 8.9.)
+    const int k = a.k_total > 0 ? a.k_total : a.K;
+    const bool pieces = (a_trans ? a.M : k) >= 4 && (b_trans ? k : a.N) >= 4;
+    if (gemm_trace()) fprintf(stderr, "nzhip_gemm: loads by %s\n", pieces ? "pieces" : "elements");
     return pieces ? pick(std::integral_constant<int, PIECES>{}) : pick(std::integral_constant<int, ELEMENTS>{});
 }
 

@@ -21,6 +21,7 @@ int gemm_mfma_dispatch(const nzhip_gemm_desc& d, hipStream_t stream, int force_t
 // Tile (64 or 128) and number of contraction chunks (1 = no split) for a product that goes to the fused kernel.
 struct GemmPlan { int tile; int64_t parts; int64_t Kc; double cost_us; };
 GemmPlan gemm_fused_plan(const nzhip_gemm_desc& d);
+bool gemm_trace();                               // NZHIP_TRACE=1
 bool gemm_small_tile(const nzhip_gemm_desc& d);
 // Two-pass route for large products: fp16 rounding pass + fp16 GEMM fed by direct-to-LDS loads
 // (nzhip_gemm_h16.hip).

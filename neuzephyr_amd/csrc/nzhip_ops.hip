@@ -454,8 +454,7 @@ static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s) {
     if (!force_fused && allow_coop && gemm_h16_coop_applicable(d)) return gemm_h16_coop_dispatch(d, s);
     if (!force_fused && (force_h16 || gemm_h16_applicable(d))) return gemm_h16_dispatch(d, s);
     GemmPlan plan = gemm_fused_plan(d);
-    static const char* trace_env = getenv("NZHIP_TRACE");               // 1: one line per product on stderr (debugging only)
-    if (trace_env && atoi(trace_env))
+    if (gemm_trace())
         fprintf(stderr, "nzhip_gemm %ld x %ld x %ld batch %ld x %ld: fused kernel, %d^2 tiles, %ld chunk(s) of %ld, model %.1f us\n",
                 (long)d.M, (long)d.K, (long)d.N, (long)d.batch_n, (long)d.batch_c, plan.tile,
                 (long)plan.parts, (long)plan.Kc, plan.cost_us);

@@ -430,6 +430,35 @@ def test_fused_kernel_at_the_ends_of_its_operands(nz, M, K, N, a_trans, b_trans,
     assert torch.equal(got.double().cpu(), A @ B)
 
 
+SHORT_LAST_CHUNKS = r"""
+import torch
+from neuzephyr_amd import capi
+for M, K, N, left in ((10, 4993, 16, 1), (33, 1538, 70, 2), (512, 2307, 32, 3), (96, 1153, 65, 1)):
+    assert K % (((K + 12) // 13 + 31) // 32 * 32) == left              # in 13 chunks of whole 32-wide k tiles
+    for a_trans in (False, True):
+        for b_trans in (False, True):
+            g = torch.Generator().manual_seed(M + K + N)
+            A, B = torch.randint(-4, 5, (M, K), generator=g).double(), torch.randint(-4, 5, (K, N), generator=g).double()
+            got = capi.gemm((A.t() if a_trans else A).contiguous().float().cuda(), (B.t() if b_trans else B).contiguous().float().cuda(),
+                            a_trans=a_trans, b_trans=b_trans)
+            assert torch.equal(got.double().cpu(), A @ B), (M, K, N, a_trans, b_trans)
+            print("exact", flush=True)
+"""
+
+
+def test_split_contractions_with_a_last_chunk_shorter_than_a_piece():
+    """One to three elements left for the last chunk: exact on integers in all layouts, and loaded by pieces like the other chunks."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    p = subprocess.run([sys.executable, "-c", SHORT_LAST_CHUNKS], capture_output=True, text=True, timeout=100, cwd=root,
+                       env={**os.environ, "NZHIP_TRACE": "1", "NZHIP_SPLITK": "13", "PYTHONPATH": root})
+    assert p.returncode == 0, p.stderr[-2000:]
+    assert p.stdout.count("exact") == 16
+    assert p.stderr.count("loads by pieces") == 16 and "loads by elements" not in p.stderr
+
+
 @pytest.mark.parametrize("M,K,N,a_trans,b_trans,slack,offset,bias_form,seed", _embedded_cases())
 def test_embedded_operands_random_sweep(nz, M, K, N, a_trans, b_trans, slack, offset, bias_form, seed):
     # random shapes, layouts, leading dimensions and base offsets through the default route choice (streaming,
