@@ -482,9 +482,9 @@ bool gemm_vec_legal(const nzhip_gemm_desc& d) {
 // ---- tile and split choice for products that do not fill the device -------------------------------
 // The fused kernel's k loop is bound by the rate at which one CU takes fp32 tiles in through its L1
 // (about 50 GB/s per CU, 45 in the instance that keeps its accesses inside ragged operands), so the time of a launch is
-// the bytes the busiest CU streams: rounds of workgroups x (tile rows + tile columns, as far as the
-// operands reach) x chunk length x 4 bytes. 64 x 64 tiles stream twice the bytes of 128 x 128 tiles in total but put four times
-// as many CUs to work (1024^3: 23.6 us -> 14.2 us); a split contraction adds a pass over the partial sums.
+// the bytes the busiest CU streams: rounds of workgroups x (tile rows + tile columns) x chunk length x 4 bytes. 64 x 64
+// tiles stream twice the bytes of 128 x 128 tiles in total but put four times as many CUs to work (1024^3: 23.6 us ->
+// 14.2 us); a split contraction adds a pass over the partial sums.
 struct FusedCostInput {
     int64_t M, N, K, members;       // members: batch_n * batch_c of the product as given
     double cus;
@@ -495,21 +495,20 @@ static double fused_cost_us(const FusedCostInput& q, int tile, int64_t parts, in
     const int64_t tiles = ((q.M + tile - 1) / tile) * ((q.N + tile - 1) / tile) * q.members * parts;
     const double rounds = (double)((tiles + (int64_t)q.cus - 1) / (int64_t)q.cus);
     const bool full = q.aligned && q.M % tile == 0 && q.N % tile == 0 && Kc % 32 == 0 && q.K % 32 == 0;   // unpredicated instance
-    // rows past the operand's extent are repeats of its last row, served by L1: a narrow operand costs what it has
-    const double rows = (double)(q.M < tile ? q.M : tile) + (double)(q.N < tile ? q.N : tile);
+    // A narrow operand costs what a whole tile of it would: the loads of rows past its end are issued all the same, and a k step
+    // has a latency that few rows do not shorten (two chunks of 1024 steps with 64 x 64 tiles: 4 x 65536 x 16 272 us, 63 x 65536 x 61
+    // 281). Charged by the rows it has, a product that leaves CUs idle gets too few chunks (10 x 260100 x 16: 233 chunks 16.7 us,
+    // 452, two workgroups per CU, 14.8; 48 x 1024 x 4096 15.9 and 12.3; the other way round only 16 x 8192 x 2048, whose operands
+    // arrive no faster: 15.8 and 17.4).
+    const double rows = 2.0 * tile;
     // two or more workgroups on a CU overlap their waits: the CU takes in up to 1.3 x what one workgroup draws
     // (16 x 8192 x 8192: 50 us in eight chunks, two workgroups per CU, against 57 us in four)
     const double per_cu = (double)tiles / q.cus;
     const double overlap = per_cu >= 2.0 ? 1.3 : per_cu > 1.0 ? 1.0 + 0.3 * (per_cu - 1.0) : 1.0;
-    // One tile of results: all there is to choose is the number of chunks, and these want more of them than the rate says
-    // (10 x 260100 x 16: 452 chunks 14.8 us, 233 chunks, the choice at 45, 16.7; 10 x 259081 x 16 450 and 232, 14.6 and 16.6;
-    // 4 x 80772 x 16 level from 181 to 505). The lower rates also keep the grouping of sums of that length, whose last bits
-    // decide roundings to fp16 further down a network.
-    const bool one_tile = q.M <= 64 && q.N <= 64;
-    const double rate = full ? 50e3 : !one_tile ? 45e3 : q.aligned ? 36e3 : 9e3;                            // bytes per us
-    const double stream = rounds * rows * (double)Kc * 4.0 / (rate * overlap);
+    const double stream = rounds * rows * (double)Kc * 4.0 / ((full ? 50e3 : 45e3) * overlap);      // bytes / (bytes per us)
     const double out = (double)q.M * q.N * q.members * 4.0;
-    const double reduce = parts > 1 ? 6.0 + (double)(parts + 1) * out / 3e6 : 0.0;
+    // the second launch: 16 x 736 x 1905 12.7 us unsplit, 8.6 in four chunks, 33 x 512 x 33 7.6 either way (charged 6 it kept the first unsplit)
+    const double reduce = parts > 1 ? 4.5 + (double)(parts + 1) * out / 3e6 : 0.0;
     // what a workgroup spends outside its k loop (first requests, predicated epilogue): 17 x 33 x 15 takes 10 us with a
     // 128 x 128 tile and 5 us with a 64 x 64 tile; rounds that share a CU pay it side by side
     const double ends = (tile == 64 ? 1.5 : 4.0) * (rounds > 2.0 ? rounds / 2.0 : 1.0);

@@ -459,6 +459,28 @@ def test_split_contractions_with_a_last_chunk_shorter_than_a_piece():
     assert p.stderr.count("loads by pieces") == 16 and "loads by elements" not in p.stderr
 
 
+PLANS = r"""
+import torch
+from neuzephyr_amd import capi
+for M, K, N in ((33, 512, 33), (63, 512, 61), (64, 512, 10), (10, 512, 10), (10, 4096, 10), (10, 260100, 16)):
+    capi.gemm(torch.zeros(M, K, device="cuda"), torch.zeros(N, K, device="cuda"), b_trans=True)
+"""
+
+
+def test_one_tile_products_are_split_by_their_length_and_not_by_the_alignment_of_their_result():
+    import os
+    import re
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    p = subprocess.run([sys.executable, "-c", PLANS], capture_output=True, text=True, timeout=100, cwd=root,
+                       env={**os.environ, "NZHIP_TRACE": "1", "PYTHONPATH": root})
+    assert p.returncode == 0, p.stderr[-2000:]
+    chunks = [int(c) for c in re.findall(r"(\d+) chunk\(s\)", p.stderr)]
+    assert len(chunks) == 6 and chunks[:4] == [1] * 4               # too short to pay for a second launch
+    assert 8 <= chunks[4] <= 32 and 256 < chunks[5] <= 512           # two workgroups per compute unit for the longest
+
+
 @pytest.mark.parametrize("M,K,N,a_trans,b_trans,slack,offset,bias_form,seed", _embedded_cases())
 def test_embedded_operands_random_sweep(nz, M, K, N, a_trans, b_trans, slack, offset, bias_form, seed):
     # random shapes, layouts, leading dimensions and base offsets through the default route choice (streaming,
