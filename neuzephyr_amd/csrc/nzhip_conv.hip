@@ -206,7 +206,7 @@ __global__ __launch_bounds__(256) void conv3x3_direct_kernel(float* __restrict__
 }
 
 // ---- streaming variant of the direct route (C <= 4, O <= 2, 16-byte aligned rows) ----------
-// A wave owns a strip of 256 columns x ST_ROWS output rows and walks DOWN it: every input row
+// A wave owns a strip of 256 columns x up to ST_ROWS output rows and walks DOWN it: every input row
 // is requested once, ST_AHEAD rows ahead of its use, rounded to fp16 once, and kept in a
 // rolling window of three rows per channel; as soon as a row arrives, the output row above it
 // is complete and is computed in the reference's k order (c, r, s) and stored. Loads of later
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256) void conv3x3_direct_kernel(float* __restrict__
 // one extra 4-byte request per row and channel that every lane issues (the others re-read a word
 // of their own quad). PIX_BIAS: the bias varies per pixel and travels with the row ring; otherwise
 // it is absent or per channel and is fetched once.
-constexpr int ST_ROWS = 16, ST_AHEAD = 3;         // ST_AHEAD: a multiple of 3 (the window depth)
+constexpr int ST_ROWS = 16, ST_AHEAD = 3;         // the tallest strip; ST_AHEAD: a multiple of 3 (the window depth)
 
 // value of `v` in lane - 1 (lane 0 keeps its own)
 __device__ __forceinline__ float from_lane_below(float v) {
@@ -256,7 +256,7 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
                                                              const float* __restrict__ w_ref,
                                                              const float* __restrict__ bias, int H, int W,
                                                              long w_batch_stride, long bias_sp, long bias_sc,
-                                                             int relu, int mirror) {
+                                                             int relu, int mirror, int strip_rows) {
     static_assert(VEC || PIX_BIAS != 2 || O_T == 1, "runs of bias for several channels need aligned rows");
     __shared__ float wsm[C_T * 9 * O_T];
     int bx, by, b;
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int strip = by * 4 + wave;
-    const int h0 = strip * ST_ROWS;
+    const int h0 = strip * strip_rows;
     if (h0 >= H) {                                               // a whole wave with nothing to do but the workgroup's one barrier
         park_weights();
         return;
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
     const bool has_l = w0 > 0, has_r = w0 + 4 < W;
     // column of the extra request: left halo for the first lane, right halo for the last, else own quad
     const int wx = lane == 0 ? (has_l ? w0 - 1 : w0) : (lane == 63 && has_r ? w0 + 4 : w0);
-    const int rows = (H - h0) < ST_ROWS ? (H - h0) : ST_ROWS;   // output rows of this strip
+    const int rows = (H - h0) < strip_rows ? (H - h0) : strip_rows;   // output rows of this strip
     const int T = rows + 2;                                      // input rows h0-1 .. h0+rows
     // Odd strips walk upwards. A strip shares its first and its last input rows with its neighbours;
     // with alternating directions both neighbours touch a shared row at the same moment (both at the
@@ -451,6 +451,23 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
     else walk(std::false_type{});
 }
 
+// Rows of a strip of the streaming kernels. A strip reads two rows more than it owns, so tall ones move fewer bytes; but its rows
+// are a serial chain of about 0.8 us each, and a strip is all the work a wave has. The tallest that still makes `strips_per_cu`:
+// 4.5 for the forward (a wave per SIMD and some), 2.5 for the weight gradient, whose waves do more per row. In us with strips of
+//                                        1     2     4     8     16 rows
+//   forward  2 x 3 x 50 x 50             5.6   5.5   6.5   9.4   14.9
+//            8 x 4 x 255 x 255 -> 2      17.6  11.6  15.1  22.0  35.2
+//            10 x 3 x 500 x 655          34.5  22.2  17.7  14.7  17.9
+//            16 x 3 x 600 x 601          58.4  37.8  30.1  25.5  21.8
+//   weights  16 x 4 x 57 x 57 -> 2       21.8  23.2  24.0  28.2  34.4
+//            10 x 3 x 300 x 300          27.3  19.0  15.9  15.7  18.3
+//            10 x 3 x 500 x 655          57.8  41.9  28.7  22.8  20.7
+static int stream_strip_rows(size_t N, size_t H, size_t W, int least, double strips_per_cu) {
+    int rows = ST_ROWS;
+    while (rows > least && (double)N * (double)((W + 255) / 256) * (double)((H + rows - 1) / rows) < strips_per_cu * device_cu_count()) rows /= 2;
+    return rows;
+}
+
 static bool conv_direct_applicable(size_t C, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad) {
     return K_h == 3 && K_w == 3 && stride == 1 && pad == 1 && C <= DC_MAX_C && O <= DC_MAX_O && O >= 1;
 }
@@ -462,13 +479,14 @@ static int conv_direct(float* y, const float* x, const float* w_ref, const float
     dim3 grid((unsigned)((W + 255) / 256), (unsigned)((H + 4 * DC_ROWS - 1) / (4 * DC_ROWS)), (unsigned)N);
     const long wbs = w_batch > 1 ? (long)(C * 9 * O) : 0;
     if (C <= 4 && O <= 2 && H >= 8 && W >= 4) {
-        dim3 sgrid((unsigned)((W + 255) / 256), (unsigned)((H + 4 * ST_ROWS - 1) / (4 * ST_ROWS)), (unsigned)N);
+        const int strip_rows = stream_strip_rows(N, H, W, 2, 4.5);
+        dim3 sgrid((unsigned)((W + 255) / 256), (unsigned)((H + 4 * strip_rows - 1) / (4 * strip_rows)), (unsigned)N);
         const bool pixb = bias && bias_sp != 0;
         // the reference's Bias node: [pixel][channel], so the bias of a lane's 4 pixels is one aligned run
         const bool pixlayout = pixb && bias_sp == (int64_t)O && bias_sc == 1, pixrun = pixlayout && (reinterpret_cast<uintptr_t>(bias) & 15) == 0;
 #define NZHIP_STK(OT, CT, PB, V)                                                                                      \
     hipLaunchKernelGGL((conv3x3_stream_kernel<OT, CT, PB, V>), sgrid, dim3(256), 0, s, y, x, w_ref, bias, (int)H, (int)W, wbs, \
-                       (long)bias_sp, (long)bias_sc, act == NZHIP_ACT_RELU, w_mirror ? 1 : 0)
+                       (long)bias_sp, (long)bias_sc, act == NZHIP_ACT_RELU, w_mirror ? 1 : 0, strip_rows)
 #define NZHIP_ST(OT, CT)                                                                                             \
     do {                                                                                                             \
         if (vec && pixrun) NZHIP_STK(OT, CT, 2, true);                                                                \
@@ -2645,7 +2663,7 @@ __global__ __launch_bounds__(256) void conv_dw_reduce_few_kernel(float* __restri
 // ---- weight gradient of the 3x3, stride 1, pad 1 convolution with a handful of channels -------------
 // With C <= 4 and O <= 2 the gradient has at most 72 entries per weight copy, each a sum over every pixel:
 // a stream over x and dy, not a matrix product. Same thread mapping as the forward stream kernel (a lane
-// owns 4 adjacent columns of a 16-row strip, three rounded x rows in a rolling register window, halo
+// owns 4 adjacent columns of a strip of rows, three rounded x rows in a rolling register window, halo
 // columns from the neighbour lanes), and C*9*O running sums per lane:
 //     acc[(c, r, s)][o] += f16(x[c][h + r - 1][w + s - 1]) * f16(dy[o][h][w]).
 // A wave adds its lanes in a fixed tree and writes one partial vector per strip; small_dw_reduce_kernel
@@ -2664,14 +2682,14 @@ __global__ __launch_bounds__(256) void conv_dw_reduce_few_kernel(float* __restri
 // channels, two waves per SIMD instead of three) 10 x 3 x 1000 x 1023 took 43.8 us, with one (158) 37.9, as without the masks.
 template <int O_T, int C_T, bool VEC, int REM>
 __global__ __launch_bounds__(256) void conv3x3_dw_stream_kernel(float* __restrict__ partial, const float* __restrict__ x,
-                                                                const float* __restrict__ dy, int H, int W) {
+                                                                const float* __restrict__ dy, int H, int W, int strip_rows) {
     static_assert(REM >= 0 && REM < 4 && (!VEC || REM == 0), "aligned rows end with a whole quad");
     constexpr int Q = C_T * 9 * O_T, AHEAD = 3;
     int bx, by, b;
     xcd_contiguous_block(bx, by, b);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int strip = by * 4 + wave, n_strips = gridDim.y * 4;
-    const int h0 = strip * ST_ROWS;
+    const int h0 = strip * strip_rows;
     float acc[Q];
 #pragma unroll
     for (int q = 0; q < Q; q++) acc[q] = 0.f;
@@ -2687,7 +2705,7 @@ __global__ __launch_bounds__(256) void conv3x3_dw_stream_kernel(float* __restric
         const float* xb = x + (long)b * C_T * H * W;
         const float* gb = dy + (long)b * O_T * H * W;
         const long plane = (long)H * W;
-        const int rows = (H - h0) < ST_ROWS ? (H - h0) : ST_ROWS;
+        const int rows = (H - h0) < strip_rows ? (H - h0) : strip_rows;
         const int T = rows + 2;
         auto walk = [&](auto upwards) {
             constexpr bool UP = decltype(upwards)::value;
@@ -4133,7 +4151,8 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
     if (C <= 4 && O <= 2) {
         const bool pieces = W % 4 == 0 && ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dy)) & 15) == 0;
         // a handful of channels: stream x and dy once, C*9*O running sums per lane
-        dim3 grid((unsigned)((W + 255) / 256), (unsigned)((H + 4 * ST_ROWS - 1) / (4 * ST_ROWS)), (unsigned)N);
+        const int strip_rows = stream_strip_rows(N, H, W, 1, 2.5);
+        dim3 grid((unsigned)((W + 255) / 256), (unsigned)((H + 4 * strip_rows - 1) / (4 * strip_rows)), (unsigned)N);
         const size_t Q = C * 9 * O, per_image = (size_t)grid.x * grid.y * 4;
         if (per_image * N > 0x7fffffffull) return set_error(NZHIP_E_UNSUPPORTED, "nzhip_conv2d_backward_weights: too many strips");
         float* partial = nullptr;
@@ -4144,7 +4163,7 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
                         : W % 4 == 1 ? conv3x3_dw_stream_kernel<OT, CT, false, 1>                                        \
                         : W % 4 == 2 ? conv3x3_dw_stream_kernel<OT, CT, false, 2>                                        \
                                      : conv3x3_dw_stream_kernel<OT, CT, false, 3>),                                      \
-                       grid, dim3(256), 0, s, partial, x, dy, (int)H, (int)W)
+                       grid, dim3(256), 0, s, partial, x, dy, (int)H, (int)W, strip_rows)
         switch ((int)(O * 10 + C)) {
             case 11: NZHIP_DWS(1, 1); break;
             case 12: NZHIP_DWS(1, 2); break;

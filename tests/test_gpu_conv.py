@@ -383,10 +383,10 @@ def test_config4b_conv_memory_bound_single_channel_out(nz, oracle):
 
 
 @pytest.mark.parametrize("O,C,bias", [(1, 3, "pixel"), (2, 4, "channel"), (1, 1, "none"), (2, 1, "pixel")])
-@pytest.mark.parametrize("H,W", [(8, 5), (17, 254), (33, 255), (16, 257), (66, 259), (19, 512), (9, 1)])
+@pytest.mark.parametrize("H,W", [(8, 5), (17, 254), (33, 255), (16, 257), (66, 259), (19, 512), (9, 1), (1201, 6), (2399, 8), (4799, 5), (6150, 4)])
 def test_thin_layers_on_rows_of_any_width_forward_and_gradients(nz, H, W, O, C, bias):
     """The row-streaming kernels (up to four channels in, two out) on rows that are and are not whole 16-byte pieces, quads cut by
-    the end of the row, one and several 256-column blocks, whole and partial 16-row strips walked both ways, mirrored weights:
+    the end of the row, one and several 256-column blocks, whole and partial strips of 1 to 16 rows walked both ways, mirrored weights:
     integers, so exact whatever the order of the sums."""
     import torch
     import torch.nn.functional as F
