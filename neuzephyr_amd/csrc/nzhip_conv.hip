@@ -250,13 +250,14 @@ __device__ __forceinline__ void load_ragged_quad(const float* row, int at, int b
 // addresses, which the memory path takes at nearly the aligned rate: 10 x 3 x 1000 x 1023 -> 1 42 us against 39 for 1024
 // columns. (83 us on the four-row blocks of the direct kernel, which re-reads half its rows element by element; 72 us with
 // this kernel's quads as four 4-byte accesses each.) The quad cut by the end of the row is moved left into it and turned back.
-// mirror: the weights are those of the convolution whose data gradient this is (weight_source_index).
-template <int O_T, int C_T, int PIX_BIAS, bool VEC>
+// MIRROR: the weights are those of the convolution whose data gradient this is (weight_source_index); no bias per pixel then.
+template <int O_T, int C_T, int PIX_BIAS, bool VEC, bool MIRROR>
 __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__ y, const float* __restrict__ x,
                                                              const float* __restrict__ w_ref,
                                                              const float* __restrict__ bias, int H, int W,
                                                              long w_batch_stride, long bias_sp, long bias_sc,
-                                                             int relu, int mirror, int strip_rows) {
+                                                             int relu, int strip_rows) {
+    __builtin_assume(strip_rows >= 1 && strip_rows <= ST_ROWS);
     static_assert(VEC || PIX_BIAS != 2 || O_T == 1, "runs of bias for several channels need aligned rows");
     __shared__ float wsm[C_T * 9 * O_T];
     int bx, by, b;
@@ -265,8 +266,7 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
     static_assert(C_T * 9 * O_T <= 128, "one weight per thread");
     // requested now, parked in LDS after the first input rows have been requested (the rows then do not
     // queue up behind the round trip of the weights)
-    long w_i = threadIdx.x;
-    if (mirror) w_i = weight_source_index(threadIdx.x / (9 * O_T), threadIdx.x / O_T % 9, threadIdx.x % O_T, C_T, O_T, 9, 1);
+    const long w_i = MIRROR ? weight_source_index(threadIdx.x / (9 * O_T), threadIdx.x / O_T % 9, threadIdx.x % O_T, C_T, O_T, 9, 1) : threadIdx.x;
     const float w_mine = threadIdx.x < C_T * 9 * O_T ? wb[w_i] : 0.f;
     auto park_weights = [&]() {
         if (threadIdx.x < C_T * 9 * O_T) wsm[threadIdx.x] = round_f16(w_mine);   // [q][o]
@@ -283,7 +283,9 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
     // Lanes past the last column stay in the walk (the barrier in park_weights() must not sit in a branch that
     // only some lanes of a wave take): they work on the image's last quad of columns and store nothing.
     const bool active = (bx * 64 + lane) * 4 < W;
-    const int w0 = active ? (bx * 64 + lane) * 4 : (W - 1) / 4 * 4;
+    // (VEC spelled out here and where rows are rounded: left to the general expressions the aligned instance schedules its requests
+    // differently, 10 x 3 x 1024 x 1024 -> 1 40.1 instead of 39.8 us)
+    const int w0 = active ? (bx * 64 + lane) * 4 : VEC ? W - 4 : (W - 1) / 4 * 4;
     bool col[4];                                                 // the lane's columns inside the row
 #pragma unroll
     for (int e = 0; e < 4; e++) col[e] = VEC || w0 + e < W;
@@ -382,7 +384,7 @@ __global__ __launch_bounds__(256) void conv3x3_stream_kernel(float* __restrict__
                     // load and the wave waits for every row as soon as it has asked for it.
                     float v = raw[u][c][e];
                     asm volatile("" : "+v"(v));
-                    r5[e] = in_img && (e == 4 || col[e == 4 ? 0 : e]) ? round_f16(v) : 0.f;
+                    r5[e] = in_img && (VEC || e == 4 || col[e == 4 ? 0 : e]) ? round_f16(v) : 0.f;
                 }
                 const float below = from_lane_below(r5[3]), above = from_lane_above(r5[0]);
                 win[wu][c][0] = has_l ? (lane == 0 ? r5[4] : below) : 0.f;
@@ -482,19 +484,22 @@ static int conv_direct(float* y, const float* x, const float* w_ref, const float
         const int strip_rows = stream_strip_rows(N, H, W, 2, 4.5);
         dim3 sgrid((unsigned)((W + 255) / 256), (unsigned)((H + 4 * strip_rows - 1) / (4 * strip_rows)), (unsigned)N);
         const bool pixb = bias && bias_sp != 0;
+        if (w_mirror && pixb) return set_error(NZHIP_E_UNSUPPORTED, "conv_direct: mirrored weights with a bias per pixel");
         // the reference's Bias node: [pixel][channel], so the bias of a lane's 4 pixels is one aligned run
         const bool pixlayout = pixb && bias_sp == (int64_t)O && bias_sc == 1, pixrun = pixlayout && (reinterpret_cast<uintptr_t>(bias) & 15) == 0;
-#define NZHIP_STK(OT, CT, PB, V)                                                                                      \
-    hipLaunchKernelGGL((conv3x3_stream_kernel<OT, CT, PB, V>), sgrid, dim3(256), 0, s, y, x, w_ref, bias, (int)H, (int)W, wbs, \
-                       (long)bias_sp, (long)bias_sc, act == NZHIP_ACT_RELU, w_mirror ? 1 : 0, strip_rows)
+#define NZHIP_STK(OT, CT, PB, V, MI)                                                                                  \
+    hipLaunchKernelGGL((conv3x3_stream_kernel<OT, CT, PB, V, MI>), sgrid, dim3(256), 0, s, y, x, w_ref, bias, (int)H, (int)W, wbs, \
+                       (long)bias_sp, (long)bias_sc, act == NZHIP_ACT_RELU, strip_rows)
 #define NZHIP_ST(OT, CT)                                                                                             \
     do {                                                                                                             \
-        if (vec && pixrun) NZHIP_STK(OT, CT, 2, true);                                                                \
-        else if (vec && pixb) NZHIP_STK(OT, CT, 1, true);                                                             \
-        else if (vec) NZHIP_STK(OT, CT, 0, true);                                                                     \
-        else if (OT == 1 && pixlayout) NZHIP_STK(OT, CT, OT == 1 ? 2 : 1, false);                                     \
-        else if (pixb) NZHIP_STK(OT, CT, 1, false);                                                                   \
-        else NZHIP_STK(OT, CT, 0, false);                                                                             \
+        if (w_mirror && vec) NZHIP_STK(OT, CT, 0, true, true);                                                        \
+        else if (w_mirror) NZHIP_STK(OT, CT, 0, false, true);                                                         \
+        else if (vec && pixrun) NZHIP_STK(OT, CT, 2, true, false);                                                    \
+        else if (vec && pixb) NZHIP_STK(OT, CT, 1, true, false);                                                      \
+        else if (vec) NZHIP_STK(OT, CT, 0, true, false);                                                              \
+        else if (OT == 1 && pixlayout) NZHIP_STK(OT, CT, OT == 1 ? 2 : 1, false, false);                              \
+        else if (pixb) NZHIP_STK(OT, CT, 1, false, false);                                                            \
+        else NZHIP_STK(OT, CT, 0, false, false);                                                                      \
     } while (0)
         switch ((int)(O * 10 + C)) {
             case 11: NZHIP_ST(1, 1); break;
@@ -2683,6 +2688,7 @@ __global__ __launch_bounds__(256) void conv_dw_reduce_few_kernel(float* __restri
 template <int O_T, int C_T, bool VEC, int REM>
 __global__ __launch_bounds__(256) void conv3x3_dw_stream_kernel(float* __restrict__ partial, const float* __restrict__ x,
                                                                 const float* __restrict__ dy, int H, int W, int strip_rows) {
+    __builtin_assume(strip_rows >= 1 && strip_rows <= ST_ROWS);
     static_assert(REM >= 0 && REM < 4 && (!VEC || REM == 0), "aligned rows end with a whole quad");
     constexpr int Q = C_T * 9 * O_T, AHEAD = 3;
     int bx, by, b;
