@@ -3457,33 +3457,33 @@ namespace nzhip {
 // MASK: dz is not given but made here, dz[n][o][p] = y[n][o][p] > 0 ? dy[n][o][p] : 0 (the gradient through the ReLU
 // that follows the convolution, ReLUNode::backward), written out for the other gradient kernels and summed on the way.
 //
-// A workgroup owns 256 V / TO pixels x TO channels, a thread V adjacent pixels of one channel; with more than one channel
-// the tile of dbias is turned in LDS on the way in and on the way out, with one channel dbias and dz have the same layout
-// and LDS is not used. Bound by memory: the loads of eight images are requested before the first is added. (A fixed tile
-// of 64 pixels x 32 channels left 31 of 32 threads idle for one channel and gave a 14 x 14 layer 32 workgroups:
-// 10 x 1 x 1024 x 1024 54 -> 9.6 us (4.8 TB/s), masked 72 -> 22; 16 x 256 x 14 x 14 masked 17 -> 5.5, 16 x 128 x 28 x 28 masked 23 -> 7.5.)
-template <bool MASK, int V, int TO>
+// A workgroup owns TP pixels x TO channels, a thread V adjacent pixels of R channels; with more than one channel the tile
+// of dbias is turned in LDS on the way in and on the way out, with one channel dbias and dz have the same layout and LDS is
+// not used. Bound by memory: the loads of several images are requested before the first is added, those of the tile of dbias
+// before the first is parked. (A fixed tile of 64 pixels x 32 channels left 31 of 32 threads idle for one channel and gave a 14 x 14
+// layer 32 workgroups: 10 x 1 x 1024 x 1024 54 -> 9.6 us (4.8 TB/s), masked 72 -> 22; 16 x 256 x 14 x 14 masked 17 -> 5.5,
+// 16 x 128 x 28 x 28 masked 23 -> 7.5.)
+template <bool MASK, int V, int TP, int TO>
 __global__ __launch_bounds__(256) void conv_bias_grad_kernel(float* __restrict__ dbias, const float* __restrict__ dz, int N,
                                                              int O, long HW, float* __restrict__ dz_out,
                                                              const float* __restrict__ y, int pixel_folds) {
-    constexpr int TP = 256 * V / TO, PT = TP / V;                // pixels of the tile; threads along them
-    constexpr int U = 8;                                         // images in flight
+    constexpr int PT = TP / V, OT = 256 / PT, R = TO / OT;       // threads along the pixels and the channels; channels a thread
+    constexpr int U = R > 4 || (MASK && R > 1) ? 2 : R > 1 ? 4 : 8;      // images in flight
+    static_assert(R >= 1 && R * OT == TO && PT * OT == 256, "whole threads");
     __shared__ float tile[TO > 1 ? TP : 1][TO + 1];              // [pixel][channel]
-    const long p0 = ((long)(blockIdx.z % pixel_folds) * gridDim.x + blockIdx.x) * TP;
-    const long o0 = ((long)(blockIdx.z / pixel_folds) * gridDim.y + blockIdx.y) * TO;
-    if (p0 >= HW || o0 >= O) return;
+    long p0 = (long)blockIdx.x * TP, o0 = (long)blockIdx.y * TO;
+    if (pixel_folds) {                                           // (0: none; the grid's own extents are a trip to memory more)
+        p0 += (long)(blockIdx.z % pixel_folds) * gridDim.x * TP;
+        o0 += (long)(blockIdx.z / pixel_folds) * gridDim.y * TO;
+        if (p0 >= HW || o0 >= O) return;
+    }
     const int px = (threadIdx.x % PT) * V, oc = threadIdx.x / PT;
     const long p = p0 + px;
-    const bool live = p < HW && o0 + oc < O;                     // V == 4: HW % 4 == 0, the four pixels are inside together
-    auto turn = [&](auto&& element) {                            // channels fastest, as dbias lies
-        constexpr int ROWS = 256 / TO;
-        const int tx = threadIdx.x % TO, ty = threadIdx.x / TO;
+    bool live[R];                                                // V == 4: HW % 4 == 0, the four pixels are inside together
 #pragma unroll
-        for (int r = 0; r < TP; r += ROWS) {
-            const long pp = p0 + ty + r;
-            if (pp < HW && o0 + tx < O) element(dbias[pp * O + o0 + tx], tile[ty + r][tx]);
-        }
-    };
+    for (int r = 0; r < R; r++) live[r] = p < HW && o0 + oc + r * OT < O;
+    constexpr int ROWS = 256 / TO;                               // dbias lies with the channels fastest
+    const int tx = threadIdx.x % TO, ty = threadIdx.x / TO;
     auto load = [&](const float* src, float (&v)[V]) {
         if constexpr (V == 4) {
             const floatx4 q = *reinterpret_cast<const floatx4*>(src);
@@ -3497,55 +3497,84 @@ __global__ __launch_bounds__(256) void conv_bias_grad_kernel(float* __restrict__
         if constexpr (V == 4) *reinterpret_cast<floatx4*>(dst) = floatx4{v[0], v[1], v[2], v[3]};
         else *dst = v[0];
     };
-    float acc[V];
+    float acc[R][V];
     if constexpr (TO > 1) {
-        turn([](float& d, float& t) { t = d; });
+        const long o = o0 + tx < O ? o0 + tx : O - 1;            // elements past the edges are copies of one inside: no test between the loads
+        float v[TP / ROWS];
+#pragma unroll
+        for (int r = 0; r < TP / ROWS; r++) {
+            const long pp = p0 + ty + r * ROWS;
+            v[r] = dbias[(pp < HW ? pp : HW - 1) * O + o];
+        }
+#pragma unroll
+        for (int r = 0; r < TP / ROWS; r++) tile[ty + r * ROWS][tx] = v[r];
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < V; e++) acc[e] = tile[px + e][oc];
-    } else if (live) {
-        load(dbias + p, acc);
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int e = 0; e < V; e++) acc[r][e] = tile[px + e][oc + r * OT];
+    } else if (live[0]) {
+        load(dbias + p, acc[0]);
     }
-    if (live) {
-        const long image = (long)O * HW, at0 = (long)(o0 + oc) * HW + p;
+    if (live[0]) {
+        const long image = (long)O * HW;
+        long at0[R];                                             // a channel past the last one re-reads the thread's first
+#pragma unroll
+        for (int r = 0; r < R; r++) at0[r] = (o0 + oc + (live[r] ? r * OT : 0)) * HW + p;
         auto some = [&](const int n0, auto count) {
             constexpr int C = decltype(count)::value;
-            float g[C][V], yy[MASK ? C : 1][V];
+            float g[C][R][V], yy[MASK ? C : 1][R][V];
 #pragma unroll
-            for (int u = 0; u < C; u++) {
-                load(dz + (long)(n0 + u) * image + at0, g[u]);
-                if constexpr (MASK) load(y + (long)(n0 + u) * image + at0, yy[u]);
-            }
+            for (int u = 0; u < C; u++)
 #pragma unroll
-            for (int u = 0; u < C; u++) {
-                if constexpr (MASK) {
-#pragma unroll
-                    for (int e = 0; e < V; e++) g[u][e] = yy[u][e] > 0.f ? g[u][e] : 0.f;
-                    store(dz_out + (long)(n0 + u) * image + at0, g[u]);
+                for (int r = 0; r < R; r++) {
+                    load(dz + (long)(n0 + u) * image + at0[r], g[u][r]);
+                    if constexpr (MASK) load(y + (long)(n0 + u) * image + at0[r], yy[u][r]);
                 }
 #pragma unroll
-                for (int e = 0; e < V; e++) acc[e] += g[u][e];
-            }
+            for (int u = 0; u < C; u++)
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    if constexpr (MASK) {
+#pragma unroll
+                        for (int e = 0; e < V; e++) g[u][r][e] = yy[u][r][e] > 0.f ? g[u][r][e] : 0.f;
+                        if (live[r]) store(dz_out + (long)(n0 + u) * image + at0[r], g[u][r]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < V; e++) acc[r][e] += g[u][r][e];
+                }
         };
         int n = 0;
         for (; n + U <= N; n += U) some(n, std::integral_constant<int, U>{});
-        for (; n + 2 <= N; n += 2) some(n, std::integral_constant<int, 2>{});
-        if (n < N) some(n, std::integral_constant<int, 1>{});
+        for (; U > 2 && n + 2 <= N; n += 2) some(n, std::integral_constant<int, 2>{});
+        for (; n < N; n++) some(n, std::integral_constant<int, 1>{});
     }
     if constexpr (TO > 1) {
         __syncthreads();
 #pragma unroll
-        for (int e = 0; e < V; e++) tile[px + e][oc] = acc[e];
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int e = 0; e < V; e++) tile[px + e][oc + r * OT] = acc[r][e];
         __syncthreads();
-        turn([](float& d, float& t) { d = t; });
-    } else if (live) {
-        store(dbias + p, acc);
+#pragma unroll
+        for (int r = 0; r < TP / ROWS; r++) {
+            const long pp = p0 + ty + r * ROWS;
+            if (pp < HW && o0 + tx < O) dbias[pp * O + o0 + tx] = tile[ty + r * ROWS][tx];
+        }
+    } else if (live[0]) {
+        store(dbias + p, acc[0]);
     }
 }
 
-// Which tile: one channel needs no turning; up to four channels take a tile of four; beyond that 32 x 32 elements with
-// 16-byte accesses when that still gives every compute unit two workgroups, else 32 pixels x 8 channels, a pixel a thread,
-// for four times the workgroups.
+// Which tile: one channel needs no turning; up to four channels take a tile of four. Beyond that small layers take 32 pixels x 8
+// channels, a pixel a thread, for the most workgroups; from 1024 elements per compute unit on runs of 64 or 128 pixels pay,
+// and with one or two images, where dbias is as much traffic as dz, runs of 32 channels. In us, unmasked and masked, 32 x 8 (or
+// 32 x 32 with 16-byte accesses) for all of these, and as chosen:
+//   16 x 64 x 223 x 223   66, 199 -> 43, 159     16 x 8 x 511 x 511    40, 128 -> 31, 102    2 x 64 x 223 x 223   23.8, 31.9 -> 10.5, 22.4
+//   16 x 256 x 113 x 113  62, 201 -> 42, 159     16 x 32 x 113 x 113   8.7, 23.4 -> 7.2, 17.6
+//   16 x 64 x 224 x 224   36, 144 -> 35, 132     16 x 8 x 224 x 224    3.5, 13.8 -> 3.5, 13.6
+// (16 x 256 x 112 x 112 unmasked is level, 35.2 and 35.7; 33.8 with 64 pixels x 32 channels and two images in flight, which costs
+// the others more.)
 template <bool MASK>
 static int conv_bias_grad_launch(float* dbias, const float* dz, size_t N, size_t O, size_t HW, float* dz_out, const float* y,
                                  hipStream_t s) {
@@ -3559,13 +3588,16 @@ static int conv_bias_grad_launch(float* dbias, const float* dz, size_t N, size_t
         const size_t ty = (O + to - 1) / to, gy = std::min<size_t>(ty, 65535), zy = (ty + gy - 1) / gy;
         if (zx * zy > 65535) return set_error(NZHIP_E_UNSUPPORTED, "conv bias gradient: extent too large");
         hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)gy, (unsigned)(zx * zy)), dim3(256), 0, s, dbias, dz, (int)N, (int)O,
-                           (long)HW, dz_out, y, (int)zx);
+                           (long)HW, dz_out, y, zx * zy > 1 ? (int)zx : 0);
         hipError_t e = hipGetLastError();
         return e == hipSuccess ? NZHIP_OK : set_hip_error(e, "conv_bias_grad kernel launch");
     };
-    if (O == 1) return vec && many ? go(conv_bias_grad_kernel<MASK, 4, 1>, 1024, 1) : go(conv_bias_grad_kernel<MASK, 1, 1>, 256, 1);
-    if (O <= 4) return vec && many ? go(conv_bias_grad_kernel<MASK, 4, 4>, 256, 4) : go(conv_bias_grad_kernel<MASK, 1, 4>, 64, 4);
-    return vec && many ? go(conv_bias_grad_kernel<MASK, 4, 32>, 32, 32) : go(conv_bias_grad_kernel<MASK, 1, 8>, 32, 8);
+    if (O == 1) return vec && many ? go(conv_bias_grad_kernel<MASK, 4, 1024, 1>, 1024, 1) : go(conv_bias_grad_kernel<MASK, 1, 256, 1>, 256, 1);
+    if (O <= 4) return vec && many ? go(conv_bias_grad_kernel<MASK, 4, 256, 4>, 256, 4) : go(conv_bias_grad_kernel<MASK, 1, 64, 4>, 64, 4);
+    if (HW * O < (size_t)device_cu_count() * 1024) return go(conv_bias_grad_kernel<MASK, 1, 32, 8>, 32, 8);
+    if (vec) return N <= 2 ? go(conv_bias_grad_kernel<MASK, 4, 32, 32>, 32, 32) : go(conv_bias_grad_kernel<MASK, 4, 64, 16>, 64, 16);
+    if (O <= 8) return go(conv_bias_grad_kernel<MASK, 1, 128, 8>, 128, 8);
+    return N <= 2 ? go(conv_bias_grad_kernel<MASK, 1, 64, 32>, 64, 32) : go(conv_bias_grad_kernel<MASK, 1, 128, 16>, 128, 16);
 }
 
 }  // namespace nzhip

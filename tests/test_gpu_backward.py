@@ -526,7 +526,8 @@ def test_conv2d_backward_relu_bias_equals_relu_backward_then_bias(nz, oracle, N,
 
 
 @pytest.mark.parametrize("N,O,H,W", [(11, 1, 512, 1028), (2, 1, 513, 1028), (3, 1, 37, 41), (9, 3, 420, 420), (10, 33, 128, 130),
-                                     (3, 33, 130, 130), (17, 34, 9, 14), (8, 4, 5, 13)])
+                                     (3, 33, 130, 130), (17, 34, 9, 14), (8, 4, 5, 13), (5, 18, 121, 124), (2, 37, 90, 92), (7, 7, 203, 197),
+                                     (2, 41, 83, 81), (5, 21, 113, 115), (4, 16, 131, 129)])
 def test_conv2d_bias_gradients_on_every_tile_shape(nz, oracle, N, O, H, W):
     """One, up to four and more channels, with and without 16-byte accesses, image counts around the eight in flight, edges in
     both directions: one chain per element, so bit for bit."""
