@@ -150,14 +150,15 @@ def shape4(s) -> C.Array:
 # Torch-facing helpers. torch is used for device memory and streams only.
 # --------------------------------------------------------------------------------------------
 def _stream_handle(stream=None) -> int:
-    """The hipStream_t a call goes to. For the current stream the handle is asked for directly: building the Stream object around
-    it costs 2.7 us, a third of a small call (relu_backward of 256 elements: 8.4 -> 6.0 us on the host)."""
+    """The hipStream_t a call goes to. For the current stream the handle is asked for directly where this torch has a function for it:
+    building the Stream object around it costs 2.7 us, a third of a small call (relu_backward of 256 elements: 8.4 -> 6.0 us on the host)."""
     import torch
     if stream is not None:
         return int(stream.cuda_stream)
-    if not torch.cuda.is_initialized():
-        torch.cuda.init()
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)       # not part of torch's public interface
+    if raw is None:
+        return int(torch.cuda.current_stream().cuda_stream)
+    return raw(torch.cuda.current_device())
 
 
 def _dev(t):

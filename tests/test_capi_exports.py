@@ -32,3 +32,14 @@ def test_python_plumbing_never_touches_the_oracle():
     for name in ("capi.py", "__init__.py", "build.py"):
         src = open(os.path.join(ROOT, "neuzephyr_amd", name)).read()
         assert "import oracle" not in src and "from oracle" not in src and "nz_oracle" not in src
+
+
+def test_stream_handle_without_torch_s_private_function(monkeypatch):
+    """A torch without the direct way to the current stream's handle: the public one answers."""
+    import types
+    import torch
+    from neuzephyr_amd import capi
+    monkeypatch.setattr(torch, "_C", types.SimpleNamespace())
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=1234))
+    assert capi._stream_handle() == 1234
+    assert capi._stream_handle(types.SimpleNamespace(cuda_stream=77)) == 77
