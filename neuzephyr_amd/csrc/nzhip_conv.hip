@@ -4177,6 +4177,18 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
         const int rc = fits ? conv_dw_generic(dw, x, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch == 1,
                                               reinterpret_cast<hipStream_t>(stream))
                             : NZHIP_E_UNSUPPORTED;
+        if (rc == NZHIP_E_UNSUPPORTED && K_h == 3 && K_w == 3 && stride == 1 && pad == 1 && C <= 4 && O <= 2 && W < 4 && H <= 0x3fffffff && N <= 65535) {
+            // thin layers of one to three columns and more rows than the gather kernel's offsets hold: four columns for the streaming kernel
+            hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+            float* x_wide = nullptr;
+            float* dy_wide = nullptr;
+            int wrc = widen_rows(&x_wide, x, N * C * H, W, s);
+            if (wrc == NZHIP_OK) wrc = widen_rows(&dy_wide, dy, N * O * H, W, s);
+            if (wrc == NZHIP_OK) wrc = nzhip_conv2d_backward_weights(dw, x_wide, dy_wide, N, C, H, 4, O, 3, 3, 1, 1, w_batch, stream);
+            const int rc2 = dy_wide ? workspace_free(dy_wide, s) : NZHIP_OK;
+            const int rc3 = x_wide ? workspace_free(x_wide, s) : NZHIP_OK;
+            return wrc ? wrc : (rc2 ? rc2 : rc3);
+        }
         if (rc == NZHIP_E_UNSUPPORTED)
             return set_error(NZHIP_E_UNSUPPORTED,
                              "nzhip_conv2d_backward_weights: more than 128 taps, a stride above 4 or extents beyond the fused kernels (use the column-matrix chain)");

@@ -574,6 +574,23 @@ def test_conv2d_bias_gradient_of_an_image_beyond_32_bit_thread_counts(nz):
         assert torch.equal(db[0, 0, p:p + (1 << 27)].t(), dz[0, :, 0, p:p + (1 << 27)])
 
 
+def test_thin_weight_gradient_of_three_columns_and_more_rows_than_the_gather_kernel_s_offsets_hold(nz):
+    import torch
+    C, H, W = 4, 180_000_000, 3
+    x, dy = torch.zeros(1, C, H, W, device="cuda"), torch.zeros(1, 1, H, W, device="cuda")
+    want = torch.zeros(C, 3, 3)
+    for k, (c, h, w) in enumerate(((0, 0, 0), (1, 5, 2), (2, 90_000_017, 1), (3, H - 1, 2), (0, H - 1, 0))):
+        x[0, c, h, w] = k + 2.0
+    for h, w, g in ((0, 0, 3.0), (4, 1, 5.0), (90_000_018, 2, 7.0), (H - 1, 1, 11.0), (H - 2, 0, 13.0)):
+        dy[0, 0, h, w] = g
+        for r in range(3):
+            for s in range(3):
+                if 0 <= h + r - 1 < H and 0 <= w + s - 1 < W:
+                    want[:, r, s] += g * x[0, :, h + r - 1, w + s - 1].cpu()
+    dw = nz.conv2d_backward_weights(torch.zeros(1, 1, C * 9, 1, device="cuda"), x, dy, 3, 3, 1, 1)
+    assert torch.equal(dw.cpu().view(C, 3, 3), want) and want.abs().sum() > 0
+
+
 @pytest.mark.parametrize("special", [70000.0, float("inf"), float("nan")])
 @pytest.mark.parametrize("C,O", [(1, 1), (3, 1), (4, 2)])
 @pytest.mark.parametrize("W,offset", [(5, 0), (6, 0), (28, 0), (28, 1), (30, 0), (31, 0), (255, 0), (256, 0), (257, 0), (260, 0), (260, 1)])
