@@ -57,7 +57,7 @@ int nzhip_device_info(int* cu_count, size_t* lds_bytes_per_cu, char* arch_name, 
  * Cutting (src/OperationKernels.cu:821-871) and the per-(n,c) launch loops of
  * TensorCoreGEMMParallel (:914-1026); the fused bias/activation replaces
  * MatrixAddKernel (:12-24) and RectifiedLinearUnitKernel (:230-235).
- * Edges are predicated in-kernel: no padded copies exist.
+ * Edges are handled in-kernel: accesses are moved into the operands, no padded copies exist.
  * Strides are in elements; a batch stride of 0 broadcasts that operand.
  * bias may be NULL; its element for output (m,n) of batch (i,j) is
  *     bias[i*bias_stride_n_batch + j*bias_stride_c_batch + m*bias_stride_row + n*bias_stride_col]
@@ -97,7 +97,9 @@ int nzhip_gemm(const nzhip_gemm_desc* desc, void* stream);
  * NZHIP_STATIC_SCRATCH_BYTES that each GPU holds from library load until the process ends; the
  * call performs no hipMalloc / hipFree and never touches the caching pool.
  * A product whose workspace would not fit is rejected with NZHIP_E_UNSUPPORTED
- * (nzhip_last_error() names the size) and leaves C untouched.
+ * (nzhip_last_error() names the size) and leaves C untouched.  Partial sums of a split contraction
+ * that would not fit are made fewer instead: such a product's sums may be grouped differently from
+ * nzhip_gemm's (same tolerance, not the same last bits).
  * All calls on one GPU share that GPU's array: calls that overlap in time on one GPU (two
  * streams, two threads) race; serialise them. */
 #define NZHIP_STATIC_SCRATCH_BYTES ((size_t)32 << 20)

@@ -523,7 +523,10 @@ GemmPlan gemm_fused_plan(const nzhip_gemm_desc& d) {
     const FusedCostInput q = fused_cost_input(d);
     GemmPlan best = {128, 1, d.K, 0.0};
     double best_cost = fused_cost_us(q, 128, 1, d.K);
+    // in the call that allocates nothing the partial sums have to fit its scratch: fewer chunks, or none, instead of a refusal
+    const double most = (double)workspace_limit() / ((double)d.M * d.N * d.batch_n * sizeof(float));
     auto consider = [&](int tile, int64_t parts, int64_t Kc) {
+        if (parts > 1 && (double)parts > most) return;
         const double c = fused_cost_us(q, tile, parts, Kc);
         if (c < best_cost * 0.97) { best_cost = c; best = {tile, parts, Kc, 0.0}; }    // keep the plainer plan on a near tie
     };

@@ -47,6 +47,7 @@ int gemm_thin_dispatch(const nzhip_gemm_desc& d, hipStream_t stream);
 
 // Stream-ordered workspace from the caching allocator (nzhip_runtime.cpp).
 int workspace_alloc(void** ptr, size_t bytes, hipStream_t stream);
+size_t workspace_limit();                        // bytes a workspace may have: what is left of the static scratch inside nzhip_gemm_static
 int workspace_free(void* ptr, hipStream_t stream);
 
 // ---- prepared operand images (nzhip_prepared) -------------------------------------------------------------

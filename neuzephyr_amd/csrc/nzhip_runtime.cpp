@@ -129,6 +129,8 @@ int workspace_alloc(void** ptr, size_t bytes, hipStream_t s) {
     return NZHIP_OK;
 }
 
+size_t workspace_limit() { return t_arena.active ? STATIC_SCRATCH_BYTES - t_arena.used : SIZE_MAX; }
+
 int workspace_free(void* ptr, hipStream_t s) {
     if (t_arena.active) return NZHIP_OK;                      // the arena is reset by the next call
     return Runtime::instance().pool().free_async(ptr, reinterpret_cast<uintptr_t>(s)) == 0

@@ -36,7 +36,7 @@ ROUTES = {
     "split contraction": [(256, 4096, 256), (128, 2048, 192)],
     "streamed skinny": [(1, 4096, 4096), (1, 1024, 512)],
     "two-pass fp16": [(3072, 768, 3072), (2000, 800, 2000)],
-    "padded operand copies": [(1000, 777, 513), (333, 331, 335)],
+    "ragged rows": [(1000, 777, 513), (333, 331, 335)],
     "no workspace": [(300, 100, 200), (17, 33, 15)],
 }
 
@@ -87,3 +87,13 @@ def test_static_entry_rejects_a_workspace_beyond_its_array(nz):
     got = torch.empty((256, 256), device="cuda")
     nz.gemm(a, b, out=got, static=True)
     assert torch.equal(got, nz.gemm(a, b))
+
+
+@pytest.mark.parametrize("M,K,N", [(320, 5728, 6400), (96, 21392, 6640)])
+def test_static_entry_splits_less_where_the_partial_sums_would_not_fit(nz, M, K, N):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M)
+    A, B = (torch.randint(-2, 3, s, device="cuda", generator=g).float() for s in ((M, K), (K, N)))
+    out = torch.full((M, N), float("nan"), device="cuda")
+    nz.gemm(A, B, out=out, static=True)
+    assert torch.equal(out, nz.gemm(A, B))          # integers: exact whatever the grouping
