@@ -8,6 +8,7 @@
 #include <cstdlib>
 
 #include "nzhip_internal.h"
+#include "nzhip_pieces.h"
 
 namespace nzhip {
 
@@ -233,14 +234,10 @@ __device__ __forceinline__ float from_lane_above(float v) {
 // A lane's quad of a row whose 16-byte pieces are not aligned, cut by the end of the row or past it: one 16-byte access at a
 // 4-byte aligned address, moved left into the row (W >= 4) where the quad does not fit, and turned back in registers. `back`
 // is how far it was moved; elements past the end of the row come out as some element of the row.
-typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ void load_ragged_quad(const float* row, int at, int back, float (&v)[4]) {
-    const floatx4 q = *reinterpret_cast<const floatx4u*>(row + at);
-    const float a = back & 1 ? q[1] : q[0], b = back & 1 ? q[2] : q[1], c = back & 1 ? q[3] : q[2];
-    v[0] = back & 2 ? c : a;
-    v[1] = back & 2 ? q[3] : b;
-    v[2] = c;
-    v[3] = q[3];
+    const floatx4 q = turn_back(*reinterpret_cast<const floatx4u*>(row + at), back);
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = q[e];
 }
 
 // PIX_BIAS: 0 none or per channel; 1 per pixel with any strides; 2 per pixel in the layout of the
@@ -3107,7 +3104,7 @@ static int conv2d_forward_impl(float* y, const float* x, const float* w_ref, con
     // kernels (16 x 64 x 56 x 56 -> 64: 12 against 18 us; 16 x 120 x 56 x 56 -> 120 with the reference's per-pixel bias: 23 against
     // 30 us), and with at least 128 well ahead
     // (16 x 512 x 28 x 28 -> 128: 16 against 31 us; 16 x 256 x 14 x 14 -> 1024: 20 against 55 us), tiny images included since
-    // their planes are widened to whole 16-byte pieces (16 x 512 x 7 x 7 -> 128: 14 against 47 us through the column matrix).
+    // planes of 49 pixels are rows like any other to the product (16 x 512 x 7 x 7 -> 128: 14 against 47 us through the column matrix).
     static const char* gemm1x1_env = getenv("NZHIP_CONV_1X1_GEMM");     // benchmarking only: 0 never, 1 always
     const bool as_product = K_h == 1 && K_w == 1 && stride == 1 && pad == 0 && H * W < 0x3fffffff && C < 0x3fffffff && O < 0x3fffffff &&
                             N <= 65535 &&

@@ -18,6 +18,7 @@
 #include <type_traits>
 
 #include "nzhip_internal.h"
+#include "nzhip_pieces.h"
 
 namespace nzhip {
 
@@ -64,14 +65,8 @@ __device__ __forceinline__ int phys_row(int r) {
 // per k tile finds the last one, whose missing k are zeroed, and one per tile the pieces that have to be turned back.
 // 16-byte accesses need no more than the 4-byte alignment of their elements: rows of 777 or 513 floats stream at the rate of
 // rows of 776 or 512 (1000 x 777 x 513: 14.9 us; element by element it was 33, through zero-padded copies of the operands 21).
-typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
 
-// element e of a piece that was moved back by `back` elements; what lies beyond the extent comes out as some element of it
-__device__ __forceinline__ floatx4 turn_back(const floatx4 q, int back) {
-    const float a = back & 1 ? q[1] : q[0], b = back & 1 ? q[2] : q[1], c = back & 1 ? q[3] : q[2];
-    return floatx4{back & 2 ? c : a, back & 2 ? q[3] : b, c, q[3]};
-}
 // How the accesses of an instance are kept inside the operands. INTERIOR: they are. PIECES: rows and 16-byte pieces are moved.
 // ELEMENTS: some contiguous extent is below 4, so pieces are made of single elements (an instance of its own: the choice made
 // in the kernel, at every load, cost the loads their place in the order the waits rely on, 1040 x 1280 x 1968 35 -> 55 us).
@@ -354,7 +349,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
         }
     }
 
-    // ---- epilogue: bias, activation, predicated (vector when legal) store ------------------
+    // ---- epilogue: bias, activation, masked store ------------------
     // Bias values are fetched in batches (all of a 32-row block at once, or once per lane when
     // the bias does not vary along rows) so the stores never wait on one load each.
     const float* bias = p.bias ? p.bias + bi * p.bias_sn + bj * p.bias_sc : nullptr;
@@ -456,6 +451,8 @@ static int launch_cfg(const GemmKernelArgs& a, bool a_trans, bool b_trans, bool 
         return launch(gemm_f16mfma_kernel<BM, BN, BK, WM, WN, true, true, E>);
     };
     if (full) return pick(std::integral_constant<int, INTERIOR>{});
+    if constexpr (BK > 32) return set_error(NZHIP_E_INVALID, "gemm: the %d-wide k step is for whole tiles", BK);
+    else {
     // By pieces where no contiguous extent is below 4. Along k that is the whole contraction, also of a split one: however few
     // elements its last chunk has, those before it in the row are the previous chunk's, so a piece moved left out of the chunk
     // is still inside the operand, and what it brings along is zeroed like anything past the end. (Judged by the last chunk
@@ -465,6 +462,7 @@ static int launch_cfg(const GemmKernelArgs& a, bool a_trans, bool b_trans, bool 
     const bool pieces = (a_trans ? a.M : k) >= 4 && (b_trans ? k : a.N) >= 4;
     if (gemm_trace()) fprintf(stderr, "nzhip_gemm: loads by %s\n", pieces ? "pieces" : "elements");
     return pieces ? pick(std::integral_constant<int, PIECES>{}) : pick(std::integral_constant<int, ELEMENTS>{});
+    }
 }
 
 static bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -494,7 +492,7 @@ struct FusedCostInput {
 static double fused_cost_us(const FusedCostInput& q, int tile, int64_t parts, int64_t Kc) {
     const int64_t tiles = ((q.M + tile - 1) / tile) * ((q.N + tile - 1) / tile) * q.members * parts;
     const double rounds = (double)((tiles + (int64_t)q.cus - 1) / (int64_t)q.cus);
-    const bool full = q.aligned && q.M % tile == 0 && q.N % tile == 0 && Kc % 32 == 0 && q.K % 32 == 0;   // unpredicated instance
+    const bool full = q.aligned && q.M % tile == 0 && q.N % tile == 0 && Kc % 32 == 0 && q.K % 32 == 0;   // the INTERIOR instance
     // A narrow operand costs what a whole tile of it would: the loads of rows past its end are issued all the same, and a k step
     // has a latency that few rows do not shorten (two chunks of 1024 steps with 64 x 64 tiles: 4 x 65536 x 16 272 us, 63 x 65536 x 61
     // 281). Charged by the rows it has, a product that leaves CUs idle gets too few chunks (10 x 260100 x 16: 233 chunks 16.7 us,
@@ -509,7 +507,7 @@ static double fused_cost_us(const FusedCostInput& q, int tile, int64_t parts, in
     const double out = (double)q.M * q.N * q.members * 4.0;
     // the second launch: 16 x 736 x 1905 12.7 us unsplit, 8.6 in four chunks, 33 x 512 x 33 7.6 either way (charged 6 it kept the first unsplit)
     const double reduce = parts > 1 ? 4.5 + (double)(parts + 1) * out / 3e6 : 0.0;
-    // what a workgroup spends outside its k loop (first requests, predicated epilogue): 17 x 33 x 15 takes 10 us with a
+    // what a workgroup spends outside its k loop (first requests, epilogue): 17 x 33 x 15 takes 10 us with a
     // 128 x 128 tile and 5 us with a 64 x 64 tile; rounds that share a CU pay it side by side
     const double ends = (tile == 64 ? 1.5 : 4.0) * (rounds > 2.0 ? rounds / 2.0 : 1.0);
     return 3.0 + ends + stream + reduce;
@@ -584,9 +582,9 @@ int gemm_mfma_dispatch(const nzhip_gemm_desc& d, hipStream_t stream, int force_t
     const bool vec = gemm_vec_legal(d);
     const int64_t batch = d.batch_n * d.batch_c;
 
-    // Tile choice: 256x256 tiles need enough of them to fill the 256 CUs and pay only in their
-    // unpredicated instance (5000x1000x5000: 379 us with predicated 256x256 tiles, 156 us with
-    // 128x128 tiles).
+    // Tile choice: 256x256 tiles need enough of them to fill the 256 CUs, and are kept to whole products. (That line was drawn when
+    // ragged ones were loaded under predicates; by moved pieces they too are faster with 256x256 tiles where the two-pass route does
+    // not take them, 5001x999x5001 104 us against 142 with 128x128, 8000x500x3000 64 against 74: it could move.)
     const int64_t t256 = ((d.M + 255) / 256) * ((d.N + 255) / 256) * batch;
     const bool whole256 = vec && d.M % 256 == 0 && d.N % 256 == 0 && d.K % 32 == 0 && (k_total <= 0 || k_total % d.K == 0);
     static const char* tile_env = getenv("NZHIP_GEMM_TILE");         // 128 | 256: benchmarking only
@@ -607,8 +605,8 @@ int gemm_mfma_dispatch(const nzhip_gemm_desc& d, hipStream_t stream, int force_t
         return launch_cfg<256, 256, 32, 2, 2>(a, a_trans, b_trans, vec, (int)batch, stream);
     if (tile == 256) return launch_cfg<256, 256, 32, 4, 2>(a, a_trans, b_trans, vec, (int)batch, stream);
     if (tile == 64) {
-        // whole tiles: 64-wide k steps halve the number of barriers (1024^3: 14.2 -> 13.0 us); with predicates
-        // the wider step only adds padding (1000 x 777 x 513: 22.0 -> 23.2 us)
+        // whole tiles: 64-wide k steps halve the number of barriers (1024^3: 14.2 -> 13.0 us). Ragged ones keep 32, also a line from
+        // the predicated loads: with moved pieces 64 is better from about 500 on (1000 x 777 x 513 15.0 -> 13.9 us, 700 x 300 x 900 8.2 -> 9.0).
         const bool whole = vec && d.M % 64 == 0 && d.N % 64 == 0 && d.K % 64 == 0 && (k_total <= 0 || k_total % d.K == 0);
         if (whole) return launch_cfg<64, 64, 64, 2, 2>(a, a_trans, b_trans, vec, (int)batch, stream);
         return launch_cfg<64, 64, 32, 2, 2>(a, a_trans, b_trans, vec, (int)batch, stream);

@@ -1040,8 +1040,8 @@ bool gemm_h16_applicable(const nzhip_gemm_desc& d) {
     // (microseconds, fused / two-pass): 3072^3 136 / 102, 4096^3 197 / 163, 4096x4096x1024 60 / 52,
     // but 2048^3 44 / 53, 4096x1024x4096 67 / 77, 4096x256x4096 30 / 36, 8192x512x8192 160 / 168 (short contractions leave
     // the rounding pass and the C stores nothing to hide behind). Shapes that are not whole
-    // 256x256x32 tiles take the fused kernel's predicated instance, which is much slower, so the
-    // threshold is lower for them: 2500^3 101 / 68, 5000x1000x5000 156 / 94, 2000^3 56 / 55.
+    // 256x256x32 tiles take 128x128 tiles in the fused kernel, which is slower, so the threshold is lower
+    // for them (2500^3 101 / 68, 2000^3 56 / 55 when it loaded ragged operands under predicates; 5000x1000x5000 now 142 / 86).
     if (d.M < 512 || d.N < 512 || d.K < 768) return false;
     const double flops = 2.0 * d.M * d.N * d.K;
     const double cvt_bytes = 6.0 * ((double)d.M * d.K + (double)d.N * d.K);

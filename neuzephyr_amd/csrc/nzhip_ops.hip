@@ -445,7 +445,7 @@ static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s) {
     // Products that leave CUs idle with 128 x 128 tiles (weight gradients with K = batch x pixels, mid-size
     // products): smaller tiles, or the contraction cut into chunks that run as a batch into a workspace and are
     // then added in order, whichever the cost model in gemm_fused_plan prefers. A chunk keeps at least 512 of the
-    // contraction when loads are vectorised and 128 otherwise. A batch over n alone (batch_c == 1: shared-weight
+    // contraction, 128 where the result is narrow. A batch over n alone (batch_c == 1: shared-weight
     // layers, the conv column-matrix route) splits the same way; its chunks take the c dimension of the launch.
     static const char* route = getenv("NZHIP_GEMM_ROUTE");         // fused | h16: overrides the route choice (benchmarking only)
     const bool force_fused = route && route[0] == 'f', force_h16 = route && route[0] == 'h';
