@@ -362,7 +362,7 @@ CONV1X1_BWD_W = [  # N, C, H, W, O, w_batch   (1x1, stride 1, no padding: one ba
     (1, 1, 1, 1, 1, 1), (1, 3, 4, 5, 2, 1), (2, 5, 7, 9, 6, 1), (3, 16, 8, 8, 24, 3), (2, 64, 16, 16, 128, 1), (4, 70, 9, 11, 33, 1),
     (2, 128, 12, 20, 64, 2), (5, 3, 30, 33, 1, 1), (1, 256, 8, 8, 256, 1), (6, 8, 5, 5, 8, 6),
     # per-sample weights (dw is read and written in place as the product's bias matrix) with a long contraction
-    # that is split into chunks, with pixel rows that forbid 16-byte loads (padded copies), and on the two-pass route
+    # that is split into chunks, with pixel rows off 16-byte boundaries, and on the two-pass route
     (2, 40, 32, 40, 24, 2), (2, 24, 31, 35, 40, 2), (3, 130, 45, 23, 70, 3), (2, 512, 48, 48, 512, 2)]
 
 
@@ -416,12 +416,16 @@ def test_conv_backward_weights_any_geometry_is_bit_exact_on_integers(nz, oracle,
     assert np.array_equal(got, expect)
 
 
-@pytest.mark.parametrize("N,C,H,W,O,Kh,Kw,stride,pad,wb", [c for c in CONV_GEN_BWD_W if c[3] % 4 != 0 or ((c[3] + 2 * c[8] - c[6]) // c[7] + 1) % 4 != 0] +
-                         [(3, 40, 7, 7, 24, 1, 1, 1, 0, 1), (2, 20, 5, 5, 33, 1, 1, 1, 0, 2), (2, 70, 35, 35, 9, 1, 1, 1, 0, 1)])   # and 1x1 products on planes of 49, 25, 1225 pixels
+@pytest.mark.parametrize("N,C,H,W,O,Kh,Kw,stride,pad,wb", [c for c in CONV_GEN_BWD_W if c[3] % 4 != 0 or ((c[3] + 2 * c[8] - c[6]) // c[7] + 1) % 4 != 0])
 def test_conv_backward_weights_on_rows_widened_to_16_byte_pieces(nz, oracle, monkeypatch, N, C, H, W, O, Kh, Kw, stride, pad, wb):
     # Large layers whose rows of x or dy are not whole 16-byte pieces run on zero-filled copies with rows of the next
     # multiple of 4; the library reads NZHIP_CONV_WIDEN per call, so the copies can be forced for these small shapes.
     monkeypatch.setenv("NZHIP_CONV_WIDEN", "1")
+    test_conv_backward_weights_any_geometry_is_bit_exact_on_integers(nz, oracle, N, C, H, W, O, Kh, Kw, stride, pad, wb)
+
+
+@pytest.mark.parametrize("N,C,H,W,O,Kh,Kw,stride,pad,wb", [(3, 40, 7, 7, 24, 1, 1, 1, 0, 1), (2, 20, 5, 5, 33, 1, 1, 1, 0, 2), (2, 70, 35, 35, 9, 1, 1, 1, 0, 1)])
+def test_conv1x1_backward_weights_on_planes_of_any_size(nz, oracle, N, C, H, W, O, Kh, Kw, stride, pad, wb):
     test_conv_backward_weights_any_geometry_is_bit_exact_on_integers(nz, oracle, N, C, H, W, O, Kh, Kw, stride, pad, wb)
 
 

@@ -197,8 +197,9 @@ WIDENED = [  # N, C, H, W, O, k, stride, pad, w_batch, per-pixel bias: rows that
     # (5x5; stride 2 with the per-pixel bias; a split contraction; per-sample weights; two chunks per loop step, which such
     # rows only reach through the copy; 7x7 stride 2 on three channels)
     (64, 16, 14, 14, 32, 5, 1, 2, 1, False), (64, 24, 21, 30, 70, 3, 2, 1, 1, True), (16, 256, 14, 14, 96, 3, 1, 1, 1, False),
-    (16, 5, 30, 30, 9, 3, 1, 1, 16, False), (256, 64, 14, 14, 48, 5, 1, 2, 1, False), (8, 3, 97, 97, 20, 7, 2, 3, 1, False),
-    # 1x1 layers as products: planes of 49, 35 and 1225 pixels widened to 52, 36 and 1228 (shared and per-sample weights,
+    (16, 5, 30, 30, 9, 3, 1, 1, 16, False), (256, 64, 14, 14, 48, 5, 1, 2, 1, False), (8, 3, 97, 97, 20, 7, 2, 3, 1, False)]
+
+RAGGED_1X1 = [  # the same columns: 1x1 layers as products on planes of 49, 35 and 1225 pixels (shared and per-sample weights,
     # per-channel and per-pixel bias)
     (8, 130, 7, 7, 140, 1, 1, 0, 1, False), (6, 128, 5, 7, 130, 1, 1, 0, 6, True), (2, 136, 35, 35, 20, 1, 1, 0, 1, False)]
 
@@ -209,6 +210,15 @@ def test_conv2d_on_rows_widened_to_16_byte_pieces_is_bit_exact(nz, oracle, monke
     # NZHIP_CONV_WIDEN per call, so the copy can be forced for shapes an oracle finishes quickly. Forward, and the
     # stride-1 data gradient (the same kernel on the output gradient, mirrored weights, accumulating in place).
     monkeypatch.setenv("NZHIP_CONV_WIDEN", "1")
+    forward_and_data_gradient_are_bit_exact(nz, oracle, N, C, H, W, O, k, stride, pad, w_batch, pix)
+
+
+@pytest.mark.parametrize("N,C,H,W,O,k,stride,pad,w_batch,pix", RAGGED_1X1)
+def test_conv1x1_on_planes_of_any_size_is_bit_exact(nz, oracle, N, C, H, W, O, k, stride, pad, w_batch, pix):
+    forward_and_data_gradient_are_bit_exact(nz, oracle, N, C, H, W, O, k, stride, pad, w_batch, pix)
+
+
+def forward_and_data_gradient_are_bit_exact(nz, oracle, N, C, H, W, O, k, stride, pad, w_batch, pix):
     rng = np.random.default_rng(N * 3 + C * 5 + H * 7 + W * 11 + O * 13 + k + stride)
     Ho, Wo = oracle.out_hw(H, W, k, k, stride, pad)
     x = rng.integers(-4, 5, size=(N, C, H, W)).astype(np.float32)

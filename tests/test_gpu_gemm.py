@@ -146,7 +146,7 @@ def test_long_contractions_with_few_tiles_are_bit_exact_on_integers(nz, M, K, N,
 @pytest.mark.parametrize("force", [0, 64, 128, 256, 18, 12])
 def test_bias_may_alias_the_output(nz, M, K, N, force):
     # "C += A B": the bias operand is C itself, element for element. Every route reads bias(m, n) in the
-    # thread that writes C(m, n), also behind a split contraction or padded operand copies.
+    # thread that writes C(m, n), also behind a split contraction or on ragged rows.
     rng = np.random.default_rng(M + 3 * K + 5 * N + force)
     A = rng.integers(-4, 5, size=(M, K)).astype(np.float32)
     B = rng.integers(-4, 5, size=(K, N)).astype(np.float32)
@@ -355,9 +355,9 @@ def test_skinny_batched_linear_single_sample(nz, oracle):
 @pytest.mark.parametrize("M,K,N", [(1000, 777, 513), (700, 701, 333), (999, 1001, 1003), (516, 1030, 520)])
 @pytest.mark.parametrize("a_trans,b_trans", [(False, False), (False, True), (True, False), (True, True)])
 def test_operands_without_16_byte_rows_are_bit_exact_on_integers(nz, M, K, N, a_trans, b_trans):
-    # products big enough for it are computed from zero-padded copies of the operands whose rows do not allow
-    # 16-byte loads; rows are embedded in NaN-filled storage with a leading dimension of their own and an odd base
-    # offset, so a read past a row's end or a missing zero in the padding poisons the result
+    # rows off 16-byte boundaries are loaded by 16-byte pieces moved into the operand; rows are embedded in NaN-filled
+    # storage with a leading dimension of their own and an odd base offset, so a read past a row's end or a missing
+    # zero past the contraction's poisons the result
     import ctypes as C
     import torch
     rng = np.random.default_rng(M + 3 * K + 7 * N)
@@ -484,7 +484,7 @@ def test_one_tile_products_are_split_by_their_length_and_not_by_the_alignment_of
 @pytest.mark.parametrize("M,K,N,a_trans,b_trans,slack,offset,bias_form,seed", _embedded_cases())
 def test_embedded_operands_random_sweep(nz, M, K, N, a_trans, b_trans, slack, offset, bias_form, seed):
     # random shapes, layouts, leading dimensions and base offsets through the default route choice (streaming,
-    # thin, split, 64 / 128 tiles, padded copies): exact on integers, nothing read or written outside the rows
+    # thin, split, 64 / 128 tiles): exact on integers, nothing read or written outside the rows
     import ctypes as C
     import torch
     rng = np.random.default_rng(seed)
