@@ -206,7 +206,7 @@ __global__ __launch_bounds__(256) void conv3x3_direct_kernel(float* __restrict__
     }
 }
 
-// ---- streaming variant of the direct route (C <= 4, O <= 2, 16-byte aligned rows) ----------
+// ---- streaming variant of the direct route (C <= 4, O <= 2, H >= 8, W >= 4) ----------------
 // A wave owns a strip of 256 columns x up to ST_ROWS output rows and walks DOWN it: every input row
 // is requested once, ST_AHEAD rows ahead of its use, rounded to fp16 once, and kept in a
 // rolling window of three rows per channel; as soon as a row arrives, the output row above it
