@@ -11,12 +11,14 @@
 //              waves and grid.y split k; partial sums meet in LDS, then (if k is split over
 //              blocks) in a workspace that a small second kernel reduces deterministically.
 //   LK kernel: L is stored with k contiguous  (L(k,l) at L[l*ld + k]); a wave owns 4 rows l,
-//              lanes stride k, and the 64 partial sums are folded with cross-lane shuffles.
+//              lanes stride k, and the 64 partial sums are folded with cross-lane shuffles; where the long
+//              extent gives few waves and k is long, grid.y splits k as in the KL kernel.
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>
 
 #include "nzhip_internal.h"
+#include "nzhip_pieces.h"
 
 namespace nzhip {
 
@@ -212,7 +214,10 @@ __global__ __launch_bounds__(KLC_THREADS) void skinny_kl_cols_kernel(const Skinn
 }
 
 // ---- LK: rows of L are dot products ------------------------------------------------------------
-template <int SR>
+// PLAIN: rows of L and S that are whole 16-byte pieces, the contraction in one workgroup. Otherwise rows of any alignment, S rows
+// of any stride and, where p.ksplit > 1, a chunk of the contraction per grid.y. (One kernel for both costs the plain case 0.6 us of
+// prologue: 1 x 1024 x 512 6.2 instead of 5.6 us.)
+template <int SR, bool PLAIN>
 __global__ __launch_bounds__(256) void skinny_lk_kernel(const SkinnyArgs p) {
     constexpr int LR = 4;                                          // rows of L per wave
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -221,6 +226,7 @@ __global__ __launch_bounds__(256) void skinny_lk_kernel(const SkinnyArgs p) {
     const float* __restrict__ L = p.L + bi * p.L_sn + bj * p.L_sc;
     const int l0 = (blockIdx.x * 4 + wave) * LR;
     if (l0 >= p.LN) return;
+    const int kb = PLAIN ? 0 : blockIdx.y * p.kslice, ke = PLAIN || kb + p.kslice >= p.K ? p.K : kb + p.kslice;
 
     float acc[SR][LR];
 #pragma unroll
@@ -228,23 +234,32 @@ __global__ __launch_bounds__(256) void skinny_lk_kernel(const SkinnyArgs p) {
 #pragma unroll
         for (int r = 0; r < LR; r++) acc[s][r] = 0.f;
 
-    const bool s_contig = p.s_sk == 1;
-    int k0 = lane * 4;
-    // Whole rows with 16-byte loads: U k steps at a time, their U x (SR + LR) loads issued before any is used -- a
-    // wave has only 64 KiB to stream, and one step per round trip to memory would leave it waiting for latency.
-    if (p.vec && s_contig && (p.SR == 1 || (p.s_ss & 3) == 0) && l0 + LR <= p.LN) {
+    // row r of the wave, row s of the narrow side: past the end the last one, loaded like the others and not stored
+    auto lrow = [&](int r) { return L + (long)(l0 + r < p.LN ? l0 + r : p.LN - 1) * p.ldl; };
+    auto srow = [&](int s) { return S + (s < p.SR ? s : p.SR - 1) * p.s_ss; };
+    const bool s_contig = PLAIN || p.s_sk == 1;
+    int k0 = kb + lane * 4;
+    // U k steps at a time, their U x (SR + LR) loads issued before any is used -- a wave has only 64 KiB to stream, and one
+    // step per round trip to memory would leave it waiting for latency. 16-byte loads need no more than 4-byte alignment
+    // (2 x 114622 x 16, rows that end 2 floats past a 16-byte piece, element by element: 1.8 us for each 256 k).
+    if (PLAIN ? l0 + LR <= p.LN : s_contig) {
         constexpr int U = 4;
-        for (; k0 + 256 * (U - 1) + 4 <= p.K; k0 += 256 * U) {
-            floatx4 sv[U][SR], lv[U][LR];
+        for (; k0 + 256 * (U - 1) + 4 <= ke; k0 += 256 * U) {
+            piece4 sv[U][SR], lv[U][LR];
 #pragma unroll
             for (int u = 0; u < U; u++) {
 #pragma unroll
                 for (int s = 0; s < SR; s++) {
-                    const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
-                    sv[u][s] = s < p.SR ? *reinterpret_cast<const floatx4*>(S + s * p.s_ss + k0 + 256 * u) : zero;
+                    if constexpr (PLAIN) {
+                        const piece4 zero = {0.f, 0.f, 0.f, 0.f};
+                        sv[u][s] = s < p.SR ? *reinterpret_cast<const piece4*>(S + s * p.s_ss + k0 + 256 * u) : zero;
+                    } else sv[u][s] = *reinterpret_cast<const floatx4u*>(srow(s) + k0 + 256 * u);
                 }
 #pragma unroll
-                for (int r = 0; r < LR; r++) lv[u][r] = *reinterpret_cast<const floatx4*>(L + (long)(l0 + r) * p.ldl + k0 + 256 * u);
+                for (int r = 0; r < LR; r++) {
+                    if constexpr (PLAIN) lv[u][r] = *reinterpret_cast<const piece4*>(L + (long)(l0 + r) * p.ldl + k0 + 256 * u);
+                    else lv[u][r] = *reinterpret_cast<const floatx4u*>(lrow(r) + k0 + 256 * u);
+                }
             }
 #pragma unroll
             for (int u = 0; u < U; u++)
@@ -256,20 +271,20 @@ __global__ __launch_bounds__(256) void skinny_lk_kernel(const SkinnyArgs p) {
                         for (int e = 0; e < 4; e++) acc[s][r] = __builtin_fmaf(rnd16(sv[u][s][e]), rnd16(lv[u][r][e]), acc[s][r]);
         }
     }
-    for (; k0 < p.K; k0 += 256) {
-        const bool fullk = p.vec && (k0 + 4 <= p.K);
-        floatx4 sv[SR];
+    for (; k0 < ke; k0 += 256) {
+        const bool fullk = k0 + 4 <= ke;
+        piece4 sv[SR];
 #pragma unroll
         for (int s = 0; s < SR; s++) {
-            floatx4 v = {0.f, 0.f, 0.f, 0.f};
+            piece4 v = {0.f, 0.f, 0.f, 0.f};
             if (s < p.SR) {
-                const float* q = S + s * p.s_ss + (long)k0 * p.s_sk;
-                if (fullk && s_contig && ((p.s_ss & 3) == 0)) {
-                    v = *reinterpret_cast<const floatx4*>(q);
+                const float* q = srow(s) + (long)k0 * p.s_sk;
+                if (fullk && s_contig) {
+                    v = *reinterpret_cast<const floatx4u*>(q);
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; e++)
-                        if (k0 + e < p.K) v[e] = q[e * p.s_sk];
+                        if (k0 + e < ke) v[e] = q[e * p.s_sk];
                 }
             }
 #pragma unroll
@@ -278,15 +293,15 @@ __global__ __launch_bounds__(256) void skinny_lk_kernel(const SkinnyArgs p) {
         }
 #pragma unroll
         for (int r = 0; r < LR; r++) {
-            floatx4 v = {0.f, 0.f, 0.f, 0.f};
+            piece4 v = {0.f, 0.f, 0.f, 0.f};
             if (l0 + r < p.LN) {
                 const float* q = L + (long)(l0 + r) * p.ldl + k0;
                 if (fullk) {
-                    v = *reinterpret_cast<const floatx4*>(q);
+                    v = *reinterpret_cast<const floatx4u*>(q);
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; e++)
-                        if (k0 + e < p.K) v[e] = q[e];
+                        if (k0 + e < ke) v[e] = q[e];
                 }
             }
 #pragma unroll
@@ -314,6 +329,10 @@ __global__ __launch_bounds__(256) void skinny_lk_kernel(const SkinnyArgs p) {
                 const int l = l0 + r;
                 if (s >= p.SR || l >= p.LN) continue;
                 float x = acc[s][r];
+                if (!PLAIN && p.ksplit > 1) {
+                    p.partial[(((long)bz * p.ksplit + blockIdx.y) * p.SR + s) * p.LN + l] = x;
+                    continue;
+                }
                 if (p.bias) x += p.bias[bi * p.b_sn + bj * p.b_sc + s * p.b_ss + l * p.b_sl];
                 if (p.relu) x = x > 0.f ? x : 0.f;
                 p.out[bi * p.o_sn + bj * p.o_sc + s * p.o_ss + l * p.o_sl] = x;
@@ -419,13 +438,33 @@ int gemm_skinny_dispatch(const nzhip_gemm_desc& d, hipStream_t stream) {
             hipLaunchKernelGGL(skinny_reduce_kernel, g2, dim3(256), 0, stream, p);
         }
     } else {
-        dim3 grid((unsigned)((p.LN + 15) / 16), 1, batch);
-        if (grid.x > 0x7fffffffu / 2) return set_error(NZHIP_E_UNSUPPORTED, "nzhip_gemm: long extent too large");
-        switch (sr_t) {
-            case 1: hipLaunchKernelGGL(skinny_lk_kernel<1>, grid, dim3(256), 0, stream, p); break;
-            case 2: hipLaunchKernelGGL(skinny_lk_kernel<2>, grid, dim3(256), 0, stream, p); break;
-            case 4: hipLaunchKernelGGL(skinny_lk_kernel<4>, grid, dim3(256), 0, stream, p); break;
-            default: hipLaunchKernelGGL(skinny_lk_kernel<8>, grid, dim3(256), 0, stream, p); break;
+        const int64_t lblocks = ((int64_t)p.LN + 15) / 16;
+        if (lblocks > 0x7fffffff / 2) return set_error(NZHIP_E_UNSUPPORTED, "nzhip_gemm: long extent too large");
+        // A wave owns four rows and 1024 k take it about 1.2 us, a trip to memory and back. Where the rows give at most every other
+        // CU a workgroup, k is split into chunks of 2048 and more, if that saves more than the second launch costs, 4.5 us:
+        // 2 x 114622 x 16 812 -> 10.8 us, 1 x 16384 x 1024 22.6 -> 15.8, 300 x 8192 x 3 15.3 -> 10.0; on more workgroups the stream
+        // itself is the limit (1 x 4096 x 4096 16.6 unsplit, 21.1 in two, 1 x 16384 x 4096 49.1 and 53.2).
+        int64_t ksplit = 512 / (lblocks * batch);
+        if (ksplit > p.K / 2048) ksplit = p.K / 2048;
+        if (lblocks * batch > device_cu_count() / 2 || (double)p.K / 1024 * (1.0 - 1.0 / (double)(ksplit < 1 ? 1 : ksplit)) < 5.0) ksplit = 1;
+        if (ksplit < 2 || (double)sizeof(float) * batch * ksplit * p.SR * p.LN > (double)workspace_limit()) ksplit = 1;
+        p.kslice = (int)(((p.K + ksplit - 1) / ksplit + 1023) / 1024 * 1024);
+        p.ksplit = (p.K + p.kslice - 1) / p.kslice;
+        if (p.ksplit > 1) {
+            rc = workspace_alloc(reinterpret_cast<void**>(&partial), sizeof(float) * batch * p.ksplit * p.SR * p.LN, stream);
+            if (rc) return rc;
+            p.partial = partial;
+        }
+        dim3 grid((unsigned)lblocks, (unsigned)p.ksplit, batch);
+        const bool plain = p.vec && p.ksplit == 1 && p.s_sk == 1 && (p.SR == 1 || (p.s_ss & 3) == 0);
+        auto kfn = sr_t == 1   ? (plain ? skinny_lk_kernel<1, true> : skinny_lk_kernel<1, false>)
+                   : sr_t == 2 ? (plain ? skinny_lk_kernel<2, true> : skinny_lk_kernel<2, false>)
+                   : sr_t == 4 ? (plain ? skinny_lk_kernel<4, true> : skinny_lk_kernel<4, false>)
+                               : (plain ? skinny_lk_kernel<8, true> : skinny_lk_kernel<8, false>);
+        hipLaunchKernelGGL(kfn, grid, dim3(256), 0, stream, p);
+        if (p.ksplit > 1) {
+            dim3 g2((unsigned)(((long)p.SR * p.LN + 63) / 64), 1, batch);
+            hipLaunchKernelGGL(skinny_reduce_kernel, g2, dim3(256), 0, stream, p);
         }
     }
     hipError_t e = hipGetLastError();

@@ -127,6 +127,37 @@ SPLITK = [(130, 9000, 70), (576, 16384, 128), (64, 4096, 64), (33, 20001, 300), 
           (10, 70000, 16), (16, 33000, 10)]       # a handful of outputs, hundreds of chunks: one wave per output adds them
 
 
+# dot products along contiguous rows, split over workgroups (rows for at most half the CUs, k long enough) and not, on rows of any
+# alignment: (M, K, N, batch)
+DOT_ROWS = [(2, 114622, 16, 1), (1, 9000, 1, 1), (1, 8193, 257, 1), (2, 10242, 18, 1), (300, 8195, 3, 1), (1, 6144, 640, 1), (33, 9217, 1, 3),
+            (20, 8199, 5, 2), (1, 6143, 7, 1), (2, 1027, 5, 1), (1, 3, 70, 1)]
+
+
+@pytest.mark.parametrize("M,K,N,batch", DOT_ROWS)
+def test_skinny_dot_products_of_any_alignment_are_bit_exact_on_integers(nz, M, K, N, batch):
+    import torch
+    rng = np.random.default_rng(M + K + N)
+    A = rng.integers(-2, 3, (batch, 1, M, K)).astype(np.float32)
+    B = rng.integers(-2, 3, (batch, 1, N, K)).astype(np.float32)
+    want = np.maximum(A.astype(np.float64) @ B.transpose(0, 1, 3, 2) + np.arange(N) % 5, 0)          # whole numbers below 2^24
+
+    def embedded(a):                                                   # at an odd offset, NaN on both sides
+        buf = torch.full((a.size + 14,), float("nan"), device="cuda")
+        buf[7:7 + a.size] = torch.from_numpy(a.ravel()).cuda()
+        return buf[7:7 + a.size].view(a.shape)
+
+    bias = dev(np.arange(N) % 5)
+    a, b = embedded(A), embedded(B)
+    if batch == 1:
+        got = [nz.gemm(a[0, 0], b[0, 0], b_trans=True, bias=bias, bias_strides=(0, 1), relu=True) for _ in range(2)]
+        got.append(nz.gemm(a[0, 0], b[0, 0], b_trans=True, bias=bias, bias_strides=(0, 1), relu=True, static=True))
+        for g in got:
+            assert np.array_equal(host(g), want[0, 0])
+    else:
+        got = nz.tensorcore_gemm(a, dev(B.transpose(0, 1, 3, 2)))
+        assert np.array_equal(np.maximum(host(got) + np.arange(N, dtype=np.float32) % 5, 0), want)
+
+
 @pytest.mark.parametrize("M,K,N", SPLITK)
 @pytest.mark.parametrize("a_trans,b_trans", [(False, False), (False, True), (True, False), (True, True)])
 def test_long_contractions_with_few_tiles_are_bit_exact_on_integers(nz, M, K, N, a_trans, b_trans):
