@@ -78,6 +78,34 @@ def test_avgpool_random_geometries_bit_exact(nz, oracle, shape, pool, stride, pa
     assert np.array_equal(host(dx), oracle.avgpool2d_backward(np.zeros(shape, np.float32), dy, pool, stride, pad))
 
 
+# the strip kernels (stride 2, no padding; forward from 48 output columns on): widths that leave 1 to 3 columns of the last quad and an
+# odd last output column, heights that leave part of a strip, images of one strip and less, rows that no window reaches
+STRIP_CASES = [((2, 1, 5, 101), 5), ((1, 2, 13, 102), 5), ((3, 1, 16, 103), 5), ((1, 1, 24, 104), 5), ((2, 2, 9, 97), 3), ((1, 1, 33, 98), 3),
+               ((1, 3, 8, 99), 2), ((2, 1, 7, 100), 2), ((1, 1, 2, 2), 2), ((5, 1, 3, 3), 3), ((1, 2, 6, 7), 5), ((1, 1, 41, 519), 5)]
+
+
+@pytest.mark.parametrize("shape,pool", STRIP_CASES)
+def test_avgpool_strips_bit_exact(nz, oracle, shape, pool):
+    import torch
+    rng = np.random.default_rng(sum(shape) * 3 + pool)
+    x = rng.uniform(-1, 1, shape).astype(np.float32)
+
+    def embedded(a):                                                  # at an odd offset, NaN on both sides
+        buf = torch.full((a.size + 14,), float("nan"), device="cuda")
+        buf[7:7 + a.size] = torch.from_numpy(a.ravel()).cuda()
+        return buf, buf[7:7 + a.size].view(a.shape)
+
+    want = oracle.avgpool2d(x, pool, 2, 0)
+    assert np.array_equal(host(nz.avgpool2d(embedded(x)[1], pool, 2, 0)), want)
+    dy = rng.uniform(-1, 1, want.shape).astype(np.float32)
+    base = rng.uniform(-1, 1, shape).astype(np.float32)
+    for overwrite, start in ((False, base), (True, np.full(shape, np.nan, np.float32))):
+        buf, dx = embedded(start)
+        nz.avgpool2d_backward(dx, embedded(dy)[1], pool, 2, 0, overwrite=overwrite)
+        assert np.array_equal(host(dx), oracle.avgpool2d_backward(np.zeros(shape, np.float32) if overwrite else base, dy, pool, 2, 0))
+        assert torch.isnan(buf[:7]).all() and torch.isnan(buf[7 + x.size:]).all()
+
+
 def test_avgpool_rejects_bad_geometry(nz):
     x = dev(np.zeros((1, 1, 4, 4)))
     with pytest.raises(nz.NzHipError):
