@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cstdlib>
 
+#include "nzhip_conv_cl.h"
 #include "nzhip_internal.h"
 #include "nzhip_pieces.h"
 
@@ -2983,6 +2984,56 @@ using namespace nzhip;
 
 // bias_stride_image != 0: the bias varies per image too (used to add into an existing tensor: bias = y with
 // strides (1, H_out*W_out, O*H_out*W_out)); only the implicit-GEMM kernels take it.
+// Whether a layer (its forward's extents; `src`: the tensor the direction reads in rows of W, x or dy) takes the channel-last kernels
+// (nzhip_conv_cl.hip). They pay for their fp16 copies with a launch and 1.5 times the bytes of what they copy, and have no chain over
+// windows after that: ahead on everything but large images whose rows are whole 16-byte pieces, where the window kernels have
+// enough windows for every CU and read fp32 once. Lines drawn on 130 layers, both sides measured (us, window kernels / these):
+static bool conv_cl_wanted(ClDirection dir, const float* src, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride,
+                           size_t pad, size_t w_batch, double other_us = 0.0) {
+    const int fits = cl_conv_fits(dir, N, C, H, W, O, K_h, K_w, stride, pad, w_batch);
+    if (fits != 1) return fits != 0;
+    // a run that asks for one of the other routes gets it
+    static const bool others = getenv("NZHIP_CONV_ROUTE") || getenv("NZHIP_CONV_DX") || getenv("NZHIP_CONV_DW") || getenv("NZHIP_CONV_DW_FOLD");
+    if (others || getenv("NZHIP_CONV_WIDEN")) return false;
+    const size_t Ho = (H + 2 * pad - K_h) / stride + 1, Wo = (W + 2 * pad - K_w) / stride + 1, out = N * Ho * Wo, px = N * H * W;
+    const bool pieces = W % 4 == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0, k3 = K_h == 3 && K_w == 3 && stride == 1;
+    // few channels either side of large images: 8x16x112x112 -> 16 23.2 / 27.5, 16x4x192x92 -> 16 5x5 45.8 / 56.5
+    if (stride == 1 && C <= 16 && O <= 16 && px >= 100000) return false;
+    // one weight copy per image, each for a few pixels: the fp16 copies cost more than they save (4x208x13x13 -> 312 at stride 2, 49
+    // pixels: 15.0 / 16.6, gradient 13.3 / 15.3; 10x256x11x11 -> 395 5x5, 121 pixels: 78.6 / 56.4, gradient 50.8 / 58.6)
+    if (w_batch > 1 && dir != CL_WEIGHTS && Ho * Wo * (dir == CL_FORWARD ? 4 : 2) <= O) return false;
+    if (dir == CL_WEIGHTS) {
+        if (K_h == 1 && K_w == 1) return false;                    // products
+        // what the gather kernel refuses stays refused: taps, strides and staged windows (of one channel) beyond it
+        size_t sw = 16;
+        while (sw < 128 && sw < Wo) sw *= 2;
+        if (!k3 && (K_h * K_w > 128 || stride > 4 || ((128 / sw - 1) * stride + K_h) * ((sw - 1) * stride + K_w + 8) > 14000)) return false;
+        // 4x64x128x128 -> 128 38 / 57, 16x32x64x64 -> 128 37 / 39, 16x64x128x128 -> 128 at stride 2 59 / 74; 8x128x64x64 -> 64 39 / 32
+        if (pieces && Wo % 4 == 0 && out >= 60000 && C >= 32) return false;
+        return !(pieces && k3 && W <= 64 && out >= 45000 && C >= 64 && O == 128);      // 16x128x56x56 -> 128 51 / 55, -> 256 84 / 78
+    }
+    if (K_h == 1 && K_w == 1) return dir == CL_FORWARD && stride == 1;                  // too few channels for a product: 16x16x176x67 -> 20 51 / 31
+    if (k3) {                                                      // (a 3x3 data gradient of stride 1 as well)
+        // weights that stay in LDS and windows that are full: 16x64x56x56 -> 64 22.0 / 21.8, per-channel bias 16.6 / 22.1, gradient 16.4 / 20.7;
+        // 16x32x64x64 -> 128 23.6 / 27.3; 16x13x76x76 -> 82, windows 59 % full, 40.2 / 30.0
+        const size_t in = dir == CL_FORWARD ? C : O, to = dir == CL_FORWARD ? O : C, bn = to > 64 ? 128 : 64, tw = W >= 64 ? 64 : 32, th = 256 / tw;
+        const bool resident = ((in + 15) / 16) * bn * 288 <= 148 * 1024 && (w_batch == 1 || N * ((to + bn - 1) / bn) <= (size_t)device_cu_count());
+        const bool full = H * W * 10 >= ((W + tw - 1) / tw * tw) * ((H + th - 1) / th * th) * 7;
+        if (resident && full && pieces && in >= 8) return px < 40000;
+        // weights beyond LDS: level on the largest, 16x256x56x56 -> 256 115 / 111, gradient 104 / 104; 16x512x28x28 -> 512 102 / 99
+        return true;
+    }
+    if (dir == CL_DATA && stride == 1) return true;                // 16x64x128x128 -> 128 5x5 233 / 177
+    if (dir == CL_DATA) {
+        // The other ways multiply zeros or move a column gradient; `other_us` is the caller's estimate for the better of them.
+        // (16x320x18x18 <- 80 7x7 at stride 2 261 / 21, 16x64x128x128 <- 128 100 / 64; 16x3x224x224 <- 64 7x7, three channels of a tile of
+        // 64, 106 / 140)
+        return cl_conv_cost(dir, N, C, H, W, O, K_h, K_w, stride, pad, w_batch) < other_us;
+    }
+    // 16x64x128x128 -> 128 at stride 2 47 / 54, 5x5 167 / 184; 8x14x144x144 -> 64 7x7 at stride 2, 41472 outputs, 38 / 25
+    return !(pieces && out >= 50000);
+}
+
 // Which kernel family a forward convolution takes (a per-image bias, which only the data gradient uses, does not change
 // the choice; the two implicit-GEMM families support it, the others do not).
 enum ConvRoute { CONV_ROUTE_DIRECT, CONV_ROUTE_FIXED, CONV_ROUTE_ANY, CONV_ROUTE_WORKSPACE };
@@ -3136,6 +3187,9 @@ static int conv2d_forward_impl(float* y, const float* x, const float* w_ref, con
     }
     bool wide = false, bn128 = false;
     const ConvRoute route = conv_forward_route(x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, H_out, W_out, wide, bn128);
+    if (!w_mirror && route != CONV_ROUTE_DIRECT && conv_cl_wanted(CL_FORWARD, x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch))
+        return cl_conv_forward(y, x, w_ref, bias, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, bias_stride_pixel, bias_stride_channel,
+                               bias_stride_image, activation == NZHIP_ACT_RELU, route != CONV_ROUTE_WORKSPACE, s);    // (the column matrix keeps no image)
     const bool fixed_geometry = route == CONV_ROUTE_FIXED, any_geometry = route == CONV_ROUTE_ANY;
     if (bias_stride_image != 0 && !fixed_geometry && !any_geometry)
         return set_error(NZHIP_E_UNSUPPORTED, "conv2d: a per-image bias needs an implicit-GEMM route");
@@ -3366,6 +3420,9 @@ extern "C" int nzhip_conv2d_backward_data(float* dx, const float* dy, const floa
         }
         return nzhip_gemm(&g, s);
     }
+    if (stride == 1 && !conv_direct_applicable(O, C, K_h, K_w, 1, K_h - 1 - pad) &&
+        conv_cl_wanted(CL_DATA, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch))
+        return cl_conv_backward_data(dx, dy, w_ref, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, accumulate, s);
     if (stride > 1) {
         const size_t Ho = (H + 2 * pad - K_h) / stride + 1, Wo = (W + 2 * pad - K_w) / stride + 1;
         // The convolution of the zero-filled gradient does stride^2 times the multiply-adds; the reference's own chain
@@ -3391,6 +3448,9 @@ extern "C" int nzhip_conv2d_backward_data(float* dx, const float* dy, const floa
         const size_t P = Ho * Wo, CKK = C * K_h * K_w;
         const bool chain_fits = N * P < 0x3fffffff && CKK < 0x3fffffff && O < 0x3fffffff && N <= 65535 && P * O < 0x7fffffffull &&
                                 N * P * CKK <= ((size_t)1 << 29);      // a column gradient of at most 2 GiB
+        // one sum per remainder of the position modulo the stride, on channel-last copies
+        if (!dx_env && conv_cl_wanted(CL_DATA, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, chain_fits && as_chain < as_conv ? as_chain : as_conv))
+            return cl_conv_backward_data(dx, dy, w_ref, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, accumulate, s);
         if (chain_fits && (dx_env && dx_env[0] ? dx_env[1] == 'h' : as_conv >= as_chain))
             return conv_dx_chain(dx, dy, w_ref, N, C, H, W, O, K_h, K_w, stride, pad, Ho, Wo, w_batch, accumulate, stream);
         const size_t Hu = H + 2 * pad - K_h + 1, Wu = W + 2 * pad - K_w + 1, total = N * O * Hu * Wu;
@@ -4100,6 +4160,10 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
                                              size_t w_batch, void* stream) {
     if (!dw || !x || !dy) return set_error(NZHIP_E_INVALID, "nzhip_conv2d_backward_weights: null pointer");
     if (w_batch != 1 && w_batch != N) return set_error(NZHIP_E_SHAPE, "Shapes are not broadcast compatible.");
+    if (stride != 0 && K_h != 0 && K_w != 0 && H + 2 * pad >= K_h && W + 2 * pad >= K_w &&
+        !(K_h == 3 && K_w == 3 && stride == 1 && pad == 1 && C <= 4 && O <= 2 && W >= 4) &&                 // streamed
+        !(K_h == 1 && K_w == 1 && pad == 0) && conv_cl_wanted(CL_WEIGHTS, x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch))
+        return cl_conv_backward_weights(dw, x, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, reinterpret_cast<hipStream_t>(stream));
     // Images of fewer than 64 output pixels (7 x 7 outputs of a network's last stage) with shared weights: a product per
     // image has a contraction of 49, and a 128-pixel segment of the gather kernel is mostly padding. The column matrices
     // of all images follow each other in memory as ONE [N pixels, C K_h K_w] matrix, so the reference's own chain

@@ -1,0 +1,157 @@
+"""The Conv2d kernels on channel-last fp16 copies (forward, data gradient, weight gradient) against float64 convolutions of
+whole numbers, bit for bit, on every workgroup tile and with and without parts. The library reads NZHIP_CONV_CL and
+NZHIP_CONV_CL_PLAN ("tile,parts") per call, so layers and plans it would choose only at large sizes can be forced."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TILES = range(5)          # 64 x 64, 64 x 64 with two groups of waves, 128 x 64, 64 x 128, 128 x 128
+
+
+@pytest.fixture(scope="module")
+def nz():
+    import torch
+    assert torch.cuda.is_available(), "these tests need the MI355X"
+    from neuzephyr_amd import capi
+    capi.load()
+    return capi
+
+
+def whole(rng, *shape):
+    return rng.integers(-2, 3, shape).astype(np.float32)
+
+
+def embedded(a):
+    """a at an odd offset in NaN-filled storage: (storage, view)"""
+    import torch
+    buf = torch.full((a.size + 14,), float("nan"), device="cuda")
+    buf[7:7 + a.size] = torch.from_numpy(np.ascontiguousarray(a).ravel()).cuda()
+    return buf, buf[7:7 + a.size].view(a.shape)
+
+
+def untouched(buf, n):
+    import torch
+    return bool(torch.isnan(buf[:7]).all() and torch.isnan(buf[7 + n:]).all())
+
+
+def oihw(w, C, K_h, K_w):
+    """the library's [copy, 1, (c, r, s), o] as [copy][o][c][r][s]"""
+    return w.reshape(w.shape[0], C, K_h, K_w, w.shape[3]).transpose(0, 4, 1, 2, 3)
+
+
+def reference(x, w, dy, K_h, K_w, stride, pad):
+    """forward sums and both gradients in float64 (whole numbers: exact)"""
+    import torch
+    import torch.nn.functional as F
+    X = torch.from_numpy(x.astype(np.float64)).requires_grad_()
+    Wt = torch.from_numpy(oihw(w, x.shape[1], K_h, K_w).astype(np.float64).copy()).requires_grad_()
+    per = Wt.shape[0] > 1
+    y = torch.cat([F.conv2d(X[n:n + 1], Wt[n if per else 0], stride=stride, padding=pad) for n in range(x.shape[0])])
+    y.backward(torch.from_numpy(dy.astype(np.float64)))
+    dw = Wt.grad.numpy().transpose(0, 2, 3, 4, 1).reshape(w.shape)
+    return y.detach().numpy(), X.grad.numpy(), dw
+
+
+# N, C, H, W, O, K_h, K_w, stride, pad, copies
+LAYERS = [
+    (2, 8, 9, 11, 64, 3, 3, 1, 1, 1),          # one group of 8 channels; 198 pixels: part of every tile
+    (3, 13, 8, 8, 65, 3, 3, 1, 1, 3),          # 13 channels in 16, a copy per image, a second channel tile with one row
+    (1, 3, 7, 7, 5, 7, 7, 2, 3, 1),            # 3 channels in 8, 49 taps, more taps than pixels
+    (5, 20, 6, 5, 17, 5, 5, 1, 2, 1),          # kernel as large as the image
+    (2, 70, 14, 14, 130, 3, 3, 2, 1, 1),       # stride 2: four sums of 1, 2, 2 and 4 taps
+    (2, 33, 10, 13, 9, 3, 3, 3, 0, 2),         # stride 3, no padding, columns that no window reaches
+    (2, 17, 12, 12, 24, 2, 2, 3, 0, 1),        # kernel below the stride: sums without a tap
+    (1, 9, 1, 40, 8, 1, 1, 1, 0, 1),           # no window at all, one row
+    (4, 40, 4, 4, 72, 4, 4, 2, 3, 1),          # even kernel, padding up to its edge, 16-pixel images
+    (1, 130, 23, 3, 66, 3, 3, 1, 2, 1),        # output larger than the input
+]
+
+
+@pytest.mark.parametrize("layer", LAYERS)
+@pytest.mark.parametrize("tile", TILES)
+def test_every_tile_is_bit_exact_on_whole_numbers(nz, monkeypatch, tile, layer):
+    import torch
+    N, C, H, W, O, K_h, K_w, stride, pad, copies = layer
+    rng = np.random.default_rng(sum(layer) + tile)
+    Ho, Wo = (H + 2 * pad - K_h) // stride + 1, (W + 2 * pad - K_w) // stride + 1
+    x, w, dy = whole(rng, N, C, H, W), whole(rng, copies, 1, C * K_h * K_w, O), whole(rng, N, O, Ho, Wo)
+    b, old_dx, old_dw = whole(rng, 1, 1, Ho * Wo, O), whole(rng, *x.shape), whole(rng, *w.shape)
+    y64, dx64, dw64 = reference(x, w, dy, K_h, K_w, stride, pad)
+    bias = b.reshape(Ho * Wo, O).T.reshape(1, O, Ho, Wo)
+    monkeypatch.setenv("NZHIP_CONV_CL", "1")
+    X, Wt, DY, B = embedded(x)[1], embedded(w)[1], embedded(dy)[1], embedded(b)[1]
+    for parts in (1, 3):
+        monkeypatch.setenv("NZHIP_CONV_CL_PLAN", f"{tile},{parts}")
+        buf, out = embedded(np.full(y64.shape, np.nan, np.float32))
+        nz.conv2d_forward(X, Wt, B, K_h, K_w, stride, pad, bias_strides=(O, 1), relu=True, out=out)
+        assert np.array_equal(out.cpu().numpy(), np.maximum(y64 + bias, 0)) and untouched(buf, y64.size)
+        nz.conv2d_forward(X, Wt, torch.from_numpy(b.ravel()[:O].copy()).cuda(), K_h, K_w, stride, pad, bias_strides=(0, 1), out=out)
+        assert np.array_equal(out.cpu().numpy(), y64 + b.ravel()[:O].reshape(1, O, 1, 1))
+        nz.conv2d_forward(X, Wt, None, K_h, K_w, stride, pad, out=out)
+        assert np.array_equal(out.cpu().numpy(), y64) and untouched(buf, y64.size)
+        if K_h == K_w and pad <= K_h - 1:
+            buf, dx = embedded(np.full(x.shape, np.nan, np.float32))
+            nz.conv2d_backward_data(dx, DY, Wt, K_h, K_w, stride, pad, accumulate=False)
+            assert np.array_equal(dx.cpu().numpy(), dx64) and untouched(buf, x.size)
+            buf, dx = embedded(old_dx)
+            nz.conv2d_backward_data(dx, DY, Wt, K_h, K_w, stride, pad)
+            assert np.array_equal(dx.cpu().numpy(), dx64 + old_dx) and untouched(buf, x.size)
+        buf, dw = embedded(old_dw)
+        nz.conv2d_backward_weights(dw, X, DY, K_h, K_w, stride, pad)
+        assert np.array_equal(dw.cpu().numpy(), dw64 + old_dw) and untouched(buf, w.size)
+
+
+@pytest.mark.parametrize("special", [float("inf"), float("nan"), 7e4])             # 7e4 is infinite in fp16
+@pytest.mark.parametrize("K,stride,pad", [(3, 1, 1), (3, 2, 1), (5, 1, 2)])
+def test_a_special_value_stays_in_the_sums_it_is_a_term_of(nz, monkeypatch, special, K, stride, pad):
+    import torch
+    N, C, H, W, O = 2, 9, 11, 10, 20                                  # 9 channels in 16, pixel counts that fill no tile
+    rng = np.random.default_rng(5)
+    Ho, Wo = (H + 2 * pad - K) // stride + 1, (W + 2 * pad - K) // stride + 1
+    x = rng.integers(1, 3, (N, C, H, W)).astype(np.float32)
+    w, dy = rng.integers(1, 3, (1, 1, C * K * K, O)).astype(np.float32), rng.integers(1, 3, (N, O, Ho, Wo)).astype(np.float32)
+    monkeypatch.setenv("NZHIP_CONV_CL", "1")
+    at = (1, 4, H - 1, W - 1)                                         # the last pixel: beside the padding, before the next plane
+    xs, mark = x.copy(), np.zeros_like(x)
+    xs[at], mark[at] = special, 1
+    y_hit, _, dw_hit = reference(mark, w, dy, K, K, stride, pad)
+    y64, dx64, dw64 = reference(x, w, dy, K, K, stride, pad)
+    cu = lambda a: torch.from_numpy(a).cuda()
+    y = nz.conv2d_forward(cu(xs), cu(w), None, K, K, stride, pad).cpu().numpy()
+    assert np.array_equal(np.isfinite(y), y_hit == 0) and np.array_equal(y[y_hit == 0], y64[y_hit == 0])
+    dw = torch.zeros(w.shape, device="cuda")
+    nz.conv2d_backward_weights(dw, cu(xs), cu(dy), K, K, stride, pad)
+    dw = dw.cpu().numpy()
+    assert np.array_equal(np.isfinite(dw), dw_hit == 0) and np.array_equal(dw[dw_hit == 0], dw64[dw_hit == 0])
+    dys, mark = dy.copy(), np.zeros_like(dy)
+    dys[1, 3, Ho - 1, Wo - 1], mark[1, 3, Ho - 1, Wo - 1] = special, 1
+    _, dx_hit, _ = reference(x, w, mark, K, K, stride, pad)
+    dx = nz.conv2d_backward_data(torch.empty(x.shape, device="cuda"), cu(dys), cu(w), K, K, stride, pad, accumulate=False).cpu().numpy()
+    assert np.array_equal(np.isfinite(dx), dx_hit == 0) and np.array_equal(dx[dx_hit == 0], dx64[dx_hit == 0])
+    dw = torch.zeros(w.shape, device="cuda")
+    nz.conv2d_backward_weights(dw, cu(x), cu(dys), K, K, stride, pad)
+    dw = dw.cpu().numpy()
+    dw_hit = np.broadcast_to(np.arange(O) == 3, dw.shape)              # padding is a term too: the column matrix holds zeros there, 0 x Inf
+    assert np.array_equal(np.isfinite(dw), ~dw_hit) and np.array_equal(dw[~dw_hit], dw64[~dw_hit])
+
+
+@pytest.mark.parametrize("layer", [(16, 256, 14, 14, 256, 3, 1, 1, 1), (2, 208, 16, 16, 144, 5, 1, 2, 2), (4, 64, 48, 48, 45, 7, 2, 3, 1),
+                                   (1, 16, 192, 96, 24, 3, 2, 1, 1)])
+def test_chosen_plans_are_bit_exact_on_whole_numbers(nz, layer):
+    import torch
+    N, C, H, W, O, K, stride, pad, copies = layer
+    rng = np.random.default_rng(sum(layer))
+    Ho, Wo = (H + 2 * pad - K) // stride + 1, (W + 2 * pad - K) // stride + 1
+    x, w, dy = whole(rng, N, C, H, W), whole(rng, copies, 1, C * K * K, O), whole(rng, N, O, Ho, Wo)
+    y64, dx64, dw64 = reference(x, w, dy, K, K, stride, pad)
+    cu = lambda a: torch.from_numpy(a).cuda()
+    handle, weights = nz.Prepared(), cu(w)
+    for _ in range(2):                                                # the second time on the kept copy of the weights
+        y = nz.conv2d_forward(cu(x), weights, None, K, K, stride, pad, prepared_w=handle)
+        assert np.array_equal(y.cpu().numpy(), y64)
+    dx = nz.conv2d_backward_data(torch.empty(x.shape, device="cuda"), cu(dy), cu(w), K, K, stride, pad, accumulate=False)
+    assert np.array_equal(dx.cpu().numpy(), dx64)
+    dw = torch.zeros(w.shape, device="cuda")
+    nz.conv2d_backward_weights(dw, cu(x), cu(dy), K, K, stride, pad)
+    assert np.array_equal(dw.cpu().numpy(), dw64)
