@@ -43,6 +43,13 @@ struct ClPrepJob {
     int ptiles, ctiles, blocks;
 };
 struct ClPrepArgs { ClPrepJob job[2]; };
+static int round8(int c) { return (c + 7) / 8 * 8; }
+// Elements from one row of a copy to the next, for rows of n: an odd number of 128-byte lines. A tile loads the same lines of 64 rows at
+// once, and the channels of a level-2 cache take 256 bytes in turn: rows an even number of lines apart crowd on half of them and fewer.
+static int cl_pitch(int n) {
+    const int lines = (n + 63) / 64;
+    return n <= 64 ? round8(n) : (lines | 1) * 64;
+}
 
 constexpr int CLP_PX = 64, CLP_CH = 64, CLP_PITCH = CLP_CH * 2 + 16;
 
@@ -70,7 +77,8 @@ __global__ __launch_bounds__(256) void cl_prep_kernel(const ClPrepArgs a) {
 #pragma unroll
             for (int e = 0; e < 8; e++) h[e] = c + e < j.C ? (_Float16)s[e] : (_Float16)0.f;
         }
-        *reinterpret_cast<half8_t*>(j.dst + u * 8) = h;
+        const long set = row / j.T;
+        *reinterpret_cast<half8_t*>(j.dst + set * j.dp + (row - set * j.T) * j.Cp + c) = h;
         return;
     }
     const int per = j.ptiles * j.ctiles;
@@ -113,7 +121,7 @@ static void prep_planes(ClPrepJob& j, const float* src, _Float16* dst, long imag
     j.src = src; j.dst = dst;
     j.T = 1; j.C = C; j.Cp = Cp; j.H = H; j.W = W; j.Hp = Hp; j.Wp = Wp; j.pt = pt; j.pl = pl;
     j.s1 = (long)C * H * W; j.sc = (long)H * W;
-    j.d1 = (long)Hp * Wp * Cp; j.dp = Cp;
+    j.dp = cl_pitch(C); j.d1 = (long)Hp * Wp * j.dp;
     j.ptiles = (Hp * Wp + CLP_PX - 1) / CLP_PX; j.ctiles = (Cp + CLP_CH - 1) / CLP_CH;
     j.blocks = (int)(images * j.ptiles * j.ctiles);
 }
@@ -123,15 +131,15 @@ static void prep_weights(ClPrepJob& j, const float* src, _Float16* dst, long cop
     j.src = src; j.dst = dst;
     j.T = taps; j.C = C; j.Cp = Cp; j.H = 1; j.W = O; j.Hp = 1; j.Wp = O;
     j.s1 = (long)C * taps * O; j.s2 = O; j.sc = (long)taps * O;
-    j.d1 = (long)O * taps * Cp; j.d2 = Cp; j.dp = (long)taps * Cp;
+    j.dp = cl_pitch(taps * Cp); j.d1 = (long)O * j.dp; j.d2 = Cp;
     j.ptiles = (O + CLP_PX - 1) / CLP_PX; j.ctiles = (Cp + CLP_CH - 1) / CLP_CH;
     j.blocks = (int)(copies * taps * j.ptiles * j.ctiles);
 }
-// rows of C elements -> rows of Cp
-static void prep_rows(ClPrepJob& j, const float* src, _Float16* dst, long rows, int C, int Cp) {
+// sets of `taps` rows of C elements -> the set's rows of Cp one after the other
+static void prep_rows(ClPrepJob& j, const float* src, _Float16* dst, long rows, int taps, int C, int Cp) {
     j = {};
     j.src = src; j.dst = dst;
-    j.T = 1; j.C = C; j.Cp = Cp; j.H = (int)rows;
+    j.T = taps; j.C = C; j.Cp = Cp; j.H = (int)rows; j.dp = cl_pitch(taps * Cp);
     j.blocks = (int)((rows * (Cp / 8) + 255) / 256);
 }
 static int prep_launch(const ClPrepArgs& a, hipStream_t s) {
@@ -427,7 +435,7 @@ struct ClDwArgs {
     const _Float16* dz;                 // channel-last, pixels of all images one after the other
     float* dw;
     float* partial;                     // [part][dw] bare sums, or null
-    int units, cu, Kw, C, taps, O, Op;  // units (tap, 8 channels); per tap
+    int units, cu, Kw, C, taps, O, Op, Os;  // units (tap, 8 channels); per tap; dz channels in whole units, dz row
     int dr, ds;                         // x copy offset between tap rows / columns, elements
     int Ho, Wo, pixels;                 // pixels of the contraction: of all images, or of one with a weight copy per image
     unsigned step_w, step_h;            // x copy offset between output columns / rows, elements
@@ -496,7 +504,7 @@ __global__ __launch_bounds__(T::THREADS) void cl_dw_kernel(const ClDwArgs p) {
 #pragma unroll
         for (int q = 0; q < Q; q++) {
             const bool in = px[q] < limit;
-            const unsigned bx = at[q], bz = (unsigned)px[q] * (unsigned)p.Op * 2u;
+            const unsigned bx = at[q], bz = (unsigned)px[q] * (unsigned)p.Os * 2u;
 #pragma unroll
             for (int t = 0; t < MT; t++) cl_load(rx, sa + t * 8192 + q * 1024, in ? bx + off_x[t][q] : CL_OUT);
 #pragma unroll
@@ -627,7 +635,6 @@ __global__ __launch_bounds__(T::THREADS) void cl_dw_kernel(const ClDwArgs p) {
 }
 
 // ---- host side ----------------------------------------------------------------------------------------------------------
-static int round8(int c) { return (c + 7) / 8 * 8; }
 
 struct ClPlan { int tile, parts; };                                 // tile: index into the list of cl_pick
 struct ClTileShape { int bm, bn, kg; };
@@ -774,8 +781,8 @@ static int conv_product(ClArgs& a, int copies, hipStream_t s) {
 // 0: not, 1: yes, 2: yes and to be taken whatever the layer.
 int cl_conv_fits(ClDirection dir, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad, size_t w_batch) {
     if (!N || !C || !O || (dir == CL_DATA && stride > 3) || K_h > 64 || K_w > 64 || H > 16384 || W > 16384 || pad > 64 || stride > 64 || C > 65535 || O > 65535 || N > 32768) return 0;
-    const size_t taps = K_h * K_w, Cp = (C + 7) / 8 * 8, Op = (O + 7) / 8 * 8, Hp = H + 2 * pad + K_h, Wp = W + 2 * pad + K_w, lim = 1u << 30;
-    if (!(N * Hp * Wp * Cp < lim && N * Hp * Wp * Op < lim && w_batch * taps * Cp * O < lim && w_batch * taps * Op * C < lim &&
+    const size_t taps = K_h * K_w, Cp = (C + 7) / 8 * 8, Op = (O + 7) / 8 * 8, Cs = C + 128, Os = O + 128, Hp = H + 2 * pad + K_h, Wp = W + 2 * pad + K_w, lim = 1u << 30;
+    if (!(N * Hp * Wp * Cs < lim && N * Hp * Wp * Os < lim && w_batch * (taps * Cp + 128) * O < lim && w_batch * (taps * Op + 128) * C < lim &&
            N * (H + 2 * pad) * (W + 2 * pad) * (C > O ? C : O) < lim / 2 && w_batch * taps * C * O < lim && taps * Cp / 8 <= 3500 && taps * Op / 8 <= 3500)) return 0;
     const char* env = getenv("NZHIP_CONV_CL");                       // read per call (tests, benchmarking): 0 never, 1 wherever they fit
     return env ? (atoi(env) ? 2 : 0) : 1;
@@ -785,14 +792,15 @@ int cl_conv_fits(ClDirection dir, size_t N, size_t C, size_t H, size_t W, size_t
 static void forward_args(ClArgs& a, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad, size_t w_batch) {
     const int Ho = (int)((H + 2 * pad - K_h) / stride + 1), Wo = (int)((W + 2 * pad - K_w) / stride + 1);
     const int Cp = round8((int)C), taps = (int)(K_h * K_w), Hp = (int)(H + 2 * pad), Wp = (int)(W + 2 * pad);
-    a.M = (int)O; a.w_row = taps * Cp; a.cu = Cp / 8; a.Kw = (int)K_w;
-    a.step_h = (int)stride * Wp * Cp; a.step_w = (int)stride * Cp;
+    const int Cs = cl_pitch((int)C);
+    a.M = (int)O; a.w_row = cl_pitch(taps * Cp); a.cu = Cp / 8; a.Kw = (int)K_w;
+    a.step_h = (int)stride * Wp * Cs; a.step_w = (int)stride * Cs;
     a.images = w_batch > 1 ? 1 : (int)N;
-    a.x_img = (long)Hp * Wp * Cp; a.w_img = (long)O * taps * Cp; a.y_img = (long)O * Ho * Wo;
+    a.x_img = (long)Hp * Wp * Cs; a.w_img = (long)O * a.w_row; a.y_img = (long)O * Ho * Wo;
     a.w_bytes = (unsigned)(a.w_img * 2); a.x_bytes = (unsigned)(a.images * a.x_img * 2);
     a.plane = (long)Ho * Wo; a.y_total = (long)N * a.y_img;
     a.n_classes = 1;
-    a.cls[0] = {(int)K_h, (int)K_w, 0, 1, 0, 1, Wp * Cp, Cp, Ho, Wo, 0, 0, Wo, 1, 0, {}, {}, {}};
+    a.cls[0] = {(int)K_h, (int)K_w, 0, 1, 0, 1, Wp * Cs, Cs, Ho, Wo, 0, 0, Wo, 1, 0, {}, {}, {}};
 }
 
 static void data_args(ClArgs& a, int (&edge)[4], size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad,
@@ -818,17 +826,18 @@ static void data_args(ClArgs& a, int (&edge)[4], size_t N, size_t C, size_t H, s
         if (v.n) { edge[2] = std::max(edge[2], v.t - 1 - v.lo); edge[3] = std::max(edge[3], v.lo + v.n - Wo); }
     }
     const int Hp = Ho + edge[0] + edge[1], Wp = Wo + edge[2] + edge[3];
-    a.M = (int)C; a.w_row = taps * Op; a.cu = Op / 8; a.Kw = (int)K_w;
-    a.step_h = Wp * Op; a.step_w = Op;
+    const int Os = cl_pitch((int)O);
+    a.M = (int)C; a.w_row = cl_pitch(taps * Op); a.cu = Op / 8; a.Kw = (int)K_w;
+    a.step_h = Wp * Os; a.step_w = Os;
     a.images = w_batch > 1 ? 1 : (int)N;
-    a.x_img = (long)Hp * Wp * Op; a.w_img = (long)C * taps * Op; a.y_img = (long)C * H * W;
+    a.x_img = (long)Hp * Wp * Os; a.w_img = (long)C * a.w_row; a.y_img = (long)C * H * W;
     a.w_bytes = (unsigned)(a.w_img * 2); a.x_bytes = (unsigned)(a.images * a.x_img * 2);
     a.plane = (long)H * W; a.y_total = (long)N * a.y_img;
     for (int i = 0; i < st; i++)
         for (int j = 0; j < st; j++) {
             const Side h = side(i, (int)H, (int)K_h), v = side(j, (int)W, (int)K_w);
             if (!h.n || !v.n) continue;
-            a.cls[a.n_classes++] = {h.t, v.t, i, st, j, st, -Wp * Op, -Op, h.n, v.n, ((h.lo + edge[0]) * Wp + v.lo + edge[2]) * Op,
+            a.cls[a.n_classes++] = {h.t, v.t, i, st, j, st, -Wp * Os, -Os, h.n, v.n, ((h.lo + edge[0]) * Wp + v.lo + edge[2]) * Os,
                                     (st * h.lo + i - (int)pad) * (int)W + st * v.lo + j - (int)pad, st * (int)W, st, 0, {}, {}, {}};
         }
 }
@@ -878,7 +887,7 @@ int cl_conv_backward_data(float* dx, const float* dy, const float* w, size_t N, 
     }
     ClPrepArgs pa = {};
     prep_planes(pa.job[0], dy, zc, (long)N, (int)O, Op, Ho, Wo, Ho + edge[0] + edge[1], Wo + edge[2] + edge[3], edge[0], edge[2]);
-    prep_rows(pa.job[1], w, wc, (long)(w_batch * C * K_h * K_w), (int)O, Op);
+    prep_rows(pa.job[1], w, wc, (long)(w_batch * C * K_h * K_w), (int)(K_h * K_w), (int)O, Op);
     rc = prep_launch(pa, s);
     if (rc == NZHIP_OK) {
         a.w = wc; a.x = zc; a.y = dx;
@@ -921,7 +930,8 @@ int cl_conv_backward_weights(float* dw, const float* x, const float* dy, size_t 
                              size_t stride, size_t pad, size_t w_batch, hipStream_t s) {
     const int Ho = (int)((H + 2 * pad - K_h) / stride + 1), Wo = (int)((W + 2 * pad - K_w) / stride + 1);
     const int Cp = round8((int)C), Op = round8((int)O), taps = (int)(K_h * K_w), Hp = (int)(H + 2 * pad), Wp = (int)(W + 2 * pad);
-    const size_t x_elems = N * Hp * Wp * (size_t)Cp, z_elems = N * Ho * Wo * (size_t)Op;
+    const int Cs = cl_pitch((int)C), Os = cl_pitch((int)O);
+    const size_t x_elems = N * Hp * Wp * (size_t)Cs, z_elems = N * Ho * Wo * (size_t)Os;
     _Float16* xc = nullptr;
     if (int rc = workspace_alloc(reinterpret_cast<void**>(&xc), (x_elems + z_elems) * 2, s)) return rc;      // (rows of whole 16 bytes)
     _Float16* zc = xc + x_elems;
@@ -935,10 +945,10 @@ int cl_conv_backward_weights(float* dw, const float* x, const float* dy, size_t 
         const int copies = w_batch > 1 ? (int)N : 1, images = w_batch > 1 ? 1 : (int)N;
         a.x = xc; a.dz = zc; a.dw = dw;
         a.cu = Cp / 8; a.units = taps * a.cu; a.Kw = (int)K_w; a.C = (int)C; a.taps = taps; a.O = (int)O; a.Op = Op;
-        a.dr = Wp * Cp; a.ds = Cp;
+        a.dr = Wp * Cs; a.ds = Cs; a.Os = Os;
         a.Ho = Ho; a.Wo = Wo; a.pixels = images * Ho * Wo;
-        a.step_h = (unsigned)(stride * Wp * Cp); a.step_w = (unsigned)(stride * Cp); a.x_img = (long)Hp * Wp * Cp;
-        a.z_img = (long)Ho * Wo * Op; a.dw_img = (long)C * taps * O; a.total = copies * a.dw_img;
+        a.step_h = (unsigned)(stride * Wp * Cs); a.step_w = (unsigned)(stride * Cs); a.x_img = (long)Hp * Wp * Cs;
+        a.z_img = (long)Ho * Wo * Os; a.dw_img = (long)C * taps * O; a.total = copies * a.dw_img;
         a.x_bytes = (unsigned)(images * a.x_img * 2); a.z_bytes = (unsigned)(images * a.z_img * 2);
         ClPlan pl = {0, 1};
         cl_plan(dw_work(N, C, O, taps, (size_t)Ho * Wo, w_batch), pl);
