@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
+#include <utility>
 
 #include "nzhip_internal.h"
 
@@ -433,6 +434,13 @@ int nzhip_gemm(const nzhip_gemm_desc* desc, void* stream) {
 
 }  // extern "C"
 
+// Estimated time of a product on its own, in us; 0 for those that stream an operand.
+static double gemm_single_cost(const nzhip_gemm_desc& d) {
+    if (gemm_thin_applicable(d) || gemm_skinny_applicable(d)) return 0.0;
+    if (gemm_h16_applicable(d)) return 6.0 + 6.0 * (double)d.K * (double)(d.M + d.N) / 5e6 + 2.0 * d.M * d.N * d.K / 0.78e9;
+    return gemm_fused_plan(d).cost_us;
+}
+
 // The route choice behind nzhip_gemm, for a validated descriptor with M, N > 0.
 static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s) {
     if (d.K == 0) {
@@ -452,8 +460,17 @@ static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s) {
     static const char* coop_env = getenv("NZHIP_H16_COOP");              // 0: never the single-kernel route (benchmarking only)
     const bool allow_coop = !(coop_env && atoi(coop_env) == 0);
     if (!force_fused && allow_coop && gemm_h16_coop_applicable(d)) return gemm_h16_coop_dispatch(d, s);
-    if (!force_fused && (force_h16 || gemm_h16_applicable(d))) return gemm_h16_dispatch(d, s);
+    if (!force_fused && (force_h16 || gemm_h16_applicable(d))) {
+        // On rows of C that are no whole 16-byte pieces the block images' kernel stores element by element, and short of 2.8e10 flops its 256-wide
+        // tiles are few: there the products on plain copies (2831 x 1296 x 2781 77 -> 43 us, 5001 x 999 x 5001 141 -> 106, 4192 x 3031 x 7535
+        // 285 -> 276; 2128 x 1984 x 1904 44.5 -> 34, 4096 x 1024 x 2048 35 -> 33; above, 4096 x 1024 x 4096 58 / 65, 6864 x 864 x 3216 69 / 75).
+        // A caller that keeps B's image keeps this one.
+        const bool plain = !force_h16 && !image_kept_by_caller(PREPARED_GEMM_B) && (((d.N | d.ldc) & 3) != 0 || 2.0 * d.M * d.N * d.K < 2.8e10);
+        if (plain && gemm_copy_wanted(&d, 1, 1e30)) return gemm_copy_run(&d, 1, s);
+        return gemm_h16_dispatch(d, s);
+    }
     GemmPlan plan = gemm_fused_plan(d);
+    if (gemm_copy_wanted(&d, 1, plan.cost_us)) return gemm_copy_run(&d, 1, s);
     if (gemm_trace())
         fprintf(stderr, "nzhip_gemm %ld x %ld x %ld batch %ld x %ld: fused kernel, %d^2 tiles, %ld chunk(s) of %ld, model %.1f us\n",
                 (long)d.M, (long)d.K, (long)d.N, (long)d.batch_n, (long)d.batch_c, plan.tile,
@@ -719,9 +736,17 @@ struct BwdOperand {
 // Reductions are folded into the contraction (K' = members x K, one launch) when both operands are
 // laid out so that the member index continues the k index; otherwise the members are added one
 // launch after the other, which fixes the summation order.
+// `only`: nothing is launched; if the whole sum is one unbatched product, that product is put there and the answer is NZHIP_OK.
+constexpr int NOT_ONE_PRODUCT = 1;
 static int accumulate_products(float* C, int64_t ldc, int64_t c_sn, int64_t c_sc, BwdOperand A, BwdOperand B, int64_t M,
-                        int64_t N, int64_t K, int64_t bn, int64_t bc, void* stream) {
-    if (bn == 0 || bc == 0 || M == 0 || N == 0) return NZHIP_OK;
+                        int64_t N, int64_t K, int64_t bn, int64_t bc, void* stream, nzhip_gemm_desc* only = nullptr) {
+    if (bn == 0 || bc == 0 || M == 0 || N == 0) return only ? NOT_ONE_PRODUCT : NZHIP_OK;
+    auto issue = [&](const nzhip_gemm_desc& g) {
+        if (!only) return nzhip_gemm(&g, stream);
+        if (g.batch_n * g.batch_c != 1) return NOT_ONE_PRODUCT;
+        *only = g;
+        return (int)NZHIP_OK;
+    };
     auto launch = [&](const float* a, const float* b, float* c, int64_t k, int la, int64_t lda, int lb, int64_t ldb,
                       int64_t nb_n, int64_t nb_c, int64_t csn, int64_t csc) {
         nzhip_gemm_desc g = {};
@@ -736,7 +761,7 @@ static int accumulate_products(float* C, int64_t ldc, int64_t c_sn, int64_t c_sc
         g.bias = c;
         g.bias_stride_row = ldc; g.bias_stride_col = 1;
         g.bias_stride_n = csn; g.bias_stride_c = csc;
-        return nzhip_gemm(&g, stream);
+        return issue(g);
     };
     const bool red_n = c_sn == 0 && bn > 1, red_c = c_sc == 0 && bc > 1;
     // distance between consecutive batch members of an operand, if it is the same for all of them
@@ -763,7 +788,7 @@ static int accumulate_products(float* C, int64_t ldc, int64_t c_sn, int64_t c_sc
             g.b_layout = A.layout == NZHIP_LAYOUT_ROW ? NZHIP_LAYOUT_TRANS : NZHIP_LAYOUT_ROW;
             g.batch_n = g.batch_c = 1;
             g.bias = C; g.bias_stride_row = sc_; g.bias_stride_col = 1;
-            return nzhip_gemm(&g, stream);
+            return issue(g);
         }
         if (M == 1 && b_shared && uc && ua && sc_ >= N && sa >= K && (A.layout == NZHIP_LAYOUT_ROW || A.ld == 1)) {
             // C_t[1,N] = A_t[1,K] * B[K,N]   ->   Cmat[T,N] = Amat[T,K] * B
@@ -774,7 +799,7 @@ static int accumulate_products(float* C, int64_t ldc, int64_t c_sn, int64_t c_sc
             g.a_layout = NZHIP_LAYOUT_ROW; g.b_layout = B.layout;
             g.batch_n = g.batch_c = 1;
             g.bias = C; g.bias_stride_row = sc_; g.bias_stride_col = 1;
-            return nzhip_gemm(&g, stream);
+            return issue(g);
         }
     }
     if (!red_n && !red_c) {
@@ -808,6 +833,7 @@ static int accumulate_products(float* C, int64_t ldc, int64_t c_sn, int64_t c_sc
             return rc;
         }
     }
+    if (only) return NOT_ONE_PRODUCT;
     // members one after the other; a dimension that does not reduce stays a batch of the launch
     for (int64_t i = 0; i < (red_n ? bn : 1); i++)
         for (int64_t j = 0; j < (red_c ? bc : 1); j++) {
@@ -818,6 +844,27 @@ static int accumulate_products(float* C, int64_t ldc, int64_t c_sn, int64_t c_sc
                 return rc;
         }
     return NZHIP_OK;
+}
+
+// whether two products write nothing the other one reads or writes, nor their own operands
+static bool apart(const nzhip_gemm_desc& p, const nzhip_gemm_desc& q) {
+    struct Range { const float *lo, *hi; };
+    auto rows = [](const float* x, int64_t ld, int64_t n, int64_t len) { return Range{x, x + (n - 1) * ld + len}; };
+    auto meet = [](const Range& a, const Range& b) { return a.lo < b.hi && b.lo < a.hi; };
+    Range in[4], out[2];
+    const nzhip_gemm_desc* d[2] = {&p, &q};
+    for (int i = 0; i < 2; i++) {
+        const nzhip_gemm_desc& g = *d[i];
+        const bool ta = g.a_layout == NZHIP_LAYOUT_TRANS, tb = g.b_layout == NZHIP_LAYOUT_TRANS;
+        if (g.K == 0) return false;
+        in[2 * i] = rows(g.A, g.lda, ta ? g.K : g.M, ta ? g.M : g.K);
+        in[2 * i + 1] = rows(g.B, g.ldb, tb ? g.N : g.K, tb ? g.K : g.N);
+        out[i] = rows(g.C, g.ldc, g.M, g.N);
+    }
+    for (const Range& o : out)
+        for (const Range& r : in)
+            if (meet(o, r)) return false;
+    return !meet(out[0], out[1]);
 }
 
 inline int64_t bstride_n(const size_t s[4]) { return s[0] > 1 ? (int64_t)(s[1] * s[2] * s[3]) : 0; }
@@ -844,6 +891,19 @@ int nzhip_matmul_backward(float* dA, float* dB, const float* A, const float* B, 
         return set_error(NZHIP_E_SHAPE, "nzhip_matmul_backward: shapes do not describe C = A * B");
     const int64_t bn = (int64_t)sC[0], bc = (int64_t)sC[1];
     const BwdOperand g = {dC, NZHIP_LAYOUT_ROW, N, (int64_t)(sC[1] * sC[2] * sC[3]), (int64_t)(sC[2] * sC[3])};
+    if (dA && dB) {
+        // Both gradients as one product each (a Linear layer): rounded once and multiplied in one launch, where that is faster than one
+        // after the other. dA and dB may overlap neither each other nor an operand then, since both are written in no order.
+        const BwdOperand bt = {B, NZHIP_LAYOUT_TRANS, N, bstride_n(sB), bstride_c(sB)}, at = {A, NZHIP_LAYOUT_TRANS, K, bstride_n(sA), bstride_c(sA)};
+        nzhip_gemm_desc d[2];
+        if (accumulate_products(dA, K, bstride_n(sA), bstride_c(sA), g, bt, M, K, N, bn, bc, stream, &d[0]) == NZHIP_OK &&
+            accumulate_products(dB, N, bstride_n(sB), bstride_c(sB), at, g, K, N, M, bn, bc, stream, &d[1]) == NZHIP_OK &&
+            validate_gemm(d[0]) == NZHIP_OK && validate_gemm(d[1]) == NZHIP_OK && apart(d[0], d[1])) {
+            // the product whose shared operand runs along its rows first
+            if (d[0].a_layout == NZHIP_LAYOUT_TRANS) std::swap(d[0], d[1]);
+            if (gemm_copy_wanted(d, 2, gemm_single_cost(d[0]) + gemm_single_cost(d[1]))) return gemm_copy_run(d, 2, as_stream(stream));
+        }
+    }
     if (dA) {                                              // dA += dC * B^T   (src/Nodes.cu:171-175)
         const BwdOperand bt = {B, NZHIP_LAYOUT_TRANS, N, bstride_n(sB), bstride_c(sB)};
         if (int rc = accumulate_products(dA, K, bstride_n(sA), bstride_c(sA), g, bt, M, K, N, bn, bc, stream)) return rc;
