@@ -23,6 +23,7 @@
 #include "nzhip_internal.h"
 #include "nzhip_lds_tiles.h"
 #include "nzhip_pieces.h"
+#include "nzhip_plan_cache.h"
 
 namespace nzhip {
 
@@ -587,17 +588,14 @@ static int cl_pick(int tile, F go) {
 // How a product is cut: `list` workgroup tiles of each kind (CL_TILES) for one weight copy, `steps` k steps of 8 units or 64 pixels in
 // the longest sum and `mean` on average (the classes of a data gradient differ), `copies` weight copies, `out` bytes of result.
 struct ClWork {
-    bool dw;
-    long tiles[5];
-    int copies;
-    long steps;
+    long dw, tiles[5], copies, steps;
     double mean, prep, out;             // prep: bytes the first launch moves
 };
 
 // Estimated time in us, and the plan it is for. Measured on 249 (layer, direction) pairs with 15 plans each (layers of 1 to 32 images, 3 to 512
 // channels, 7 x 7 to 224 x 224, kernels 3, 5 and 7, strides 1 and 2) and fitted: the plan chosen is 1.3 % slower than the best of the 15
 // in the geometric mean, 16 % at worst. A k step of a workgroup alone on its CU takes `alone`, of two that share one `pair` together.
-static double cl_plan(const ClWork& w, ClPlan& best) {
+static double cl_plan_search(const ClWork& w, ClPlan& best) {
     static const double alone[2][5] = {{0.191, 0.295, 0.346, 0.423, 0.484}, {0.358, 0.515, 0.493, 0.468, 0.575}};
     static const double pair[2][5] = {{0.375, 0.360, 0.579, 0.461, 0.500}, {0.441, 0.560, 0.633, 0.427, 0.600}};
     static const double first[5] = {4.2, 5.1, 4.2, 4.2, 4.8};        // launch, first request and result of a workgroup
@@ -629,6 +627,16 @@ static double cl_plan(const ClWork& w, ClPlan& best) {
         }
     }
     return 3.9 + w.prep / 5e6 + least;
+}
+static double cl_plan(const ClWork& w, ClPlan& best) {
+    struct Found { ClPlan plan; double cost; };
+    struct Key { ClWork w; long cus; };
+    static thread_local PlanCache<Key, Found> cache;
+    bool known;
+    Found& f = cache.at(Key{w, device_cu_count()}, known);
+    if (!known) f.cost = cl_plan_search(w, f.plan);
+    best = f.plan;
+    return f.cost;
 }
 // read per call (tests, benchmarking): "tile,parts"
 static void plan_env(ClPlan& pl) {
@@ -836,7 +844,7 @@ int cl_conv_backward_data(float* dx, const float* dy, const float* w, size_t N, 
 static ClWork dw_work(size_t N, size_t C, size_t O, size_t taps, size_t P, size_t w_batch) {
     ClWork w = {};
     const long rows = (long)(taps * ((C + 7) / 8) * 8), pixels = (long)((w_batch > 1 ? 1 : N) * P);
-    w.dw = true;
+    w.dw = 1;
     w.copies = w_batch > 1 ? (int)N : 1;
     for (int t = 0; t < 5; t++) w.tiles[t] = ((rows + CL_TILES[t].bm - 1) / CL_TILES[t].bm) * (((long)O + CL_TILES[t].bn - 1) / CL_TILES[t].bn);
     w.steps = (pixels + 63) / 64;

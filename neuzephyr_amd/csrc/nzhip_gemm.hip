@@ -19,6 +19,7 @@
 
 #include "nzhip_internal.h"
 #include "nzhip_pieces.h"
+#include "nzhip_plan_cache.h"
 
 namespace nzhip {
 
@@ -517,7 +518,7 @@ static FusedCostInput fused_cost_input(const nzhip_gemm_desc& d) {
     return {d.M, d.N, d.K, d.batch_n * d.batch_c, (double)device_cu_count(), gemm_vec_legal(d)};
 }
 
-GemmPlan gemm_fused_plan(const nzhip_gemm_desc& d) {
+static GemmPlan gemm_fused_plan_search(const nzhip_gemm_desc& d) {
     const FusedCostInput q = fused_cost_input(d);
     GemmPlan best = {128, 1, d.K, 0.0};
     double best_cost = fused_cost_us(q, 128, 1, d.K);
@@ -543,6 +544,15 @@ GemmPlan gemm_fused_plan(const nzhip_gemm_desc& d) {
     }
     best.cost_us = best_cost;
     return best;
+}
+
+GemmPlan gemm_fused_plan(const nzhip_gemm_desc& d) {
+    struct Key { int64_t m, n, k, batch_n, batch_c, aligned, cus, scratch; };
+    static thread_local PlanCache<Key, GemmPlan> cache;
+    bool known;
+    GemmPlan& plan = cache.at(Key{d.M, d.N, d.K, d.batch_n, d.batch_c, gemm_vec_legal(d), device_cu_count(), (int64_t)workspace_limit()}, known);
+    if (!known) plan = gemm_fused_plan_search(d);
+    return plan;
 }
 
 bool gemm_small_tile(const nzhip_gemm_desc& d) {

@@ -16,6 +16,7 @@
 #include "nzhip_internal.h"
 #include "nzhip_lds_tiles.h"
 #include "nzhip_pieces.h"
+#include "nzhip_plan_cache.h"
 
 namespace nzhip {
 
@@ -303,7 +304,7 @@ static bool copy_plan_env(CopyPlan& pl) {
 // Estimated time in us and the plan it is for, fitted on 66 products and pairs of 16 to 4096 rows, columns and k with 15 plans each: the plan
 // chosen is 1.4 % slower than the best of the 15 in the geometric mean, 13 % at worst. A k step (64) of a workgroup alone on its CU
 // takes `alone`, of two that share one `pair` together.
-static CopyPlan copy_plan(const nzhip_gemm_desc* d, int count, double* cost) {
+static CopyPlan copy_plan_search(const nzhip_gemm_desc* d, int count, double* cost) {
     static const double alone[COPY_TILES] = {0.207, 0.482, 0.385, 0.296, 0.530, 0.800}, pair[COPY_TILES] = {0.329, 0.482, 0.453, 0.469, 0.530, 0.800};
     static const double first[COPY_TILES] = {4.4, 4.7, 4.1, 4.3, 5.9, 6.0};      // launch, first request and result of a workgroup
     static const int cuts[] = {1, 2, 3, 4, 6, 8, 12, 16};
@@ -344,8 +345,21 @@ static CopyPlan copy_plan(const nzhip_gemm_desc* d, int count, double* cost) {
             }
         }
     }
-    if (cost) *cost = 2.8 + rounding / 7.9e6 + least;
+    *cost = 2.8 + rounding / 7.9e6 + least;
     return best;
+}
+
+static CopyPlan copy_plan(const nzhip_gemm_desc* d, int count, double* cost) {
+    struct Key { int64_t count, m, n, k, m2, n2, k2; };
+    struct Found { CopyPlan plan; double cost; };
+    static thread_local PlanCache<Key, Found> cache;
+    const bool pair = count == 2;
+    const Key key = {count + (int64_t)device_cu_count() * 4, d[0].M, d[0].N, d[0].K, pair ? d[1].M : 0, pair ? d[1].N : 0, pair ? d[1].K : 0};
+    bool known;
+    Found& f = cache.at(key, known);
+    if (!known) f.plan = copy_plan_search(d, count, &f.cost);
+    if (cost) *cost = f.cost;
+    return f.plan;
 }
 
 // halfs of the copy of an operand of `rows` rows, a whole number of 128-byte lines
