@@ -482,11 +482,13 @@ bool gemm_copy_wanted(const nzhip_gemm_desc* d, int count, double other_us) {
     copy_plan_env(pl);
     if (copy_bytes(d, count, pl) > workspace_limit()) return false;   // in the call that allocates nothing the copies have to fit its scratch
     if (env) return true;
-    // One product has to be ahead by an eighth, which is how far off the other estimate is where it matters (256 x 4096 x 4096 estimated
-    // at 39, 31 measured, 33 here). Ahead: 1235 x 1116 x 1766 31.1 -> 19.5 us, 2800 x 1312 x 928 35.2 -> 24.0, 1000 x 777 x 513 15.4 -> 11.7; not
-    // taken: 1024^3 13.4 / 13.7, 256^3 6.9 / 9.5, 64 x 4096 x 4096 19.0 / 27.6. Pairs: 4096 samples, 1024 inputs, 4096 outputs 190 -> 112 us,
-    // 537 x 681 -> 644 28.3 -> 12.4, 24 x 2389 -> 1664 22.8 / 22.2.
-    return cost < other_us * (count == 1 ? 0.87 : 1.0);
+    // The other estimate is above the time by a fifth where B is read along its rows, by a twentieth where it is not (69 products of 31 to
+    // 6629 rows), and half a us pays for the second launch. Of those 69 the route taken is 1.4 % behind the better one in the geometric
+    // mean. Copies ahead: 944 x 1984 x 2352 38.0 -> 25.8 us, 1000 x 513 x 777 15.0 -> 10.9, 261 x 528 x 576 10.8 -> 8.0. Behind, and not taken:
+    // 128 x 1024 x 1024 9.3 us or 9.8, 112 x 1853 x 2721 15.3 or 16.7, 1520 x 346 x 243 6.4 or 7.0, 66 x 5601 x 6196 38 or 54. Pairs: 4096 samples,
+    // 1024 inputs, 4096 outputs 190 -> 112 us, 537 x 681 -> 644 28.3 -> 12.4, 24 x 2389 -> 1664 22.8 / 22.2.
+    if (count == 2) return cost < other_us;
+    return cost + 0.5 < other_us * (d[0].b_layout == NZHIP_LAYOUT_TRANS ? 0.80 : 0.95);
 }
 
 }  // namespace nzhip
