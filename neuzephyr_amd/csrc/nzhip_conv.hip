@@ -3025,10 +3025,12 @@ static bool conv_cl_wanted(ClDirection dir, const float* src, size_t N, size_t C
     }
     if (dir == CL_DATA && stride == 1) return true;                // 16x64x128x128 -> 128 5x5 233 / 177
     if (dir == CL_DATA) {
-        // The other ways multiply zeros or move a column gradient; `other_us` is the caller's estimate for the better of them.
-        // (16x320x18x18 <- 80 7x7 at stride 2 261 / 21, 16x64x128x128 <- 128 100 / 64; 16x3x224x224 <- 64 7x7, three channels of a tile of
-        // 64, 106 / 140)
-        return cl_conv_cost(dir, N, C, H, W, O, K_h, K_w, stride, pad, w_batch) < other_us;
+        // The other ways multiply zeros or move a column gradient; `other_us` is the caller's estimate for the better of them. The estimate
+        // of this one is up to half again above the time on large images, whose lines are written whole: it counts 0.72 (of 69 layers
+        // one then takes the slower way by more than 5 %, 10x101x96x96 <- 8 28 / 20). 16x320x18x18 <- 80 7x7 at stride 2 261 / 20, 16x64x128x128
+        // <- 128 100 / 43, 16x320x64x52 <- 39 63 / 32, 8x32x85x85 <- 151 36 / 18; few of a tile's 64 channels: 16x3x224x224 <- 64 7x7 106 / 129,
+        // 8x5x208x208 <- 194 7x7 78 / 178, 16x4x192x192 <- 112 35 / 68
+        return cl_conv_cost(dir, N, C, H, W, O, K_h, K_w, stride, pad, w_batch) * 0.72 < other_us;
     }
     // 16x64x128x128 -> 128 at stride 2 47 / 54, 5x5 167 / 184; 8x14x144x144 -> 64 7x7 at stride 2, 41472 outputs, 38 / 25
     return !(pieces && out >= 50000);

@@ -145,7 +145,6 @@ struct ClClass {
     int di, dj;                         // copy offset of tap (i, j): i di + j dj elements
     int Hc, Wc, base;                   // pixels per image, copy offset of pixel (0, 0) in elements
     int out, out_h, out_w;              // place of pixel (i, j) in its output plane: out + i out_h + j out_w
-    int first;                          // first tile of the class
     ClDiv by_ns, by_hw, by_w;           // ns, Hc Wc, Wc
 };
 struct ClArgs {
@@ -161,8 +160,8 @@ struct ClArgs {
     int images;                         // images in one launch row: N, or 1 with a weight copy per image
     long plane, y_total;                // output plane; elements of y
     long bias_sp, bias_sc, bias_sn;
-    int relu, parts, part_units, tiles_m, tiles, n_classes;
-    ClDiv by_cu, by_tiles_m;
+    int relu, parts, part_units, tiles_m, tiles, n_classes;      // tiles: of all classes, as if each had as many as the largest
+    ClDiv by_cu, by_tiles_m, by_classes;
     ClClass cls[CL_MAX_CLASSES];
 };
 
@@ -181,14 +180,22 @@ __global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
     const int wm = wave / T::WN, wn = wave % T::WN, li = lane & 31, lh = lane >> 5;
 
     const int lin = cl_xcd_place(blockIdx.x, p.tiles);
-    int ci = 0;
-    if (MANY)
-        while (ci + 1 < p.n_classes && lin >= p.cls[ci + 1].first) ci++;
+    int ci = 0, in_class = lin;
+    // The classes of a strided data gradient take turns: each writes every stride-th pixel of dx, so that the workgroups which write the
+    // same lines run together and the L2 of their XCD writes whole ones (16 x 64 x 128 x 128 <- 128 61.6 -> 42.8 us, 16 x 128 x 56 x 56 <- 128
+    // 31.4 -> 23.5, against one class after the other). Every second run of eight is reversed: a CU gets each 32nd workgroup of
+    // its XCD, and would get only long sums or only short ones (45.3 -> 42.8, 21.0 -> 19.3 on 16 x 256 x 28 x 28 <- 256).
+    if (MANY) {
+        in_class = cl_quot(lin, p.by_classes);
+        ci = lin - in_class * p.n_classes;
+        if (in_class & 8) ci = p.n_classes - 1 - ci;
+    }
     const ClClass& c = p.cls[MANY ? ci : 0];
-    const int in_class = MANY ? lin - c.first : lin, tile_n = cl_quot(in_class, p.by_tiles_m), tile_m = in_class - tile_n * p.tiles_m;
+    const int tile_n = cl_quot(in_class, p.by_tiles_m), tile_m = in_class - tile_n * p.tiles_m;
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const int z = blockIdx.z;
     const int hw = c.Hc * c.Wc, pixels = p.images * hw;
+    if (MANY && n0 >= pixels) return;                               // a class of fewer tiles than the largest
 
     // units of this part, a whole number of steps per group; the table of their offsets in the two copies, in bytes
     const int units = c.nr * c.ns * p.cu, u_first = blockIdx.y * p.part_units;
@@ -689,14 +696,16 @@ static int conv_product(ClArgs& a, int copies, hipStream_t s) {
     a.parts = (units + a.part_units - 1) / a.part_units;
     if (a.parts < 1) a.parts = 1;
     a.tiles_m = (a.M + sh.bm - 1) / sh.bm;
-    a.tiles = 0;
+    int most = 0;
     a.by_cu = cl_div(a.cu); a.by_tiles_m = cl_div(a.tiles_m);
     for (int i = 0; i < a.n_classes; i++) {
         ClClass& c = a.cls[i];
         c.by_ns = cl_div(c.ns ? c.ns : 1); c.by_hw = cl_div(c.Hc * c.Wc); c.by_w = cl_div(c.Wc);
-        a.cls[i].first = a.tiles;
-        a.tiles += (int)(((long)a.images * a.cls[i].Hc * a.cls[i].Wc + sh.bn - 1) / sh.bn) * a.tiles_m;
+        const int tiles = (int)(((long)a.images * c.Hc * c.Wc + sh.bn - 1) / sh.bn) * a.tiles_m;
+        if (tiles > most) most = tiles;
     }
+    a.tiles = most * a.n_classes;
+    a.by_classes = cl_div(a.n_classes);
     float* partial = nullptr;
     if (a.parts > 1)
         if (int rc = workspace_alloc(reinterpret_cast<void**>(&partial), (size_t)a.parts * a.y_total * sizeof(float), s)) return rc;
@@ -743,7 +752,7 @@ static void forward_args(ClArgs& a, size_t N, size_t C, size_t H, size_t W, size
     a.w_bytes = (unsigned)(a.w_img * 2); a.x_bytes = (unsigned)(a.images * a.x_img * 2);
     a.plane = (long)Ho * Wo; a.y_total = (long)N * a.y_img;
     a.n_classes = 1;
-    a.cls[0] = {(int)K_h, (int)K_w, 0, 1, 0, 1, Wp * Cs, Cs, Ho, Wo, 0, 0, Wo, 1, 0, {}, {}, {}};
+    a.cls[0] = {(int)K_h, (int)K_w, 0, 1, 0, 1, Wp * Cs, Cs, Ho, Wo, 0, 0, Wo, 1, {}, {}, {}};
 }
 
 static void data_args(ClArgs& a, int (&edge)[4], size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad,
@@ -781,7 +790,7 @@ static void data_args(ClArgs& a, int (&edge)[4], size_t N, size_t C, size_t H, s
             const Side h = side(i, (int)H, (int)K_h), v = side(j, (int)W, (int)K_w);
             if (!h.n || !v.n) continue;
             a.cls[a.n_classes++] = {h.t, v.t, i, st, j, st, -Wp * Os, -Os, h.n, v.n, ((h.lo + edge[0]) * Wp + v.lo + edge[2]) * Os,
-                                    (st * h.lo + i - (int)pad) * (int)W + st * v.lo + j - (int)pad, st * (int)W, st, 0, {}, {}, {}};
+                                    (st * h.lo + i - (int)pad) * (int)W + st * v.lo + j - (int)pad, st * (int)W, st, {}, {}, {}};
         }
 }
 

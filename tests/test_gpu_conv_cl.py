@@ -60,6 +60,7 @@ LAYERS = [
     (1, 3, 7, 7, 5, 7, 7, 2, 3, 1),            # 3 channels in 8, 49 taps, more taps than pixels
     (5, 20, 6, 5, 17, 5, 5, 1, 2, 1),          # kernel as large as the image
     (2, 70, 14, 14, 130, 3, 3, 2, 1, 1),       # stride 2: four sums of 1, 2, 2 and 4 taps
+    (3, 20, 29, 31, 12, 3, 3, 2, 1, 1),        # four sums of 720 to 630 pixels, 12 to 10 tiles
     (2, 33, 10, 13, 9, 3, 3, 3, 0, 2),         # stride 3, no padding, columns that no window reaches
     (2, 17, 12, 12, 24, 2, 2, 3, 0, 1),        # kernel below the stride: sums without a tap
     (1, 9, 1, 40, 8, 1, 1, 1, 0, 1),           # no window at all, one row
