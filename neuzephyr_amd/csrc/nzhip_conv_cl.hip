@@ -282,14 +282,17 @@ __global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
             request(t);
         }
         look_up(NST - 1);
+        ClSums<TM, TN> sums;
         int slot = 0;
         for (int t = 0; t < steps; t++) {
             cl_wait_vmcnt<(NST - 2) * LOADS>();                     // this wave's share of step t has landed
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // everybody's has, and step t - 1 is read by all
             request(slot == 0 ? NST - 1 : slot - 1);
             multiply(ring + slot * STAGE, t + NST);
+            sums.take(acc, t);
             slot = slot == NST - 1 ? 0 : slot + 1;
         }
+        sums.finish(acc);
         cl_wait_vmcnt<0>();
     }
 
@@ -498,6 +501,7 @@ __global__ __launch_bounds__(T::THREADS) void cl_dw_kernel(const ClDwArgs p) {
         request(t);
         advance();
     }
+    ClSums<TM, TN> sums;
     int slot = 0;
     for (int t = 0; t < steps; t++) {
         cl_wait_vmcnt<(NST - 2) * LOADS>();
@@ -522,8 +526,10 @@ __global__ __launch_bounds__(T::THREADS) void cl_dw_kernel(const ClDwArgs p) {
 #pragma unroll
                 for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[k][i], bf[k][j], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
+        sums.take(acc, t);
         slot = slot == NST - 1 ? 0 : slot + 1;
     }
+    sums.finish(acc);
     cl_wait_vmcnt<0>();
 
     if constexpr (KG > 1) {

@@ -150,6 +150,7 @@ __device__ __forceinline__ void copy_tile(const CopyProduct& p, const int lin, c
         return cl_read_turned(q + turned[0][block & 1], q + turned[1][block & 1]);
     };
 
+    ClSums<TM, TN> sums;
     for (int s = 0; s < NST - 1; s++) request(s);
     int slot = 0;
     for (int s = 0; s < steps; s++) {
@@ -173,8 +174,10 @@ __device__ __forceinline__ void copy_tile(const CopyProduct& p, const int lin, c
 #pragma unroll
                 for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[k][i], bf[k][j], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
+        sums.take(acc, s);
         slot = slot == NST - 1 ? 0 : slot + 1;
     }
+    sums.finish(acc);
     cl_wait_vmcnt<0>();
 
     if constexpr (KG > 1) {
@@ -484,9 +487,9 @@ bool gemm_copy_wanted(const nzhip_gemm_desc* d, int count, double other_us) {
     if (env) return true;
     // The other estimate is above the time by a fifth where B is read along its rows, by a twentieth where it is not (69 products of 31 to
     // 6629 rows), and half a us pays for the second launch. Of those 69 the route taken is 1.4 % behind the better one in the geometric
-    // mean. Copies ahead: 944 x 1984 x 2352 38.0 -> 25.8 us, 1000 x 513 x 777 15.0 -> 10.9, 261 x 528 x 576 10.8 -> 8.0. Behind, and not taken:
-    // 128 x 1024 x 1024 9.3 us or 9.8, 112 x 1853 x 2721 15.3 or 16.7, 1520 x 346 x 243 6.4 or 7.0, 66 x 5601 x 6196 38 or 54. Pairs: 4096 samples,
-    // 1024 inputs, 4096 outputs 190 -> 112 us, 537 x 681 -> 644 28.3 -> 12.4, 24 x 2389 -> 1664 22.8 / 22.2.
+    // mean. Copies ahead: 944 x 2352 x 1984 38.0 -> 25.8 us, 1000 x 777 x 513 14.9 -> 11.5, 261 x 576 x 528 10.8 -> 8.0. Behind, and not taken:
+    // 128 x 1024 x 1024 9.3 us or 9.8, 112 x 2721 x 1853 15.3 or 16.7, 1520 x 243 x 346 6.4 or 7.0, 66 x 6196 x 5601 38 or 54. Pairs: 4096 samples,
+    // 1024 inputs, 4096 outputs 190 -> 115 us, 537 x 681 -> 644 28.3 -> 12.4, 24 x 2389 -> 1664 22.8 / 22.2.
     if (count == 2) return cost < other_us;
     return cost + 0.5 < other_us * (d[0].b_layout == NZHIP_LAYOUT_TRANS ? 0.80 : 0.95);
 }

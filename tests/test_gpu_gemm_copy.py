@@ -63,6 +63,24 @@ def test_every_tile_and_layout_is_bit_exact_on_whole_numbers(nz, monkeypatch, ti
             assert np.array_equal(out.cpu().numpy(), want + old) and untouched(buf, M * N), tag
 
 
+@pytest.mark.parametrize("K", [512, 576, 16384])
+@pytest.mark.parametrize("tile", TILES)
+def test_a_long_contraction_is_summed_in_chains_of_512(nz, monkeypatch, tile, K):
+    """Unsplit: bit-exact on whole numbers, and the error of chains, not of one long sum. Each addition of a chain of n terms of equal variance
+    rounds a partial sum of i terms by u sqrt(i / n) at most, evenly distributed: relative variance n u^2 / 6, with u = 2^-24. n = 512 for the
+    chains, K / 512 for their sum: 5.7e-7 at 16384 (one sum: up to 3.1e-6, 8e-7 as MFMAs add several terms at once)."""
+    import torch
+    monkeypatch.setenv("NZHIP_GEMM_COPY", "1")
+    monkeypatch.setenv("NZHIP_GEMM_COPY_PLAN", f"{tile},1")
+    rng = np.random.default_rng(K + tile)
+    A, B = whole(rng, 70, K), whole(rng, K, 130)
+    assert np.array_equal(nz.gemm(torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()).cpu().numpy(), A.astype(np.float64) @ B)
+    A, B = (rng.standard_normal(x.shape).astype(np.float16).astype(np.float32) for x in (A, B))
+    want = A.astype(np.float64) @ B
+    err = nz.gemm(torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()).cpu().numpy() - want
+    assert np.linalg.norm(err) <= np.linalg.norm(want) * 2.0 ** -24 * np.sqrt((512 + K / 512) / 6)
+
+
 @pytest.mark.parametrize("S,inputs,outputs", [(65, 130, 63), (9, 300, 200), (257, 65, 10), (128, 64, 256), (40, 9, 600)])
 @pytest.mark.parametrize("tile", TILES)
 def test_both_gradients_of_a_linear_layer_are_bit_exact_on_whole_numbers(nz, monkeypatch, tile, S, inputs, outputs):
