@@ -60,7 +60,7 @@ struct CopyProduct {
     int M, N, K, lda, ldb, ldc;
     unsigned a_bytes, b_bytes;
     long bias_sm, bias_sn;
-    int relu, parts, part_steps, tiles, tiles_m, tiles_n;
+    int relu, parts, part_steps, tiles, tiles_m, tiles_n, chain;      // chain: steps, a power of two
     ClDiv by_tiles, by_panel, by_tiles_m;   // panels of up to 8 tile columns
 };
 struct CopyPair {
@@ -174,7 +174,7 @@ __device__ __forceinline__ void copy_tile(const CopyProduct& p, const int lin, c
 #pragma unroll
                 for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[k][i], bf[k][j], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        sums.take(acc, s);
+        sums.take(acc, s, p.chain);
         slot = slot == NST - 1 ? 0 : slot + 1;
     }
     sums.finish(acc);
@@ -307,7 +307,7 @@ static bool copy_plan_env(CopyPlan& pl) {
 // Estimated time in us and the plan it is for, fitted on 66 products and pairs of 16 to 4096 rows, columns and k with 15 plans each: the plan
 // chosen is 1.4 % slower than the best of the 15 in the geometric mean, 13 % at worst. A k step (64) of a workgroup alone on its CU
 // takes `alone`, of two that share one `pair` together.
-static CopyPlan copy_plan_search(const nzhip_gemm_desc* d, int count, double* cost) {
+static CopyPlan copy_plan_search(const nzhip_gemm_desc* d, int count, bool one_sum, double* cost) {
     static const double alone[COPY_TILES] = {0.207, 0.482, 0.385, 0.296, 0.530, 0.800}, pair[COPY_TILES] = {0.329, 0.482, 0.453, 0.469, 0.530, 0.800};
     static const double first[COPY_TILES] = {4.4, 4.7, 4.1, 4.3, 5.9, 6.0};      // launch, first request and result of a workgroup
     static const int cuts[] = {1, 2, 3, 4, 6, 8, 12, 16};
@@ -322,7 +322,9 @@ static CopyPlan copy_plan_search(const nzhip_gemm_desc* d, int count, double* co
     for (int t = 0; t < COPY_TILES; t++) {
         const CopyShape& sh = COPY_SHAPES[t];
         const bool two = t == 0 || t == 2 || t == 3;
+        if (one_sum && sh.kg > 1) continue;
         for (int cut : cuts) {
+            if (one_sum && cut > 1) break;
             double wgs = 0.0, work = 0.0, longest = 0.0, summed = 0.0;
             for (int i = 0; i < count; i++) {
                 const int64_t steps = (d[i].K + 63) / 64, per = (steps + cut - 1) / cut, parts = (steps + per - 1) / per, own = (per + sh.kg - 1) / sh.kg;
@@ -352,15 +354,15 @@ static CopyPlan copy_plan_search(const nzhip_gemm_desc* d, int count, double* co
     return best;
 }
 
-static CopyPlan copy_plan(const nzhip_gemm_desc* d, int count, double* cost) {
+static CopyPlan copy_plan(const nzhip_gemm_desc* d, int count, bool one_sum, double* cost) {
     struct Key { int64_t count, m, n, k, m2, n2, k2; };
     struct Found { CopyPlan plan; double cost; };
     static thread_local PlanCache<Key, Found> cache;
     const bool pair = count == 2;
-    const Key key = {count + (int64_t)device_cu_count() * 4, d[0].M, d[0].N, d[0].K, pair ? d[1].M : 0, pair ? d[1].N : 0, pair ? d[1].K : 0};
+    const Key key = {count + one_sum * 4 + (int64_t)device_cu_count() * 8, d[0].M, d[0].N, d[0].K, pair ? d[1].M : 0, pair ? d[1].N : 0, pair ? d[1].K : 0};
     bool known;
     Found& f = cache.at(key, known);
-    if (!known) f.plan = copy_plan_search(d, count, &f.cost);
+    if (!known) f.plan = copy_plan_search(d, count, one_sum, &f.cost);
     if (cost) *cost = f.cost;
     return f.plan;
 }
@@ -379,8 +381,8 @@ static size_t copy_bytes(const nzhip_gemm_desc* d, int count, const CopyPlan& pl
     return bytes;
 }
 
-int gemm_copy_run(const nzhip_gemm_desc* d, int count, hipStream_t s) {
-    CopyPlan pl = copy_plan(d, count, nullptr);
+int gemm_copy_run(const nzhip_gemm_desc* d, int count, hipStream_t s, bool one_sum) {
+    CopyPlan pl = copy_plan(d, count, one_sum, nullptr);
     copy_plan_env(pl);
     const CopyShape sh = COPY_SHAPES[pl.tile];
     struct Operand { const float* p; int64_t ld, rows, cols; size_t at; int pitch; };
@@ -408,6 +410,7 @@ int gemm_copy_run(const nzhip_gemm_desc* d, int count, hipStream_t s) {
         p.bias_sm = g.bias_stride_row; p.bias_sn = g.bias_stride_col; p.relu = g.activation == NZHIP_ACT_RELU;
         const int steps = (p.K + 63) / 64;
         p.part_steps = (steps + pl.parts - 1) / pl.parts;
+        p.chain = one_sum ? 1 << 30 : CL_CHAIN;
         p.parts = (steps + p.part_steps - 1) / p.part_steps;
         p.tiles_m = (p.M + sh.bm - 1) / sh.bm; p.tiles_n = (p.N + sh.bn - 1) / sh.bn;
         p.tiles = p.tiles_m * p.tiles_n;
@@ -469,7 +472,7 @@ int gemm_copy_run(const nzhip_gemm_desc* d, int count, hipStream_t s) {
     return rc ? rc : rc2 ? rc2 : rc3;
 }
 
-bool gemm_copy_wanted(const nzhip_gemm_desc* d, int count, double other_us) {
+bool gemm_copy_wanted(const nzhip_gemm_desc* d, int count, double other_us, bool one_sum) {
     const char* env = getenv("NZHIP_GEMM_COPY");                      // read per call (tests, benchmarking): 0 never, 1 wherever it fits
     if (env && !atoi(env)) return false;
     // a run that asks for one of the other routes, or for a plan of theirs, gets it
@@ -481,9 +484,12 @@ bool gemm_copy_wanted(const nzhip_gemm_desc* d, int count, double other_us) {
                        d[1].b_layout != NZHIP_LAYOUT_ROW)) return false;
     if (!env && count == 1 && d[0].M <= 64 && d[0].N <= 64) return false;      // one tile: the fused kernel is over before a second launch begins (33 x 512 x 33 7.6 us)
     double cost;
-    CopyPlan pl = copy_plan(d, count, &cost);
+    CopyPlan pl = copy_plan(d, count, one_sum, &cost);
     copy_plan_env(pl);
-    if (copy_bytes(d, count, pl) > workspace_limit()) return false;   // in the call that allocates nothing the copies have to fit its scratch
+    // The call that allocates nothing has to give the same bits: one product takes this route only where its copies fit that call's
+    // scratch as well (one sum over k has the same bits on either route).
+    const size_t bytes = copy_bytes(d, count, pl);
+    if (bytes > workspace_limit() || (!env && count == 1 && !one_sum && bytes > NZHIP_STATIC_SCRATCH_BYTES)) return false;
     if (env) return true;
     // The other estimate is above the time by a fifth where B is read along its rows, by a twentieth where it is not (69 products of 31 to
     // 6629 rows), and half a us pays for the second launch. Of those 69 the route taken is 1.4 % behind the better one in the geometric

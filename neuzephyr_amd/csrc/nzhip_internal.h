@@ -40,8 +40,9 @@ void gemm_h16_coop_test_mode(unsigned spin_limit, int mute);   // test hook: bou
 int gemm_h16_coop_timeouts(unsigned* count);     // polls that gave up since the library was loaded (expected: 0)
 // Products on rounded copies of their operands, one or the two gradients of a product in one launch (nzhip_gemm_copy.hip);
 // other_us: the estimate for the other ways
-bool gemm_copy_wanted(const nzhip_gemm_desc* d, int count, double other_us);
-int gemm_copy_run(const nzhip_gemm_desc* d, int count, hipStream_t stream);
+// one_sum: every element is one sum over all of k, bit for bit the two-pass kernel's result (a caller that keeps B's image gets that kernel)
+bool gemm_copy_wanted(const nzhip_gemm_desc* d, int count, double other_us, bool one_sum = false);
+int gemm_copy_run(const nzhip_gemm_desc* d, int count, hipStream_t stream, bool one_sum = false);
 // Bandwidth-bound kernels for M <= 8 (nzhip_skinny.hip).
 int gemm_skinny_dispatch(const nzhip_gemm_desc& d, hipStream_t stream);
 bool gemm_skinny_applicable(const nzhip_gemm_desc& d);

@@ -85,8 +85,8 @@ struct ClSums {
 #pragma unroll
                 for (int r = 0; r < 16; r++) sum[i][j][r] = 0.f;
     }
-    __device__ __forceinline__ void take(floatx16 (&acc)[TM][TN], int step) {
-        if ((step & (CL_CHAIN - 1)) != CL_CHAIN - 1) return;
+    __device__ __forceinline__ void take(floatx16 (&acc)[TM][TN], int step, int chain = CL_CHAIN) {
+        if ((step & (chain - 1)) != chain - 1) return;
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll

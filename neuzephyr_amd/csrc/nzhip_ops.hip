@@ -464,9 +464,9 @@ static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s) {
         // On rows of C that are no whole 16-byte pieces the block images' kernel stores element by element, and short of 2.8e10 flops its 256-wide
         // tiles are few: there the products on plain copies (2831 x 1296 x 2781 77 -> 43 us, 5001 x 999 x 5001 141 -> 106, 4192 x 3031 x 7535
         // 285 -> 276; 2128 x 1984 x 1904 44.5 -> 34, 4096 x 1024 x 2048 35 -> 33; above, 4096 x 1024 x 4096 58 / 65, 6864 x 864 x 3216 69 / 75).
-        // A caller that keeps B's image keeps this one.
+        // A caller that keeps B's image keeps this one, with the same result: one sum over k either way.
         const bool plain = !force_h16 && !image_kept_by_caller(PREPARED_GEMM_B) && (((d.N | d.ldc) & 3) != 0 || 2.0 * d.M * d.N * d.K < 2.8e10);
-        if (plain && gemm_copy_wanted(&d, 1, 1e30)) return gemm_copy_run(&d, 1, s);
+        if (plain && gemm_copy_wanted(&d, 1, 1e30, true)) return gemm_copy_run(&d, 1, s, true);
         return gemm_h16_dispatch(d, s);
     }
     GemmPlan plan = gemm_fused_plan(d);
