@@ -143,3 +143,23 @@ def test_chosen_plans_are_bit_exact_on_whole_numbers(nz, M, K, N, b_trans):
     A, B = whole(rng, M, K), whole(rng, K, N)
     got = nz.gemm(torch.from_numpy(A).cuda(), torch.from_numpy(np.ascontiguousarray(B.T if b_trans else B)).cuda(), b_trans=b_trans)
     assert np.array_equal(got.cpu().numpy(), A.astype(np.float64) @ B)
+
+
+@pytest.mark.parametrize("M,K,N", [(600, 9000, 600), (1400, 1296, 1001), (520, 4100, 2052), (3072, 768, 3072)])
+def test_a_kept_image_gives_the_bits_of_the_plain_call(nz, M, K, N):
+    import torch
+    rng = np.random.default_rng(M)
+    A, B = (torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda() for s in ((M, K), (K, N)))
+    h = nz.Prepared()
+    try:
+        assert torch.equal(nz.gemm(A, B, prepared_b=h), nz.gemm(A, B))
+    finally:
+        h.close()
+
+
+@pytest.mark.parametrize("M,K,N", [(200, 5000, 5000), (1000, 777, 513), (381, 3820, 2880)])
+def test_the_call_without_allocations_gives_the_same_bits(nz, M, K, N):
+    import torch
+    rng = np.random.default_rng(M)
+    A, B = (torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda() for s in ((M, K), (K, N)))
+    assert torch.equal(nz.gemm(A, B, static=True), nz.gemm(A, B))
