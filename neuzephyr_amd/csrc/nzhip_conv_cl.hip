@@ -145,6 +145,7 @@ struct ClClass {
     int di, dj;                         // copy offset of tap (i, j): i di + j dj elements
     int Hc, Wc, base;                   // pixels per image, copy offset of pixel (0, 0) in elements
     int out, out_h, out_w;              // place of pixel (i, j) in its output plane: out + i out_h + j out_w
+    int lo_h, lo_w;                     // tap (i, j) of pixel (k, l) reads row lo_h + k - i, column lo_w + l - j of dy (a data gradient)
     ClDiv by_ns, by_hw, by_w;           // ns, Hc Wc, Wc
 };
 struct ClArgs {
@@ -161,11 +162,31 @@ struct ClArgs {
     long plane, y_total;                // output plane; elements of y
     long bias_sp, bias_sc, bias_sn;
     int relu, parts, part_units, tiles_m, tiles, n_classes;      // tiles: of all classes, as if each had as many as the largest
+    int dy_h, dy_w;                     // dy's extents; 0 in a forward
     ClDiv by_cu, by_tiles_m, by_classes;
     ClClass cls[CL_MAX_CLASSES];
 };
 
-// 64 TM output channels x 64 TN pixels per workgroup, 2 x 2 waves of 32 TM x 32 TN per k group; KG groups of four waves take alternate
+// Units u_first .. + n_units of one element of a data gradient, taps outside dy left out: the zeros around dy are no terms of the sum, and
+// times an infinite weight they are not nothing either.
+__device__ __forceinline__ float cl_terms(const ClArgs& p, const ClClass& c, const int z, const int img, const int i, const int j, const int o,
+                                          const int u_first, const int n_units) {
+    const _Float16* x = p.x + z * p.x_img + img * p.x_img + c.base + (long)i * p.step_h + (long)j * p.step_w;
+    const _Float16* w = p.w + z * p.w_img + (long)o * p.w_row;
+    float s = 0.f;
+#pragma unroll 1
+    for (int u = u_first; u < u_first + n_units; u++) {
+        const int t = cl_quot(u, p.by_cu), ti = cl_quot(t, c.by_ns), tj = t - ti * c.ns, e = (u - t * p.cu) * 8;
+        if ((unsigned)(c.lo_h + i - ti) >= (unsigned)p.dy_h || (unsigned)(c.lo_w + j - tj) >= (unsigned)p.dy_w) continue;
+        const half8_t a = *reinterpret_cast<const half8_t*>(w + ((c.r0 + ti * c.rs) * p.Kw + c.s0 + tj * c.ss) * p.cu * 8 + e);
+        const half8_t b = *reinterpret_cast<const half8_t*>(x + (long)ti * c.di + (long)tj * c.dj + e);
+#pragma unroll
+        for (int q = 0; q < 8; q++) s = __builtin_fmaf((float)a[q], (float)b[q], s);
+    }
+    return s;
+}
+
+// 64 TM output channels x 32 WN TN pixels per workgroup, 2 x WN waves of 32 TM x 32 TN per k group; KG groups take alternate
 // k steps into rings of their own and meet in LDS at the end, where a layer gives fewer tiles than CUs.
 // LDS rows are 128 bytes, 8 units; unit u of row r lies at u ^ (r >> 1 & 7), which puts the 16 rows that share a pass of a
 // 128-bit read on 16 bank groups. The lane that loads a slot asks for the unit that belongs there, so a lane needs the
@@ -332,6 +353,24 @@ __global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
         bpix[j] = (long)(z + img) * p.bias_sn + pl * p.bias_sp;
     }
     const bool split = p.parts > 1;
+    // A data gradient's NaN at a pixel with taps outside dy may come from those (an infinite weight times the zeros there): summed again below
+    unsigned again[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) again[i][j] = 0;
+    if (p.dy_h) {
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+            const int px = n0 + (wn * TN + j) * 32 + li, q = px - cl_quot(px, c.by_hw) * hw, h = cl_quot(q, c.by_w), fh = c.lo_h + h, fw = c.lo_w + q - h * c.Wc;
+            if (!live[j] || (fh < p.dy_h && fh >= c.nr - 1 && fw < p.dy_w && fw >= c.ns - 1)) continue;
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    if (acc[i][j][r] != acc[i][j][r]) again[i][j] |= 1u << r;
+        }
+    }
     if (p.bias && !split) {
         const bool quads = p.bias_sc == 1;
 #pragma unroll
@@ -361,7 +400,20 @@ __global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
                 const int o = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
                 float v = acc[i][j][r];
                 if (p.relu && !split) v = v > 0.f ? v : 0.f;
-                if (live[j] && o < p.M) y[out[j] + (unsigned)o * (unsigned)p.plane] = v;
+                if (live[j] && o < p.M && !(again[i][j] >> r & 1)) y[out[j] + (unsigned)o * (unsigned)p.plane] = v;
+            }
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+#pragma unroll 1
+            for (unsigned left = again[i][j]; left; left &= left - 1) {
+                const int r = __builtin_ctz(left), o = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
+                if (o >= p.M) continue;
+                const int px = n0 + (wn * TN + j) * 32 + li, img = cl_quot(px, c.by_hw), q = px - img * hw, h = cl_quot(q, c.by_w);
+                float v = cl_terms(p, c, z, img, h, q - h * c.Wc, o, u_first, n_units);
+                if (p.bias && !split) v += p.bias[bpix[j] + o * p.bias_sc];
+                y[out[j] + (unsigned)o * (unsigned)p.plane] = v;
             }
 }
 
@@ -758,7 +810,7 @@ static void forward_args(ClArgs& a, size_t N, size_t C, size_t H, size_t W, size
     a.w_bytes = (unsigned)(a.w_img * 2); a.x_bytes = (unsigned)(a.images * a.x_img * 2);
     a.plane = (long)Ho * Wo; a.y_total = (long)N * a.y_img;
     a.n_classes = 1;
-    a.cls[0] = {(int)K_h, (int)K_w, 0, 1, 0, 1, Wp * Cs, Cs, Ho, Wo, 0, 0, Wo, 1, {}, {}, {}};
+    a.cls[0] = {(int)K_h, (int)K_w, 0, 1, 0, 1, Wp * Cs, Cs, Ho, Wo, 0, 0, Wo, 1, 0, 0, {}, {}, {}};
 }
 
 static void data_args(ClArgs& a, int (&edge)[4], size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad,
@@ -785,7 +837,7 @@ static void data_args(ClArgs& a, int (&edge)[4], size_t N, size_t C, size_t H, s
     }
     const int Hp = Ho + edge[0] + edge[1], Wp = Wo + edge[2] + edge[3];
     const int Os = cl_pitch((int)O);
-    a.M = (int)C; a.w_row = cl_pitch(taps * Op); a.cu = Op / 8; a.Kw = (int)K_w;
+    a.M = (int)C; a.w_row = cl_pitch(taps * Op); a.cu = Op / 8; a.Kw = (int)K_w; a.dy_h = Ho; a.dy_w = Wo;
     a.step_h = Wp * Os; a.step_w = Os;
     a.images = w_batch > 1 ? 1 : (int)N;
     a.x_img = (long)Hp * Wp * Os; a.w_img = (long)C * a.w_row; a.y_img = (long)C * H * W;
@@ -796,7 +848,7 @@ static void data_args(ClArgs& a, int (&edge)[4], size_t N, size_t C, size_t H, s
             const Side h = side(i, (int)H, (int)K_h), v = side(j, (int)W, (int)K_w);
             if (!h.n || !v.n) continue;
             a.cls[a.n_classes++] = {h.t, v.t, i, st, j, st, -Wp * Os, -Os, h.n, v.n, ((h.lo + edge[0]) * Wp + v.lo + edge[2]) * Os,
-                                    (st * h.lo + i - (int)pad) * (int)W + st * v.lo + j - (int)pad, st * (int)W, st, {}, {}, {}};
+                                    (st * h.lo + i - (int)pad) * (int)W + st * v.lo + j - (int)pad, st * (int)W, st, h.lo, v.lo, {}, {}, {}};
         }
 }
 

@@ -137,6 +137,34 @@ def test_a_special_value_stays_in_the_sums_it_is_a_term_of(nz, monkeypatch, spec
     assert np.array_equal(np.isfinite(dw), ~dw_hit) and np.array_equal(dw[~dw_hit], dw64[~dw_hit])
 
 
+@pytest.mark.parametrize("special", [float("inf"), float("nan"), -7e4])            # -7e4 is infinite in fp16
+@pytest.mark.parametrize("tile,parts", [(0, 1), (1, 3), (2, 1), (3, 2), (4, 1)])
+@pytest.mark.parametrize("K,stride,pad,copies", [(3, 2, 1, 1), (3, 1, 1, 2), (5, 2, 2, 1), (4, 3, 2, 2)])
+def test_a_special_weight_reaches_only_the_data_gradients_it_is_a_term_of(nz, monkeypatch, special, tile, parts, K, stride, pad, copies):
+    """At the border of dx some taps lie outside dy: no terms of the sum, whatever their weight."""
+    import torch
+    N, C, H, W, O = 2, 70, 11, 10, 20
+    rng = np.random.default_rng(6)
+    Ho, Wo = (H + 2 * pad - K) // stride + 1, (W + 2 * pad - K) // stride + 1
+    x, dy, old = np.zeros((N, C, H, W), np.float32), rng.integers(1, 3, (N, O, Ho, Wo)).astype(np.float32), whole(rng, N, C, H, W)
+    w = rng.integers(1, 3, (copies, 1, C * K * K, O)).astype(np.float32)
+    _, dx64, _ = reference(x, w, dy, K, K, stride, pad)
+    monkeypatch.setenv("NZHIP_CONV_CL", "1")
+    monkeypatch.setenv("NZHIP_CONV_CL_PLAN", f"{tile},{parts}")
+    cu = lambda a: torch.from_numpy(a.copy()).cuda()
+    for c, tap, o in ((0, 0, 0), (C - 1, K * K - 1, O - 1), (33, K // 2 * K, 7), (64, 1, 8)):
+        at = (copies - 1, 0, c * K * K + tap, o)
+        ws, mark = w.copy(), np.zeros_like(w)
+        ws[at], mark[at] = special, 1
+        _, hit, _ = reference(x, mark, dy, K, K, stride, pad)
+        assert (hit != 0).any() and (hit[:, c] == 0).any()
+        for accumulate in (False, True):
+            dx = cu(old)
+            nz.conv2d_backward_data(dx, cu(dy), cu(ws), K, K, stride, pad, accumulate=accumulate)
+            got, want = dx.cpu().numpy(), dx64 + (old if accumulate else 0)
+            assert np.array_equal(np.isfinite(got), hit == 0) and np.array_equal(got[hit == 0], want[hit == 0]), (at, accumulate)
+
+
 @pytest.mark.parametrize("layer", [(16, 256, 14, 14, 256, 3, 1, 1, 1), (2, 208, 16, 16, 144, 5, 1, 2, 2), (4, 64, 48, 48, 45, 7, 2, 3, 1),
                                    (1, 16, 192, 96, 24, 3, 2, 1, 1)])
 def test_chosen_plans_are_bit_exact_on_whole_numbers(nz, layer):
