@@ -191,8 +191,8 @@ __device__ __forceinline__ float cl_terms(const ClArgs& p, const ClClass& c, con
 // LDS rows are 128 bytes, 8 units; unit u of row r lies at u ^ (r >> 1 & 7), which puts the 16 rows that share a pass of a
 // 128-bit read on 16 bank groups. The lane that loads a slot asks for the unit that belongs there, so a lane needs the
 // offsets of two units per step (rows of even and odd groups of 8), from a table in LDS, one step ahead.
-// MANY: more than one class.
-template <typename T, bool MANY>
+// DATA: a data gradient. MANY: more than one class.
+template <typename T, bool DATA, bool MANY>
 __global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
     constexpr int TM = T::TM, TN = T::TN, KG = T::KG, BM = T::BM, BN = T::BN, NST = T::NST, STAGE = T::STAGE, LA = T::LA, LB = T::LB, LOADS = LA + LB;
     extern __shared__ __attribute__((aligned(1024))) char lds[];
@@ -339,6 +339,8 @@ __global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
             }
     }
 
+    if (m0 + wm * TM * 32 >= p.M) return;                           // nothing of this wave's is stored
+
     // ---- epilogue: lane = pixel, registers = channels (r >> 2) * 8 + lh * 4 + (r & 3); bias first, then the stores
     unsigned out[TN];
     long bpix[TN];
@@ -353,68 +355,79 @@ __global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
         bpix[j] = (long)(z + img) * p.bias_sn + pl * p.bias_sp;
     }
     const bool split = p.parts > 1;
-    // A data gradient's NaN at a pixel with taps outside dy may come from those (an infinite weight times the zeros there): summed again below
-    unsigned again[TM][TN];
+    float* y = split ? p.partial + blockIdx.y * p.y_total : p.y;
+    // AGAIN: NaNs of pixels with taps outside dy may come from an infinite weight times the zeros there, and are summed again
+    auto finish = [&](auto again_tag) {
+        constexpr bool AGAIN = decltype(again_tag)::value;
+        unsigned again[TM][TN];
+        if (AGAIN)
 #pragma unroll
-    for (int i = 0; i < TM; i++)
+            for (int j = 0; j < TN; j++) {
+                const int px = n0 + (wn * TN + j) * 32 + li, q = px - cl_quot(px, c.by_hw) * hw, h = cl_quot(q, c.by_w), row = c.lo_h + h, col = c.lo_w + q - h * c.Wc;
+                const bool edge = live[j] && (row >= p.dy_h || row < c.nr - 1 || col >= p.dy_w || col < c.ns - 1);
 #pragma unroll
-        for (int j = 0; j < TN; j++) again[i][j] = 0;
-    if (p.dy_h) {
+                for (int i = 0; i < TM; i++) {
+                    again[i][j] = 0;
 #pragma unroll
-        for (int j = 0; j < TN; j++) {
-            const int px = n0 + (wn * TN + j) * 32 + li, q = px - cl_quot(px, c.by_hw) * hw, h = cl_quot(q, c.by_w), fh = c.lo_h + h, fw = c.lo_w + q - h * c.Wc;
-            if (!live[j] || (fh < p.dy_h && fh >= c.nr - 1 && fw < p.dy_w && fw >= c.ns - 1)) continue;
+                    for (int r = 0; r < 16; r++) again[i][j] |= edge && acc[i][j][r] != acc[i][j][r] ? 1u << r : 0u;
+                }
+            }
+        if (p.bias && !split) {
+            const bool quads = p.bias_sc == 1;
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int r = 0; r < 16; r++)
-                    if (acc[i][j][r] != acc[i][j][r]) again[i][j] |= 1u << r;
+                for (int j = 0; j < TN; j++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        const int o = m0 + (wm * TM + i) * 32 + g * 8 + lh * 4;
+                        if (quads && o + 4 <= p.M) {
+                            const piece4 v = *reinterpret_cast<const floatx4u*>(p.bias + bpix[j] + o);
+#pragma unroll
+                            for (int e = 0; e < 4; e++) acc[i][j][g * 4 + e] += v[e];
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 4; e++) acc[i][j][g * 4 + e] += p.bias[bpix[j] + (long)(o + e < p.M ? o + e : p.M - 1) * p.bias_sc];
+                        }
+                    }
         }
-    }
-    if (p.bias && !split) {
-        const bool quads = p.bias_sc == 1;
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
             for (int j = 0; j < TN; j++)
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int o = m0 + (wm * TM + i) * 32 + g * 8 + lh * 4;
-                    if (quads && o + 4 <= p.M) {
-                        const piece4 v = *reinterpret_cast<const floatx4u*>(p.bias + bpix[j] + o);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) acc[i][j][g * 4 + e] += v[e];
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; e++) acc[i][j][g * 4 + e] += p.bias[bpix[j] + (long)(o + e < p.M ? o + e : p.M - 1) * p.bias_sc];
-                    }
+                for (int r = 0; r < 16; r++) {
+                    const int o = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
+                    float v = acc[i][j][r];
+                    if (p.relu && !split) v = v > 0.f ? v : 0.f;
+                    if (live[j] && o < p.M && !(AGAIN && again[i][j] >> r & 1)) y[out[j] + (unsigned)o * (unsigned)p.plane] = v;
                 }
-    }
-    float* y = split ? p.partial + blockIdx.y * p.y_total : p.y;
+        if (AGAIN)
 #pragma unroll
-    for (int i = 0; i < TM; i++)
+            for (int i = 0; i < TM; i++)
 #pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int o = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
-                float v = acc[i][j][r];
-                if (p.relu && !split) v = v > 0.f ? v : 0.f;
-                if (live[j] && o < p.M && !(again[i][j] >> r & 1)) y[out[j] + (unsigned)o * (unsigned)p.plane] = v;
-            }
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
+                for (int j = 0; j < TN; j++)
 #pragma unroll 1
-            for (unsigned left = again[i][j]; left; left &= left - 1) {
-                const int r = __builtin_ctz(left), o = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
-                if (o >= p.M) continue;
-                const int px = n0 + (wn * TN + j) * 32 + li, img = cl_quot(px, c.by_hw), q = px - img * hw, h = cl_quot(q, c.by_w);
-                float v = cl_terms(p, c, z, img, h, q - h * c.Wc, o, u_first, n_units);
-                if (p.bias && !split) v += p.bias[bpix[j] + o * p.bias_sc];
-                y[out[j] + (unsigned)o * (unsigned)p.plane] = v;
-            }
+                    for (unsigned left = again[i][j]; left; left &= left - 1) {
+                        const int r = __builtin_ctz(left), o = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
+                        if (o >= p.M) continue;
+                        const int px = n0 + (wn * TN + j) * 32 + li, img = cl_quot(px, c.by_hw), q = px - img * hw, h = cl_quot(q, c.by_w);
+                        float v = cl_terms(p, c, z, img, h, q - h * c.Wc, o, u_first, n_units);
+                        if (p.bias && !split) v += p.bias[bpix[j] + o * p.bias_sc];
+                        y[out[j] + (unsigned)o * (unsigned)p.plane] = v;
+                    }
+    };
+    if constexpr (DATA) {
+        float all = 0.f;                                            // NaN if one of them is
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) all += acc[i][j][r];
+        if (__builtin_expect(__any(all != all), 0)) return finish(std::true_type{});
+    }
+    finish(std::false_type{});
 }
 
 // y = act(sum of the parts, in order, + bias): element idx is (image, channel, pixel)
@@ -774,7 +787,7 @@ static int conv_product(ClArgs& a, int copies, hipStream_t s) {
     int rc;
     auto go = [&](auto tile) {
         using T = decltype(tile);
-        return launch(a.n_classes > 1 ? cl_conv_kernel<T, true> : cl_conv_kernel<T, false>, grid, T::THREADS, T::RING + table, a, s, "cl_conv kernel launch");
+        return launch(a.n_classes > 1 ? cl_conv_kernel<T, true, true> : a.dy_h ? cl_conv_kernel<T, true, false> : cl_conv_kernel<T, false, false>, grid, T::THREADS, T::RING + table, a, s, "cl_conv kernel launch");
     };
     rc = cl_pick(pl.tile, go);
     if (rc == NZHIP_OK && a.parts > 1) {
