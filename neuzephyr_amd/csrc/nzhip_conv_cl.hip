@@ -193,7 +193,7 @@ __device__ __forceinline__ float cl_terms(const ClArgs& p, const ClClass& c, con
 // offsets of two units per step (rows of even and odd groups of 8), from a table in LDS, one step ahead.
 // DATA: a data gradient. MANY: more than one class.
 template <typename T, bool DATA, bool MANY>
-__global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
+__global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) {
     constexpr int TM = T::TM, TN = T::TN, KG = T::KG, BM = T::BM, BN = T::BN, NST = T::NST, STAGE = T::STAGE, LA = T::LA, LB = T::LB, LOADS = LA + LB;
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -272,7 +272,9 @@ __global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
     const int sw = (li >> 1) & 7;
     // One step: every fragment is requested before the first MFMA (a read takes 100 clocks and more to come back, an MFMA 32), then
     // the offsets of the next request.
-    auto multiply = [&](const char* base, int ahead) {
+    ClSums<TM, TN> sums;
+    const int chain = cl_chain(steps);
+    auto multiply = [&](const char* base, int t, int ahead) {
         half8_t af[4][TM], bf[4][TN];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -284,6 +286,7 @@ __global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
             __builtin_amdgcn_sched_barrier(0);                      // in the order of their use
         }
         look_up(ahead);
+        sums.take(acc, t, chain);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int k = 0; k < 4; k++)
@@ -303,14 +306,12 @@ __global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
             request(t);
         }
         look_up(NST - 1);
-        ClSums<TM, TN> sums;
         int slot = 0;
         for (int t = 0; t < steps; t++) {
             cl_wait_vmcnt<(NST - 2) * LOADS>();                     // this wave's share of step t has landed
             asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // everybody's has, and step t - 1 is read by all
             request(slot == 0 ? NST - 1 : slot - 1);
-            multiply(ring + slot * STAGE, t + NST);
-            sums.take(acc, t);
+            multiply(ring + slot * STAGE, t, t + NST);
             slot = slot == NST - 1 ? 0 : slot + 1;
         }
         sums.finish(acc);
@@ -430,14 +431,12 @@ __global__ __launch_bounds__(T::THREADS) void cl_conv_kernel(const ClArgs p) {
     finish(std::false_type{});
 }
 
-// y = act(sum of the parts, in order, + bias): element idx is (image, channel, pixel)
+// y = act(sum of the parts + bias): element idx is (image, channel, pixel)
 __global__ __launch_bounds__(256) void cl_sum_kernel(float* y, const float* __restrict__ partial, const float* bias, unsigned total, int parts,
                                                      unsigned plane, unsigned M, long sp, long sc, long sn, int relu) {
     const unsigned i = blockIdx.x * 256 + threadIdx.x;
     if (i >= total) return;
-    float s = 0.f;
-#pragma unroll 8
-    for (int q = 0; q < parts; q++) s += partial[(long)q * total + i];
+    float s = cl_sum_parts(parts, [&](int q) { return partial[(long)q * total + i]; });
     if (bias) {
         const unsigned pl = i / plane, px = i - pl * plane, img = pl / M, o = pl - img * M;
         s += bias[img * sn + o * sc + px * sp];
@@ -471,7 +470,7 @@ struct ClDwArgs {
 // LDS load: 16 lanes read 4 pixels x 16 channels and each gets 4 pixels of one channel. Swizzle and ring as above. A pixel past
 // the end is zeros in both operands (an offset outside the buffer), so nothing of a neighbour enters a sum.
 template <typename T>
-__global__ __launch_bounds__(T::THREADS) void cl_dw_kernel(const ClDwArgs p) {
+__global__ __launch_bounds__(T::THREADS, 2) void cl_dw_kernel(const ClDwArgs p) {
     constexpr int TM = T::TM, TN = T::TN, KG = T::KG, NST = T::NST, STAGE = T::STAGE;
     constexpr int MT = T::BM / 64, NT = T::BN / 64, Q = 4 / T::WN, LOADS = Q * (MT + NT);     // 64-channel tiles; groups of 8 pixels per wave and step
     extern __shared__ __attribute__((aligned(1024))) char lds[];
@@ -567,6 +566,7 @@ __global__ __launch_bounds__(T::THREADS) void cl_dw_kernel(const ClDwArgs p) {
         advance();
     }
     ClSums<TM, TN> sums;
+    const int chain = cl_chain(steps);
     int slot = 0;
     for (int t = 0; t < steps; t++) {
         cl_wait_vmcnt<(NST - 2) * LOADS>();
@@ -583,6 +583,7 @@ __global__ __launch_bounds__(T::THREADS) void cl_dw_kernel(const ClDwArgs p) {
             __builtin_amdgcn_sched_barrier(0);                      // in the order of their use
         }
         advance();                                                  // in the time the reads take
+        sums.take(acc, t, chain);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int k = 0; k < 4; k++)
@@ -591,7 +592,6 @@ __global__ __launch_bounds__(T::THREADS) void cl_dw_kernel(const ClDwArgs p) {
 #pragma unroll
                 for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[k][i], bf[k][j], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        sums.take(acc, t);
         slot = slot == NST - 1 ? 0 : slot + 1;
     }
     sums.finish(acc);

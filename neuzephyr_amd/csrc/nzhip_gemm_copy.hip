@@ -167,6 +167,8 @@ __device__ __forceinline__ void copy_tile(const CopyProduct& p, const int lin, c
             for (int j = 0; j < TN; j++) bf[k][j] = read(base + BM * 128, B_KC, wn * TN + j, k);
             __builtin_amdgcn_sched_barrier(0);                      // in the order of their use
         }
+        sums.take(acc, s, p.chain);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int k = 0; k < 4; k++)
 #pragma unroll
@@ -174,7 +176,6 @@ __device__ __forceinline__ void copy_tile(const CopyProduct& p, const int lin, c
 #pragma unroll
                 for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[k][i], bf[k][j], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        sums.take(acc, s, p.chain);
         slot = slot == NST - 1 ? 0 : slot + 1;
     }
     sums.finish(acc);
@@ -244,28 +245,26 @@ __device__ __forceinline__ void copy_tile(const CopyProduct& p, const int lin, c
 
 // FORM: bit 0 A_KC, bit 1 B_KC
 template <int FORM, typename T>
-__global__ __launch_bounds__(T::THREADS) void copy_product_kernel(const CopyPair a) {
+__global__ __launch_bounds__(T::THREADS, 2) void copy_product_kernel(const CopyPair a) {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     copy_tile<(FORM & 1) != 0, (FORM & 2) != 0, T>(a.p[0], cl_xcd_place(blockIdx.x, a.total), lds);
 }
 // both gradients of C = A B: dA += dC B^T with dC along its rows, and dB += A^T dC across them
 template <int FORM1, int FORM2, typename T>
-__global__ __launch_bounds__(T::THREADS) void copy_pair_kernel(const CopyPair a) {
+__global__ __launch_bounds__(T::THREADS, 2) void copy_pair_kernel(const CopyPair a) {
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int lin = cl_xcd_place(blockIdx.x, a.total);
     if (lin < a.first2) copy_tile<(FORM1 & 1) != 0, (FORM1 & 2) != 0, T>(a.p[0], lin, lds);
     else copy_tile<(FORM2 & 1) != 0, (FORM2 & 2) != 0, T>(a.p[1], lin - a.first2, lds);
 }
 
-// C = act(the parts' sums, in order, + bias)
+// C = act(the parts' sums + bias)
 __global__ __launch_bounds__(256) void copy_sum_kernel(const CopyPair a, const int blocks1, const ClDiv by_n1, const ClDiv by_n2) {
     const bool second = (int)blockIdx.x >= blocks1;
     const CopyProduct& p = a.p[second];
     const int i = ((int)blockIdx.x - (second ? blocks1 : 0)) * 256 + threadIdx.x;
     if (i >= p.M * p.N) return;
-    float s = 0.f;
-#pragma unroll 8
-    for (int q = 0; q < p.parts; q++) s += p.partial[(long)q * p.M * p.N + i];
+    float s = cl_sum_parts(p.parts, [&](int q) { return p.partial[(long)q * p.M * p.N + i]; });
     const int m = cl_quot(i, second ? by_n2 : by_n1), n = i - m * p.N;
     if (p.bias) s += p.bias[m * p.bias_sm + n * p.bias_sn];
     if (p.relu) s = s > 0.f ? s : 0.f;
@@ -410,7 +409,7 @@ int gemm_copy_run(const nzhip_gemm_desc* d, int count, hipStream_t s, bool one_s
         p.bias_sm = g.bias_stride_row; p.bias_sn = g.bias_stride_col; p.relu = g.activation == NZHIP_ACT_RELU;
         const int steps = (p.K + 63) / 64;
         p.part_steps = (steps + pl.parts - 1) / pl.parts;
-        p.chain = one_sum ? 1 << 30 : CL_CHAIN;
+        p.chain = one_sum ? 1 << 30 : p.M <= 64 || p.N <= 64 ? cl_chain(p.part_steps / sh.kg) : CL_CHAIN;      // narrow ones: the fused kernel's chunks are of 128
         p.parts = (steps + p.part_steps - 1) / p.part_steps;
         p.tiles_m = (p.M + sh.bm - 1) / sh.bm; p.tiles_n = (p.N + sh.bn - 1) / sh.bn;
         p.tiles = p.tiles_m * p.tiles_n;

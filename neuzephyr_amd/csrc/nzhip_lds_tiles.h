@@ -69,11 +69,28 @@ __device__ __forceinline__ half8_t cl_read_turned(const char* lo, const char* hi
     return v;
 }
 
-// Sums of the steps so far, which a chain leaves after every CL_CHAIN of them: the error of an fp32 sum grows with the length of its chain,
-// and the kernels these take the place of cut a long contraction into chunks. With chains of 512, 944 x 2352 x 1984 has a relative error
-// of 1.5e-7 against 64 bits, 3.1e-7 without, 2.2e-7 on the fused kernel; 16 x 256 x 14 x 14 -> 256 1.4e-7, 2.1e-7, 1.5e-7. It costs 1 to 2 %
+// Sums of the steps so far, which a chain leaves after every `chain` of them: the error of an fp32 sum grows with the length of its chain,
+// and the kernels these take the place of cut a long contraction into chunks. Products: chains of CL_CHAIN steps, 512 elements. 944 x 2352 x 1984
+// has a relative error of 1.5e-7 against 64 bits then, 3.1e-7 without, 2.2e-7 on the fused kernel. It costs 1 to 2 %
 // (1000 x 777 x 513 11.3 -> 11.5 us, both gradients of 4096 x 1024 -> 4096 112 -> 115).
 constexpr int CL_CHAIN = 8;
+// Convolutions and products of at most 64 rows or columns: the kernels before sum in chunks of 16 channels, 128 pixels, 128 elements. n steps a chain of S leave an error of about 8.7 n + S / n
+// squared (fitted to chains of 1, 2, 4 and 8 steps), least at these n. Chains of 512 were up to 1.8 times as far off as those kernels
+// (weight gradient 8 x 13 x 16 x 16 -> 128, 7x7 at stride 2 1.4e-7, 0.8e-7 before and now). They cost 1 % more than those.
+__host__ __device__ __forceinline__ int cl_chain(int steps) { return steps < 18 ? 1 : steps < 70 ? 2 : steps < 280 ? 4 : steps < 1120 ? 8 : 16; }
+// The parts' sums, eight chains side by side for the same reason (64 in one chain: 1.6e-7, weight gradient 4 x 16 x 32 x 32 -> 16, 1.0e-7 so)
+template <typename F>
+__device__ __forceinline__ float cl_sum_parts(int parts, F part) {
+    float s[8] = {};
+    for (int q = 0; q < parts; q += 8) {                              // all eight requested before the first is added
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = part(q + e < parts ? q + e : parts - 1);
+#pragma unroll
+        for (int e = 0; e < 8; e++) s[e] += q + e < parts ? v[e] : 0.f;
+    }
+    return ((s[0] + s[4]) + (s[2] + s[6])) + ((s[1] + s[5]) + (s[3] + s[7]));
+}
 template <int TM, int TN>
 struct ClSums {
     floatx16 sum[TM][TN];
@@ -85,8 +102,9 @@ struct ClSums {
 #pragma unroll
                 for (int r = 0; r < 16; r++) sum[i][j][r] = 0.f;
     }
-    __device__ __forceinline__ void take(floatx16 (&acc)[TM][TN], int step, int chain = CL_CHAIN) {
-        if ((step & (chain - 1)) != chain - 1) return;
+    // before the MFMAs of a step, between the requests of its fragments and their use: the time these take covers it. chain: a power of two
+    __device__ __forceinline__ void take(floatx16 (&acc)[TM][TN], int step, int chain) {
+        if (step & (chain - 1)) return;
 #pragma unroll
         for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -107,6 +125,8 @@ struct ClSums {
     }
 };
 
+// The kernels ask for two waves per SIMD, the most that LDS has room for: with up to 256 registers the compiler keeps the sums in ordinary ones, with
+// up to 512 in accumulation registers, and every sum that a chain leaves would be moved there and back.
 // A tile: TM x TN fragments of 32 x 32 per wave, 2 x WN waves in each of KG groups.
 template <int TM_, int TN_, int WN_, int KG_>
 struct ClTile {

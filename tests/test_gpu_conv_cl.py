@@ -165,6 +165,33 @@ def test_a_special_weight_reaches_only_the_data_gradients_it_is_a_term_of(nz, mo
             assert np.array_equal(np.isfinite(got), hit == 0) and np.array_equal(got[hit == 0], want[hit == 0]), (at, accumulate)
 
 
+# N, C, H, W, O, K, stride, pad, copies: short sums, sums of 64 parts, strided gradients of many short sums, long sums
+PRECISION = [(8, 13, 16, 16, 128, 7, 2, 3, 1), (1, 32, 23, 23, 15, 5, 1, 2, 1), (8, 8, 48, 48, 8, 7, 2, 3, 8), (4, 16, 32, 32, 16, 3, 1, 1, 1), (4, 32, 48, 48, 33, 3, 2, 1, 4),
+             (16, 16, 30, 30, 113, 7, 2, 3, 1), (4, 160, 65, 65, 16, 3, 2, 1, 1), (16, 272, 17, 17, 99, 5, 1, 2, 16), (16, 256, 14, 14, 256, 3, 1, 1, 1)]
+
+
+@pytest.mark.parametrize("layer", PRECISION)
+def test_sums_are_as_exact_as_those_of_the_kernels_that_round_as_they_stage(nz, monkeypatch, layer):
+    """Error in the 2-norm against float64 on operands that fp16 holds exactly, so that only the order of the fp32 sums counts."""
+    import torch
+    N, C, H, W, O, K, stride, pad, copies = layer
+    rng = np.random.default_rng(7)
+    Ho, Wo = (H + 2 * pad - K) // stride + 1, (W + 2 * pad - K) // stride + 1
+    x, w, dy = (rng.standard_normal(s).astype(np.float16).astype(np.float32) for s in ((N, C, H, W), (copies, 1, C * K * K, O), (N, O, Ho, Wo)))
+    want = reference(x, w, dy, K, K, stride, pad)
+    X, Wt, DY = (torch.from_numpy(a).cuda() for a in (x, w, dy))
+    err = {}
+    for route in ("0", "1"):
+        monkeypatch.setenv("NZHIP_CONV_CL", route)
+        dw = torch.zeros(w.shape, device="cuda")
+        nz.conv2d_backward_weights(dw, X, DY, K, K, stride, pad)
+        dx = nz.conv2d_backward_data(torch.empty(x.shape, device="cuda"), DY, Wt, K, K, stride, pad, accumulate=False)
+        got = nz.conv2d_forward(X, Wt, None, K, K, stride, pad), dx, dw
+        err[route] = [np.linalg.norm(g.cpu().numpy() - r) / np.linalg.norm(r) for g, r in zip(got, want)]
+    for name, before, now in zip(("y", "dx", "dw"), err["0"], err["1"]):
+        assert now <= 1.05 * before, (name, before, now)              # (the 2-norm over thousands of elements moves by a few hundredths with their order)
+
+
 @pytest.mark.parametrize("layer", [(16, 256, 14, 14, 256, 3, 1, 1, 1), (2, 208, 16, 16, 144, 5, 1, 2, 2), (4, 64, 48, 48, 45, 7, 2, 3, 1),
                                    (1, 16, 192, 96, 24, 3, 2, 1, 1)])
 def test_chosen_plans_are_bit_exact_on_whole_numbers(nz, layer):

@@ -81,6 +81,22 @@ def test_a_long_contraction_is_summed_in_chains_of_512(nz, monkeypatch, tile, K)
     assert np.linalg.norm(err) <= np.linalg.norm(want) * 2.0 ** -24 * np.sqrt((512 + K / 512) / 6)
 
 
+@pytest.mark.parametrize("S,inputs,outputs", [(29, 466, 640), (64, 848, 786), (48, 880, 1984), (16, 792, 2752)])
+def test_gradients_of_few_samples_are_as_exact_as_one_product_after_the_other(nz, monkeypatch, S, inputs, outputs):
+    """Error in the 2-norm against float64 on operands that fp16 holds exactly: only the order of the fp32 sums counts."""
+    import torch
+    rng = np.random.default_rng(S)
+    W, x, dz = (rng.standard_normal(s).astype(np.float16).astype(np.float32) for s in ((1, 1, outputs, inputs), (S, 1, inputs, 1), (S, 1, outputs, 1)))
+    want = dz[:, 0, :, 0].T.astype(np.float64) @ x[:, 0, :, 0], dz[:, 0, :, 0].astype(np.float64) @ W[0, 0]
+    err = {}
+    for route in ("0", "1"):
+        monkeypatch.setenv("NZHIP_GEMM_COPY", route)
+        gw, gx = torch.zeros(W.shape, device="cuda"), torch.zeros(x.shape, device="cuda")
+        nz.matmul_backward(gw, gx, *(torch.from_numpy(a).cuda() for a in (W, x, dz)))
+        err[route] = [np.linalg.norm(g.cpu().numpy().reshape(r.shape) - r) / np.linalg.norm(r) for g, r in zip((gw, gx), want)]
+    assert all(now <= 1.05 * before for now, before in zip(err["1"], err["0"])), err      # (the norm moves by a few hundredths with the order)
+
+
 @pytest.mark.parametrize("S,inputs,outputs", [(65, 130, 63), (9, 300, 200), (257, 65, 10), (128, 64, 256), (40, 9, 600)])
 @pytest.mark.parametrize("tile", TILES)
 def test_both_gradients_of_a_linear_layer_are_bit_exact_on_whole_numbers(nz, monkeypatch, tile, S, inputs, outputs):
