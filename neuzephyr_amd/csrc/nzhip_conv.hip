@@ -3049,6 +3049,7 @@ static ConvRoute conv_forward_route(const float* x, size_t N, size_t C, size_t H
     static const char* bn_env = getenv("NZHIP_CONV_BN");
     wide = tw_env ? atoi(tw_env) == 64 : W_out >= 64;
     bn128 = bn_env ? atoi(bn_env) == 128 : O > 64;
+    if (H == 0 || W == 0) return CONV_ROUTE_WORKSPACE;               // nothing but padding: the others clamp their loads to an element that is not there
     if (conv_direct_applicable(C, O, K_h, K_w, stride, pad)) return CONV_ROUTE_DIRECT;
     const bool force_ws = route_env && route_env[0] == 'w', force_gen = route_env && route_env[0] == 'g';
     if (force_ws) return CONV_ROUTE_WORKSPACE;
@@ -4211,6 +4212,7 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
     if (stride == 0 || K_h == 0 || K_w == 0) return set_error(NZHIP_E_INVALID, "nzhip_conv2d_backward_weights: zero stride or kernel extent");
     if (H + 2 * pad < K_h || W + 2 * pad < K_w)
         return set_error(NZHIP_E_SHAPE, "nzhip_conv2d_backward_weights: kernel larger than the padded input");
+    if (H == 0 || W == 0) return NZHIP_OK;                            // nothing but padding
     if (conv1x1_strided(K_h, K_w, stride, pad, N, C, H, W)) {
         // 1x1 with a stride: the pixels the convolution looked at, gathered once, then the 1x1 stride-1 product
         // (16 x 1024 x 14 x 14 -> 2048 at stride 2: 351 -> 35 us)

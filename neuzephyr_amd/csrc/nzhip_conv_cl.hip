@@ -31,13 +31,13 @@ namespace nzhip {
 // One job turns `images` sets of (channel, pixel) planes into channel-last rows: pixel p of image i, channel c is read at
 //   src + (i / T) * s1 + (i % T) * s2 + c * sc + (p's place in an H x W plane)
 // and written, with channels C..Cp-1 zero, to dst + (i / T) * d1 + (i % T) * d2 + p * dp + c. p runs over Hp x Wp pixels of which
-// H x W from (pt, pl) on are read and the others are zero. ROWS jobs (sc == 0) copy rows of C contiguous elements to rows of Cp.
+// H x W from (pt, pl) on are read and the others are zero. Jobs with `rows` copy rows of C contiguous elements to rows of Cp.
 struct ClPrepJob {
     const float* src;
     _Float16* dst;
     long s1, s2, sc, d1, d2, dp;
     int T, C, Cp, H, W, Hp, Wp, pt, pl;
-    int ptiles, ctiles, blocks;
+    int ptiles, ctiles, blocks, rows;
 };
 struct ClPrepArgs { ClPrepJob job[2]; };
 constexpr int CLP_PX = 64, CLP_CH = 64, CLP_PITCH = CLP_CH * 2 + 16;
@@ -51,11 +51,11 @@ __global__ __launch_bounds__(256) void cl_prep_kernel(const ClPrepArgs a) {
     if (second) b -= a.job[0].blocks;
     const ClPrepJob& j = a.job[second];
     const int tid = threadIdx.x;
-    if (j.sc == 0) {                                              // rows of contiguous elements: only rounded
+    if (j.rows) {                                                 // rows of contiguous elements: only rounded
         const int upr = j.Cp / 8;
         const long u = (long)b * 256 + tid, row = u / upr;
         const int c = (int)(u - row * upr) * 8;
-        if (row >= (long)j.H) return;
+        if (row >= (long)j.rows) return;
         const float* s = j.src + row * j.C + c;
         half8_t h;
         if (c + 8 <= j.C) {
@@ -128,7 +128,7 @@ static void prep_weights(ClPrepJob& j, const float* src, _Float16* dst, long cop
 static void prep_rows(ClPrepJob& j, const float* src, _Float16* dst, long rows, int taps, int C, int Cp) {
     j = {};
     j.src = src; j.dst = dst;
-    j.T = taps; j.C = C; j.Cp = Cp; j.H = (int)rows; j.dp = cl_pitch(taps * Cp);
+    j.T = taps; j.C = C; j.Cp = Cp; j.rows = (int)rows; j.dp = cl_pitch(taps * Cp);
     j.blocks = (int)((rows * (Cp / 8) + 255) / 256);
 }
 static int prep_launch(const ClPrepArgs& a, hipStream_t s) {
@@ -803,7 +803,7 @@ static int conv_product(ClArgs& a, int copies, hipStream_t s) {
 // The extents the kernels' 32-bit offsets and tables hold: copies and result below 2 GiB, a unit table beside the largest ring.
 // 0: not, 1: yes, 2: yes and to be taken whatever the layer.
 int cl_conv_fits(ClDirection dir, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad, size_t w_batch) {
-    if (!N || !C || !O || (dir == CL_DATA && stride > 3) || K_h > 64 || K_w > 64 || H > 16384 || W > 16384 || pad > 64 || stride > 64 || C > 65535 || O > 65535 || N > 32768) return 0;
+    if (!N || !C || !O || !H || !W || (dir == CL_DATA && stride > 3) || K_h > 64 || K_w > 64 || H > 16384 || W > 16384 || pad > 64 || stride > 64 || C > 65535 || O > 65535 || N > 32768) return 0;
     const size_t taps = K_h * K_w, Cp = (C + 7) / 8 * 8, Op = (O + 7) / 8 * 8, Cs = C + 128, Os = O + 128, Hp = H + 2 * pad + K_h, Wp = W + 2 * pad + K_w, lim = 1u << 30;
     if (!(N * Hp * Wp * Cs < lim && N * Hp * Wp * Os < lim && w_batch * (taps * Cp + 128) * O < lim && w_batch * (taps * Op + 128) * C < lim &&
            N * (H + 2 * pad) * (W + 2 * pad) * (C > O ? C : O) < lim / 2 && w_batch * taps * C * O < lim && taps * Cp / 8 <= 3500 && taps * Op / 8 <= 3500)) return 0;

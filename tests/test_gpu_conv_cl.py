@@ -165,6 +165,22 @@ def test_a_special_weight_reaches_only_the_data_gradients_it_is_a_term_of(nz, mo
             assert np.array_equal(np.isfinite(got), hit == 0) and np.array_equal(got[hit == 0], want[hit == 0]), (at, accumulate)
 
 
+@pytest.mark.parametrize("H,W,pad", [(0, 0, 3), (0, 0, 2), (0, 5, 2), (3, 0, 2)])
+def test_an_empty_plane_is_all_padding(nz, H, W, pad):
+    """y is the bias (here nothing), not what a copy of the same size left in the workspace; dw gets nothing."""
+    import torch
+    N, C, O, K = 2, 16, 24, 3
+    lib, stream = nz.load(), torch.cuda.current_stream().cuda_stream
+    Ho, Wo = H + 2 * pad - K + 1, W + 2 * pad - K + 1
+    w = torch.ones(1, 1, C * K * K, O, device="cuda")
+    nz.conv2d_forward(torch.ones(N, C, H + 2 * pad, W + 2 * pad, device="cuda"), w, None, K, K, 1, 0)
+    y, dw, one = torch.full((N, O, Ho, Wo), 7.0, device="cuda"), torch.full_like(w, 3.0), torch.ones(64, device="cuda")
+    nz.check(lib.nzhip_conv2d_forward(y.data_ptr(), one.data_ptr(), w.data_ptr(), None, N, C, H, W, O, K, K, 1, pad, 1, 0, 1, 0, stream))
+    assert bool((y == 0).all())
+    nz.check(lib.nzhip_conv2d_backward_weights(dw.data_ptr(), one.data_ptr(), y.data_ptr(), N, C, H, W, O, K, K, 1, pad, 1, stream))
+    assert bool((dw == 3).all())
+
+
 # N, C, H, W, O, K, stride, pad, copies: short sums, sums of 64 parts, strided gradients of many short sums, long sums
 PRECISION = [(8, 13, 16, 16, 128, 7, 2, 3, 1), (1, 32, 23, 23, 15, 5, 1, 2, 1), (8, 8, 48, 48, 8, 7, 2, 3, 8), (4, 16, 32, 32, 16, 3, 1, 1, 1), (4, 32, 48, 48, 33, 3, 2, 1, 4),
              (16, 16, 30, 30, 113, 7, 2, 3, 1), (4, 160, 65, 65, 16, 3, 2, 1, 1), (16, 272, 17, 17, 99, 5, 1, 2, 16), (16, 256, 14, 14, 256, 3, 1, 1, 1)]
