@@ -61,7 +61,7 @@ struct CopyProduct {
     unsigned a_bytes, b_bytes;
     long bias_sm, bias_sn;
     int relu, parts, part_steps, tiles, tiles_m, tiles_n, chain;      // chain: steps, a power of two
-    ClDiv by_tiles, by_panel, by_tiles_m;   // panels of up to 8 tile columns
+    ClDiv by_tiles, by_panel;           // panels of up to 8 tile columns
 };
 struct CopyPair {
     CopyProduct p[2];
@@ -413,7 +413,7 @@ int gemm_copy_run(const nzhip_gemm_desc* d, int count, hipStream_t s, bool one_s
         p.parts = (steps + p.part_steps - 1) / p.part_steps;
         p.tiles_m = (p.M + sh.bm - 1) / sh.bm; p.tiles_n = (p.N + sh.bn - 1) / sh.bn;
         p.tiles = p.tiles_m * p.tiles_n;
-        p.by_tiles = cl_div(p.tiles); p.by_panel = cl_div(8 * p.tiles_m); p.by_tiles_m = cl_div(p.tiles_m);
+        p.by_tiles = cl_div(p.tiles); p.by_panel = cl_div(8 * p.tiles_m);
         if (p.parts > 1) partials += (size_t)p.parts * p.M * p.N;
         if (i == 1) a.first2 = a.total;
         a.total += p.tiles * p.parts;
