@@ -3190,9 +3190,11 @@ static int conv2d_forward_impl(float* y, const float* x, const float* w_ref, con
     }
     bool wide = false, bn128 = false;
     const ConvRoute route = conv_forward_route(x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, H_out, W_out, wide, bn128);
-    if (!w_mirror && route != CONV_ROUTE_DIRECT && conv_cl_wanted(CL_FORWARD, x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch))
-        return cl_conv_forward(y, x, w_ref, bias, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, bias_stride_pixel, bias_stride_channel,
+    if (!w_mirror && route != CONV_ROUTE_DIRECT && conv_cl_wanted(CL_FORWARD, x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch)) {
+        const int rc = cl_conv_forward(y, x, w_ref, bias, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, bias_stride_pixel, bias_stride_channel,
                                bias_stride_image, activation == NZHIP_ACT_RELU, route != CONV_ROUTE_WORKSPACE, s);    // (the column matrix keeps no image)
+        if (rc != NZHIP_E_NOMEM) return rc;
+    }
     const bool fixed_geometry = route == CONV_ROUTE_FIXED, any_geometry = route == CONV_ROUTE_ANY;
     if (bias_stride_image != 0 && !fixed_geometry && !any_geometry)
         return set_error(NZHIP_E_UNSUPPORTED, "conv2d: a per-image bias needs an implicit-GEMM route");
@@ -3424,8 +3426,10 @@ extern "C" int nzhip_conv2d_backward_data(float* dx, const float* dy, const floa
         return nzhip_gemm(&g, s);
     }
     if (stride == 1 && !conv_direct_applicable(O, C, K_h, K_w, 1, K_h - 1 - pad) &&
-        conv_cl_wanted(CL_DATA, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch))
-        return cl_conv_backward_data(dx, dy, w_ref, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, accumulate, s);
+        conv_cl_wanted(CL_DATA, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch)) {
+        const int rc = cl_conv_backward_data(dx, dy, w_ref, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, accumulate, s);
+        if (rc != NZHIP_E_NOMEM) return rc;
+    }
     if (stride > 1) {
         const size_t Ho = (H + 2 * pad - K_h) / stride + 1, Wo = (W + 2 * pad - K_w) / stride + 1;
         // The convolution of the zero-filled gradient does stride^2 times the multiply-adds; the reference's own chain
@@ -3452,8 +3456,10 @@ extern "C" int nzhip_conv2d_backward_data(float* dx, const float* dy, const floa
         const bool chain_fits = N * P < 0x3fffffff && CKK < 0x3fffffff && O < 0x3fffffff && N <= 65535 && P * O < 0x7fffffffull &&
                                 N * P * CKK <= ((size_t)1 << 29);      // a column gradient of at most 2 GiB
         // one sum per remainder of the position modulo the stride, on channel-last copies
-        if (!dx_env && conv_cl_wanted(CL_DATA, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, chain_fits && as_chain < as_conv ? as_chain : as_conv))
-            return cl_conv_backward_data(dx, dy, w_ref, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, accumulate, s);
+        if (!dx_env && conv_cl_wanted(CL_DATA, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, chain_fits && as_chain < as_conv ? as_chain : as_conv)) {
+            const int rc = cl_conv_backward_data(dx, dy, w_ref, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, accumulate, s);
+            if (rc != NZHIP_E_NOMEM) return rc;
+        }
         if (chain_fits && (dx_env && dx_env[0] ? dx_env[1] == 'h' : as_conv >= as_chain))
             return conv_dx_chain(dx, dy, w_ref, N, C, H, W, O, K_h, K_w, stride, pad, Ho, Wo, w_batch, accumulate, stream);
         const size_t Hu = H + 2 * pad - K_h + 1, Wu = W + 2 * pad - K_w + 1, total = N * O * Hu * Wu;
@@ -4165,8 +4171,10 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
     if (w_batch != 1 && w_batch != N) return set_error(NZHIP_E_SHAPE, "Shapes are not broadcast compatible.");
     if (stride != 0 && K_h != 0 && K_w != 0 && H + 2 * pad >= K_h && W + 2 * pad >= K_w &&
         !(K_h == 3 && K_w == 3 && stride == 1 && pad == 1 && C <= 4 && O <= 2 && W >= 4) &&                 // streamed
-        !(K_h == 1 && K_w == 1 && pad == 0) && conv_cl_wanted(CL_WEIGHTS, x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch))
-        return cl_conv_backward_weights(dw, x, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, reinterpret_cast<hipStream_t>(stream));
+        !(K_h == 1 && K_w == 1 && pad == 0) && conv_cl_wanted(CL_WEIGHTS, x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch)) {
+        const int rc = cl_conv_backward_weights(dw, x, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, reinterpret_cast<hipStream_t>(stream));
+        if (rc != NZHIP_E_NOMEM) return rc;
+    }
     // Images of fewer than 64 output pixels (7 x 7 outputs of a network's last stage) with shared weights: a product per
     // image has a contraction of 49, and a 128-pixel segment of the gather kernel is mostly padding. The column matrices
     // of all images follow each other in memory as ONE [N pixels, C K_h K_w] matrix, so the reference's own chain

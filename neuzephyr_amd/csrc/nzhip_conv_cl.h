@@ -13,6 +13,7 @@ enum ClDirection { CL_FORWARD, CL_DATA, CL_WEIGHTS };
 int cl_conv_fits(ClDirection dir, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad, size_t w_batch);
 // estimated time in us of one that is
 double cl_conv_cost(ClDirection dir, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad, size_t w_batch);
+// The three take all their memory before their first launch; NZHIP_E_NOMEM: nothing was launched, and the caller's other ways need less.
 // may_keep: a prepared handle of the caller may keep the weights' copy
 int cl_conv_forward(float* y, const float* x, const float* w, const float* bias, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h,
                     size_t K_w, size_t stride, size_t pad, size_t w_batch, int64_t bias_sp, int64_t bias_sc, int64_t bias_sn, int relu,

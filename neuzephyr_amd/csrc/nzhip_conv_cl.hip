@@ -163,6 +163,7 @@ struct ClArgs {
     long bias_sp, bias_sc, bias_sn;
     int relu, parts, part_units, tiles_m, tiles, n_classes;      // tiles: of all classes, as if each had as many as the largest
     int dy_h, dy_w;                     // dy's extents; 0 in a forward
+    int units;                          // of the longest sum (host)
     ClDiv by_cu, by_tiles_m, by_classes;
     ClClass cls[CL_MAX_CLASSES];
 };
@@ -750,18 +751,18 @@ static ClWork conv_work(const ClArgs& a, int copies, double prep) {
     return w;
 }
 
-// tiles, parts and launch of a product whose operands are in place; a.M, a.cls (taps and pixels) and everything but tiles and parts is set
-static int conv_product(ClArgs& a, int copies, hipStream_t s) {
+// Tiles and parts of a product; a.M, a.cls (taps and pixels) and everything else but the addresses is set. Bytes of its partial sums.
+static size_t conv_cut(ClArgs& a, int copies, ClPlan& pl) {
     int units = 0;
     for (int i = 0; i < a.n_classes; i++) {
         const int u = a.cls[i].nr * a.cls[i].ns * a.cu;
         if (u > units) units = u;
     }
     const int steps = (units + 7) / 8;
-    ClPlan pl = {0, 1};
     cl_plan(conv_work(a, copies, 0.0), pl);
     plan_env(pl);
     const ClTileShape sh = CL_TILES[pl.tile];
+    a.units = units;
     a.part_units = ((steps + pl.parts - 1) / pl.parts) * 8;
     if (a.part_units < 8) a.part_units = 8;
     a.parts = (units + a.part_units - 1) / a.part_units;
@@ -777,12 +778,13 @@ static int conv_product(ClArgs& a, int copies, hipStream_t s) {
     }
     a.tiles = most * a.n_classes;
     a.by_classes = cl_div(a.n_classes);
-    float* partial = nullptr;
-    if (a.parts > 1)
-        if (int rc = workspace_alloc(reinterpret_cast<void**>(&partial), (size_t)a.parts * a.y_total * sizeof(float), s)) return rc;
-    a.partial = partial;
+    return a.parts > 1 ? (size_t)a.parts * a.y_total * sizeof(float) : 0;
+}
+
+// its launches, operands and partial sums in place
+static int conv_product(const ClArgs& a, int copies, const ClPlan& pl, hipStream_t s) {
     const dim3 grid((unsigned)a.tiles, (unsigned)a.parts, (unsigned)copies);
-    const int mu = a.part_units < units ? a.part_units : units, kgs = sh.kg;
+    const int mu = a.part_units < a.units ? a.part_units : a.units, kgs = CL_TILES[pl.tile].kg;
     const size_t table = (size_t)(((mu + 7) / 8 + kgs - 1) / kgs + 4) * kgs * 8 * sizeof(int2);      // (steps + stages) of every group
     int rc;
     auto go = [&](auto tile) {
@@ -791,13 +793,12 @@ static int conv_product(ClArgs& a, int copies, hipStream_t s) {
     };
     rc = cl_pick(pl.tile, go);
     if (rc == NZHIP_OK && a.parts > 1) {
-        hipLaunchKernelGGL(cl_sum_kernel, dim3((unsigned)((a.y_total + 255) / 256)), dim3(256), 0, s, a.y, partial, a.bias, (unsigned)a.y_total, a.parts,
+        hipLaunchKernelGGL(cl_sum_kernel, dim3((unsigned)((a.y_total + 255) / 256)), dim3(256), 0, s, a.y, a.partial, a.bias, (unsigned)a.y_total, a.parts,
                            (unsigned)a.plane, (unsigned)a.M, a.bias_sp, a.bias_sc, a.bias_sn, a.relu);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) rc = set_hip_error(e, "cl_sum kernel launch");
     }
-    const int rc2 = partial ? workspace_free(partial, s) : NZHIP_OK;
-    return rc ? rc : rc2;
+    return rc;
 }
 
 // The extents the kernels' 32-bit offsets and tables hold: copies and result below 2 GiB, a unit table beside the largest ring.
@@ -880,6 +881,14 @@ int cl_conv_forward(float* y, const float* x, const float* w, const float* bias,
         workspace_free(xc, s);
         return rc;
     }
+    const int copies = w_batch > 1 ? (int)N : 1;
+    ClPlan pl = {0, 1};
+    if (const size_t bytes = conv_cut(a, copies, pl)) rc = workspace_alloc(reinterpret_cast<void**>(&a.partial), bytes, s);
+    if (rc) {
+        may_keep ? image_release(lease, s, false) : workspace_free(lease.ptr, s);
+        workspace_free(xc, s);
+        return rc;
+    }
     ClPrepArgs pa = {};
     prep_planes(pa.job[0], x, xc, (long)N, (int)C, Cp, (int)H, (int)W, (int)(H + 2 * pad), (int)(W + 2 * pad), (int)pad, (int)pad);
     if (lease.fill) prep_weights(pa.job[1], w, reinterpret_cast<_Float16*>(lease.ptr), (long)w_batch, (int)C, Cp, taps, (int)O);
@@ -888,10 +897,11 @@ int cl_conv_forward(float* y, const float* x, const float* w, const float* bias,
     if (rc == NZHIP_OK) {
         a.w = reinterpret_cast<const _Float16*>(lease.ptr); a.x = xc; a.y = y; a.bias = bias;
         a.bias_sp = bias_sp; a.bias_sc = bias_sc; a.bias_sn = bias_sn; a.relu = relu;
-        rc = conv_product(a, w_batch > 1 ? (int)N : 1, s);
+        rc = conv_product(a, copies, pl, s);
     }
     const int rc2 = may_keep ? image_release(lease, s, enqueued) : workspace_free(lease.ptr, s), rc3 = workspace_free(xc, s);
-    return rc ? rc : rc2 ? rc2 : rc3;
+    const int rc4 = a.partial ? workspace_free(a.partial, s) : NZHIP_OK;
+    return rc ? rc : rc2 ? rc2 : rc3 ? rc3 : rc4;
 }
 
 int cl_conv_backward_data(float* dx, const float* dy, const float* w, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w,
@@ -903,8 +913,12 @@ int cl_conv_backward_data(float* dx, const float* dy, const float* w, size_t N, 
     _Float16* zc = nullptr;
     _Float16* wc = nullptr;
     if (int rc = workspace_alloc(reinterpret_cast<void**>(&zc), N * (size_t)a.x_img * 2, s)) return rc;
+    const int copies = w_batch > 1 ? (int)N : 1;
+    ClPlan pl = {0, 1};
     int rc = workspace_alloc(reinterpret_cast<void**>(&wc), w_batch * (size_t)a.w_img * 2, s);
+    if (const size_t bytes = rc ? 0 : conv_cut(a, copies, pl)) rc = workspace_alloc(reinterpret_cast<void**>(&a.partial), bytes, s);
     if (rc) {
+        if (wc) workspace_free(wc, s);
         workspace_free(zc, s);
         return rc;
     }
@@ -915,10 +929,10 @@ int cl_conv_backward_data(float* dx, const float* dy, const float* w, size_t N, 
     if (rc == NZHIP_OK) {
         a.w = wc; a.x = zc; a.y = dx;
         if (accumulate) { a.bias = dx; a.bias_sp = 1; a.bias_sc = a.plane; a.bias_sn = a.y_img; }
-        rc = conv_product(a, w_batch > 1 ? (int)N : 1, s);
+        rc = conv_product(a, copies, pl, s);
     }
-    const int rc2 = workspace_free(wc, s), rc3 = workspace_free(zc, s);
-    return rc ? rc : rc2 ? rc2 : rc3;
+    const int rc2 = workspace_free(wc, s), rc3 = workspace_free(zc, s), rc4 = a.partial ? workspace_free(a.partial, s) : NZHIP_OK;
+    return rc ? rc : rc2 ? rc2 : rc3 ? rc3 : rc4;
 }
 
 static ClWork dw_work(size_t N, size_t C, size_t O, size_t taps, size_t P, size_t w_batch) {
@@ -958,45 +972,49 @@ int cl_conv_backward_weights(float* dw, const float* x, const float* dy, size_t 
     _Float16* xc = nullptr;
     if (int rc = workspace_alloc(reinterpret_cast<void**>(&xc), (x_elems + z_elems) * 2, s)) return rc;      // (rows of whole 16 bytes)
     _Float16* zc = xc + x_elems;
+    ClDwArgs a = {};
+    const int copies = w_batch > 1 ? (int)N : 1, images = w_batch > 1 ? 1 : (int)N;
+    a.x = xc; a.dz = zc; a.dw = dw;
+    a.cu = Cp / 8; a.units = taps * a.cu; a.Kw = (int)K_w; a.C = (int)C; a.taps = taps; a.O = (int)O; a.Op = Op;
+    a.dr = Wp * Cs; a.ds = Cs; a.Os = Os;
+    a.Ho = Ho; a.Wo = Wo; a.pixels = images * Ho * Wo;
+    a.step_h = (unsigned)(stride * Wp * Cs); a.step_w = (unsigned)(stride * Cs); a.x_img = (long)Hp * Wp * Cs;
+    a.z_img = (long)Ho * Wo * Os; a.dw_img = (long)C * taps * O; a.total = copies * a.dw_img;
+    a.x_bytes = (unsigned)(images * a.x_img * 2); a.z_bytes = (unsigned)(images * a.z_img * 2);
+    ClPlan pl = {0, 1};
+    cl_plan(dw_work(N, C, O, taps, (size_t)Ho * Wo, w_batch), pl);
+    plan_env(pl);
+    const ClTileShape sh = CL_TILES[pl.tile];
+    const int adv = 64 * sh.kg, hw = Ho * Wo;
+    a.adv_h = adv % hw / Wo; a.adv_w = adv % hw % Wo;
+    a.adv = (unsigned)(adv / hw * a.x_img + a.adv_h * (long)a.step_h + a.adv_w * (long)a.step_w) * 2u;
+    a.wrap_w = (unsigned)((long)a.step_h - (long)Wo * a.step_w) * 2u;
+    a.wrap_h = (unsigned)(a.x_img - (long)Ho * a.step_h) * 2u;
+    const int steps = (a.pixels + 63) / 64;
+    a.part_steps = (steps + pl.parts - 1) / pl.parts;
+    a.parts = (steps + a.part_steps - 1) / a.part_steps;
+    a.by_cu = cl_div(a.cu); a.by_kw = cl_div(a.Kw); a.by_hw = cl_div(hw); a.by_w = cl_div(Wo);
+    a.tiles_m = (a.units * 8 + sh.bm - 1) / sh.bm;
+    a.by_tiles_m = cl_div(a.tiles_m);
+    a.tiles = a.tiles_m * (int)((O + sh.bn - 1) / sh.bn);
+    float* partial = nullptr;
+    if (a.parts > 1)
+        if (int rc = workspace_alloc(reinterpret_cast<void**>(&partial), (size_t)a.parts * a.total * sizeof(float), s)) {
+            workspace_free(xc, s);
+            return rc;
+        }
+    a.partial = partial;
     ClPrepArgs pa = {};
     prep_planes(pa.job[0], x, xc, (long)N, (int)C, Cp, (int)H, (int)W, Hp, Wp, (int)pad, (int)pad);
     prep_planes(pa.job[1], dy, zc, (long)N, (int)O, Op, Ho, Wo, Ho, Wo, 0, 0);
     int rc = prep_launch(pa, s);
-    float* partial = nullptr;
     if (rc == NZHIP_OK) {
-        ClDwArgs a = {};
-        const int copies = w_batch > 1 ? (int)N : 1, images = w_batch > 1 ? 1 : (int)N;
-        a.x = xc; a.dz = zc; a.dw = dw;
-        a.cu = Cp / 8; a.units = taps * a.cu; a.Kw = (int)K_w; a.C = (int)C; a.taps = taps; a.O = (int)O; a.Op = Op;
-        a.dr = Wp * Cs; a.ds = Cs; a.Os = Os;
-        a.Ho = Ho; a.Wo = Wo; a.pixels = images * Ho * Wo;
-        a.step_h = (unsigned)(stride * Wp * Cs); a.step_w = (unsigned)(stride * Cs); a.x_img = (long)Hp * Wp * Cs;
-        a.z_img = (long)Ho * Wo * Os; a.dw_img = (long)C * taps * O; a.total = copies * a.dw_img;
-        a.x_bytes = (unsigned)(images * a.x_img * 2); a.z_bytes = (unsigned)(images * a.z_img * 2);
-        ClPlan pl = {0, 1};
-        cl_plan(dw_work(N, C, O, taps, (size_t)Ho * Wo, w_batch), pl);
-        plan_env(pl);
-        const ClTileShape sh = CL_TILES[pl.tile];
-        const int adv = 64 * sh.kg, hw = Ho * Wo;
-        a.adv_h = adv % hw / Wo; a.adv_w = adv % hw % Wo;
-        a.adv = (unsigned)(adv / hw * a.x_img + a.adv_h * (long)a.step_h + a.adv_w * (long)a.step_w) * 2u;
-        a.wrap_w = (unsigned)((long)a.step_h - (long)Wo * a.step_w) * 2u;
-        a.wrap_h = (unsigned)(a.x_img - (long)Ho * a.step_h) * 2u;
-        const int steps = (a.pixels + 63) / 64;
-        a.part_steps = (steps + pl.parts - 1) / pl.parts;
-        a.parts = (steps + a.part_steps - 1) / a.part_steps;
-        a.by_cu = cl_div(a.cu); a.by_kw = cl_div(a.Kw); a.by_hw = cl_div(hw); a.by_w = cl_div(Wo);
-        a.tiles_m = (a.units * 8 + sh.bm - 1) / sh.bm;
-        a.by_tiles_m = cl_div(a.tiles_m);
-        a.tiles = a.tiles_m * (int)((O + sh.bn - 1) / sh.bn);
-        if (a.parts > 1) rc = workspace_alloc(reinterpret_cast<void**>(&partial), (size_t)a.parts * a.total * sizeof(float), s);
-        a.partial = partial;
         const dim3 grid((unsigned)a.tiles, (unsigned)a.parts, (unsigned)copies);
         auto go = [&](auto tile) {
             using T = decltype(tile);
             return launch(cl_dw_kernel<T>, grid, T::THREADS, T::RING, a, s, "cl_dw kernel launch");
         };
-        if (rc == NZHIP_OK) rc = cl_pick(pl.tile, go);
+        rc = cl_pick(pl.tile, go);
         if (rc == NZHIP_OK && a.parts > 1) {
             hipLaunchKernelGGL(cl_sum_kernel, dim3((unsigned)((a.total + 255) / 256)), dim3(256), 0, s, dw, partial, dw, (unsigned)a.total, a.parts,
                                (unsigned)a.total, 1u, 1L, 0L, 0L, 0);

@@ -380,6 +380,7 @@ static size_t copy_bytes(const nzhip_gemm_desc* d, int count, const CopyPlan& pl
     return bytes;
 }
 
+// NZHIP_E_NOMEM: no memory for the copies or partial sums, and nothing was launched
 int gemm_copy_run(const nzhip_gemm_desc* d, int count, hipStream_t s, bool one_sum) {
     CopyPlan pl = copy_plan(d, count, one_sum, nullptr);
     copy_plan_env(pl);

@@ -466,11 +466,13 @@ static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s) {
         // 285 -> 276; 2128 x 1984 x 1904 44.5 -> 34, 4096 x 1024 x 2048 35 -> 33; above, 4096 x 1024 x 4096 58 / 65, 6864 x 864 x 3216 69 / 75).
         // A caller that keeps B's image keeps this one, with the same result: one sum over k either way.
         const bool plain = !force_h16 && !image_kept_by_caller(PREPARED_GEMM_B) && (((d.N | d.ldc) & 3) != 0 || 2.0 * d.M * d.N * d.K < 2.8e10);
-        if (plain && gemm_copy_wanted(&d, 1, 1e30, true)) return gemm_copy_run(&d, 1, s, true);
+        if (plain && gemm_copy_wanted(&d, 1, 1e30, true))
+            if (const int rc = gemm_copy_run(&d, 1, s, true); rc != NZHIP_E_NOMEM) return rc;
         return gemm_h16_dispatch(d, s);
     }
     GemmPlan plan = gemm_fused_plan(d);
-    if (gemm_copy_wanted(&d, 1, plan.cost_us)) return gemm_copy_run(&d, 1, s);
+    if (gemm_copy_wanted(&d, 1, plan.cost_us))
+        if (const int rc = gemm_copy_run(&d, 1, s); rc != NZHIP_E_NOMEM) return rc;                 // no memory for the copies: the ways below need less
     if (gemm_trace())
         fprintf(stderr, "nzhip_gemm %ld x %ld x %ld batch %ld x %ld: fused kernel, %d^2 tiles, %ld chunk(s) of %ld, model %.1f us\n",
                 (long)d.M, (long)d.K, (long)d.N, (long)d.batch_n, (long)d.batch_c, plan.tile,
@@ -901,7 +903,8 @@ int nzhip_matmul_backward(float* dA, float* dB, const float* A, const float* B, 
             validate_gemm(d[0]) == NZHIP_OK && validate_gemm(d[1]) == NZHIP_OK && apart(d[0], d[1])) {
             // the product whose shared operand runs along its rows first
             if (d[0].a_layout == NZHIP_LAYOUT_TRANS) std::swap(d[0], d[1]);
-            if (gemm_copy_wanted(d, 2, gemm_single_cost(d[0]) + gemm_single_cost(d[1]))) return gemm_copy_run(d, 2, as_stream(stream));
+            if (gemm_copy_wanted(d, 2, gemm_single_cost(d[0]) + gemm_single_cost(d[1])))
+                if (const int rc = gemm_copy_run(d, 2, as_stream(stream)); rc != NZHIP_E_NOMEM) return rc;
         }
     }
     if (dA) {                                              // dA += dC * B^T   (src/Nodes.cu:171-175)

@@ -452,6 +452,11 @@ int gemm_skinny_dispatch(const nzhip_gemm_desc& d, hipStream_t stream) {
         p.ksplit = (p.K + p.kslice - 1) / p.kslice;
         if (p.ksplit > 1) {
             rc = workspace_alloc(reinterpret_cast<void**>(&partial), sizeof(float) * batch * p.ksplit * p.SR * p.LN, stream);
+            if (rc == NZHIP_E_NOMEM) {                              // in one piece, then
+                rc = NZHIP_OK;
+                p.ksplit = 1;
+                p.kslice = p.K;
+            }
             if (rc) return rc;
             p.partial = partial;
         }
