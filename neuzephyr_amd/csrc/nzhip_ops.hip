@@ -434,10 +434,14 @@ int nzhip_gemm(const nzhip_gemm_desc* desc, void* stream) {
 
 }  // extern "C"
 
-// Estimated time of a product on its own, in us; 0 for those that stream an operand.
+// Estimated time in us of a product with its result's old value added, on its own; 0 for those that stream an operand. The single kernel and the two-pass
+// kernel as measured on the two gradients of layers of 2304 to 8192 rows, columns and k (both 4096^3 304 us, 305 here, both 8192^3 1951 and 2006, both
+// 6000^3 1051 and 1035): a launch, the result's read and write where it does not hide, half as fast in single elements, and the products' rate.
 static double gemm_single_cost(const nzhip_gemm_desc& d) {
     if (gemm_thin_applicable(d) || gemm_skinny_applicable(d)) return 0.0;
-    if (gemm_h16_applicable(d)) return 6.0 + 6.0 * (double)d.K * (double)(d.M + d.N) / 5e6 + 2.0 * d.M * d.N * d.K / 0.78e9;
+    const double flops = 2.0 * d.M * d.N * d.K;
+    if (gemm_h16_coop_applicable(d)) return 30.0 + flops / 1.13e9;
+    if (gemm_h16_applicable(d)) return 28.0 + 8.0 * d.M * d.N / (((d.N | d.ldc) & 3) != 0 ? 3.0e6 : 5.9e6) + flops / 0.98e9;
     return gemm_fused_plan(d).cost_us;
 }
 

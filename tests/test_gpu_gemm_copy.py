@@ -173,6 +173,23 @@ def test_a_kept_image_gives_the_bits_of_the_plain_call(nz, M, K, N):
         h.close()
 
 
+@pytest.mark.parametrize("S,inputs,outputs,copies", [(4096, 4096, 4096, False), (5000, 3000, 3500, False), (8192, 2048, 8192, False),
+                                                     (4096, 1024, 4096, True), (1024, 4096, 4096, True)])
+def test_gradients_of_large_layers_take_the_faster_way(nz, monkeypatch, S, inputs, outputs, copies):
+    """Both in one launch on copies are summed in chains of 512, one after the other in one sum: other bits."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(S)
+    W, x, dz = (torch.randn(s, device="cuda", generator=g) for s in ((1, 1, outputs, inputs), (S, 1, inputs, 1), (S, 1, outputs, 1)))
+
+    def gradients(route):
+        monkeypatch.setenv("NZHIP_GEMM_COPY", route) if route else monkeypatch.delenv("NZHIP_GEMM_COPY")
+        return nz.matmul_backward(torch.zeros_like(W), torch.zeros_like(x), W, x, dz)
+
+    one_launch, two, chosen = gradients("1"), gradients("0"), gradients(None)
+    for way, taken in ((one_launch, copies), (two, not copies)):
+        assert all(torch.equal(a, b) for a, b in zip(way, chosen)) == taken
+
+
 @pytest.mark.parametrize("M,K,N", [(200, 5000, 5000), (1000, 777, 513), (381, 3820, 2880)])
 def test_the_call_without_allocations_gives_the_same_bits(nz, M, K, N):
     import torch
