@@ -466,10 +466,14 @@ static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s) {
     if (!force_fused && allow_coop && gemm_h16_coop_applicable(d)) return gemm_h16_coop_dispatch(d, s);
     if (!force_fused && (force_h16 || gemm_h16_applicable(d))) {
         // On rows of C that are no whole 16-byte pieces the block images' kernel stores element by element, and short of 2.8e10 flops its 256-wide
-        // tiles are few: there the products on plain copies (2831 x 1296 x 2781 77 -> 43 us, 5001 x 999 x 5001 141 -> 106, 4192 x 3031 x 7535
-        // 285 -> 276; 2128 x 1984 x 1904 44.5 -> 34, 4096 x 1024 x 2048 35 -> 33; above, 4096 x 1024 x 4096 58 / 65, 6864 x 864 x 3216 69 / 75).
+        // tiles are few: there the products on plain copies (2831 x 1296 x 2781 77 -> 43 us, 5001 x 999 x 5001 141 -> 106, 2128 x 1984 x 1904 44.5 -> 34,
+        // 4096 x 1024 x 2048 35 -> 33; above, 4096 x 1024 x 4096 58 / 65, 6864 x 864 x 3216 69 / 75). The stores weigh less as a product grows, and
+        // the 256-wide tiles read less: of 45 odd products the copies are ahead up to 1.6e11 flops (two-pass / copies: 3000 x 8191 x 3001 280 / 259,
+        // 1879 x 5382 x 7781 244 / 237) and level or behind from 1.9e11 on (4192 x 7535 x 3031 296 / 320, 4502 x 5068 x 6369 375 / 395, 6001^3 608 / 595,
+        // 5001 x 8000 x 5001 523 / 598, 8191^3 1138 / 1303).
         // A caller that keeps B's image keeps this one, with the same result: one sum over k either way.
-        const bool plain = !force_h16 && !image_kept_by_caller(PREPARED_GEMM_B) && (((d.N | d.ldc) & 3) != 0 || 2.0 * d.M * d.N * d.K < 2.8e10);
+        const double flops = 2.0 * d.M * d.N * d.K;
+        const bool plain = !force_h16 && !image_kept_by_caller(PREPARED_GEMM_B) && (((d.N | d.ldc) & 3) != 0 ? flops < 1.75e11 : flops < 2.8e10);
         if (plain && gemm_copy_wanted(&d, 1, 1e30, true))
             if (const int rc = gemm_copy_run(&d, 1, s, true); rc != NZHIP_E_NOMEM) return rc;
         return gemm_h16_dispatch(d, s);
