@@ -161,16 +161,20 @@ def test_chosen_plans_are_bit_exact_on_whole_numbers(nz, M, K, N, b_trans):
     assert np.array_equal(got.cpu().numpy(), A.astype(np.float64) @ B)
 
 
-@pytest.mark.parametrize("M,K,N", [(600, 9000, 600), (1400, 1296, 1001), (520, 4100, 2052), (3072, 768, 3072)])
-def test_a_kept_image_gives_the_bits_of_the_plain_call(nz, M, K, N):
+@pytest.mark.parametrize("b_trans", [False, True])
+@pytest.mark.parametrize("M,K,N", [(2831, 1296, 2781), (2000, 777, 2001), (1801, 801, 1803), (3072, 768, 3072)])
+def test_a_kept_image_gives_the_bits_of_the_plain_call(nz, M, K, N, b_trans):
+    """The plain call multiplies copies, the one that keeps B's image takes the two-pass kernel: one sum over k in either."""
     import torch
     rng = np.random.default_rng(M)
-    A, B = (torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda() for s in ((M, K), (K, N)))
-    h = nz.Prepared()
-    try:
-        assert torch.equal(nz.gemm(A, B, prepared_b=h), nz.gemm(A, B))
-    finally:
-        h.close()
+    A, B, b = (torch.from_numpy(rng.standard_normal(s).astype(np.float32)).cuda() for s in ((M, K), (N, K) if b_trans else (K, N), (N,)))
+    for how in ({}, {"bias": b, "bias_strides": (0, 1), "relu": True}):
+        h = nz.Prepared()
+        try:
+            assert torch.equal(nz.gemm(A, B, b_trans=b_trans, prepared_b=h, **how), nz.gemm(A, B, b_trans=b_trans, **how))
+            assert h.fills() == 1                                     # else the handle was not used, and both calls were the same one
+        finally:
+            h.close()
 
 
 @pytest.mark.parametrize("S,inputs,outputs,copies", [(4096, 4096, 4096, False), (5000, 3000, 3500, False), (8192, 2048, 8192, False),
