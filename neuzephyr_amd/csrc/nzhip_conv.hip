@@ -3010,7 +3010,9 @@ static bool conv_cl_wanted(ClDirection dir, const float* src, size_t N, size_t C
         if (!k3 && (K_h * K_w > 128 || stride > 4 || ((128 / sw - 1) * stride + K_h) * ((sw - 1) * stride + K_w + 8) > 14000)) return false;
         // 4x64x128x128 -> 128 38 / 57, 16x32x64x64 -> 128 37 / 39, 16x64x128x128 -> 128 at stride 2 59 / 74; 8x128x64x64 -> 64 39 / 32
         if (pieces && Wo % 4 == 0 && out >= 60000 && C >= 32) return false;
-        return !(pieces && k3 && W <= 64 && out >= 45000 && C >= 64 && O == 128);      // 16x128x56x56 -> 128 51 / 55, -> 256 84 / 78
+        // The window kernel's tile is 128 outputs wide: ahead where one holds them all and is two thirds full. 16x128x56x56 -> 64 51 / 44,
+        // -> 96 51 / 54, -> 112 51 / 55, -> 127 52 / 56, -> 128 51 / 56, -> 136 81 / 67, -> 256 88 / 80; 15x96x64x60 -> 128 49 / 58
+        return !(pieces && k3 && W <= 64 && out >= 45000 && C >= 64 && O > 85 && O <= 128);
     }
     if (K_h == 1 && K_w == 1) return dir == CL_FORWARD && stride == 1;                  // too few channels for a product: 16x16x176x67 -> 20 51 / 31
     if (k3) {                                                      // (a 3x3 data gradient of stride 1 as well)

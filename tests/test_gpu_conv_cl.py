@@ -227,3 +227,31 @@ def test_chosen_plans_are_bit_exact_on_whole_numbers(nz, layer):
     dw = torch.zeros(w.shape, device="cuda")
     nz.conv2d_backward_weights(dw, cu(x), cu(dy), K, K, stride, pad)
     assert np.array_equal(dw.cpu().numpy(), dw64)
+
+
+# direction, layer (N, C, H, W, O, K, stride, pad, copies), a bias per pixel, whether the kernels on copies are the faster ones
+CHOICES = [
+    ("weights", (16, 128, 56, 56, 112, 3, 1, 1, 1), False, False), ("weights", (16, 128, 56, 56, 128, 3, 1, 1, 1), False, False),
+    ("weights", (16, 128, 56, 56, 64, 3, 1, 1, 1), False, True), ("weights", (16, 128, 56, 56, 136, 3, 1, 1, 1), False, True),
+]
+
+
+@pytest.mark.parametrize("direction,layer,pixel_bias,copies", CHOICES)
+def test_layers_take_the_faster_kernels(nz, monkeypatch, direction, layer, pixel_bias, copies):
+    """Told apart by their bits: the kernels leave a chain of sums at other places."""
+    import torch
+    N, C, H, W, O, K, stride, pad, w_copies = layer
+    g = torch.Generator(device="cuda").manual_seed(sum(layer))
+    normal = lambda *s: torch.randn(s, device="cuda", generator=g)
+    Ho, Wo = (H + 2 * pad - K) // stride + 1, (W + 2 * pad - K) // stride + 1
+    x, w, dy = normal(N, C, H, W), normal(w_copies, 1, C * K * K, O), normal(N, O, Ho, Wo)
+    b, strides = (normal(1, 1, Ho * Wo, O), (O, 1)) if pixel_bias else (normal(O), (0, 1))
+
+    def result(route):
+        monkeypatch.setenv("NZHIP_CONV_CL", route) if route else monkeypatch.delenv("NZHIP_CONV_CL")
+        if direction == "forward": return nz.conv2d_forward(x, w, b, K, K, stride, pad, bias_strides=strides)
+        if direction == "data": return nz.conv2d_backward_data(torch.empty_like(x), dy, w, K, K, stride, pad, accumulate=False)
+        return nz.conv2d_backward_weights(torch.zeros_like(w), x, dy, K, K, stride, pad)
+
+    on_copies, other, chosen = result("1"), result("0"), result(None)
+    assert torch.equal(on_copies, chosen) == copies and torch.equal(other, chosen) == (not copies)
