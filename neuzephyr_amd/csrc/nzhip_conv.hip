@@ -3010,6 +3010,13 @@ static bool conv_cl_wanted(ClDirection dir, const float* src, size_t N, size_t C
         if (!k3 && (K_h * K_w > 128 || stride > 4 || ((128 / sw - 1) * stride + K_h) * ((sw - 1) * stride + K_w + 8) > 14000)) return false;
         // 4x64x128x128 -> 128 38 / 57, 16x32x64x64 -> 128 37 / 39, 16x64x128x128 -> 128 at stride 2 59 / 74; 8x128x64x64 -> 64 39 / 32
         if (pieces && Wo % 4 == 0 && out >= 60000 && C >= 32) return false;
+        // The window kernels take 16 channels at once and read dy once: ahead where those are more than half used and dy is large. 16x10x96x96 -> 87 33 / 47,
+        // 8x15x96x96 -> 242 36 / 53, 10x12x60x60 -> 149 18.4 / 25.7; 8x12x64x64 -> 96 23 / 22, 32x10x9x32 -> 240 24 / 17, 32x6x48x48 -> 160 47 / 36
+        if (pieces && k3 && C > 8 && C <= 16 && O > 64 && out >= 36000) return false;
+        // With a weight copy per image they add no partial sums up: 32x9x128x128 -> 480 at stride 2 65 / 158, 16x6x32x180 -> 192 5x5 35 / 59, 16x7x64x64 -> 84 at
+        // stride 2 13 / 17, 8x4x32x32 -> 96 5x5 11.7 / 14.1; 16x11x10x36 -> 384 5x5 28 / 27; rows of up to 16 outputs, of which a step takes
+        // eight, 16x6x32x32 -> 225 at stride 2 17.6 / 12.0; shared weights 16x7x32x32 -> 128 5x5 42 / 19
+        if (pieces && Wo % 4 == 0 && Wo > 16 && !k3 && w_batch > 1 && C <= 16 && O > 64 && K_h <= 5) return false;
         // The window kernel's tile is 128 outputs wide: ahead where one holds them all and is two thirds full. 16x128x56x56 -> 64 51 / 44,
         // -> 96 51 / 54, -> 112 51 / 55, -> 127 52 / 56, -> 128 51 / 56, -> 136 81 / 67, -> 256 88 / 80; 15x96x64x60 -> 128 49 / 58
         return !(pieces && k3 && W <= 64 && out >= 45000 && C >= 64 && O > 85 && O <= 128);

@@ -233,6 +233,9 @@ def test_chosen_plans_are_bit_exact_on_whole_numbers(nz, layer):
 CHOICES = [
     ("weights", (16, 128, 56, 56, 112, 3, 1, 1, 1), False, False), ("weights", (16, 128, 56, 56, 128, 3, 1, 1, 1), False, False),
     ("weights", (16, 128, 56, 56, 64, 3, 1, 1, 1), False, True), ("weights", (16, 128, 56, 56, 136, 3, 1, 1, 1), False, True),
+    ("weights", (8, 15, 96, 96, 242, 3, 1, 1, 1), False, False), ("weights", (32, 6, 48, 48, 160, 3, 1, 1, 1), False, True),
+    ("weights", (16, 6, 32, 180, 192, 5, 1, 2, 16), False, False), ("weights", (16, 7, 32, 32, 128, 5, 1, 2, 1), False, True),
+    ("weights", (16, 7, 64, 64, 84, 3, 2, 1, 16), False, False), ("weights", (16, 6, 32, 32, 225, 3, 2, 1, 16), False, True),
 ]
 
 
