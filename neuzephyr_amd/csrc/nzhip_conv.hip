@@ -2987,9 +2987,10 @@ using namespace nzhip;
 // Whether a layer (its forward's extents; `src`: the tensor the direction reads in rows of W, x or dy) takes the channel-last kernels
 // (nzhip_conv_cl.hip). They pay for their fp16 copies with a launch and 1.5 times the bytes of what they copy, and have no chain over
 // windows after that: ahead on everything but large images whose rows are whole 16-byte pieces, where the window kernels have
-// enough windows for every CU and read fp32 once. Lines drawn on 130 layers, both sides measured (us, window kernels / these):
+// enough windows for every CU and read fp32 once. pixel_bias: a forward whose bias the other kernels turn into planes with a launch of its own.
+// Lines drawn on 130 layers and checked on 575 (3 to 512 channels, 7 x 7 to 224 x 224, kernels 3, 5 and 7), both sides measured (us, window kernels / these):
 static bool conv_cl_wanted(ClDirection dir, const float* src, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride,
-                           size_t pad, size_t w_batch, double other_us = 0.0) {
+                           size_t pad, size_t w_batch, bool pixel_bias = false, double other_us = 0.0) {
     const int fits = cl_conv_fits(dir, N, C, H, W, O, K_h, K_w, stride, pad, w_batch);
     if (fits != 1) return fits != 0;
     // a run that asks for one of the other routes gets it
@@ -3028,7 +3029,9 @@ static bool conv_cl_wanted(ClDirection dir, const float* src, size_t N, size_t C
         const size_t in = dir == CL_FORWARD ? C : O, to = dir == CL_FORWARD ? O : C, bn = to > 64 ? 128 : 64, tw = W >= 64 ? 64 : 32, th = 256 / tw;
         const bool resident = ((in + 15) / 16) * bn * 288 <= 148 * 1024 && (w_batch == 1 || N * ((to + bn - 1) / bn) <= (size_t)device_cu_count());
         const bool full = H * W * 10 >= ((W + tw - 1) / tw * tw) * ((H + th - 1) / th * th) * 7;
-        if (resident && full && pieces && in >= 8) return px < 40000;
+        // one tile of outputs and a bias that the window kernels read as it lies: 8x128x64x64 -> 64 19.1 / 21.8, 16x66x48x48 -> 16 15.8 / 22.4, 8x83x64x64
+        // -> 32 17.3 / 18.7; below 24000 pixels 10x64x32x32 -> 60 13.4 / 10.9, 8x96x32x32 -> 64 15.1 / 12.8, up to 64 channels 8x16x64x64 -> 48 11.5 / 11.2
+        if (resident && full && pieces && in >= 8) return px < (dir == CL_FORWARD && !pixel_bias && in > 64 && to <= 64 ? 24000 : 40000);
         // weights beyond LDS: level on the largest, 16x256x56x56 -> 256 115 / 111, gradient 104 / 104; 16x512x28x28 -> 512 102 / 99
         return true;
     }
@@ -3199,7 +3202,7 @@ static int conv2d_forward_impl(float* y, const float* x, const float* w_ref, con
     }
     bool wide = false, bn128 = false;
     const ConvRoute route = conv_forward_route(x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, H_out, W_out, wide, bn128);
-    if (!w_mirror && route != CONV_ROUTE_DIRECT && conv_cl_wanted(CL_FORWARD, x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch)) {
+    if (!w_mirror && route != CONV_ROUTE_DIRECT && conv_cl_wanted(CL_FORWARD, x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, bias && bias_stride_pixel != 0)) {
         const int rc = cl_conv_forward(y, x, w_ref, bias, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, bias_stride_pixel, bias_stride_channel,
                                bias_stride_image, activation == NZHIP_ACT_RELU, route != CONV_ROUTE_WORKSPACE, s);    // (the column matrix keeps no image)
         if (rc != NZHIP_E_NOMEM) return rc;
@@ -3465,7 +3468,7 @@ extern "C" int nzhip_conv2d_backward_data(float* dx, const float* dy, const floa
         const bool chain_fits = N * P < 0x3fffffff && CKK < 0x3fffffff && O < 0x3fffffff && N <= 65535 && P * O < 0x7fffffffull &&
                                 N * P * CKK <= ((size_t)1 << 29);      // a column gradient of at most 2 GiB
         // one sum per remainder of the position modulo the stride, on channel-last copies
-        if (!dx_env && conv_cl_wanted(CL_DATA, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, chain_fits && as_chain < as_conv ? as_chain : as_conv)) {
+        if (!dx_env && conv_cl_wanted(CL_DATA, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, false, chain_fits && as_chain < as_conv ? as_chain : as_conv)) {
             const int rc = cl_conv_backward_data(dx, dy, w_ref, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, accumulate, s);
             if (rc != NZHIP_E_NOMEM) return rc;
         }

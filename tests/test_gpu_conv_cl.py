@@ -236,6 +236,8 @@ CHOICES = [
     ("weights", (8, 15, 96, 96, 242, 3, 1, 1, 1), False, False), ("weights", (32, 6, 48, 48, 160, 3, 1, 1, 1), False, True),
     ("weights", (16, 6, 32, 180, 192, 5, 1, 2, 16), False, False), ("weights", (16, 7, 32, 32, 128, 5, 1, 2, 1), False, True),
     ("weights", (16, 7, 64, 64, 84, 3, 2, 1, 16), False, False), ("weights", (16, 6, 32, 32, 225, 3, 2, 1, 16), False, True),
+    ("forward", (8, 128, 64, 64, 64, 3, 1, 1, 1), False, False), ("forward", (8, 128, 64, 64, 64, 3, 1, 1, 1), True, True),
+    ("forward", (10, 64, 32, 32, 60, 3, 1, 1, 1), False, True),
 ]
 
 
