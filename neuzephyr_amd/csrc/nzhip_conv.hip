@@ -3000,9 +3000,13 @@ static bool conv_cl_wanted(ClDirection dir, const float* src, size_t N, size_t C
     const bool pieces = W % 4 == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0, k3 = K_h == 3 && K_w == 3 && stride == 1;
     // few channels either side of large images: 8x16x112x112 -> 16 23.2 / 27.5, 16x4x192x92 -> 16 5x5 45.8 / 56.5
     if (stride == 1 && C <= 16 && O <= 16 && px >= 100000) return false;
+    // and with fewer than 8, which the copy fills up to 8: 16x7x192x192 -> 32 52 / 70, 16x4x176x176 -> 64 52 / 64
+    if (dir == CL_FORWARD && k3 && C < 8 && O <= 64 && px >= 400000) return false;
     // one weight copy per image, each for a few pixels: the fp16 copies cost more than they save (4x208x13x13 -> 312 at stride 2, 49
-    // pixels: 15.0 / 16.6, gradient 13.3 / 15.3; 10x256x11x11 -> 395 5x5, 121 pixels: 78.6 / 56.4, gradient 50.8 / 58.6)
-    if (w_batch > 1 && dir != CL_WEIGHTS && Ho * Wo * (dir == CL_FORWARD ? 4 : 2) <= O) return false;
+    // pixels: 15.0 / 16.6, gradient 13.3 / 15.3; 10x256x11x11 -> 395 5x5, 121 pixels: 78.6 / 56.4, gradient 50.8 / 58.6). What counts is the copy
+    // with its channels filled up to 8 (16x4x12x12 -> 425 5x5, 144 pixels, 12.1 / 16.5; 16x9x16x16 -> 176 7x7 at stride 2, 64 pixels, 13.3 / 16.8)
+    if (w_batch > 1 && dir == CL_FORWARD && Ho * Wo * 4 * C <= O * ((C + 7) / 8 * 8)) return false;
+    if (w_batch > 1 && dir == CL_DATA && Ho * Wo * 2 <= O) return false;
     if (dir == CL_WEIGHTS) {
         if (K_h == 1 && K_w == 1) return false;                    // products
         // what the gather kernel refuses stays refused: taps, strides and staged windows (of one channel) beyond it

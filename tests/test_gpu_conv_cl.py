@@ -238,6 +238,8 @@ CHOICES = [
     ("weights", (16, 7, 64, 64, 84, 3, 2, 1, 16), False, False), ("weights", (16, 6, 32, 32, 225, 3, 2, 1, 16), False, True),
     ("forward", (8, 128, 64, 64, 64, 3, 1, 1, 1), False, False), ("forward", (8, 128, 64, 64, 64, 3, 1, 1, 1), True, True),
     ("forward", (10, 64, 32, 32, 60, 3, 1, 1, 1), False, True),
+    ("forward", (16, 4, 12, 12, 425, 5, 1, 2, 16), False, False), ("forward", (16, 5, 16, 16, 403, 5, 1, 2, 16), False, True),
+    ("forward", (16, 4, 176, 176, 64, 3, 1, 1, 16), False, False), ("forward", (10, 4, 160, 160, 192, 3, 1, 1, 10), False, True),
 ]
 
 
