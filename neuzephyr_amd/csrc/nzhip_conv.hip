@@ -2982,8 +2982,23 @@ static int conv_subsample(float** sub, const float* x, size_t planes, size_t H, 
 
 using namespace nzhip;
 
-// bias_stride_image != 0: the bias varies per image too (used to add into an existing tensor: bias = y with
-// strides (1, H_out*W_out, O*H_out*W_out)); only the implicit-GEMM kernels take it.
+// Which kernel family a forward convolution takes (a per-image bias, which only the data gradient uses, does not change
+// the choice; the two implicit-GEMM families support it, the others do not).
+enum ConvRoute { CONV_ROUTE_DIRECT, CONV_ROUTE_FIXED, CONV_ROUTE_ANY, CONV_ROUTE_WORKSPACE };
+static ConvRoute conv_forward_route(const float* x, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride,
+                                    size_t pad, size_t w_batch, size_t H_out, size_t W_out, bool& wide, bool& bn128);
+
+// Whether the any-geometry kernel takes a convolution in whole rounds of the CUs, with all pixels of its windows in use.
+static bool conv_windows_full(const float* x, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad,
+                              size_t w_batch) {
+    const size_t Ho = (H + 2 * pad - K_h) / stride + 1, Wo = (W + 2 * pad - K_w) / stride + 1;
+    bool wide, bn128;
+    if (conv_forward_route(x, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, Ho, Wo, wide, bn128) != CONV_ROUTE_ANY) return false;
+    const size_t sw = (size_t)1 << conv_igemm_gen_sw_log(Wo, O, K_h, K_w, stride, pad), sr = CG_PX / sw;
+    const size_t windows = N * ((Ho + sr - 1) / sr) * ((Wo + sw - 1) / sw), tiles = O > 64 ? (O + 127) / 128 : 1;
+    return windows * tiles % (size_t)device_cu_count() == 0 && N * Ho * Wo * 100 >= windows * CG_PX * 97;
+}
+
 // Whether a layer (its forward's extents; `src`: the tensor the direction reads in rows of W, x or dy) takes the channel-last kernels
 // (nzhip_conv_cl.hip). They pay for their fp16 copies with a launch and 1.5 times the bytes of what they copy, and have no chain over
 // windows after that: ahead on everything but large images whose rows are whole 16-byte pieces, where the window kernels have
@@ -3037,8 +3052,12 @@ static bool conv_cl_wanted(ClDirection dir, const float* src, size_t N, size_t C
         // -> 32 17.3 / 18.7; below 24000 pixels 10x64x32x32 -> 60 13.4 / 10.9, 8x96x32x32 -> 64 15.1 / 12.8, up to 64 channels 8x16x64x64 -> 48 11.5 / 11.2
         if (resident && full && pieces && in >= 8) return px < (dir == CL_FORWARD && !pixel_bias && in > 64 && to <= 64 ? 24000 : 40000);
         // weights beyond LDS: level on the largest, 16x256x56x56 -> 256 115 / 111, gradient 104 / 104; 16x512x28x28 -> 512 102 / 99
-        return true;
     }
+    // The any-geometry windows where they fill every round of the CUs and leave no pixel of a window idle: 16x352x64x64 -> 128 84 / 121, 16x212x64x64 -> 208
+    // 105 / 141, gradient 105 / 126, 32x83x64x64 -> 192 at stride 2 43 / 53, 16x95x32x64 -> 144 5x5 52 / 61; with 2.5 rounds 10x287x128x128 -> 32 167 / 147
+    if (pieces && (dir == CL_FORWARD ? conv_windows_full(src, N, C, H, W, O, K_h, K_w, stride, pad, w_batch)
+                                     : k3 && pad <= 2 && conv_windows_full(src, N, O, Ho, Wo, C, 3, 3, 1, 2 - pad, w_batch))) return false;
+    if (k3) return true;
     if (dir == CL_DATA && stride == 1) return true;                // 16x64x128x128 -> 128 5x5 233 / 177
     if (dir == CL_DATA) {
         // The other ways multiply zeros or move a column gradient; `other_us` is the caller's estimate for the better of them. The estimate
@@ -3051,10 +3070,6 @@ static bool conv_cl_wanted(ClDirection dir, const float* src, size_t N, size_t C
     // 16x64x128x128 -> 128 at stride 2 47 / 54, 5x5 167 / 184; 8x14x144x144 -> 64 7x7 at stride 2, 41472 outputs, 38 / 25
     return !(pieces && out >= 50000);
 }
-
-// Which kernel family a forward convolution takes (a per-image bias, which only the data gradient uses, does not change
-// the choice; the two implicit-GEMM families support it, the others do not).
-enum ConvRoute { CONV_ROUTE_DIRECT, CONV_ROUTE_FIXED, CONV_ROUTE_ANY, CONV_ROUTE_WORKSPACE };
 
 static ConvRoute conv_forward_route(const float* x, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride,
                                     size_t pad, size_t w_batch, size_t H_out, size_t W_out, bool& wide, bool& bn128) {
@@ -3114,6 +3129,8 @@ static ConvRoute conv_forward_route(const float* x, size_t N, size_t C, size_t H
     return fixed_ok && !few_patches ? CONV_ROUTE_FIXED : CONV_ROUTE_WORKSPACE;
 }
 
+// bias_stride_image != 0: the bias varies per image too (used to add into an existing tensor: bias = y with
+// strides (1, H_out*W_out, O*H_out*W_out)); only the implicit-GEMM kernels take it.
 // w_mirror: w_ref is the parameter of the convolution whose DATA GRADIENT this call computes ([(c_f, tap)][o_f] with
 // c_f running over this call's O channels and o_f over its C), to be used with channels swapped and taps mirrored.
 // The implicit-GEMM routes read it that way while they build their fp16 weight image, the direct kernels while they fetch

@@ -240,6 +240,8 @@ CHOICES = [
     ("forward", (10, 64, 32, 32, 60, 3, 1, 1, 1), False, True),
     ("forward", (16, 4, 12, 12, 425, 5, 1, 2, 16), False, False), ("forward", (16, 5, 16, 16, 403, 5, 1, 2, 16), False, True),
     ("forward", (16, 4, 176, 176, 64, 3, 1, 1, 16), False, False), ("forward", (10, 4, 160, 160, 192, 3, 1, 1, 10), False, True),
+    ("forward", (16, 352, 64, 64, 128, 3, 1, 1, 1), False, False), ("forward", (10, 287, 128, 128, 32, 3, 1, 1, 1), False, True),
+    ("data", (16, 212, 64, 64, 208, 3, 1, 1, 16), False, False), ("data", (16, 352, 64, 64, 128, 3, 1, 1, 1), False, True),
 ]
 
 
