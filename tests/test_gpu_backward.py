@@ -241,6 +241,14 @@ def test_conv2d_backward_data_matches_the_chain_on_integers(nz, oracle, N, C, H,
     assert np.array_equal(got, expect)
 
 
+@pytest.mark.parametrize("N,C,H,W,O,K,pad,wb", CONV_BWD_DATA)
+@pytest.mark.parametrize("accumulate", [True, False])
+def test_conv2d_backward_data_without_copies_matches_the_chain_on_integers(nz, oracle, monkeypatch, N, C, H, W, O, K, pad, wb, accumulate):
+    # the kernels and chains that large layers and calls without memory for copies still take
+    monkeypatch.setenv("NZHIP_CONV_CL", "0")
+    test_conv2d_backward_data_matches_the_chain_on_integers(nz, oracle, N, C, H, W, O, K, pad, wb, accumulate)
+
+
 def test_conv2d_backward_data_float_tolerance_and_adjoint(nz, oracle):
     N, C, H, W, O, K, pad = 2, 32, 24, 40, 48, 3, 1
     rng = np.random.default_rng(5)
@@ -289,6 +297,13 @@ def test_strided_conv2d_backward_data_is_exact_on_integers(nz, oracle, N, C, H, 
     expect = oracle.conv2d_backward_data(dx0.copy() if accumulate else np.zeros_like(dx0), dy, w, K, K, pad, stride)
     got = host(nz.conv2d_backward_data(dev(dx0), dev(dy), dev(w), K, K, stride, pad, accumulate=accumulate))
     assert np.array_equal(got, expect)
+
+
+@pytest.mark.parametrize("N,C,H,W,O,K,stride,pad,wb", CONV_BWD_DATA_STRIDED)
+@pytest.mark.parametrize("accumulate", [True, False])
+def test_strided_conv2d_backward_data_without_copies_is_exact_on_integers(nz, oracle, monkeypatch, N, C, H, W, O, K, stride, pad, wb, accumulate):
+    monkeypatch.setenv("NZHIP_CONV_CL", "0")
+    test_strided_conv2d_backward_data_is_exact_on_integers(nz, oracle, N, C, H, W, O, K, stride, pad, wb, accumulate)
 
 
 def test_conv2d_backward_data_rejects_what_it_does_not_cover(nz):
@@ -414,6 +429,18 @@ def test_conv_backward_weights_any_geometry_is_bit_exact_on_integers(nz, oracle,
     expect = oracle.conv2d_backward_weights(dw0.copy(), x, dy, Kh, Kw, pad, stride)
     got = host(nz.conv2d_backward_weights(dev(dw0), dev(x), dev(dy), Kh, Kw, stride, pad))
     assert np.array_equal(got, expect)
+
+
+@pytest.mark.parametrize("N,C,H,W,O,Kh,Kw,stride,pad,wb", CONV_GEN_BWD_W)
+def test_conv_backward_weights_any_geometry_without_copies_is_bit_exact_on_integers(nz, oracle, monkeypatch, N, C, H, W, O, Kh, Kw, stride, pad, wb):
+    monkeypatch.setenv("NZHIP_CONV_CL", "0")
+    test_conv_backward_weights_any_geometry_is_bit_exact_on_integers(nz, oracle, N, C, H, W, O, Kh, Kw, stride, pad, wb)
+
+
+@pytest.mark.parametrize("N,C,H,W,O,wb", CONV_BWD_W)
+def test_conv2d_backward_weights_without_copies_is_bit_exact_on_integers(nz, oracle, monkeypatch, N, C, H, W, O, wb):
+    monkeypatch.setenv("NZHIP_CONV_CL", "0")
+    test_conv2d_backward_weights_is_bit_exact_on_integers(nz, oracle, N, C, H, W, O, wb)
 
 
 @pytest.mark.parametrize("N,C,H,W,O,Kh,Kw,stride,pad,wb", [c for c in CONV_GEN_BWD_W if c[3] % 4 != 0 or ((c[3] + 2 * c[8] - c[6]) // c[7] + 1) % 4 != 0])

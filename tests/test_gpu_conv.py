@@ -193,6 +193,19 @@ def test_conv2d_any_geometry_integers_bit_exact(nz, oracle, N, C, H, W, O, k_h, 
         assert np.array_equal(got[n:n + 1].astype(np.float64), truth), (n,)
 
 
+@pytest.mark.parametrize("N,C,H,W,O,k_h,k_w,stride,pad,w_batch,pix", CONV_ANY_GEOMETRY)
+def test_conv2d_any_geometry_without_copies_integers_bit_exact(nz, oracle, monkeypatch, N, C, H, W, O, k_h, k_w, stride, pad, w_batch, pix):
+    # the window kernels that large images and calls without memory for copies still take
+    monkeypatch.setenv("NZHIP_CONV_CL", "0")
+    test_conv2d_any_geometry_integers_bit_exact(nz, oracle, N, C, H, W, O, k_h, k_w, stride, pad, w_batch, pix)
+
+
+@pytest.mark.parametrize("N,C,H,W,O,k_h,k_w,stride,pad,w_batch", CONV_CASES)
+def test_conv2d_without_copies_integers_bit_exact(nz, oracle, monkeypatch, N, C, H, W, O, k_h, k_w, stride, pad, w_batch):
+    monkeypatch.setenv("NZHIP_CONV_CL", "0")
+    test_conv2d_integers_bit_exact(nz, oracle, N, C, H, W, O, k_h, k_w, stride, pad, w_batch)
+
+
 WIDENED = [  # N, C, H, W, O, k, stride, pad, w_batch, per-pixel bias: rows that are not whole 16-byte pieces on the any-geometry kernel
     # (5x5; stride 2 with the per-pixel bias; a split contraction; per-sample weights; two chunks per loop step, which such
     # rows only reach through the copy; 7x7 stride 2 on three channels)
