@@ -503,9 +503,9 @@ bool gemm_copy_wanted(const nzhip_gemm_desc* d, int count, double other_us, bool
     // 128 x 1024 x 1024 9.3 us or 9.8, 112 x 2721 x 1853 15.3 or 16.7, 1520 x 243 x 346 6.4 or 7.0, 66 x 6196 x 5601 38 or 54.
     if (count == 2) {
         // Two products' operands and results outgrow the caches as they grow, which the steps' times do not know: 12 % at 3e11 flops, 24 % at 2e12.
-        // 113 pairs of 256 to 8192 samples, inputs and outputs: one taken is more than 4 % behind two calls, 2560 x 6336 -> 2112 212 / 234. Taken: 4096 samples, 1024 inputs, 4096
-        // outputs 168 -> 104 us, 3072^3 205 / 191, 4001^3 420 / 377, 537 x 681 -> 644 28.3 -> 12.4. Not taken: 4096^3 304 / 369, 8192 x 4096 -> 4096
-        // 551 / 690, 5000 x 3000 -> 3500 313 / 332, 8192^3 1951 / 2594.
+        // 113 pairs of 256 to 8192 samples, inputs and outputs: one taken is more than 4 % behind two calls, 2560 x 6336 -> 2112 212 / 234. Taken: 4096
+        // samples, 1024 inputs, 4096 outputs 168 -> 104 us, 3072^3 205 / 191, 4001^3 420 / 377, 537 x 681 -> 644 28.3 -> 12.4. Not taken: 4096^3
+        // 304 / 369, 8192 x 4096 -> 4096 551 / 690, 5000 x 3000 -> 3500 313 / 332, 8192^3 1951 / 2594.
         const double flops = 4.0 * d[0].M * d[0].N * d[0].K;
         return cost * std::max(1.0, 1.0 + 0.045 * std::log2(flops / 5e10)) < other_us;
     }
