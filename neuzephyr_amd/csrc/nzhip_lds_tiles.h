@@ -36,9 +36,12 @@ __device__ __forceinline__ int4_t cl_buffer(const void* base, unsigned bytes) {
     const uint64_t a = reinterpret_cast<uint64_t>(base);
     return int4_t{(int)(uint32_t)a, (int)(uint32_t)(a >> 32), (int)bytes, (int)CL_RSRC};
 }
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"                   // m0 is reserved: that it is not preserved across the assembly is what is said here
 __device__ __forceinline__ void cl_load(int4_t r, unsigned lds, unsigned off) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(r), "s"(lds) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 __device__ __forceinline__ unsigned cl_lds(const char* p) { return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const char*)p; }
 // n / d for n below 2^31: one product and a shift (a division by a run-time value is some 40 instructions, and a workgroup needs a
 // dozen of them before its first request)
