@@ -2420,7 +2420,7 @@ static int conv2d_via_workspace(float* y, const float* x, const float* w_ref, co
         g.bias_stride_row = bias_sc;       // output row = channel
         g.bias_stride_col = bias_sp;       // output column = pixel
         g.activation = act;
-        rc = nzhip_gemm(&g, s);
+        rc = gemm_of_columns(&g, s);
     }
     int rc2 = workspace_free(col, s);
     return rc ? rc : rc2;
@@ -3217,7 +3217,7 @@ static int conv2d_forward_impl(float* y, const float* x, const float* w_ref, con
             }
             g.bias = bias_planes; g.bias_stride_row = (int64_t)(H * W); g.bias_stride_col = 1;
         }
-        const int rc = nzhip_gemm(&g, s);
+        const int rc = gemm_of_columns(&g, s);
         const int rc2 = bias_planes ? workspace_free(bias_planes, s) : NZHIP_OK;
         return rc ? rc : rc2;
     }
@@ -3356,7 +3356,7 @@ static int conv_dx_chain_planes(float* dx, const float* dy, const float* w_ref, 
         g.batch_n = (int64_t)N; g.batch_c = 1;
         g.a_stride_n = w_batch > 1 ? (int64_t)(CKK * O) : 0; g.b_stride_n = (int64_t)(O * P); g.c_stride_n = (int64_t)(CKK * Pp);
         g.activation = NZHIP_ACT_NONE;
-        rc = nzhip_gemm(&g, s);
+        rc = gemm_of_columns(&g, s);
     }
     if (rc == NZHIP_OK) {
         hipLaunchKernelGGL(col_t_gather_kernel, dim3((unsigned)((C * H * W + 255) / 256), (unsigned)N), dim3(256), 0, s, dx, colT, (int)Ho,
@@ -3397,7 +3397,7 @@ static int conv_dx_chain_rows(float* dx, const float* dy, const float* w_ref, si
             g.M = (int64_t)(N * P); g.batch_n = 1;
         }
         g.activation = NZHIP_ACT_NONE;
-        rc = nzhip_gemm(&g, s);
+        rc = gemm_of_columns(&g, s);
     }
     if (rc == NZHIP_OK && !accumulate) rc = nzhip_fill(dx, 0.f, N * C * H * W, stream);
     if (rc == NZHIP_OK) rc = nzhip_im2col_backward(dx, dcol, Ho, Wo, C, K_h, K_w, stride, pad, H, W, N, stream);
@@ -3456,7 +3456,7 @@ extern "C" int nzhip_conv2d_backward_data(float* dx, const float* dy, const floa
         if (accumulate) {
             g.bias = dx; g.bias_stride_n = g.c_stride_n; g.bias_stride_row = g.ldc; g.bias_stride_col = 1;
         }
-        return nzhip_gemm(&g, s);
+        return gemm_of_columns(&g, s);
     }
     if (stride == 1 && !conv_direct_applicable(O, C, K_h, K_w, 1, K_h - 1 - pad) &&
         conv_cl_wanted(CL_DATA, dy, N, C, H, W, O, K_h, K_w, stride, pad, w_batch)) {
@@ -3749,12 +3749,12 @@ static int conv1x1_backward_weights(float* dw, const float* x, const float* dy, 
     if (!shared || N == 1) {
         g.C = dw;
         g.bias = dw; g.bias_stride_n = (int64_t)(C * O); g.bias_stride_row = (int64_t)O; g.bias_stride_col = 1;
-        return nzhip_gemm(&g, s);
+        return gemm_of_columns(&g, s);
     }
     float* P = nullptr;
     if (int rc = workspace_alloc(reinterpret_cast<void**>(&P), N * C * O * sizeof(float), s)) return rc;
     g.C = P;
-    int rc = nzhip_gemm(&g, s);
+    int rc = gemm_of_columns(&g, s);
     if (rc == NZHIP_OK) {
         const long n = (long)(C * O);
         hipLaunchKernelGGL(dw_add_members_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, dw, P, (int)N, n);
@@ -4238,7 +4238,7 @@ extern "C" int nzhip_conv2d_backward_weights(float* dw, const float* x, const fl
                 g.bias = dw; g.bias_stride_row = (int64_t)O; g.bias_stride_col = 1;                    // dw += ...
                 g.batch_n = 1; g.batch_c = 1;
                 g.activation = NZHIP_ACT_NONE;
-                rc = nzhip_gemm(&g, s);
+                rc = gemm_of_columns(&g, s);
             }
             const int rc2 = workspace_free(dyt, s), rc3 = workspace_free(col, s);
             return rc ? rc : (rc2 ? rc2 : rc3);

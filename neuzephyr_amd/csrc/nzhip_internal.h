@@ -43,6 +43,13 @@ int gemm_h16_coop_timeouts(unsigned* count);     // polls that gave up since the
 // one_sum: every element is one sum over all of k, bit for bit the two-pass kernel's result (a caller that keeps B's image gets that kernel)
 bool gemm_copy_wanted(const nzhip_gemm_desc* d, int count, double other_us, bool one_sum = false);
 int gemm_copy_run(const nzhip_gemm_desc* d, int count, hipStream_t stream, bool one_sum = false);
+// Products of few tiles in one launch, the contraction cut between the waves of a workgroup (nzhip_gemm_slices.hip)
+// the shape to run a product with, -1: not with these; its estimated time
+int gemm_slices_plan(const nzhip_gemm_desc& d);
+double gemm_slices_cost(const nzhip_gemm_desc& d, int shape);
+int gemm_slices_run(const nzhip_gemm_desc& d, int shape, hipStream_t stream);
+// A convolution's product on its column matrix: nzhip_gemm without those. The lines between the convolution kernels were drawn against it.
+int gemm_of_columns(const nzhip_gemm_desc* desc, hipStream_t stream);
 // Bandwidth-bound kernels for M <= 8 (nzhip_skinny.hip).
 int gemm_skinny_dispatch(const nzhip_gemm_desc& d, hipStream_t stream);
 bool gemm_skinny_applicable(const nzhip_gemm_desc& d);

@@ -421,7 +421,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_wide_kernel(nzhip_gemm_desc
 
 using namespace nzhip;
 
-static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s);
+static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s, bool slices = true);
 
 extern "C" {
 
@@ -434,11 +434,18 @@ int nzhip_gemm(const nzhip_gemm_desc* desc, void* stream) {
 
 }  // extern "C"
 
+int nzhip::gemm_of_columns(const nzhip_gemm_desc* desc, hipStream_t s) {
+    if (int rc = validate_gemm(*desc)) return rc;
+    return desc->M == 0 || desc->N == 0 ? NZHIP_OK : gemm_routed(*desc, s, false);
+}
+
 // Estimated time in us of a product with its result's old value added, on its own; 0 for those that stream an operand. The single kernel and the two-pass
 // kernel as measured on the two gradients of layers of 2304 to 8192 rows, columns and k (both 4096^3 304 us, 305 here, both 8192^3 1951 and 2006, both
 // 6000^3 1051 and 1035): a launch, the result's read and write where it does not hide, half as fast in single elements, and the products' rate.
 static double gemm_single_cost(const nzhip_gemm_desc& d) {
-    if (gemm_thin_applicable(d) || gemm_skinny_applicable(d)) return 0.0;
+    if (gemm_thin_applicable(d)) return 0.0;
+    if (const int shape = gemm_slices_plan(d); shape >= 0) return gemm_slices_cost(d, shape);
+    if (gemm_skinny_applicable(d)) return 0.0;
     const double flops = 2.0 * d.M * d.N * d.K;
     if (gemm_h16_coop_applicable(d)) return 30.0 + flops / 1.13e9;
     if (gemm_h16_applicable(d)) return 28.0 + 8.0 * d.M * d.N / (((d.N | d.ldc) & 3) != 0 ? 3.0e6 : 5.9e6) + flops / 0.98e9;
@@ -446,13 +453,19 @@ static double gemm_single_cost(const nzhip_gemm_desc& d) {
 }
 
 // The route choice behind nzhip_gemm, for a validated descriptor with M, N > 0.
-static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s) {
+static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s, bool slices) {
     if (d.K == 0) {
         dim3 grid((unsigned)((d.M * d.N + 255) / 256), (unsigned)(d.batch_n * d.batch_c));
         hipLaunchKernelGGL(fill_bias_act_kernel, grid, dim3(256), 0, s, d);
         return check_launch("fill_bias_act_kernel");
     }
     if (gemm_thin_applicable(d)) return gemm_thin_dispatch(d, s);
+    if (const int shape = slices ? gemm_slices_plan(d) : -1; shape >= 0) {
+        if (gemm_trace())
+            fprintf(stderr, "nzhip_gemm %ld x %ld x %ld batch %ld x %ld: sliced kernel, shape %d, 1 chunk(s) of %ld, model %.1f us\n", (long)d.M, (long)d.K,
+                    (long)d.N, (long)d.batch_n, (long)d.batch_c, shape, (long)d.K, gemm_slices_cost(d, shape));
+        return gemm_slices_run(d, shape, s);
+    }
     if (gemm_skinny_applicable(d)) return gemm_skinny_dispatch(d, s);
     // Products that leave CUs idle with 128 x 128 tiles (weight gradients with K = batch x pixels, mid-size
     // products): smaller tiles, or the contraction cut into chunks that run as a batch into a workspace and are

@@ -1,0 +1,106 @@
+"""The kernel for products of few tiles (nzhip_gemm_slices.hip) at the edges of its tiles, chunks and rules: exact on integers, nothing read or
+written outside the operands' rows, errors no larger than those of the kernels that take the same products otherwise. The library reads
+NZHIP_GEMM_SLICES per call: 0 never, 1 to 3 one of its workgroup shapes."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def nz():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from neuzephyr_amd import capi
+    capi.load()
+    return capi
+
+
+# M, K, N: one row and column; the tiles' edges; chunks of 32 k cut anywhere; fewer chunks than waves, and more
+SIZES = [(1, 4, 1), (1, 33, 70), (33, 5, 2), (31, 31, 33), (32, 32, 32), (64, 64, 65), (65, 127, 63), (70, 130, 2), (3, 259, 129), (128, 1029, 96)]
+
+
+@pytest.mark.parametrize("shape", [1, 2, 3])
+@pytest.mark.parametrize("a_trans", [False, True])
+@pytest.mark.parametrize("b_trans", [False, True])
+@pytest.mark.parametrize("size", SIZES)
+def test_exact_on_integers_inside_larger_buffers(nz, monkeypatch, size, a_trans, b_trans, shape):
+    """Rows of odd length and offset inside buffers of NaN: what lies between the rows or past them must enter no sum."""
+    import torch
+    monkeypatch.setenv("NZHIP_GEMM_SLICES", str(shape))
+    M, K, N = size
+    rng = np.random.default_rng(M * 31 + K * 7 + N)
+    A, B, bias = (rng.integers(-3, 4, s).astype(np.float32) for s in ((M, K), (K, N), (M, N)))
+    want = (A.astype(np.int64) @ B.astype(np.int64)).astype(np.float32)
+
+    def embed(x, slack, offset):
+        rows, cols = x.shape
+        buf = torch.full((offset + rows * (cols + slack) + 3,), float("nan"), device="cuda")
+        view = buf[offset:offset + rows * (cols + slack)].view(rows, cols + slack)[:, :cols]
+        view.copy_(torch.from_numpy(np.ascontiguousarray(x)))
+        return buf, view
+
+    import ctypes as C
+    keep = [embed(A.T if a_trans else A, 1, 1), embed(B.T if b_trans else B, 2, 3), embed(np.full((M, N), 9, np.float32), 3, 2), embed(bias, 0, 1)]
+    (_, a), (_, b), (cbuf, c), (_, bv) = keep
+    for form in ("none", "bias, ReLU", "column bias", "added to"):
+        cbuf.fill_(float("nan"))
+        c.fill_(4.0)
+        d = nz.GemmDesc(A=a.data_ptr(), B=b.data_ptr(), C=c.data_ptr(), M=M, N=N, K=K, lda=a.stride(0), ldb=b.stride(0), ldc=c.stride(0),
+                        a_layout=int(a_trans), b_layout=int(b_trans), batch_n=1, batch_c=1)
+        expect = want
+        if form == "bias, ReLU":
+            d.bias, d.bias_stride_row, d.bias_stride_col, d.activation = bv.data_ptr(), bv.stride(0), 1, 1
+            expect = np.maximum(want + bias, 0)
+        elif form == "column bias":
+            d.bias, d.bias_stride_row, d.bias_stride_col = bv.data_ptr(), 0, 1
+            expect = want + bias[:1]
+        elif form == "added to":
+            d.bias, d.bias_stride_row, d.bias_stride_col = c.data_ptr(), c.stride(0), 1
+            expect = want + 4
+        nz.check(nz.load().nzhip_gemm(C.byref(d), torch.cuda.current_stream().cuda_stream))
+        assert np.array_equal(c.cpu().numpy(), expect), form
+        c.fill_(float("nan"))
+        assert bool(torch.isnan(cbuf).all()), form
+
+
+@pytest.mark.parametrize("shape", [1, 2, 3])
+@pytest.mark.parametrize("sa,sb", [((3, 2, 40, 70), (3, 2, 70, 50)), ((1, 4, 33, 36), (5, 1, 36, 65)), ((4, 1, 64, 64), (1, 1, 64, 32))])
+def test_batches_with_broadcasts(nz, monkeypatch, sa, sb, shape):
+    import torch
+    monkeypatch.setenv("NZHIP_GEMM_SLICES", str(shape))
+    rng = np.random.default_rng(3)
+    A, B = (rng.integers(-3, 4, s).astype(np.float32) for s in (sa, sb))
+    got = nz.tensorcore_gemm(torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda())
+    assert np.array_equal(got.cpu().numpy(), np.matmul(A, B))
+
+
+def test_infinities_and_nans_stay_in_their_rows_and_columns(nz, monkeypatch):
+    """K = 45: the last chunk is filled up with zeros, which must meet no infinity."""
+    import torch
+    A, B = torch.ones(40, 45, device="cuda"), torch.ones(45, 70, device="cuda")
+    A[7, 44], B[44, 11], B[0, 69] = float("inf"), float("nan"), 7e4                      # 7e4 is beyond fp16
+    for shape in (1, 2, 3):
+        for a_trans in (False, True):
+            for b_trans in (False, True):
+                monkeypatch.setenv("NZHIP_GEMM_SLICES", str(shape))
+                got = nz.gemm(A.T.contiguous() if a_trans else A, B.T.contiguous() if b_trans else B, a_trans=a_trans, b_trans=b_trans)
+                want = A.half().float().cpu() @ B.half().float().cpu()
+                assert torch.equal(got.cpu().nan_to_num(nan=-1.0), want.nan_to_num(nan=-1.0)), (shape, a_trans, b_trans)
+
+
+# one-tile and many-tile products, long and short sums, each with the shape that the rule picks
+@pytest.mark.parametrize("M,K,N", [(64, 64, 64), (256, 256, 256), (300, 300, 300), (100, 1000, 200), (48, 1943, 112), (16, 1520, 18), (1, 416, 3072), (700, 300, 900), (1024, 1024, 1024)])
+@pytest.mark.parametrize("b_trans", [False, True])
+def test_sums_are_as_exact_as_those_of_the_other_kernels(nz, monkeypatch, M, K, N, b_trans):
+    """Error in the 2-norm against float64 on operands that fp16 holds exactly."""
+    import torch
+    g = torch.Generator().manual_seed(M + K + N)
+    A, B = torch.randn(M, K, generator=g).half().float().cuda(), torch.randn(*((N, K) if b_trans else (K, N)), generator=g).half().float().cuda()
+    want = A.double() @ (B.T if b_trans else B).double()
+    err = {}
+    for route in ("0", None):
+        monkeypatch.setenv("NZHIP_GEMM_SLICES", route) if route else monkeypatch.delenv("NZHIP_GEMM_SLICES")
+        err[route] = float((nz.gemm(A, B, b_trans=b_trans).double() - want).norm() / want.norm())
+    assert err[None] <= 1.05 * err["0"], err                        # (the 2-norm of a few thousand elements moves by a few hundredths with their order)
