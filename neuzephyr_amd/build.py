@@ -10,7 +10,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libnzhip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["nzhip_gemm.hip", "nzhip_gemm_h16.hip", "nzhip_gemm_copy.hip", "nzhip_gemm_slices.hip", "nzhip_skinny.hip", "nzhip_conv.hip", "nzhip_conv_cl.hip", "nzhip_ops.hip", "nzhip_fp32.hip",
+SOURCES = ["nzhip_gemm.hip", "nzhip_gemm_h16.hip", "nzhip_gemm_copy.hip", "nzhip_gemm_slices.hip", "nzhip_skinny.hip", "nzhip_conv.hip", "nzhip_conv_cl.hip", "nzhip_conv_slices.hip", "nzhip_ops.hip", "nzhip_fp32.hip",
            "nzhip_nn.hip", "nzhip_probe.hip",
            "nzhip_runtime.cpp"]
 FLAGS = [

@@ -14,11 +14,10 @@
 #include "nzhip_internal.h"
 #include "nzhip_lds_tiles.h"
 #include "nzhip_pieces.h"
+#include "nzhip_slices.h"
 
 namespace nzhip {
 
-typedef unsigned uint2_t __attribute__((ext_vector_type(2)));
-typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
 typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
 
 struct SliceArgs {
@@ -37,13 +36,13 @@ struct SliceArgs {
 // KC: k runs along its rows in memory; 8 lanes take the 128 bytes of a row, 16 each, and the fragments are formed through LDS.
 template <bool KC, int F>
 struct Slice {
-    static constexpr int PITCH = 80;                                // bytes of an LDS row: 32 halfs, padded
+    static constexpr int PITCH = SLICE_PITCH;
     static constexpr int LDS = F * 32 * PITCH;
     uint4_t v[F * 4];
     unsigned off[F * 4];
     __amdgpu_buffer_rsrc_t from;
     __device__ __forceinline__ void start(const float* x, int ld, int row0, int rows, int K, int lane) {
-        from = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), 0, (unsigned)((rows - 1) * ld + K) * 4u, CL_RSRC);
+        from = slice_buffer(x, (unsigned)((rows - 1) * ld + K) * 4u);
 #pragma unroll
         for (int p = 0; p < F * 4; p++) {
             const int r = row0 + p * 8 + (lane >> 3);
@@ -96,7 +95,7 @@ struct Slice<false, F> {
     bool moved;
     __amdgpu_buffer_rsrc_t from;
     __device__ __forceinline__ void start(const float* x, int ld_, int row0, int rows, int K, int lane) {
-        from = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(x), 0, (unsigned)((K - 1) * ld_ + rows) * 4u, CL_RSRC);
+        from = slice_buffer(x, (unsigned)((K - 1) * ld_ + rows) * 4u);
         ld = (unsigned)ld_ * 4u;
         const int r = row0 + (lane & 31) * F, at = F > 1 && r + F > rows ? rows - F : r < rows ? r : rows - 1;       // a pair that the end cuts starts at the last two
         off = (unsigned)at * 4u + (unsigned)(lane >> 5) * 8u * ld;
@@ -141,7 +140,7 @@ template <int FM, int FN, bool A_KC, bool B_KC, int NW>
 __global__ __launch_bounds__(NW * 64, FM * FN == 4 ? 2 : 4) void gemm_slices_kernel(const SliceArgs p) {
     using SA = Slice<A_KC, FM>;
     using SB = Slice<B_KC, FN>;
-    constexpr int BM = FM * 32, BN = FN * 32, STAGE = SA::LDS + SB::LDS, UNITS = FM * FN * 4;
+    constexpr int BM = FM * 32, BN = FN * 32, STAGE = SA::LDS + SB::LDS;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 31, lh = lane >> 5;
 
@@ -185,9 +184,7 @@ __global__ __launch_bounds__(NW * 64, FM * FN == 4 ? 2 : 4) void gemm_slices_ker
             sa.load(k1, p.K, lane);
             sb.load(k1, p.K, lane);
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        slice_wave_sync();
         sa.read(a, own_a, lane);
         sb.read(b, own_b, lane);
         if (FM * FN == 1 && (odd ^= 1)) {
@@ -203,9 +200,7 @@ __global__ __launch_bounds__(NW * 64, FM * FN == 4 ? 2 : 4) void gemm_slices_ker
             for (int i = 0; i < FM; i++)
 #pragma unroll
                 for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[s][i], b[s][j], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        slice_wave_sync();
     }
 
     if constexpr (FM * FN == 1)
@@ -216,15 +211,7 @@ __global__ __launch_bounds__(NW * 64, FM * FN == 4 ? 2 : 4) void gemm_slices_ker
     const int active = chunks < NW ? chunks : NW;
     piece4* park = reinterpret_cast<piece4*>(lds);
     if (STAGE) __syncthreads();
-    if (wave < active) {
-#pragma unroll
-        for (int i = 0; i < FM; i++)
-#pragma unroll
-            for (int j = 0; j < FN; j++)
-#pragma unroll
-                for (int g = 0; g < 4; g++)
-                    park[(wave * UNITS + (i * 4 + g) * FN + j) * 64 + lane] = piece4{acc[i][j][g * 4], acc[i][j][g * 4 + 1], acc[i][j][g * 4 + 2], acc[i][j][g * 4 + 3]};
-    }
+    if (wave < active) slice_park(park, acc, wave, lane);
     __syncthreads();
     float* C = p.C + bi * p.c_sn + bj * p.c_sc;
     const float* bias = p.bias ? p.bias + bi * p.bias_sn + bj * p.bias_sc : nullptr;
@@ -234,22 +221,7 @@ __global__ __launch_bounds__(NW * 64, FM * FN == 4 ? 2 : 4) void gemm_slices_ker
         if (ig >= FM * 4) break;
         piece4 s[FN];
 #pragma unroll
-        for (int j = 0; j < FN; j++) {
-            piece4 o[NW];                                           // all requested before the first is added
-#pragma unroll
-            for (int w = 0; w < NW; w++) o[w] = park[((w < active ? w : 0) * UNITS + ig * FN + j) * 64 + lane];
-#pragma unroll
-            for (int w = 1; w < NW; w++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) o[w][e] = w < active ? o[w][e] : 0.f;
-#pragma unroll
-            for (int h = NW / 2; h > 0; h /= 2)
-#pragma unroll
-                for (int w = 0; w < h; w++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) o[w][e] += o[w + h][e];
-            s[j] = o[0];
-        }
+        for (int j = 0; j < FN; j++) s[j] = slice_collect<FM, FN, NW>(park, ig, j, active, lane);
         float bv[4][FN];
 #pragma unroll
         for (int e = 0; e < 4; e++)
