@@ -110,21 +110,22 @@ __device__ __forceinline__ void copy_tile(const CopyProduct& p, const int lin, c
 
     char* ring = lds + kg * NST * STAGE;
     const unsigned at_a = cl_lds(ring) + wave * (A_KC ? LA : Q) * 1024, at_b = cl_lds(ring) + BM * 128 + wave * (B_KC ? LB : Q) * 1024;
-    auto request = [&](int slot) {
-        const bool even = at + ch < units, odd = at + (ch ^ 4) < units, any = at < units;
-#pragma unroll
-        for (int j = 0; j < LA; j++) {
+    auto request_one = [&](int slot, int j) {                       // the step's j-th request
+        if (j < LA) {
             const unsigned to = at_a + slot * STAGE + (A_KC ? j * 1024 : (j / Q) * 8192 + (j % Q) * 1024);
-            cl_load(ra, to, (A_KC ? (j & 1 ? odd : even) : any) ? off_a[j] : CL_OUT);
+            cl_load(ra, to, at + (A_KC ? ch ^ ((j & 1) * 4) : 0) < units ? off_a[j] : CL_OUT);
             off_a[j] += add_a;
+        } else {
+            const int i = j - LA;
+            const unsigned to = at_b + slot * STAGE + (B_KC ? i * 1024 : (i / Q) * 8192 + (i % Q) * 1024);
+            cl_load(rb, to, at + (B_KC ? ch ^ ((i & 1) * 4) : 0) < units ? off_b[i] : CL_OUT);
+            off_b[i] += add_b;
         }
+        if (j == LOADS - 1) at += 8 * KG;
+    };
+    auto request = [&](int slot) {
 #pragma unroll
-        for (int j = 0; j < LB; j++) {
-            const unsigned to = at_b + slot * STAGE + (B_KC ? j * 1024 : (j / Q) * 8192 + (j % Q) * 1024);
-            cl_load(rb, to, (B_KC ? (j & 1 ? odd : even) : any) ? off_b[j] : CL_OUT);
-            off_b[j] += add_b;
-        }
-        at += 8 * KG;
+        for (int j = 0; j < LOADS; j++) request_one(slot, j);
     };
 
     floatx16 acc[TM][TN];
@@ -152,14 +153,8 @@ __device__ __forceinline__ void copy_tile(const CopyProduct& p, const int lin, c
     };
 
     ClSums<TM, TN> sums;
-    for (int s = 0; s < NST - 1; s++) request(s);
-    int slot = 0;
-    for (int s = 0; s < steps; s++) {
-        cl_wait_vmcnt<(NST - 2) * LOADS>();
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        request(slot == 0 ? NST - 1 : slot - 1);
-        const char* base = ring + slot * STAGE;
-        half8_t af[4][TM], bf[4][TN];
+    half8_t af[4][TM], bf[4][TN];
+    auto fragments = [&](const char* base) {
 #pragma unroll
         for (int k = 0; k < 4; k++) {
 #pragma unroll
@@ -168,16 +163,68 @@ __device__ __forceinline__ void copy_tile(const CopyProduct& p, const int lin, c
             for (int j = 0; j < TN; j++) bf[k][j] = read(base + BM * 128, B_KC, wn * TN + j, k);
             __builtin_amdgcn_sched_barrier(0);                      // in the order of their use
         }
-        sums.take(acc, s, p.chain);
-        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](int k) {
 #pragma unroll
-        for (int k = 0; k < 4; k++)
+        for (int i = 0; i < TM; i++)
 #pragma unroll
-            for (int i = 0; i < TM; i++)
+            for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[k][i], bf[k][j], acc[i][j], 0, 0, 0);
+    };
+    for (int s = 0; s < NST - 1; s++) request(s);
+    int slot = 0;
+    // 128 x 256: the waves of rows 0..63 and those of rows 64..127, one of each per SIMD, take turns: one half reads a step's fragments from LDS
+    // while the other's MFMAs run and issue its requests, a barrier between the turns. All in step, the three added up (2560 clocks a
+    // step of the pair below, of which the MFMAs are 1024, the reads about 900 and the issue of the requests 770): pairs of 4096 x 1024 -> 4096 116
+    // -> 110 us, 4096 x 4096 -> 1024 130 -> 124, 2048^3 on this tile 45 -> 42. Left over is that either half alone takes 67 of the 87 us: with
+    // the MFMAs out, with the requests out of bounds. Smaller tiles lose by the second barrier (2048^3 on 128 x 128 35.1 -> 36.6).
+    // Half h of a step's two: the first half of the waves reads step s in half 2 s, the second in 2 s + 1, and each waits for its share of step s + 1
+    // before the barrier that ends half 2 s + 1. A slot is free when the later half has read it: the first half fills the slot
+    // of step s - 1 in half 2 s + 1, the second that of step s in half 2 s + 2, one step further ahead.
+    if constexpr (TM == 2 && TN == 2) {
+        static_assert(KG == 1 && T::WN == 4, "the halves are the waves of the tile's upper and lower rows, on the same SIMDs");
+        const bool late = __builtin_amdgcn_readfirstlane(tid) >= T::THREADS / 2;
+        cl_wait_vmcnt<(NST - 2) * LOADS>();
+        if (late) {
+            request(NST - 1);
+            asm volatile("s_barrier" ::: "memory");
+        }
+        asm volatile("s_barrier" ::: "memory");
+        for (int s = 0; s < steps; s++) {
+            const int to = late ? slot : slot == 0 ? NST - 1 : slot - 1;
+            fragments(ring + slot * STAGE);
+            sums.take(acc, s, p.chain);
+            __builtin_amdgcn_sched_barrier(0);
+            if (late) cl_wait_vmcnt<(NST - 2) * LOADS>();
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-                for (int j = 0; j < TN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[k][i], bf[k][j], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        slot = slot == NST - 1 ? 0 : slot + 1;
+            for (int k = 0; k < 4; k++) {
+                multiply(k);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = k * LOADS / 4; j < (k + 1) * LOADS / 4; j++) request_one(to, j);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_s_setprio(0);
+            if (!late) cl_wait_vmcnt<(NST - 2) * LOADS>();
+            asm volatile("s_barrier" ::: "memory");
+            slot = slot == NST - 1 ? 0 : slot + 1;
+        }
+        if (!late) asm volatile("s_barrier" ::: "memory");
+    } else {
+        for (int s = 0; s < steps; s++) {
+            cl_wait_vmcnt<(NST - 2) * LOADS>();
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            request(slot == 0 ? NST - 1 : slot - 1);
+            fragments(ring + slot * STAGE);
+            sums.take(acc, s, p.chain);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < 4; k++) multiply(k);
+            __builtin_amdgcn_sched_barrier(0);
+            slot = slot == NST - 1 ? 0 : slot + 1;
+        }
     }
     sums.finish(acc);
     cl_wait_vmcnt<0>();

@@ -81,6 +81,22 @@ def test_a_long_contraction_is_summed_in_chains_of_512(nz, monkeypatch, tile, K)
     assert np.linalg.norm(err) <= np.linalg.norm(want) * 2.0 ** -24 * np.sqrt((512 + K / 512) / 6)
 
 
+@pytest.mark.parametrize("K", [1, 64, 65, 128, 129, 192, 257, 1000])
+def test_waves_that_take_turns_are_bit_exact_on_whole_numbers(nz, monkeypatch, K):
+    """128 x 256 tiles, 100 of them side by side, of one to 16 steps: fewer than the ring's three, as many, one more, many."""
+    import torch
+    monkeypatch.setenv("NZHIP_GEMM_COPY", "1")
+    monkeypatch.setenv("NZHIP_GEMM_COPY_PLAN", "5,1")
+    rng = np.random.default_rng(K)
+    A, B = whole(rng, 1270, K), whole(rng, K, 2500)
+    want = A @ B                                                       # whole numbers below 2^24: exact in fp32
+    a, b = torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda()
+    for a_trans in (False, True):
+        for b_trans in (False, True):
+            aa, bb = a.T.contiguous() if a_trans else a, b.T.contiguous() if b_trans else b
+            assert np.array_equal(nz.gemm(aa, bb, a_trans=a_trans, b_trans=b_trans).cpu().numpy(), want), (a_trans, b_trans)
+
+
 @pytest.mark.parametrize("S,inputs,outputs", [(29, 466, 640), (64, 848, 786), (48, 880, 1984), (16, 792, 2752)])
 def test_gradients_of_few_samples_are_as_exact_as_one_product_after_the_other(nz, monkeypatch, S, inputs, outputs):
     """Error in the 2-norm against float64 on operands that fp16 holds exactly: only the order of the fp32 sums counts."""
