@@ -161,10 +161,11 @@ struct ClArgs {
     int images;                         // images in one launch row: N, or 1 with a weight copy per image
     long plane, y_total;                // output plane; elements of y
     long bias_sp, bias_sc, bias_sn;
-    int relu, parts, part_units, tiles_m, tiles, n_classes;      // tiles: of all classes, as if each had as many as the largest
+    int relu, parts, part_units, tiles_m, tiles, n_classes;      // tiles: of all classes or pairs, as if each had as many as the largest
+    int paired;                         // classes 2 i and 2 i + 1 are the even and the odd columns of the same rows, and one workgroup's
     int dy_h, dy_w;                     // dy's extents; 0 in a forward
     int units;                          // of the longest sum (host)
-    ClDiv by_cu, by_tiles_m, by_classes;
+    ClDiv by_cu, by_tiles_m, by_groups;     // groups: the classes, or the pairs of them
     ClClass cls[CL_MAX_CLASSES];
 };
 
@@ -192,8 +193,9 @@ __device__ __forceinline__ float cl_terms(const ClArgs& p, const ClClass& c, con
 // LDS rows are 128 bytes, 8 units; unit u of row r lies at u ^ (r >> 1 & 7), which puts the 16 rows that share a pass of a
 // 128-bit read on 16 bank groups. The lane that loads a slot asks for the unit that belongs there, so a lane needs the
 // offsets of two units per step (rows of even and odd groups of 8), from a table in LDS, one step ahead.
-// DATA: a data gradient. MANY: more than one class.
-template <typename T, bool DATA, bool MANY>
+// DATA: a data gradient. MANY: more than one class. PAIRED: a workgroup has the even columns of its rows and then the odd ones: one run of k steps, two
+// sums, stores of two neighbours.
+template <typename T, bool DATA, bool MANY, bool PAIRED>
 __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) {
     constexpr int TM = T::TM, TN = T::TN, KG = T::KG, BM = T::BM, BN = T::BN, NST = T::NST, STAGE = T::STAGE, LA = T::LA, LB = T::LB, LOADS = LA + LB;
     extern __shared__ __attribute__((aligned(1024))) char lds[];
@@ -208,11 +210,14 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
     // 31.4 -> 23.5, against one class after the other). Every second run of eight is reversed: a CU gets each 32nd workgroup of
     // its XCD, and would get only long sums or only short ones (45.3 -> 42.8, 21.0 -> 19.3 on 16 x 256 x 28 x 28 <- 256).
     if (MANY) {
-        in_class = cl_quot(lin, p.by_classes);
-        ci = lin - in_class * p.n_classes;
-        if (in_class & 8) ci = p.n_classes - 1 - ci;
+        const int groups = PAIRED ? p.n_classes / 2 : p.n_classes;
+        in_class = cl_quot(lin, p.by_groups);
+        ci = lin - in_class * groups;
+        if (in_class & 8) ci = groups - 1 - ci;
+        if (PAIRED) ci *= 2;
     }
     const ClClass& c = p.cls[MANY ? ci : 0];
+    const ClClass& odd = p.cls[PAIRED ? ci + 1 : 0];                // as many rows, as many columns or one less: that one's sums are not stored
     const int tile_n = cl_quot(in_class, p.by_tiles_m), tile_m = in_class - tile_n * p.tiles_m;
     const int m0 = tile_m * BM, n0 = tile_n * BN;
     const int z = blockIdx.z;
@@ -220,15 +225,23 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
     if (MANY && n0 >= pixels) return;                               // a class of fewer tiles than the largest
 
     // units of this part, a whole number of steps per group; the table of their offsets in the two copies, in bytes
-    const int units = c.nr * c.ns * p.cu, u_first = blockIdx.y * p.part_units;
-    const int n_units = u_first + p.part_units < units ? p.part_units : units - u_first;                 // 0 or less: an empty sum
-    const int steps = n_units > 0 ? ((n_units + 7) / 8 + KG - 1) / KG : 0;
+    const int u_first = blockIdx.y * p.part_units;
+    auto part_of = [&](const ClClass& d) {                          // 0 or less: an empty sum
+        const int units = d.nr * d.ns * p.cu;
+        return u_first + p.part_units < units ? p.part_units : units - u_first;
+    };
+    const int n_units = part_of(c), n_odd = PAIRED ? part_of(odd) : 0;
+    const int steps = n_units > 0 ? ((n_units + 7) / 8 + KG - 1) / KG : 0, steps_odd = n_odd > 0 ? ((n_odd + 7) / 8 + KG - 1) / KG : 0;
     int2* tab = reinterpret_cast<int2*>(lds + KG * NST * STAGE);
-    for (int v = tid; v < (steps + NST) * KG * 8; v += T::THREADS) {
-        const int u = u_first + v, t = cl_quot(u, p.by_cu), i = cl_quot(t, c.by_ns), j = t - i * c.ns, e = (u - t * p.cu) * 8;
-        const bool in = v < n_units;
-        tab[v] = int2{in ? (((c.r0 + i * c.rs) * p.Kw + c.s0 + j * c.ss) * p.cu * 8 + e) * 2 : (int)CL_OUT,
-                      in ? (i * c.di + j * c.dj + e) * 2 : (int)CL_OUT};
+    auto unit_at = [&](int v, const ClClass& d, int n, int shift) {
+        const int u = u_first + v, t = cl_quot(u, p.by_cu), i = cl_quot(t, d.by_ns), j = t - i * d.ns, e = (u - t * p.cu) * 8;
+        const bool in = v < n;
+        return int2{in ? (((d.r0 + i * d.rs) * p.Kw + d.s0 + j * d.ss) * p.cu * 8 + e) * 2 : (int)CL_OUT,
+                    in ? (i * d.di + j * d.dj + e + shift) * 2 : (int)CL_OUT};
+    };
+    for (int v = tid; v < (steps + steps_odd + NST) * KG * 8; v += T::THREADS) {
+        const int past = v - steps * KG * 8;
+        tab[v] = PAIRED && past >= 0 ? unit_at(past, odd, n_odd, odd.base - c.base) : unit_at(v, c, n_units, 0);
     }
 
     const int4_t rw = cl_buffer(p.w + z * p.w_img, p.w_bytes), rx = cl_buffer(p.x + z * p.x_img, p.x_bytes);
@@ -274,8 +287,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
     // One step: every fragment is requested before the first MFMA (a read takes 100 clocks and more to come back, an MFMA 32), then
     // the offsets of the next request.
     ClSums<TM, TN> sums;
-    const int chain = cl_chain(steps);
-    auto multiply = [&](const char* base, int t, int ahead) {
+    auto multiply = [&](const char* base, int t, int chain, int ahead) {
         half8_t af[4][TM], bf[4][TN];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -298,7 +310,8 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    if (steps > 0) {
+    floatx16 even[PAIRED ? TM : 1][PAIRED ? TN : 1];                 // sums of the even columns
+    if (steps + steps_odd > 0) {
         __syncthreads();                                            // the table
         // Units past the end are offsets outside both buffers: zeros, in the last step and in requests nobody reads, so the
         // number in flight is the same in every step and no step is special.
@@ -308,26 +321,52 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
         }
         look_up(NST - 1);
         int slot = 0;
-        for (int t = 0; t < steps; t++) {
-            cl_wait_vmcnt<(NST - 2) * LOADS>();                     // this wave's share of step t has landed
-            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // everybody's has, and step t - 1 is read by all
-            request(slot == 0 ? NST - 1 : slot - 1);
-            multiply(ring + slot * STAGE, t, t + NST);
-            slot = slot == NST - 1 ? 0 : slot + 1;
+        auto run = [&](int from, int n) {
+            const int chain = cl_chain(n);
+            for (int t = 0; t < n; t++) {
+                cl_wait_vmcnt<(NST - 2) * LOADS>();                 // this wave's share of the step has landed
+                asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");   // everybody's has, and the step before is read by all
+                request(slot == 0 ? NST - 1 : slot - 1);
+                multiply(ring + slot * STAGE, t, chain, from + t + NST);
+                slot = slot == NST - 1 ? 0 : slot + 1;
+            }
+            sums.finish(acc);
+        };
+        run(0, steps);
+        if constexpr (PAIRED) {
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        even[i][j][r] = acc[i][j][r];
+                        acc[i][j][r] = sums.sum[i][j][r] = 0.f;
+                    }
+            run(steps, steps_odd);
         }
-        sums.finish(acc);
         cl_wait_vmcnt<0>();
+    } else if constexpr (PAIRED) {
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) even[i][j][r] = 0.f;
     }
 
     if constexpr (KG > 1) {
         static_assert(KG == 2, "two groups meet pairwise");
         __syncthreads();
-        floatx16* park = reinterpret_cast<floatx16*>(lds) + (wave * TM * TN) * 64 + lane;
+        floatx16* park = reinterpret_cast<floatx16*>(lds) + (wave * TM * TN * (PAIRED ? 2 : 1)) * 64 + lane;
         if (kg == 1) {
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
-                for (int j = 0; j < TN; j++) park[(i * TN + j) * 64] = acc[i][j];
+                for (int j = 0; j < TN; j++) {
+                    park[(i * TN + j) * 64] = acc[i][j];
+                    if constexpr (PAIRED) park[(TM * TN + i * TN + j) * 64] = even[i][j];
+                }
         }
         __syncthreads();
         if (kg == 1) return;
@@ -338,6 +377,11 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
                 const floatx16 o = park[(i * TN + j) * 64];
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[i][j][r] += o[r];
+                if constexpr (PAIRED) {
+                    const floatx16 e = park[(TM * TN + i * TN + j) * 64];
+#pragma unroll
+                    for (int r = 0; r < 16; r++) even[i][j][r] += e[r];
+                }
             }
     }
 
@@ -346,27 +390,29 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
     // ---- epilogue: lane = pixel, registers = channels (r >> 2) * 8 + lh * 4 + (r & 3); bias first, then the stores
     unsigned out[TN];
     long bpix[TN];
-    bool live[TN];
+    bool live[TN], both[TN];                                        // both: the odd column's neighbour too
 #pragma unroll
     for (int j = 0; j < TN; j++) {
         const int px = n0 + (wn * TN + j) * 32 + li;
         live[j] = px < pixels;
         const int pc = live[j] ? px : pixels - 1, img = cl_quot(pc, c.by_hw), q = pc - img * hw, i = cl_quot(q, c.by_w), k = q - i * c.Wc;
         const int pl = c.out + i * c.out_h + k * c.out_w;
+        both[j] = PAIRED && live[j] && k < odd.Wc;
         out[j] = (unsigned)((z + img) * (int)p.y_img + pl);
         bpix[j] = (long)(z + img) * p.bias_sn + pl * p.bias_sp;
     }
     const bool split = p.parts > 1;
     float* y = split ? p.partial + blockIdx.y * p.y_total : p.y;
-    // AGAIN: NaNs of pixels with taps outside dy may come from an infinite weight times the zeros there, and are summed again
-    auto finish = [&](auto again_tag) {
+    // AGAIN: NaNs of pixels with taps outside dy may come from an infinite weight times the zeros there, and are summed again.
+    // d: the class whose sums acc are, `by` columns right of the pixel at out[j]
+    auto finish = [&](auto again_tag, const ClClass& d, floatx16 (&acc)[TM][TN], const bool (&live)[TN], const int by, const int n_units) {
         constexpr bool AGAIN = decltype(again_tag)::value;
         unsigned again[TM][TN];
         if (AGAIN)
 #pragma unroll
             for (int j = 0; j < TN; j++) {
-                const int px = n0 + (wn * TN + j) * 32 + li, q = px - cl_quot(px, c.by_hw) * hw, h = cl_quot(q, c.by_w), row = c.lo_h + h, col = c.lo_w + q - h * c.Wc;
-                const bool edge = live[j] && (row >= p.dy_h || row < c.nr - 1 || col >= p.dy_w || col < c.ns - 1);
+                const int px = n0 + (wn * TN + j) * 32 + li, q = px - cl_quot(px, c.by_hw) * hw, h = cl_quot(q, c.by_w), row = d.lo_h + h, col = d.lo_w + q - h * c.Wc;
+                const bool edge = live[j] && (row >= p.dy_h || row < d.nr - 1 || col >= p.dy_w || col < d.ns - 1);
 #pragma unroll
                 for (int i = 0; i < TM; i++) {
                     again[i][j] = 0;
@@ -384,12 +430,12 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
                     for (int g = 0; g < 4; g++) {
                         const int o = m0 + (wm * TM + i) * 32 + g * 8 + lh * 4;
                         if (quads && o + 4 <= p.M) {
-                            const piece4 v = *reinterpret_cast<const floatx4u*>(p.bias + bpix[j] + o);
+                            const piece4 v = *reinterpret_cast<const floatx4u*>(p.bias + bpix[j] + o);      // (by is 0)
 #pragma unroll
                             for (int e = 0; e < 4; e++) acc[i][j][g * 4 + e] += v[e];
                         } else {
 #pragma unroll
-                            for (int e = 0; e < 4; e++) acc[i][j][g * 4 + e] += p.bias[bpix[j] + (long)(o + e < p.M ? o + e : p.M - 1) * p.bias_sc];
+                            for (int e = 0; e < 4; e++) acc[i][j][g * 4 + e] += p.bias[bpix[j] + (live[j] ? by : 0) + (long)(o + e < p.M ? o + e : p.M - 1) * p.bias_sc];
                         }
                     }
         }
@@ -402,7 +448,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
                     const int o = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
                     float v = acc[i][j][r];
                     if (p.relu && !split) v = v > 0.f ? v : 0.f;
-                    if (live[j] && o < p.M && !(AGAIN && again[i][j] >> r & 1)) y[out[j] + (unsigned)o * (unsigned)p.plane] = v;
+                    if (live[j] && o < p.M && !(AGAIN && again[i][j] >> r & 1)) y[out[j] + by + (unsigned)o * (unsigned)p.plane] = v;
                 }
         if (AGAIN)
 #pragma unroll
@@ -414,9 +460,9 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
                         const int r = __builtin_ctz(left), o = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
                         if (o >= p.M) continue;
                         const int px = n0 + (wn * TN + j) * 32 + li, img = cl_quot(px, c.by_hw), q = px - img * hw, h = cl_quot(q, c.by_w);
-                        float v = cl_terms(p, c, z, img, h, q - h * c.Wc, o, u_first, n_units);
-                        if (p.bias && !split) v += p.bias[bpix[j] + o * p.bias_sc];
-                        y[out[j] + (unsigned)o * (unsigned)p.plane] = v;
+                        float v = cl_terms(p, d, z, img, h, q - h * c.Wc, o, u_first, n_units);
+                        if (p.bias && !split) v += p.bias[bpix[j] + by + o * p.bias_sc];
+                        y[out[j] + by + (unsigned)o * (unsigned)p.plane] = v;
                     }
     };
     if constexpr (DATA) {
@@ -426,10 +472,41 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
 #pragma unroll
             for (int j = 0; j < TN; j++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) all += acc[i][j][r];
-        if (__builtin_expect(__any(all != all), 0)) return finish(std::true_type{});
+                for (int r = 0; r < 16; r++) all += PAIRED ? acc[i][j][r] + even[i][j][r] : acc[i][j][r];
+        if (__builtin_expect(__any(all != all), 0)) {
+            if constexpr (PAIRED) {
+                finish(std::true_type{}, c, even, live, 0, n_units);
+                return finish(std::true_type{}, odd, acc, both, 1, n_odd);
+            } else return finish(std::true_type{}, c, acc, live, 0, n_units);
+        }
     }
-    finish(std::false_type{});
+    if constexpr (PAIRED) {
+        if (p.bias && !split) {
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const int o = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
+                        const float* b = p.bias + bpix[j] + (long)(o < p.M ? o : p.M - 1) * p.bias_sc;
+                        even[i][j][r] += b[0];
+                        acc[i][j][r] += b[both[j] ? 1 : 0];
+                    }
+        }
+#pragma unroll
+        for (int i = 0; i < TM; i++)
+#pragma unroll
+            for (int j = 0; j < TN; j++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int o = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
+                    float* to = y + out[j] + (unsigned)o * (unsigned)p.plane;
+                    if (o >= p.M) continue;
+                    if (both[j]) *reinterpret_cast<floatx2u*>(to) = floatx2u{even[i][j][r], acc[i][j][r]};
+                    else if (live[j]) *to = even[i][j][r];
+                }
+    } else finish(std::false_type{}, c, acc, live, 0, n_units);
 }
 
 // y = act(sum of the parts + bias): element idx is (image, channel, pixel)
@@ -669,6 +746,7 @@ static int cl_pick(int tile, F go) {
 struct ClWork {
     long dw, tiles[5], copies, steps;
     double mean, prep, out;             // prep: bytes the first launch moves
+    double store;                       // bytes of result written per us
 };
 
 // Estimated time in us, and the plan it is for. Measured on 249 (layer, direction) pairs with 15 plans each (layers of 1 to 32 images, 3 to 512
@@ -697,7 +775,7 @@ static double cl_plan_search(const ClWork& w, ClPlan& best) {
                 const double step = two ? alone[w.dw][t] + (pair[w.dw][t] - alone[w.dw][t]) * share : alone[w.dw][t];
                 main += filled * (rounds > 1.0 ? load : (double)own) * step + (filled - 1.0) * 2.7;
             }
-            main += w.out / 3.3e6;
+            main += w.out / w.store;
             if (parts > 1) main += 2.6 + w.out * (2.0 * parts + 1.0) / 9.2e6;
             if (main < least) {
                 least = main;
@@ -735,12 +813,13 @@ static int launch(K kfn, dim3 grid, int threads, size_t lds, const A& a, hipStre
 static ClWork conv_work(const ClArgs& a, int copies, double prep) {
     ClWork w = {};
     w.copies = copies; w.prep = prep; w.out = (double)a.y_total * 4.0;
+    w.store = a.paired ? 5.5e6 : 3.3e6;
     for (int t = 0; t < 5; t++) {
         double all = 0.0;
-        for (int i = 0; i < a.n_classes; i++) {
+        for (int i = 0; i < a.n_classes; i += a.paired ? 2 : 1) {
             const ClClass& c = a.cls[i];
             const long n = (((long)a.images * c.Hc * c.Wc + CL_TILES[t].bn - 1) / CL_TILES[t].bn) * ((a.M + CL_TILES[t].bm - 1) / CL_TILES[t].bm);
-            const long k = ((long)c.nr * c.ns * a.cu + 7) / 8;
+            const long k = ((long)c.nr * c.ns * a.cu + 7) / 8 + (a.paired ? ((long)a.cls[i + 1].nr * a.cls[i + 1].ns * a.cu + 7) / 8 : 0);
             w.tiles[t] += n;
             all += (double)n * (double)k;
             if (k > w.steps) w.steps = k;
@@ -776,8 +855,9 @@ static size_t conv_cut(ClArgs& a, int copies, ClPlan& pl) {
         const int tiles = (int)(((long)a.images * c.Hc * c.Wc + sh.bn - 1) / sh.bn) * a.tiles_m;
         if (tiles > most) most = tiles;
     }
-    a.tiles = most * a.n_classes;
-    a.by_classes = cl_div(a.n_classes);
+    const int groups = a.paired ? a.n_classes / 2 : a.n_classes;
+    a.tiles = most * groups;
+    a.by_groups = cl_div(groups);
     return a.parts > 1 ? (size_t)a.parts * a.y_total * sizeof(float) : 0;
 }
 
@@ -785,11 +865,20 @@ static size_t conv_cut(ClArgs& a, int copies, ClPlan& pl) {
 static int conv_product(const ClArgs& a, int copies, const ClPlan& pl, hipStream_t s) {
     const dim3 grid((unsigned)a.tiles, (unsigned)a.parts, (unsigned)copies);
     const int mu = a.part_units < a.units ? a.part_units : a.units, kgs = CL_TILES[pl.tile].kg;
-    const size_t table = (size_t)(((mu + 7) / 8 + kgs - 1) / kgs + 4) * kgs * 8 * sizeof(int2);      // (steps + stages) of every group
+    size_t steps = 0;                                                 // of one workgroup's sum or two, at most
+    for (int i = 0; i < a.n_classes; i += a.paired ? 2 : 1) {
+        size_t n = 0;
+        for (int k = i; k < i + (a.paired ? 2 : 1); k++) n += ((std::min(a.cls[k].nr * a.cls[k].ns * a.cu, mu) + 7) / 8 + kgs - 1) / kgs;
+        steps = std::max(steps, n);
+    }
+    const size_t table = (steps + 4) * kgs * 8 * sizeof(int2);       // and the ring's stages
     int rc;
     auto go = [&](auto tile) {
         using T = decltype(tile);
-        return launch(a.n_classes > 1 ? cl_conv_kernel<T, true, true> : a.dy_h ? cl_conv_kernel<T, true, false> : cl_conv_kernel<T, false, false>, grid, T::THREADS, T::RING + table, a, s, "cl_conv kernel launch");
+        return launch(a.paired          ? cl_conv_kernel<T, true, true, true>
+                      : a.n_classes > 1 ? cl_conv_kernel<T, true, true, false>
+                      : a.dy_h          ? cl_conv_kernel<T, true, false, false>
+                                        : cl_conv_kernel<T, false, false, false>, grid, T::THREADS, T::RING + table, a, s, "cl_conv kernel launch");
     };
     rc = cl_pick(pl.tile, go);
     if (rc == NZHIP_OK && a.parts > 1) {
@@ -857,8 +946,10 @@ static void data_args(ClArgs& a, int (&edge)[4], size_t N, size_t C, size_t H, s
     a.x_img = (long)Hp * Wp * Os; a.w_img = (long)C * a.w_row; a.y_img = (long)C * H * W;
     a.w_bytes = (unsigned)(a.w_img * 2); a.x_bytes = (unsigned)(a.images * a.x_img * 2);
     a.plane = (long)H * W; a.y_total = (long)N * a.y_img;
+    const bool pairs = st == 2 && W > 1;                            // columns 0, 2, .. first
     for (int i = 0; i < st; i++)
-        for (int j = 0; j < st; j++) {
+        for (int q = 0; q < st; q++) {
+            const int j = pairs ? (q + (int)pad) & 1 : q;
             const Side h = side(i, (int)H, (int)K_h), v = side(j, (int)W, (int)K_w);
             if (!h.n || !v.n) continue;
             a.cls[a.n_classes++] = {h.t, v.t, i, st, j, st, -Wp * Os, -Os, h.n, v.n, ((h.lo + edge[0]) * Wp + v.lo + edge[2]) * Os,
@@ -904,6 +995,22 @@ int cl_conv_forward(float* y, const float* x, const float* w, const float* bias,
     return rc ? rc : rc2 ? rc2 : rc3 ? rc3 : rc4;
 }
 
+// Whether a data gradient at stride 2 computes neighbouring columns in one workgroup. One class of columns after the other stores every second 4 bytes
+// of a line, twice: 16 x 128 x 56 x 56 <- 128 15 of 22 us, 2.3 TB/s. In pairs 8 bytes a lane go out at 5 TB/s, by half as many workgroups with sums twice
+// as long, which layers of few tiles do not fill the chip with. The model has both; on 130 layers the way it takes at this margin is
+// 1 % behind the better one in the geometric mean and 9 % at worst but for two of long sums on small images (508 channels 16 x 16 <- 318 46 or 59 us, 32 of 80 x 80 <- 480
+// 22 or 27). 16 x 128 x 56 x 56 <- 128 30.5 -> 25.4 us, 16 x 64 x 128 x 128 <- 128 51 -> 42, 8 x 392 x 80 x 80 <- 16 41 -> 25, 4 x 320 x 160 x 160 <- 30 68 -> 38.
+// Where the stores would gain less than 1.2 % the model's last rounds decide, and not well (10 x 13 x 92 x 92 <- 389 7x7 120 or 124).
+// Not taken: 16 x 17 x 27 x 27 <- 128 7x7 15.5 or 20.9, 10 x 39 x 32 x 32 <- 240 12.8 or 15.6.
+static bool cl_paired(ClArgs& a, size_t stride, size_t W, int copies) {
+    if (stride != 2 || W < 2) return false;
+    if (const char* e = getenv("NZHIP_CONV_CL_PAIRED")) return atoi(e);      // read per call (tests, benchmarking)
+    ClPlan pl;
+    const double one = cl_plan(conv_work(a, copies, 0.0), pl);
+    a.paired = 1;
+    return 1.1 * cl_plan(conv_work(a, copies, 0.0), pl) < one && (double)a.y_total * 5e-7 > 0.012 * one;      // that the stores gain
+}
+
 int cl_conv_backward_data(float* dx, const float* dy, const float* w, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w,
                           size_t stride, size_t pad, size_t w_batch, int accumulate, hipStream_t s) {
     ClArgs a = {};
@@ -914,6 +1021,7 @@ int cl_conv_backward_data(float* dx, const float* dy, const float* w, size_t N, 
     _Float16* wc = nullptr;
     if (int rc = workspace_alloc(reinterpret_cast<void**>(&zc), N * (size_t)a.x_img * 2, s)) return rc;
     const int copies = w_batch > 1 ? (int)N : 1;
+    a.paired = cl_paired(a, stride, W, copies);
     ClPlan pl = {0, 1};
     int rc = workspace_alloc(reinterpret_cast<void**>(&wc), w_batch * (size_t)a.w_img * 2, s);
     if (const size_t bytes = rc ? 0 : conv_cut(a, copies, pl)) rc = workspace_alloc(reinterpret_cast<void**>(&a.partial), bytes, s);
@@ -944,6 +1052,7 @@ static ClWork dw_work(size_t N, size_t C, size_t O, size_t taps, size_t P, size_
     w.steps = (pixels + 63) / 64;
     w.mean = (double)w.steps;
     w.out = 8.0 * (double)w_batch * (double)(C * taps * O);
+    w.store = 3.3e6;
     return w;
 }
 

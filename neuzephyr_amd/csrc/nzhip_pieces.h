@@ -7,6 +7,7 @@
 namespace nzhip {
 
 typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef float piece4 __attribute__((ext_vector_type(4)));
 
 // element e of a piece that was moved back by `back` elements; what lies beyond the extent comes out as some element of it

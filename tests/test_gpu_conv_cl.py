@@ -103,6 +103,51 @@ def test_every_tile_is_bit_exact_on_whole_numbers(nz, monkeypatch, tile, layer):
         assert np.array_equal(dw.cpu().numpy(), dw64 + old_dw) and untouched(buf, w.size)
 
 
+# N, C, H, W, O, K, pad, copies: rows of an odd and an even number of columns, of two and three; one row; no tap for the even columns, for the odd
+# ones; a second channel tile of one row; more columns than windows reach
+PAIRS = [(2, 8, 9, 11, 24, 3, 1, 1), (3, 65, 8, 12, 13, 3, 1, 3), (2, 5, 7, 2, 9, 3, 1, 1), (2, 5, 6, 3, 9, 3, 0, 2), (1, 9, 1, 40, 8, 1, 0, 1),
+         (2, 12, 10, 9, 17, 1, 0, 1), (2, 4, 14, 15, 8, 7, 3, 1), (4, 40, 4, 4, 72, 4, 3, 1), (2, 33, 10, 13, 9, 2, 1, 2), (5, 20, 6, 6, 17, 5, 0, 1)]
+
+
+@pytest.mark.parametrize("layer", PAIRS)
+@pytest.mark.parametrize("tile", TILES)
+def test_columns_in_pairs_are_bit_exact_on_whole_numbers(nz, monkeypatch, tile, layer):
+    N, C, H, W, O, K, pad, copies = layer
+    rng = np.random.default_rng(sum(layer) + tile)
+    Ho, Wo = (H + 2 * pad - K) // 2 + 1, (W + 2 * pad - K) // 2 + 1
+    x, w, dy, old = np.zeros((N, C, H, W), np.float32), whole(rng, copies if copies == 1 else N, 1, C * K * K, O), whole(rng, N, O, Ho, Wo), whole(rng, N, C, H, W)
+    _, dx64, _ = reference(x, w, dy, K, K, 2, pad)
+    monkeypatch.setenv("NZHIP_CONV_CL", "1")
+    monkeypatch.setenv("NZHIP_CONV_CL_PAIRED", "1")
+    for parts in (1, 2):
+        monkeypatch.setenv("NZHIP_CONV_CL_PLAN", f"{tile},{parts}")
+        for accumulate in (False, True):
+            buf, dx = embedded(old if accumulate else np.full(x.shape, np.nan, np.float32))
+            nz.conv2d_backward_data(dx, embedded(dy)[1], embedded(w)[1], K, K, 2, pad, accumulate=accumulate)
+            assert np.array_equal(dx.cpu().numpy(), dx64 + (old if accumulate else 0)) and untouched(buf, x.size), (parts, accumulate)
+
+
+@pytest.mark.parametrize("special", [float("inf"), float("nan"), -7e4])
+@pytest.mark.parametrize("K,W", [(3, 10), (3, 11), (5, 10)])
+def test_a_special_weight_reaches_only_its_columns_of_a_pair(nz, monkeypatch, special, K, W):
+    import torch
+    N, C, H, O, pad = 2, 70, 11, 20, K // 2
+    rng = np.random.default_rng(7)
+    Ho, Wo = (H + 2 * pad - K) // 2 + 1, (W + 2 * pad - K) // 2 + 1
+    x, dy, w = np.zeros((N, C, H, W), np.float32), rng.integers(1, 3, (N, O, Ho, Wo)).astype(np.float32), rng.integers(1, 3, (1, 1, C * K * K, O)).astype(np.float32)
+    _, dx64, _ = reference(x, w, dy, K, K, 2, pad)
+    monkeypatch.setenv("NZHIP_CONV_CL", "1")
+    monkeypatch.setenv("NZHIP_CONV_CL_PAIRED", "1")
+    for c, tap, o in ((0, 0, 0), (C - 1, K * K - 1, O - 1), (33, K // 2 * K, 7), (64, 1, 8)):
+        ws, mark = w.copy(), np.zeros_like(w)
+        ws[0, 0, c * K * K + tap, o], mark[0, 0, c * K * K + tap, o] = special, 1
+        _, hit, _ = reference(x, mark, dy, K, K, 2, pad)
+        dx = torch.ones(x.shape, device="cuda")
+        nz.conv2d_backward_data(dx, torch.from_numpy(dy).cuda(), torch.from_numpy(ws).cuda(), K, K, 2, pad)
+        got = dx.cpu().numpy()
+        assert np.array_equal(np.isfinite(got), hit == 0) and np.array_equal(got[hit == 0], dx64[hit == 0] + 1), (c, tap, o)
+
+
 @pytest.mark.parametrize("special", [float("inf"), float("nan"), 7e4])             # 7e4 is infinite in fp16
 @pytest.mark.parametrize("K,stride,pad", [(3, 1, 1), (3, 2, 1), (5, 1, 2)])
 def test_a_special_value_stays_in_the_sums_it_is_a_term_of(nz, monkeypatch, special, K, stride, pad):
