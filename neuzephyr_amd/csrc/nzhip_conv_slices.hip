@@ -262,8 +262,10 @@ static ConvSliceArgs conv_slices_args(bool data, size_t N, size_t C, size_t H, s
 // - a wave's chain of chunks: up to 80 units, 130 where 100 tiles and more share the weights (1 x 336 x 16 x 16 -> 314 14.6 / 18.3, 189 units; 2 x 240 x 16 x 16
 //   -> 66 12.1 / 11.4, 135)
 // - what the tiles take in: 90 MB (16 x 64 x 12 x 48 -> 176, 255 MB, 13.1 / 17.6; 16 x 10 x 32 x 8 -> 224 5x5, 92 MB, 10.3 / 10.3), a data gradient 80
-//   (10 x 16 x 48 x 48 <- 80, 133 MB, 15.6 / 10.7, but 4 x 104 x 64 x 64 <- 19, 151 MB, 10.7 / 13.7), 60 at strides, where it multiplies zeros
-//   (10 x 16 x 32 x 32 <- 96 at stride 2, 71 MB, 9.8 / 10.7)
+//   (10 x 16 x 48 x 48 <- 80, 133 MB, 15.6 / 10.7, but 4 x 104 x 64 x 64 <- 19, 151 MB, 10.7 / 13.7)
+// - data gradients at strides, which multiply zeros here: up to 72 units (1 x 105 x 39 x 39 <- 126, 72, 9.7 / 9.2; 5x5 1 x 79 x 21 x 21 <- 40, 75, 9.6 / 9.8;
+//   10 x 15 x 19 x 19 <- 194, 117, 11.5 / 13.3) and 60 MB, 45 MB where some CUs get two of the tiles (16 x 11 x 25 x 25 <- 48, 35 MB, 10.3 / 8.0;
+//   4 x 26 x 46 x 46 <- 27 5x5, 268 tiles, 55 MB, 8.8 / 10.3), drawn on 45 more
 // - tiles: 3300 and 1500 (16 x 11 x 80 x 80 -> 48 1x1, 6400, 20.5 / 17.3, but 8 x 5 x 80 x 80 -> 138, 8000, 24.2 / 24.8)
 // - forwards of 1x1 at strides, which otherwise copy the pixels they look at first: 350 MB (10 x 400 x 150 x 150 -> 21 105 / 47, 4 x 288 x 158 x 158 -> 171 55 / 50)
 // - 1x1 data gradients are one product already: only those of up to 8 channels, on which the streaming kernels are slow (16 x 8 x 88 x 88 <- 480 127 / 49)
@@ -273,7 +275,8 @@ static int conv_slices_shape(bool data, const ConvSliceArgs& a, bool one, size_t
     if (one && data && stride == 1) return a.M <= 8 && a.K >= 32 && mb <= 500 ? shape : -1;
     if (one && !data && stride > 1) return mb <= 350 && a.total <= 5000 ? shape : -1;
     if (a.units > (a.total >= 100 ? 130 : 80)) return -1;
-    return mb <= (!data ? 90 : stride > 1 ? 60 : 80) && a.total <= (data ? 1500 : 3300) ? shape : -1;
+    if (data && stride > 1 && (a.units > 72 || mb > (a.total > 256 ? 45 : 60))) return -1;
+    return mb <= (!data ? 90 : 80) && a.total <= (data ? 1500 : 3300) ? shape : -1;
 }
 
 int conv_slices_plan(ClDirection dir, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad, size_t w_batch) {
