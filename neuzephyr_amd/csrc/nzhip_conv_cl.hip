@@ -165,6 +165,7 @@ struct ClArgs {
     int paired;                         // classes 2 i and 2 i + 1 are the even and the odd columns of the same rows, and one workgroup's
     int dy_h, dy_w;                     // dy's extents; 0 in a forward
     int units;                          // of the longest sum (host)
+    int early_bias;                     // requested before the first step
     ClDiv by_cu, by_tiles_m, by_groups;     // groups: the classes, or the pairs of them
     ClClass cls[CL_MAX_CLASSES];
 };
@@ -258,6 +259,51 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
         const int img = cl_quot(px, c.by_hw), q = px - img * hw, i = cl_quot(q, c.by_w), k = q - i * c.Wc;
         row_b[j] = (unsigned)(img * (int)p.x_img + c.base + i * p.step_h + k * p.step_w) * 2u;
     }
+
+    // the results: lane = pixel, registers = channels (r >> 2) * 8 + lh * 4 + (r & 3)
+    unsigned out[TN];
+    long bpix[TN];
+    bool live[TN], both[TN];                                        // both: the odd column's neighbour too
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        const int px = n0 + (wn * TN + j) * 32 + li;
+        live[j] = px < pixels;
+        const int pc = live[j] ? px : pixels - 1, img = cl_quot(pc, c.by_hw), q = pc - img * hw, i = cl_quot(q, c.by_w), k = q - i * c.Wc;
+        const int pl = c.out + i * c.out_h + k * c.out_w;
+        both[j] = PAIRED && live[j] && k < odd.Wc;
+        out[j] = (unsigned)((z + img) * (int)p.y_img + pl);
+        bpix[j] = (long)(z + img) * p.bias_sn + pl * p.bias_sp;
+    }
+    const bool split = p.parts > 1;
+    float* y = split ? p.partial + blockIdx.y * p.y_total : p.y;
+    // The bias of a forward of up to two workgroups a CU is requested before the first step: after the last one it was a trip to memory between
+    // the sums and their stores (16 x 256 x 14 x 14 -> 256 18.0 -> 17.4 us a call, 4 x 87 x 59 x 59 -> 50 14.3 -> 13.5; 36 layers 1.5 % in the geometric
+    // mean). With more, others cover that trip and first steps would wait for it (16 x 16 x 48 x 48 -> 135 21.3, asked for by all waves at the start
+    // 23.8), and waves without a result must not ask (32 x 48 x 51 x 51 -> 16 7x7 25.8 -> 27). The old values of a weight gradient, twice the registers,
+    // gained nothing that way (0 to 4 %, but 16 x 100 x 20 x 20 -> 200 with a copy per image 21.0 -> 22.2).
+    float bias[DATA ? 1 : TM][DATA ? 1 : TN][16];
+    auto request_bias = [&] {
+        if constexpr (!DATA) {
+            const bool quads = p.bias_sc == 1;
+#pragma unroll
+            for (int i = 0; i < TM; i++)
+#pragma unroll
+                for (int j = 0; j < TN; j++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        const int o = m0 + (wm * TM + i) * 32 + g * 8 + lh * 4;
+                        if (quads && o + 4 <= p.M) {
+                            const piece4 v = *reinterpret_cast<const floatx4u*>(p.bias + bpix[j] + o);
+#pragma unroll
+                            for (int e = 0; e < 4; e++) bias[i][j][g * 4 + e] = v[e];
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 4; e++) bias[i][j][g * 4 + e] = p.bias[bpix[j] + (long)(o + e < p.M ? o + e : p.M - 1) * p.bias_sc];
+                        }
+                    }
+        }
+    };
+    if (p.early_bias && kg == 0 && m0 + wm * TM * 32 < p.M) request_bias();
 
     floatx16 acc[TM][TN];
 #pragma unroll
@@ -387,22 +433,7 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
 
     if (m0 + wm * TM * 32 >= p.M) return;                           // nothing of this wave's is stored
 
-    // ---- epilogue: lane = pixel, registers = channels (r >> 2) * 8 + lh * 4 + (r & 3); bias first, then the stores
-    unsigned out[TN];
-    long bpix[TN];
-    bool live[TN], both[TN];                                        // both: the odd column's neighbour too
-#pragma unroll
-    for (int j = 0; j < TN; j++) {
-        const int px = n0 + (wn * TN + j) * 32 + li;
-        live[j] = px < pixels;
-        const int pc = live[j] ? px : pixels - 1, img = cl_quot(pc, c.by_hw), q = pc - img * hw, i = cl_quot(q, c.by_w), k = q - i * c.Wc;
-        const int pl = c.out + i * c.out_h + k * c.out_w;
-        both[j] = PAIRED && live[j] && k < odd.Wc;
-        out[j] = (unsigned)((z + img) * (int)p.y_img + pl);
-        bpix[j] = (long)(z + img) * p.bias_sn + pl * p.bias_sp;
-    }
-    const bool split = p.parts > 1;
-    float* y = split ? p.partial + blockIdx.y * p.y_total : p.y;
+    // ---- epilogue
     // AGAIN: NaNs of pixels with taps outside dy may come from an infinite weight times the zeros there, and are summed again.
     // d: the class whose sums acc are, `by` columns right of the pixel at out[j]
     auto finish = [&](auto again_tag, const ClClass& d, floatx16 (&acc)[TM][TN], const bool (&live)[TN], const int by, const int n_units) {
@@ -421,22 +452,17 @@ __global__ __launch_bounds__(T::THREADS, 2) void cl_conv_kernel(const ClArgs p) 
                 }
             }
         if (p.bias && !split) {
-            const bool quads = p.bias_sc == 1;
+            if (!p.early_bias) request_bias();
 #pragma unroll
             for (int i = 0; i < TM; i++)
 #pragma unroll
                 for (int j = 0; j < TN; j++)
 #pragma unroll
-                    for (int g = 0; g < 4; g++) {
-                        const int o = m0 + (wm * TM + i) * 32 + g * 8 + lh * 4;
-                        if (quads && o + 4 <= p.M) {
-                            const piece4 v = *reinterpret_cast<const floatx4u*>(p.bias + bpix[j] + o);      // (by is 0)
-#pragma unroll
-                            for (int e = 0; e < 4; e++) acc[i][j][g * 4 + e] += v[e];
-                        } else {
-#pragma unroll
-                            for (int e = 0; e < 4; e++) acc[i][j][g * 4 + e] += p.bias[bpix[j] + (live[j] ? by : 0) + (long)(o + e < p.M ? o + e : p.M - 1) * p.bias_sc];
-                        }
+                    for (int r = 0; r < 16; r++) {
+                        if constexpr (DATA) {
+                            const int o = m0 + (wm * TM + i) * 32 + (r >> 2) * 8 + lh * 4 + (r & 3);
+                            acc[i][j][r] += p.bias[bpix[j] + (live[j] ? by : 0) + (long)(o < p.M ? o : p.M - 1) * p.bias_sc];
+                        } else acc[i][j][r] += bias[i][j][r];
                     }
         }
 #pragma unroll
@@ -988,6 +1014,7 @@ int cl_conv_forward(float* y, const float* x, const float* w, const float* bias,
     if (rc == NZHIP_OK) {
         a.w = reinterpret_cast<const _Float16*>(lease.ptr); a.x = xc; a.y = y; a.bias = bias;
         a.bias_sp = bias_sp; a.bias_sc = bias_sc; a.bias_sn = bias_sn; a.relu = relu;
+        a.early_bias = bias && a.parts == 1 && (long)a.tiles * copies <= 2 * device_cu_count();
         rc = conv_product(a, copies, pl, s);
     }
     const int rc2 = may_keep ? image_release(lease, s, enqueued) : workspace_free(lease.ptr, s), rc3 = workspace_free(xc, s);
