@@ -1029,13 +1029,22 @@ int cl_conv_forward(float* y, const float* x, const float* w, const float* bias,
 // 22 or 27). 16 x 128 x 56 x 56 <- 128 30.5 -> 25.4 us, 16 x 64 x 128 x 128 <- 128 51 -> 42, 8 x 392 x 80 x 80 <- 16 41 -> 25, 4 x 320 x 160 x 160 <- 30 68 -> 38.
 // Where the stores would gain less than 1.2 % the model's last rounds decide, and not well (10 x 13 x 92 x 92 <- 389 7x7 120 or 124).
 // Not taken: 16 x 17 x 27 x 27 <- 128 7x7 15.5 or 20.9, 10 x 39 x 32 x 32 <- 240 12.8 or 15.6.
-static bool cl_paired(ClArgs& a, size_t stride, size_t W, int copies) {
+static bool cl_paired(const ClArgs& a, size_t N, size_t H, size_t W, size_t K_h, size_t pad, size_t stride, int copies) {
     if (stride != 2 || W < 2) return false;
     if (const char* e = getenv("NZHIP_CONV_CL_PAIRED")) return atoi(e);      // read per call (tests, benchmarking)
-    ClPlan pl;
-    const double one = cl_plan(conv_work(a, copies, 0.0), pl);
-    a.paired = 1;
-    return 1.1 * cl_plan(conv_work(a, copies, 0.0), pl) < one && (double)a.y_total * 5e-7 > 0.012 * one;      // that the stores gain
+    struct Key { long N, C, H, W, cu, K_h, K_w, pad, copies, cus; };
+    struct Found { bool paired; };
+    static thread_local PlanCache<Key, Found> cache;
+    bool known;
+    Found& f = cache.at(Key{(long)N, a.M, (long)H, (long)W, a.cu, (long)K_h, a.Kw, (long)pad, copies, device_cu_count()}, known);
+    if (!known) {
+        ClPlan pl;
+        ClArgs two = a;
+        const double one = cl_plan(conv_work(a, copies, 0.0), pl);
+        two.paired = 1;
+        f.paired = 1.1 * cl_plan(conv_work(two, copies, 0.0), pl) < one && (double)a.y_total * 5e-7 > 0.012 * one;      // that the stores gain
+    }
+    return f.paired;
 }
 
 int cl_conv_backward_data(float* dx, const float* dy, const float* w, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w,
@@ -1048,7 +1057,7 @@ int cl_conv_backward_data(float* dx, const float* dy, const float* w, size_t N, 
     _Float16* wc = nullptr;
     if (int rc = workspace_alloc(reinterpret_cast<void**>(&zc), N * (size_t)a.x_img * 2, s)) return rc;
     const int copies = w_batch > 1 ? (int)N : 1;
-    a.paired = cl_paired(a, stride, W, copies);
+    a.paired = cl_paired(a, N, H, W, K_h, pad, stride, copies);
     ClPlan pl = {0, 1};
     int rc = workspace_alloc(reinterpret_cast<void**>(&wc), w_batch * (size_t)a.w_img * 2, s);
     if (const size_t bytes = rc ? 0 : conv_cut(a, copies, pl)) rc = workspace_alloc(reinterpret_cast<void**>(&a.partial), bytes, s);
