@@ -285,28 +285,40 @@ static bool slices_fit(const nzhip_gemm_desc& d, int shape) {
     return ra * d.lda + d.K < lim && rb * d.ldb + d.K < lim && (d.M / 32 + 1) * (d.N / 32 + 1) * members < (1 << 28);
 }
 
-// The shape a product is to run with, -1: another kernel is faster. Drawn on 430 products of 1 to 4096 rows and columns and 16 to 2500 k against
-// the kernels that took them before (us there / here):
+// The shape a product is to run with, -1: another kernel is faster. Drawn on 430 products of 1 to 4096 rows and columns and 16 to 2500 k, and again on 2600
+// of 1 to 4 rows or columns and 1900 others, against the kernels that took them before (us there / here):
 // - K up to 2048: past that a CU's intake of K x 64 elements outlasts a second launch (80 x 1760 x 288 10.0 / 8.4, 48 x 1943 x 112 9.7 / 7.5; 64 x 1728 x 384
 //   9.0 / 8.4, 48 x 2279 x 576 9.4 / 11.9, 11 x 2480 x 1040 8.4 / 9.7).
 // - 95 MB that the tiles take in, 130 where both operands run along k, and at most 1024 tiles: 1472 x 231 x 464 8.1 / 6.0, 373 x 704 x 884 10.0 / 7.5,
 //   1408 x 640 x 357 11.0 / 9.0, 984 x 1328 x 366 with B along k 12.5 / 11.7; 1000 x 777 x 513 11.5 / 12.4, 601 x 1481 x 485 13.8 / 15.2, 1305 x 409 x 819 (1066 tiles) 10.3 / 11.6.
-// - one or two rows or columns whose product only streams the other operand: up to 640 k (1 x 372 x 256 3.9 / 3.9, 378 x 352 x 2 5.8 / 4.9, 2 x 528 x 576
-//   5.4 / 4.3; 1 x 1516 x 480 4.5 / 5.9, 18 x 914 x 1 5.9 / 6.4), above that only with that operand across k, where the streaming kernel
-//   needs a second launch (1 x 832 x 3314 14.9 / 5.9, 288 x 1279 x 2 10.6 / 7.5).
+//   A fourth round of the CUs pays with both operands across k only (3056 x 421 x 304 with both along it, 960 tiles, 8.3 / 9.8, 736 x 639 x 1088 9.7 / 11.4, B along it
+//   1135 x 276 x 874 7.5 / 8.1): 768 tiles with both along it, 896 with B alone, 80 MB past 768 with A alone (356 x 426 x 2167, 816 tiles, 9.8 / 11.2).
+// - one or two rows or columns whose product only streams the other operand, with a kernel that does no more than that, along k: up to 640 k (378 x 352 x 2 5.8 / 4.9,
+//   2 x 528 x 576 5.4 / 4.3; 1 x 1516 x 480 4.5 / 5.9, 18 x 914 x 1 5.9 / 6.4); one row by rows of 16-byte pieces up to 128 (1 x 208 x 2 2.9 / 3.5, 1 x 448 x 263
+//   3.6 / 3.9), one column 32 (528 x 256 x 1 3.2 / 4.2, 976 x 368 x 1 3.6 / 4.5; 96 x 16 x 1 3.5 / 3.2), with other rows 384 by up to 64 of them (2 x 465 x 1 3.4 / 4.0;
+//   1 x 323 x 128 4.5 / 4.0).
+//   Across k the streaming kernel needs a second launch (1 x 832 x 3314 14.9 / 5.9, 288 x 1279 x 2 10.6 / 7.5), but not for a handful of k (195 x 6 x 1 2.8 / 3.4, one row or
+//   column of up to 16 in pieces) and not where a workgroup keeps whole columns, up to 4096 of them (2064 x 1136 x 1 4.0 / 6.1, 2 x 1424 x 2688 4.8 / 6.9; 1 x 1760 x 6000 14.7 / 9.0).
 // - 64 x 64 tiles where they fill two thirds of the CUs or more, in one round: 1378 x 690 x 448 10.9 / 8.6, 1344 x 864 x 624 11.7 / 10.8, 541 x 1472 x 1232
-//   15.9 / 14.2, 1024^3 13.5 / 11.7; 572 x 1024 x 1153 12.2 / 12.2, 727 x 1289 x 752 (144 tiles) 13.3 / 15.7, 1221 x 816 x 848 (280) 14.4 / 20.9. Not whole tiles
-//   with both operands along k, on which the fused kernel is at its best (1024^3 10.2 / 11.6).
+//   15.9 / 14.2, 1024^3 13.5 / 11.7; 572 x 1024 x 1153 12.2 / 12.2, 727 x 1289 x 752 (144 tiles) 13.3 / 15.7, 1221 x 816 x 848 (280) 14.4 / 20.9. With both operands along k
+//   up to 1280 k (588 x 1441 x 1136 14.9 / 16.9, 991 x 1507 x 650 15.9 / 17.0), and not whole tiles, on which the fused kernel is at its best (1024^3 10.2 / 11.6).
 static int slices_shape(const nzhip_gemm_desc& d) {
     const int64_t members = d.batch_n * d.batch_c, lo = d.M < d.N ? d.M : d.N;
     const bool a_kc = d.a_layout == NZHIP_LAYOUT_ROW, b_kc = d.b_layout == NZHIP_LAYOUT_TRANS;
     const int64_t t32 = (d.M + 31) / 32 * ((d.N + 31) / 32) * members, t64 = (d.M + 63) / 64 * ((d.N + 63) / 64) * members;
     const int cus = device_cu_count();
     if (d.K > 2048) return -1;
-    if (lo <= 2 && d.K > 640 && (d.M <= d.N ? b_kc || d.N == 1 : a_kc)) return -1;
+    if (lo <= 2) {
+        const int64_t hi = d.M < d.N ? d.N : d.M;
+        const SkinnyForm f = gemm_skinny_form(d);
+        if (d.K > 640 && (f.along || hi == 1)) return -1;
+        if (f.along && lo == 1 && (f.pieces ? d.K > (d.N == 1 ? 32 : 128) : d.K > 384 && hi <= 64)) return -1;
+        if (!f.along && (d.K < 10 || (lo == 1 && f.pieces && d.K <= 16) || (f.columns && hi <= 4096))) return -1;
+    }
+    const int64_t most = !b_kc ? 1024 : a_kc ? 768 : 896, in = a_kc && b_kc ? 130000000 : a_kc && t32 > 768 ? 80000000 : 95000000;
     // more tiles than CUs: workgroups of 4 waves, of which a CU holds more (1500 x 250 x 350 6.3 us with 4, 8.2 with 8)
-    if (t32 <= 1024 && t32 * d.K * 256 <= (a_kc && b_kc ? 130000000 : 95000000)) return t32 > cus || d.K <= 128 ? 0 : 1;
-    if (lo > 2 && t64 <= cus && t64 * 3 >= cus * 2 && d.K <= 1536 && !(a_kc && b_kc && (d.M | d.N | d.K) % 64 == 0)) return 2;
+    if (t32 <= most && t32 * d.K * 256 <= in) return t32 > cus || d.K <= 128 ? 0 : 1;
+    if (lo > 2 && t64 <= cus && t64 * 3 >= cus * 2 && d.K <= (a_kc && b_kc ? 1280 : 1536) && !(a_kc && b_kc && (d.M | d.N | d.K) % 64 == 0)) return 2;
     return -1;
 }
 

@@ -53,6 +53,9 @@ int gemm_of_columns(const nzhip_gemm_desc* desc, hipStream_t stream);
 // Bandwidth-bound kernels for M <= 8 (nzhip_skinny.hip).
 int gemm_skinny_dispatch(const nzhip_gemm_desc& d, hipStream_t stream);
 bool gemm_skinny_applicable(const nzhip_gemm_desc& d);
+// How they would read a product: the long operand's rows along k; 16 bytes at a time; all k of 16 columns by one workgroup
+struct SkinnyForm { bool along, pieces, columns; };
+SkinnyForm gemm_skinny_form(const nzhip_gemm_desc& d);
 // short contraction (K <= 32), one extent <= 16, the other long: streamed, one lane per long index
 bool gemm_thin_applicable(const nzhip_gemm_desc& d);
 int gemm_thin_dispatch(const nzhip_gemm_desc& d, hipStream_t stream);

@@ -353,10 +353,11 @@ bool gemm_skinny_applicable(const nzhip_gemm_desc& d) {
     return small >= 1 && small <= lim && big >= 1 && d.batch_n * d.batch_c <= 65535;
 }
 
-int gemm_skinny_dispatch(const nzhip_gemm_desc& d, hipStream_t stream) {
+// the kernels' arguments for a product; whether the long operand is stored with l contiguous
+static bool skinny_args(const nzhip_gemm_desc& d, SkinnyArgs& p) {
     const bool a_trans = d.a_layout == NZHIP_LAYOUT_TRANS, b_trans = d.b_layout == NZHIP_LAYOUT_TRANS;
-    SkinnyArgs p = {};
-    bool l_is_kl;                    // long operand stored with l contiguous
+    bool l_is_kl;
+    p = SkinnyArgs{};
     if (d.M <= d.N) {
         // skinny side = rows of A, long side = columns of B
         p.S = d.A;
@@ -400,14 +401,30 @@ int gemm_skinny_dispatch(const nzhip_gemm_desc& d, hipStream_t stream) {
     p.vec = ((p.ldl & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.L) & 15) == 0) && ((p.L_sn & 3) == 0) &&
             ((p.L_sc & 3) == 0) && ((reinterpret_cast<uintptr_t>(p.S) & 15) == 0) && ((p.S_sn & 3) == 0) &&
             ((p.S_sc & 3) == 0);
+    return l_is_kl;
+}
+
+// enough column groups to occupy the chip, a contraction long enough to stream: one kernel, no partial sums
+static bool skinny_columns(const SkinnyArgs& p, bool l_is_kl, int64_t batch) {
+    static const char* klc_env = getenv("NZHIP_SKINNY_COLS");           // benchmarking only: 0 keeps the split-contraction kernels
+    const bool klc_on = !klc_env || atoi(klc_env) != 0;
+    return l_is_kl && klc_on && batch == 1 && p.SR <= 2 && p.vec && p.LN % KLC_COLS == 0 && p.LN >= 128 * KLC_COLS && p.K >= 1024;
+}
+
+SkinnyForm gemm_skinny_form(const nzhip_gemm_desc& d) {
+    SkinnyArgs p;
+    const bool l_is_kl = skinny_args(d, p);
+    return SkinnyForm{!l_is_kl, p.vec != 0, skinny_columns(p, l_is_kl, d.batch_n * d.batch_c)};
+}
+
+int gemm_skinny_dispatch(const nzhip_gemm_desc& d, hipStream_t stream) {
+    SkinnyArgs p;
+    const bool l_is_kl = skinny_args(d, p);
     const unsigned batch = (unsigned)(d.batch_n * d.batch_c);
     const int sr_t = p.SR <= 1 ? 1 : (p.SR <= 2 ? 2 : (p.SR <= 4 ? 4 : 8));
     int rc = NZHIP_OK;
     float* partial = nullptr;
-    static const char* klc_env = getenv("NZHIP_SKINNY_COLS");           // benchmarking only: 0 keeps the split-contraction kernels
-    const bool klc_on = !klc_env || atoi(klc_env) != 0;
-    if (l_is_kl && klc_on && batch == 1 && p.SR <= 2 && p.vec && p.LN % KLC_COLS == 0 && p.LN >= 128 * KLC_COLS && p.K >= 1024) {
-        // enough column groups to occupy the chip, a contraction long enough to stream: one kernel, no partial sums
+    if (skinny_columns(p, l_is_kl, batch)) {
         dim3 grid((unsigned)(p.LN / KLC_COLS));
         if (sr_t == 1) hipLaunchKernelGGL(skinny_kl_cols_kernel<1>, grid, dim3(KLC_THREADS), 0, stream, p);
         else hipLaunchKernelGGL(skinny_kl_cols_kernel<2>, grid, dim3(KLC_THREADS), 0, stream, p);

@@ -104,3 +104,35 @@ def test_sums_are_as_exact_as_those_of_the_other_kernels(nz, monkeypatch, M, K, 
         monkeypatch.setenv("NZHIP_GEMM_SLICES", route) if route else monkeypatch.delenv("NZHIP_GEMM_SLICES")
         err[route] = float((nz.gemm(A, B, b_trans=b_trans).double() - want).norm() / want.norm())
     assert err[None] <= 1.05 * err["0"], err                        # (the 2-norm of a few thousand elements moves by a few hundredths with their order)
+
+
+ROUTES = r"""
+import sys, torch
+from neuzephyr_amd import capi
+for line in sys.stdin:
+    M, K, N, at, bt = (int(v) for v in line.split())
+    A, B = torch.zeros((K, M) if at else (M, K), device="cuda"), torch.zeros((N, K) if bt else (K, N), device="cuda")
+    print("product", file=sys.stderr, flush=True)
+    capi.gemm(A, B, a_trans=bool(at), b_trans=bool(bt))
+"""
+
+# M, K, N, a_trans, b_trans and the shape: none where the kernels before take less time; 32 x 32 tiles of 4 and 8 waves, 64 x 64
+RULE = [((2064, 1136, 1, 1, 1), None), ((2, 1424, 2688, 0, 0), None), ((528, 256, 1, 0, 0), None), ((1, 208, 2, 0, 1), None), ((2, 465, 1, 0, 0), None),
+        ((1264, 8, 1, 1, 1), None), ((64, 16, 1, 1, 1), None), ((2, 8, 368, 0, 0), None), ((588, 1441, 1136, 0, 1), None), ((1, 1760, 6000, 0, 0), 1),
+        ((1, 100, 300, 0, 1), 0), ((1, 323, 128, 1, 1), 1), ((96, 16, 1, 0, 0), 0), ((378, 352, 2, 0, 1), 1), ((2, 40, 300, 0, 0), 0), ((588, 1200, 1136, 0, 1), 2),
+        ((900, 300, 900, 0, 0), 0), ((3056, 421, 304, 0, 1), 2), ((736, 648, 1088, 0, 1), 2), ((1135, 276, 874, 1, 1), 2), ((356, 426, 2167, 0, 0), 2)]
+
+
+def test_which_products_run_on_it():
+    """The lines of its rule: rows and columns that a streaming kernel reads in one launch, a fourth round of small tiles, long sums of large ones."""
+    import os
+    import re
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = {k: v for k, v in os.environ.items() if not k.startswith("NZHIP_")}
+    p = subprocess.run([sys.executable, "-c", ROUTES], input="\n".join(" ".join(map(str, s)) for s, _ in RULE), capture_output=True, text=True, timeout=100, cwd=root,
+                       env={**env, "NZHIP_TRACE": "1", "PYTHONPATH": root})
+    assert p.returncode == 0, p.stderr[-2000:]
+    taken = [re.search(r"sliced kernel, shape (\d)", t) for t in p.stderr.split("product\n")[1:]]
+    assert [int(t[1]) if t else None for t in taken] == [shape for _, shape in RULE]
