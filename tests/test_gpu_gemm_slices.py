@@ -136,3 +136,33 @@ def test_which_products_run_on_it():
     assert p.returncode == 0, p.stderr[-2000:]
     taken = [re.search(r"sliced kernel, shape (\d)", t) for t in p.stderr.split("product\n")[1:]]
     assert [int(t[1]) if t else None for t in taken] == [shape for _, shape in RULE]
+
+
+# samples, inputs, outputs of a Linear layer, and whether its two gradients take less time as a pair on rounded copies than one after the other
+PAIRS = [(201, 1168, 292, True), (457, 3888, 208, True), (562, 1008, 821, True), (1008, 1632, 128, False), (848, 352, 48, False), (736, 134, 8, False)]
+
+
+@pytest.mark.parametrize("S,I,O,pair", PAIRS)
+def test_gradients_of_a_layer_go_the_faster_way(nz, monkeypatch, S, I, O, pair):
+    """Told by the bits: the sums of the two ways are in different order."""
+    import torch
+    g = torch.Generator().manual_seed(S + I + O)
+    W, x, dz = (torch.randn(*s, generator=g).cuda() for s in ((1, 1, O, I), (S, 1, I, 1), (S, 1, O, 1)))
+
+    def gradients():
+        dW, dx = torch.ones(1, 1, O, I, device="cuda"), torch.ones(S, 1, I, 1, device="cuda")
+        nz.matmul_backward(dW, dx, W, x, dz)
+        return dW.view(O, I), dx.view(S, I)
+
+    def one_by_one():
+        dW, dx = torch.ones(O, I, device="cuda"), torch.ones(S, I, device="cuda")
+        nz.gemm(dz.view(S, O), x.view(S, I), a_trans=True, bias=dW, bias_strides=(I, 1), out=dW)
+        nz.gemm(dz.view(S, O), W.view(O, I), bias=dx, bias_strides=(I, 1), out=dx)
+        return dW, dx
+
+    same = lambda p, q: all(torch.equal(a, b) for a, b in zip(p, q))
+    got, apart = gradients(), one_by_one()
+    monkeypatch.setenv("NZHIP_GEMM_COPY", "1")
+    together = gradients()
+    assert not same(apart, together)
+    assert same(got, together if pair else apart)
