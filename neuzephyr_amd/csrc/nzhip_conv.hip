@@ -3175,7 +3175,7 @@ static int conv2d_forward_impl(float* y, const float* x, const float* w_ref, con
     if (w_mirror && (K_h != K_w || (K_h == 1 && K_w == 1)))     // mirrored taps as one reversed index need a square kernel; 1x1 routes take the weights as they lie
         return conv2d_forward_mirrored_copy(y, x, w_ref, bias, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, bias_stride_pixel,
                                             bias_stride_channel, bias_stride_image, activation, stream);
-    if (const int shape = w_mirror || conv_direct_applicable(C, O, K_h, K_w, stride, pad) ? -1 : conv_slices_plan(CL_FORWARD, N, C, H, W, O, K_h, K_w, stride, pad, w_batch); shape >= 0)
+    if (const int shape = w_mirror || conv_direct_applicable(C, O, K_h, K_w, stride, pad) ? -1 : conv_slices_plan(CL_FORWARD, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, bias && bias_stride_pixel != 0); shape >= 0)
         return conv_slices_run(false, shape, y, x, w_ref, bias, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, bias_stride_pixel, bias_stride_channel,
                                bias_stride_image, activation == NZHIP_ACT_RELU, 0, s);
     if (conv1x1_strided(K_h, K_w, stride, pad, N, C, H, W) && H_out * W_out >= 64) {
@@ -3434,7 +3434,7 @@ extern "C" int nzhip_conv2d_backward_data(float* dx, const float* dy, const floa
                          "nzhip_conv2d_backward_data: only square kernels, pad <= K-1 and stride <= 8 (use the column-matrix chain)");
     if (N == 0 || O == 0 || C == 0) return NZHIP_OK;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (const int shape = stride == 1 && conv_direct_applicable(O, C, K_h, K_w, 1, K_h - 1 - pad) ? -1 : conv_slices_plan(CL_DATA, N, C, H, W, O, K_h, K_w, stride, pad, w_batch); shape >= 0)
+    if (const int shape = stride == 1 && conv_direct_applicable(O, C, K_h, K_w, 1, K_h - 1 - pad) ? -1 : conv_slices_plan(CL_DATA, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, false); shape >= 0)
         return conv_slices_run(true, shape, dx, dy, w_ref, nullptr, N, C, H, W, O, K_h, K_w, stride, pad, w_batch, 0, 0, 0, 0, accumulate, s);
     if (conv1x1_strided(K_h, K_w, stride, pad, N, C, H, W) && ((H - 1) / stride + 1) * ((W - 1) / stride + 1) >= 64) {
         // 1x1 with a stride: the gradient of the pixels the convolution looked at, as a 1x1 stride-1 problem on the

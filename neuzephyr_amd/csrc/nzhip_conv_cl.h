@@ -23,9 +23,9 @@ int cl_conv_backward_data(float* dx, const float* dy, const float* w, size_t N, 
 int cl_conv_backward_weights(float* dw, const float* x, const float* dy, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w,
                              size_t stride, size_t pad, size_t w_batch, hipStream_t s);
 
-
 // Convolutions of few tiles in one launch (nzhip_conv_slices.hip). The shape to run one with, -1: not with these
-int conv_slices_plan(ClDirection dir, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad, size_t w_batch);
+// pixel_bias: a bias that differs from pixel to pixel
+int conv_slices_plan(ClDirection dir, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad, size_t w_batch, bool pixel_bias);
 int conv_slices_run(bool data, int shape, float* y, const float* x, const float* w, const float* bias, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w,
                     size_t stride, size_t pad, size_t w_batch, int64_t bias_sp, int64_t bias_sc, int64_t bias_sn, int relu, int accumulate, hipStream_t s);
 

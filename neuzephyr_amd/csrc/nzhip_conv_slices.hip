@@ -267,19 +267,34 @@ static ConvSliceArgs conv_slices_args(bool data, size_t N, size_t C, size_t H, s
 //   10 x 15 x 19 x 19 <- 194, 117, 11.5 / 13.3) and 60 MB, 45 MB where some CUs get two of the tiles (16 x 11 x 25 x 25 <- 48, 35 MB, 10.3 / 8.0;
 //   4 x 26 x 46 x 46 <- 27 5x5, 268 tiles, 55 MB, 8.8 / 10.3), drawn on 45 more
 // - tiles: 3300 and 1500 (16 x 11 x 80 x 80 -> 48 1x1, 6400, 20.5 / 17.3, but 8 x 5 x 80 x 80 -> 138, 8000, 24.2 / 24.8)
+//   shared 1x1 forwards of more than 160 outputs 2000 (32 x 16 x 18 x 18 -> 192 8.6 / 10.7, 10 x 52 x 32 x 32 -> 320 9.9 / 11.1)
 // - forwards of 1x1 at strides, which otherwise copy the pixels they look at first: 350 MB (10 x 400 x 150 x 150 -> 21 105 / 47, 4 x 288 x 158 x 158 -> 171 55 / 50)
+//   not with a bias per pixel and more than 224 outputs where that and y are most of the traffic (8 x 20 x 80 x 80 -> 336 17.2 / 21.1, 4 x 14 x 112 x 112 -> 368
+//   17.5 / 21.2; 16 x 17 x 66 x 66 -> 211 17.9 / 13.9)
 // - 1x1 data gradients are one product already: only those of up to 8 channels, on which the streaming kernels are slow (16 x 8 x 88 x 88 <- 480 127 / 49)
-static int conv_slices_shape(bool data, const ConvSliceArgs& a, bool one, size_t stride) {
+static int conv_slices_shape(bool data, const ConvSliceArgs& a, bool one, size_t stride, bool pixel_bias) {
     const double mb = (double)a.total * a.units * 4096e-6;
     const int shape = a.total <= 512 && a.units > 8;                  // 8 waves where a CU gets one or two workgroups (8 x 240 x 8 x 8 -> 235 16.5 us with 4, 13.1 with 8)
     if (one && data && stride == 1) return a.M <= 8 && a.K >= 32 && mb <= 500 ? shape : -1;
-    if (one && !data && stride > 1) return mb <= 350 && a.total <= 5000 ? shape : -1;
+    if (one && !data && stride > 1) return mb <= 350 && a.total <= 5000 && !(pixel_bias && a.units <= 2 && a.tiles_m >= 8 && a.total > 3300) ? shape : -1;
+    if (one && !data && !a.w_img && a.tiles_m >= 6 && a.total > 2000) return -1;
     if (a.units > (a.total >= 100 ? 130 : 80)) return -1;
     if (data && stride > 1 && (a.units > 72 || mb > (a.total > 256 ? 45 : 60))) return -1;
     return mb <= (!data ? 90 : 80) && a.total <= (data ? 1500 : 3300) ? shape : -1;
 }
 
-int conv_slices_plan(ClDirection dir, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad, size_t w_batch) {
+// Estimated time in us of a forward that is no 1x1 at a stride, or a data gradient at stride 1, fitted on 1399 and 500 of them (11 % and 15 % off on average):
+// a wave's chunks, what a second workgroup adds to them, and the lines that 32 pixels of a channel lie on, at a stride two to four.
+static double conv_slices_cost(bool data, const ConvSliceArgs& a, int shape, bool pixel_bias) {
+    const double r = (double)a.total / device_cu_count(), more = r > 1.0 ? r - 1.0 : 0.0, out = (double)a.y_img * (a.total / a.tiles) * 1e-6;
+    const int nw = shape ? 8 : 4, two = shape && r > 1.0, lines = a.stride == 1 ? 0 : a.Wr >= 32 ? 1 : a.Wr >= 16 ? 2 : 3;
+    const double chunks = (double)(((a.units + 1) / 2 + nw - 1) / nw);
+    if (data) return shape ? 2.8 + chunks * (1.0 + 0.54 * two) + 0.0018 * a.total : 0.3 + 1.67 * chunks + r * (1.26 - 0.13 * chunks);
+    const double first = shape ? 0.93 + 0.07 * lines : 0.54 + 0.19 * lines, next = shape ? two * (0.51 + 0.16 * lines) : 0.37 * more;
+    return 2.7 + chunks * (first + next) + out * ((shape ? 1.8 : 0.9) + (pixel_bias ? 1.1 : 0.0));
+}
+
+int conv_slices_plan(ClDirection dir, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w, size_t stride, size_t pad, size_t w_batch, bool pixel_bias) {
     static const bool others = getenv("NZHIP_CONV_ROUTE") || getenv("NZHIP_CONV_DX") || getenv("NZHIP_CONV_1X1_GEMM") || getenv("NZHIP_CONV_TW") || getenv("NZHIP_CONV_BN");
     const char* env = getenv("NZHIP_CONV_SLICES");                    // read per call (tests, benchmarking): 0 never, 1 and 2 that shape wherever it fits
     // a run that asks for one of the other routes gets it
@@ -291,7 +306,17 @@ int conv_slices_plan(ClDirection dir, size_t N, size_t C, size_t H, size_t W, si
     const size_t Ho = (Hp - K_h) / stride + 1, Wo = (Wp - K_w) / stride + 1;
     if (N * ((C + O + 62) / 32 + 1) * ((H * W + Ho * Wo) / 32 + 2) >= lim) return -1;
     if (env) return atoi(env) >= 1 && atoi(env) <= 2 ? atoi(env) - 1 : -1;
-    return conv_slices_shape(dir == CL_DATA, conv_slices_args(dir == CL_DATA, N, C, H, W, O, K_h, K_w, stride, pad, w_batch), K_h == 1 && K_w == 1, stride);
+    const bool data = dir == CL_DATA, one = K_h == 1 && K_w == 1;
+    const ConvSliceArgs a = conv_slices_args(data, N, C, H, W, O, K_h, K_w, stride, pad, w_batch);
+    const int shape = conv_slices_shape(data, a, one, stride, pixel_bias);
+    if (shape < 0 || (one && (data || stride > 1)) || (data && stride > 1)) return shape;
+    // Near those lines the copies are often ahead, most of all with few channels, whose units are filled up, and at strides: taken where this one's estimate is
+    // 10 % below theirs, or just below with a weight copy per image, which they are slow on. Of 1399 forwards 121 were more than 5 % slower here than on the
+    // ways before (16 x 112 x 16 x 16 -> 283 3x3 at stride 2 13.0 / 18.7, 2 x 3 x 107 x 107 -> 318 9.3 / 12.1, 32 x 7 x 11 x 11 -> 336 8.7 / 10.4), 32 are now, by 0.4 to 2 us;
+    // of 347 gradients 18 (16 x 96 x 16 x 16 <- 4 7x7 8.6 / 10.8) and 4. Up to 64 outputs, 20 MB and 800 tiles this one is nearly always ahead.
+    if ((data || a.tiles_m >= 3) && ((double)a.total * a.units * 4096e-6 > 20 || a.total > 800) && cl_conv_fits(dir, N, C, H, W, O, K_h, K_w, stride, pad, w_batch) &&
+        conv_slices_cost(data, a, shape, pixel_bias) >= (!data && w_batch > 1 ? 1.0 : 0.9) * cl_conv_cost(dir, N, C, H, W, O, K_h, K_w, stride, pad, w_batch)) return -1;
+    return shape;
 }
 
 int conv_slices_run(bool data, int shape, float* y, const float* x, const float* w, const float* bias, size_t N, size_t C, size_t H, size_t W, size_t O, size_t K_h, size_t K_w,

@@ -93,3 +93,46 @@ def test_sums_are_as_exact_as_those_of_the_other_kernels(nz, monkeypatch, layer)
         err[route] = [np.linalg.norm(g.cpu().numpy() - r) / np.linalg.norm(r) for g, r in zip(got, want)]
     for name, before, now in zip(("y", "dx"), err["0"], err["2"]):
         assert now <= 1.05 * before, (name, before, now)              # (the 2-norm over thousands of elements moves by a few hundredths with their order)
+
+
+# n, C, H, O, K, stride, weight copies, bias per pixel: layers that other ways compute in less time, and neighbours on which this one does
+RULE = [((16, 112, 16, 283, 3, 2, 1, False), False), ((2, 3, 107, 318, 3, 2, 1, True), False), ((32, 7, 11, 336, 3, 1, 1, True), False), ((16, 40, 16, 283, 3, 2, 1, False), True),
+        ((10, 48, 7, 384, 5, 1, 10, True), True), ((8, 3, 90, 24, 3, 1, 1, False), True), ((4, 112, 48, 237, 1, 1, 4, True), True)]
+
+
+@pytest.mark.parametrize("layer,taken", RULE)
+def test_which_forwards_run_on_it(nz, monkeypatch, layer, taken):  # noqa: F811
+    """Told by the bits: the sums of the ways are in different order."""
+    import torch
+    N, C, H, O, K, stride, copies, pixel = layer
+    Ho = (H + 2 * (K // 2) - K) // stride + 1
+    g = torch.Generator().manual_seed(sum(layer))
+    x, w, b = (torch.randn(*s, generator=g).cuda() for s in ((N, C, H, H), (copies, 1, C * K * K, O), (1, 1, Ho * Ho, O)))
+    run = lambda: nz.conv2d_forward(x, w, b, K, K, stride, K // 2, bias_strides=(O if pixel else 0, 1))
+    got = run()
+    monkeypatch.setenv("NZHIP_CONV_SLICES", "0")
+    other = run()
+    monkeypatch.setenv("NZHIP_CONV_SLICES", "1")
+    here = [run()]
+    monkeypatch.setenv("NZHIP_CONV_SLICES", "2")
+    here.append(run())
+    assert not any(torch.equal(other, h) for h in here)
+    assert any(torch.equal(got, h) for h in here) if taken else torch.equal(got, other)
+
+
+@pytest.mark.parametrize("layer,taken", [((16, 96, 16, 4, 7, 1, 1), False), ((4, 223, 27, 4, 5, 1, 1), False), ((16, 40, 16, 4, 7, 1, 1), True), ((4, 100, 27, 40, 3, 1, 1), True)])
+def test_which_gradients_run_on_it(nz, monkeypatch, layer, taken):  # noqa: F811
+    import torch
+    N, C, H, O, K, stride, copies = layer
+    g = torch.Generator().manual_seed(sum(layer))
+    dy, w = (torch.randn(*s, generator=g).cuda() for s in ((N, O, H, H), (copies, 1, C * K * K, O)))
+    run = lambda: nz.conv2d_backward_data(torch.empty(N, C, H, H, device="cuda"), dy, w, K, K, stride, K // 2, accumulate=False)
+    got = run()
+    monkeypatch.setenv("NZHIP_CONV_SLICES", "0")
+    other = run()
+    monkeypatch.setenv("NZHIP_CONV_SLICES", "1")
+    here = [run()]
+    monkeypatch.setenv("NZHIP_CONV_SLICES", "2")
+    here.append(run())
+    assert not any(torch.equal(other, h) for h in here)
+    assert any(torch.equal(got, h) for h in here) if taken else torch.equal(got, other)
