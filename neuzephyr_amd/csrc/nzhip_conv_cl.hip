@@ -768,11 +768,11 @@ static int cl_pick(int tile, F go) {
     }
 }
 // How a product is cut: `list` workgroup tiles of each kind (CL_TILES) for one weight copy, `steps` k steps of 8 units or 64 pixels in
-// the longest sum and `mean` on average (the classes of a data gradient differ), `copies` weight copies, `out` bytes of result.
+// the longest sum, `after` in the other sum of its workgroup (columns in pairs) and `mean` in both on average (the classes of a data gradient
+// differ), `copies` weight copies, `out` bytes of result.
 struct ClWork {
-    long dw, tiles[5], copies, steps;
+    long dw, tiles[5], copies, steps, after, paired;
     double mean, prep, out;             // prep: bytes the first launch moves
-    double store;                       // bytes of result written per us
 };
 
 // Estimated time in us, and the plan it is for. Measured on 249 (layer, direction) pairs with 15 plans each (layers of 1 to 32 images, 3 to 512
@@ -787,21 +787,24 @@ static double cl_plan_search(const ClWork& w, ClPlan& best) {
     double least = 1e30;
     for (int t = 0; t < 5; t++) {
         const int kg = CL_TILES[t].kg;
+        // pairs on 128 x 64, a weight copy per image (16 x 352 x 26 x 26 <- 38 7x7 50.9 us, 41.6 on 64 x 128; shared, 16 x 80 x 49 x 49 <- 87 34.3, 38.9)
+        const double slow = w.paired && t == 2 && w.copies > 1 ? 1.2 : 1.0;
         for (int cut : cuts) {
             if (cut > 1 && (cut > w.steps || (double)cut * w.out > 5e8 || (double)w.tiles[t] * w.copies * cut > 8.0 * cus)) break;
-            const long per = (w.steps + cut - 1) / cut, parts = (w.steps + per - 1) / per, own = (per + kg - 1) / kg;
+            // each sum is cut at the same steps, so the first part has most of both
+            const long per = (w.steps + cut - 1) / cut, parts = (w.steps + per - 1) / per, also = w.after < per ? w.after : per, own = (per + kg - 1) / kg + (also + kg - 1) / kg;
             if (cut > 1 && parts != cut) continue;
-            const bool two = t != 1 && t != 4 && (w.dw || per * 8 <= (t == 0 ? 1900 : 900));      // LDS for two: ring and table
+            const bool two = t != 1 && t != 4 && (w.dw || (per + also) * 8 <= (t == 0 ? 1900 : 900));      // LDS for two: ring and table
             const double wgs = (double)w.tiles[t] * w.copies * parts, load = w.mean / parts / kg;
             double main = first[t];
-            if (wgs <= cus) main += own * alone[w.dw][t];
+            if (wgs <= cus) main += own * alone[w.dw][t] * slow;
             else {
                 const double rounds = wgs / (cus * (two ? 2 : 1)), filled = rounds < 1.0 ? 1.0 : rounds < 3.0 ? std::ceil(rounds) : rounds + 0.4;
                 const double share = wgs / cus - 1.0 < 1.0 ? wgs / cus - 1.0 : 1.0;
                 const double step = two ? alone[w.dw][t] + (pair[w.dw][t] - alone[w.dw][t]) * share : alone[w.dw][t];
-                main += filled * (rounds > 1.0 ? load : (double)own) * step + (filled - 1.0) * 2.7;
+                main += filled * (rounds > 1.0 ? load : (double)own) * step * slow + (filled - 1.0) * 2.7;
             }
-            main += w.out / w.store;
+            main += w.out / (w.paired ? 5.5e6 : 3.3e6);               // stores of 8 bytes a lane, of 4
             if (parts > 1) main += 2.6 + w.out * (2.0 * parts + 1.0) / 9.2e6;
             if (main < least) {
                 least = main;
@@ -839,16 +842,19 @@ static int launch(K kfn, dim3 grid, int threads, size_t lds, const A& a, hipStre
 static ClWork conv_work(const ClArgs& a, int copies, double prep) {
     ClWork w = {};
     w.copies = copies; w.prep = prep; w.out = (double)a.y_total * 4.0;
-    w.store = a.paired ? 5.5e6 : 3.3e6;
+    w.paired = a.paired;
     for (int t = 0; t < 5; t++) {
         double all = 0.0;
         for (int i = 0; i < a.n_classes; i += a.paired ? 2 : 1) {
             const ClClass& c = a.cls[i];
             const long n = (((long)a.images * c.Hc * c.Wc + CL_TILES[t].bn - 1) / CL_TILES[t].bn) * ((a.M + CL_TILES[t].bm - 1) / CL_TILES[t].bm);
-            const long k = ((long)c.nr * c.ns * a.cu + 7) / 8 + (a.paired ? ((long)a.cls[i + 1].nr * a.cls[i + 1].ns * a.cu + 7) / 8 : 0);
+            const long k = ((long)c.nr * c.ns * a.cu + 7) / 8, k2 = a.paired ? ((long)a.cls[i + 1].nr * a.cls[i + 1].ns * a.cu + 7) / 8 : 0;
             w.tiles[t] += n;
-            all += (double)n * (double)k;
-            if (k > w.steps) w.steps = k;
+            all += (double)n * (double)(k + k2);
+            if (k + k2 > w.steps + w.after) {
+                w.steps = std::max(k, k2);
+                w.after = std::min(k, k2);
+            }
         }
         if (t == 0) w.mean = w.tiles[0] ? all / (double)w.tiles[0] : 0.0;
     }
@@ -898,6 +904,8 @@ static int conv_product(const ClArgs& a, int copies, const ClPlan& pl, hipStream
         steps = std::max(steps, n);
     }
     const size_t table = (steps + 4) * kgs * 8 * sizeof(int2);       // and the ring's stages
+    if (gemm_trace())
+        fprintf(stderr, "nzhip_conv: channel-last copies, tile %d, %d part(s), planned %d%s\n", pl.tile, a.parts, pl.parts, a.paired ? ", columns in pairs" : "");
     int rc;
     auto go = [&](auto tile) {
         using T = decltype(tile);
@@ -1024,9 +1032,10 @@ int cl_conv_forward(float* y, const float* x, const float* w, const float* bias,
 
 // Whether a data gradient at stride 2 computes neighbouring columns in one workgroup. One class of columns after the other stores every second 4 bytes
 // of a line, twice: 16 x 128 x 56 x 56 <- 128 15 of 22 us, 2.3 TB/s. In pairs 8 bytes a lane go out at 5 TB/s, by half as many workgroups with sums twice
-// as long, which layers of few tiles do not fill the chip with. The model has both; on 130 layers the way it takes at this margin is
-// 1 % behind the better one in the geometric mean and 9 % at worst but for two of long sums on small images (508 channels 16 x 16 <- 318 46 or 59 us, 32 of 80 x 80 <- 480
-// 22 or 27). 16 x 128 x 56 x 56 <- 128 30.5 -> 25.4 us, 16 x 64 x 128 x 128 <- 128 51 -> 42, 8 x 392 x 80 x 80 <- 16 41 -> 25, 4 x 320 x 160 x 160 <- 30 68 -> 38.
+// as long, which layers of few tiles do not fill the chip with. The model has both; on 744 layers the way it takes at this margin is
+// 0.7 % behind the better one in the geometric mean. 204 go in pairs, three of them 7 to 9 % slower so (16 x 288 x 19 x 19 <- 180 24.9 or 27.2 us, a weight copy per
+// image); not taken though ahead are 34 by more than 5 %, most of all long sums on small images (16 x 508 x 16 x 16 <- 318 7x7 57.9 or 44.5, 4 x 32 x 80 x 80 <- 480 25.8 or
+// 21.7). 16 x 128 x 56 x 56 <- 128 30.5 -> 25.4 us, 16 x 64 x 128 x 128 <- 128 51 -> 42, 8 x 392 x 80 x 80 <- 16 41 -> 25, 4 x 320 x 160 x 160 <- 30 68 -> 38.
 // Where the stores would gain less than 1.2 % the model's last rounds decide, and not well (10 x 13 x 92 x 92 <- 389 7x7 120 or 124).
 // Not taken: 16 x 17 x 27 x 27 <- 128 7x7 15.5 or 20.9, 10 x 39 x 32 x 32 <- 240 12.8 or 15.6.
 static bool cl_paired(const ClArgs& a, size_t N, size_t H, size_t W, size_t K_h, size_t pad, size_t stride, int copies) {
@@ -1088,7 +1097,6 @@ static ClWork dw_work(size_t N, size_t C, size_t O, size_t taps, size_t P, size_
     w.steps = (pixels + 63) / 64;
     w.mean = (double)w.steps;
     w.out = 8.0 * (double)w_batch * (double)(C * taps * O);
-    w.store = 3.3e6;
     return w;
 }
 

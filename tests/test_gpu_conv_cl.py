@@ -309,3 +309,32 @@ def test_layers_take_the_faster_kernels(nz, monkeypatch, direction, layer, pixel
 
     on_copies, other, chosen = result("1"), result("0"), result(None)
     assert torch.equal(on_copies, chosen) == copies and torch.equal(other, chosen) == (not copies)
+
+
+PLANS = r"""
+import sys, torch
+from neuzephyr_amd import capi
+for line in sys.stdin:
+    n, C, H, O, K, copies = (int(v) for v in line.split())
+    Ho = (H + 2 * (K // 2) - K) // 2 + 1
+    print("layer", file=sys.stderr, flush=True)
+    capi.conv2d_backward_data(torch.zeros(n, C, H, H, device="cuda"), torch.zeros(n, O, Ho, Ho, device="cuda"), torch.zeros(copies, 1, C * K * K, O, device="cuda"), K, K, 2, K // 2)
+"""
+
+
+def test_plans_of_columns_in_pairs_are_what_is_launched():
+    """The parts that the estimate was for, in layers whose two sums differ in length; and not on 128 x 64 tiles, on which pairs are slow."""
+    import os
+    import re
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    env = {k: v for k, v in os.environ.items() if not k.startswith("NZHIP_")}
+    layers = [(1, 233, 25, 352, 5, 1), (8, 32, 80, 480, 7, 1), (32, 13, 44, 288, 7, 1), (4, 256, 16, 288, 5, 1), (16, 352, 26, 38, 7, 16)]
+    p = subprocess.run([sys.executable, "-c", PLANS], input="\n".join(" ".join(map(str, v)) for v in layers), capture_output=True, text=True, timeout=100, cwd=root,
+                       env={**env, "NZHIP_TRACE": "1", "NZHIP_CONV_CL": "1", "NZHIP_CONV_CL_PAIRED": "1", "PYTHONPATH": root})
+    assert p.returncode == 0, p.stderr[-2000:]
+    plans = re.findall(r"channel-last copies, tile (\d), (\d+) part\(s\), planned (\d+), columns in pairs", p.stderr)
+    assert len(plans) == len(layers)
+    assert all(parts == planned for _, parts, planned in plans), plans
+    assert max(int(parts) for _, parts, _ in plans) > 1 and plans[-1][0] != "2", plans
