@@ -3065,6 +3065,8 @@ static bool conv_cl_wanted(ClDirection dir, const float* src, size_t N, size_t C
         // one then takes the slower way by more than 5 %, 10x101x96x96 <- 8 28 / 20). 16x320x18x18 <- 80 7x7 at stride 2 261 / 20, 16x64x128x128
         // <- 128 100 / 43, 16x320x64x52 <- 39 63 / 32, 8x32x85x85 <- 151 36 / 18; few of a tile's 64 channels: 16x3x224x224 <- 64 7x7 106 / 129,
         // 8x5x208x208 <- 194 7x7 78 / 178, 16x4x192x192 <- 112 35 / 68
+        // With columns in pairs the estimate is that of the pairs from 8 channels on: 16x480x80x80 <- 32 87 / 50, 10x205x144x144 <- 32 90 / 49, 16x575x103x103 <- 20 214 / 139;
+        // 32x3x144x144 <- 27 31 / 38
         return cl_conv_cost(dir, N, C, H, W, O, K_h, K_w, stride, pad, w_batch) * 0.72 < other_us;
     }
     // 16x64x128x128 -> 128 at stride 2 47 / 54, 5x5 167 / 184; 8x14x144x144 -> 64 7x7 at stride 2, 41472 outputs, 38 / 25

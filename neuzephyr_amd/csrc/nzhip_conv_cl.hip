@@ -1111,8 +1111,12 @@ double cl_conv_cost(ClDirection dir, size_t N, size_t C, size_t H, size_t W, siz
     }
     ClArgs a = {};
     int edge[4];
-    if (dir == CL_FORWARD) forward_args(a, N, C, H, W, O, K_h, K_w, stride, pad, w_batch);
-    else data_args(a, edge, N, C, H, W, O, K_h, K_w, stride, pad, w_batch);
+    if (dir == CL_FORWARD) {
+        forward_args(a, N, C, H, W, O, K_h, K_w, stride, pad, w_batch);
+    } else {
+        data_args(a, edge, N, C, H, W, O, K_h, K_w, stride, pad, w_batch);
+        a.paired = C >= 8 && cl_paired(a, N, H, W, K_h, pad, stride, w_batch > 1 ? (int)N : 1);
+    }
     return cl_plan(conv_work(a, w_batch > 1 ? (int)N : 1, 1.5 * weights + (dir == CL_FORWARD ? x : y) + 2.0 * N * (double)a.x_img), pl);
 }
 

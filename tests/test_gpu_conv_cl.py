@@ -287,6 +287,7 @@ CHOICES = [
     ("forward", (16, 4, 176, 176, 64, 3, 1, 1, 16), False, False), ("forward", (10, 4, 160, 160, 192, 3, 1, 1, 10), False, True),
     ("forward", (16, 352, 64, 64, 128, 3, 1, 1, 1), False, False), ("forward", (10, 287, 128, 128, 32, 3, 1, 1, 1), False, True),
     ("data", (16, 212, 64, 64, 208, 3, 1, 1, 16), False, False), ("data", (16, 352, 64, 64, 128, 3, 1, 1, 1), False, True),
+    ("data", (8, 480, 80, 80, 32, 3, 2, 1, 1), False, True), ("data", (10, 48, 144, 144, 5, 3, 2, 1, 10), False, True), ("data", (32, 3, 144, 144, 27, 3, 2, 1, 1), False, False),
 ]
 
 
