@@ -475,8 +475,8 @@ static int gemm_routed(const nzhip_gemm_desc& d, hipStream_t s, bool slices) {
     if (gemm_thin_applicable(d)) return gemm_thin_dispatch(d, s);
     if (const int shape = slices ? gemm_slices_plan(d) : -1; shape >= 0) {
         if (gemm_trace())
-            fprintf(stderr, "nzhip_gemm %ld x %ld x %ld batch %ld x %ld: sliced kernel, shape %d, 1 chunk(s) of %ld, model %.1f us\n", (long)d.M, (long)d.K,
-                    (long)d.N, (long)d.batch_n, (long)d.batch_c, shape, (long)d.K, gemm_slices_cost(d, shape));
+            fprintf(stderr, "nzhip_gemm %ld x %ld x %ld batch %ld x %ld: sliced kernel, shape %d, model %.1f us\n", (long)d.M, (long)d.K,
+                    (long)d.N, (long)d.batch_n, (long)d.batch_c, shape, gemm_slices_cost(d, shape));
         return gemm_slices_run(d, shape, s);
     }
     if (gemm_skinny_applicable(d)) return gemm_skinny_dispatch(d, s);

@@ -16,3 +16,21 @@ def pytest_configure(config):
 def oracle():
     from oracle import oracle as orc
     return orc
+
+
+@pytest.fixture(params=["as chosen", "without sliced kernels"])
+def sliced(request, monkeypatch):
+    """Once as the library chooses and once with the kernels it has for more tiles, which the same sizes went to before there were others for few."""
+    if request.param != "as chosen":
+        monkeypatch.setenv("NZHIP_GEMM_SLICES", "0")
+        monkeypatch.setenv("NZHIP_CONV_SLICES", "0")
+
+
+@pytest.fixture(params=["as chosen", "without sliced kernels", "without copies"])
+def conv_ways(request, monkeypatch):
+    """The same, and once with the window, gather and column kernels."""
+    if request.param == "without sliced kernels":
+        monkeypatch.setenv("NZHIP_GEMM_SLICES", "0")
+        monkeypatch.setenv("NZHIP_CONV_SLICES", "0")
+    elif request.param == "without copies":
+        monkeypatch.setenv("NZHIP_CONV_CL", "0")

@@ -70,6 +70,7 @@ MATMUL_BWD_CASES = [
 ]
 
 
+@pytest.mark.usefixtures("sliced")
 @pytest.mark.parametrize("sa,sb", MATMUL_BWD_CASES)
 def test_matmul_backward_integers_bit_exact(nz, oracle, sa, sb):
     rng = np.random.default_rng(hash((sa, sb)) % (1 << 31))
@@ -90,6 +91,7 @@ def test_matmul_backward_integers_bit_exact(nz, oracle, sa, sb):
 @pytest.mark.parametrize("sa,sb,sc", [((2, 3, 5, 7), (2, 3, 7, 6), (2, 3, 5, 6)), ((3, 1, 5, 7), (1, 2, 7, 6), (1, 1, 5, 6)),
                                      ((3, 2, 5, 7), (3, 2, 7, 6), (1, 2, 5, 6)), ((3, 2, 5, 7), (3, 2, 7, 6), (3, 1, 5, 6)),
                                      ((1, 1, 40, 33), (1, 1, 33, 50), (1, 1, 40, 50))])
+@pytest.mark.usefixtures("sliced")
 def test_gemm_backward_entry_integers_bit_exact(nz, oracle, sa, sb, sc):
     rng = np.random.default_rng(17)
     A, B, C0 = ints(rng, sa), ints(rng, sb), ints(rng, sc, -9, 10)
@@ -99,6 +101,7 @@ def test_gemm_backward_entry_integers_bit_exact(nz, oracle, sa, sb, sc):
     assert np.array_equal(host(C), want)
 
 
+@pytest.mark.usefixtures("sliced")
 def test_linear_layer_backward_float_tolerance(nz, oracle):
     # Model::Linear shapes (W[1,1,OUT,IN] * x[n,1,IN,1]) at a size the oracle finishes quickly
     n, IN, OUT = 192, 256, 320
@@ -356,6 +359,7 @@ def _conv_grad_sweep_cases(seed, count):
     return cases
 
 
+@pytest.mark.usefixtures("conv_ways")
 @pytest.mark.parametrize("N,C,H,W,O,wb", _conv_grad_sweep_cases(20252, 48))
 def test_conv2d_gradients_random_sweep_integers_bit_exact(nz, oracle, N, C, H, W, O, wb):
     # 3x3, stride 1, padding 1 (what the fused gradients cover): both gradients against the node chain's sums
@@ -677,6 +681,7 @@ def _random_conv_geometries(count, seed, many_images=False):
     return cases
 
 
+@pytest.mark.usefixtures("conv_ways")
 @pytest.mark.parametrize("N,C,H,W,O,Kh,Kw,stride,pad,wb", _random_conv_geometries(48, 2024) + _random_conv_geometries(32, 7, many_images=True))
 def test_random_conv_geometries_forward_and_gradients_bit_exact(nz, oracle, N, C, H, W, O, Kh, Kw, stride, pad, wb):
     """Forward, weight gradient and (where the entry point covers the geometry) data gradient of one seeded random layer

@@ -277,6 +277,7 @@ BIAS_SHARED_BY_IMAGES = [  # N, C, H, W, O, per-sample weights: a per-pixel bias
     (3, 64, 32, 64, 128, False), (16, 48, 32, 64, 100, True), (16, 64, 32, 128, 128, True), (5, 16, 64, 64, 40, False)]
 
 
+@pytest.mark.usefixtures("conv_ways")
 @pytest.mark.parametrize("N,C,H,W,O,per_sample", BIAS_SHARED_BY_IMAGES)
 def test_conv2d_per_pixel_bias_with_every_xcd_on_one_eighth_of_all_images(nz, oracle, N, C, H, W, O, per_sample):
     rng = np.random.default_rng(N * 7 + C * 3 + H + W + O + per_sample)
@@ -291,6 +292,7 @@ def test_conv2d_per_pixel_bias_with_every_xcd_on_one_eighth_of_all_images(nz, or
     assert np.array_equal(got.astype(np.float64), truth)
 
 
+@pytest.mark.usefixtures("conv_ways")
 @pytest.mark.parametrize("N,C,H,W,O,k,pad,pix", PER_SAMPLE)
 def test_conv2d_per_sample_weights_that_differ_between_images(nz, oracle, N, C, H, W, O, k, pad, pix):
     # the reference's Conv2d parameter holds one weight copy per sample (src/Model.cu:248-252); here every copy is
@@ -335,6 +337,7 @@ def _conv_sweep_cases(seed, count):
     return cases
 
 
+@pytest.mark.usefixtures("conv_ways")
 @pytest.mark.parametrize("N,C,H,W,O,k_h,k_w,stride,pad,w_batch", _conv_sweep_cases(20251, 64))
 def test_conv2d_random_sweep_integers_bit_exact(nz, oracle, N, C, H, W, O, k_h, k_w, stride, pad, w_batch):
     rng = np.random.default_rng(N * 7 + C * 11 + H * 13 + W * 17 + O * 19 + k_h + stride + pad)
@@ -349,6 +352,7 @@ def test_conv2d_random_sweep_integers_bit_exact(nz, oracle, N, C, H, W, O, k_h, 
         assert np.array_equal(got[n:n + 1].astype(np.float64), truth), (n,)
 
 
+@pytest.mark.usefixtures("conv_ways")
 @pytest.mark.parametrize("N,C,H,W,O", [(2, 5, 10, 9, 6), (1, 128, 9, 64, 64), (1, 64, 8, 64, 128), (2, 64, 7, 64, 48), (1, 32, 8, 128, 64)])
 def test_conv2d_per_pixel_bias_like_the_reference_parameter(nz, oracle, N, C, H, W, O):
     x = oracle.fill((N, C, H, W), 61, "normal", 0.0, 1.0)

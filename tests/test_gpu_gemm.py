@@ -82,6 +82,7 @@ SKINNY = [(1, 1, 1), (1, 4096, 64), (1, 777, 513), (3, 300, 1000), (8, 64, 260),
           (1, 4096, 4096), (2, 1500, 2064), (2048, 1100, 2), (4096, 1024, 1)]
 
 
+@pytest.mark.usefixtures("sliced")
 @pytest.mark.parametrize("M,K,N", SKINNY)
 @pytest.mark.parametrize("a_trans,b_trans", [(False, False), (False, True), (True, False), (True, True)])
 def test_skinny_products_are_bit_exact_on_integers(nz, M, K, N, a_trans, b_trans):
@@ -97,6 +98,7 @@ def test_skinny_products_are_bit_exact_on_integers(nz, M, K, N, a_trans, b_trans
     assert np.array_equal(got, expect)
 
 
+@pytest.mark.usefixtures("sliced")
 def test_skinny_split_contraction_back_to_back(nz):
     # the streaming kernel's blocks leave partial sums in a pooled workspace that a second kernel adds: calls of
     # different shapes, queued without a wait between them on two streams, must not see each other's partials
@@ -133,6 +135,7 @@ DOT_ROWS = [(2, 114622, 16, 1), (1, 9000, 1, 1), (1, 8193, 257, 1), (2, 10242, 1
             (20, 8199, 5, 2), (1, 6143, 7, 1), (2, 1027, 5, 1), (1, 3, 70, 1)]
 
 
+@pytest.mark.usefixtures("sliced")
 @pytest.mark.parametrize("M,K,N,batch", DOT_ROWS)
 def test_skinny_dot_products_of_any_alignment_are_bit_exact_on_integers(nz, M, K, N, batch):
     import torch
@@ -351,6 +354,7 @@ def _route_sweep_cases():
     return cases
 
 
+@pytest.mark.usefixtures("sliced")
 @pytest.mark.parametrize("M,K,N", _route_sweep_cases())
 def test_default_route_is_bit_exact_on_integers(nz, M, K, N):
     # no forced kernel: whatever nzhip_gemm picks for the shape must give the exact integer product
@@ -367,6 +371,7 @@ def test_default_route_is_bit_exact_on_integers(nz, M, K, N):
 
 
 
+@pytest.mark.usefixtures("sliced")
 def test_skinny_batched_linear_single_sample(nz, oracle):
     # one sample through Model::Linear: W[1,1,OUT,IN] x[1,1,IN,1]
     OUT, IN = 1000, 515
@@ -383,6 +388,7 @@ def test_skinny_batched_linear_single_sample(nz, oracle):
     assert np.max(np.abs(got - ref)) <= 1e-4
 
 
+@pytest.mark.usefixtures("sliced")
 @pytest.mark.parametrize("M,K,N", [(1000, 777, 513), (700, 701, 333), (999, 1001, 1003), (516, 1030, 520)])
 @pytest.mark.parametrize("a_trans,b_trans", [(False, False), (False, True), (True, False), (True, True)])
 def test_operands_without_16_byte_rows_are_bit_exact_on_integers(nz, M, K, N, a_trans, b_trans):
@@ -505,13 +511,14 @@ def test_one_tile_products_are_split_by_their_length_and_not_by_the_alignment_of
     import sys
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     p = subprocess.run([sys.executable, "-c", PLANS], capture_output=True, text=True, timeout=100, cwd=root,
-                       env={**os.environ, "NZHIP_TRACE": "1", "PYTHONPATH": root})
+                       env={**os.environ, "NZHIP_TRACE": "1", "NZHIP_GEMM_SLICES": "0", "PYTHONPATH": root})
     assert p.returncode == 0, p.stderr[-2000:]
     chunks = [int(c) for c in re.findall(r"(\d+) chunk\(s\)", p.stderr)]
-    assert len(chunks) == 6 and chunks[:4] == [1] * 4               # too short to pay for a second launch
+    assert len(chunks) == 6 and "sliced" not in p.stderr and chunks[:4] == [1] * 4               # too short to pay for a second launch
     assert 8 <= chunks[4] <= 32 and 256 < chunks[5] <= 512           # two workgroups per compute unit for the longest
 
 
+@pytest.mark.usefixtures("sliced")
 @pytest.mark.parametrize("M,K,N,a_trans,b_trans,slack,offset,bias_form,seed", _embedded_cases())
 def test_embedded_operands_random_sweep(nz, M, K, N, a_trans, b_trans, slack, offset, bias_form, seed):
     # random shapes, layouts, leading dimensions and base offsets through the default route choice (streaming,
@@ -568,6 +575,7 @@ def test_embedded_operands_random_sweep(nz, M, K, N, a_trans, b_trans, slack, of
     assert np.all(np.isnan(got[:, N:])) and np.all(np.isnan(flat[:offset[2]])) and np.all(np.isnan(flat[offset[2] + M * ldc:]))
 
 
+@pytest.mark.usefixtures("sliced")
 def test_unaligned_base_pointers_take_the_scalar_path(nz):
     import torch
     rng = np.random.default_rng(5)
@@ -585,6 +593,7 @@ def test_unaligned_base_pointers_take_the_scalar_path(nz):
     assert np.array_equal(got, (A.astype(np.int64) @ B.astype(np.int64)).astype(np.float32))
 
 
+@pytest.mark.usefixtures("sliced")
 def test_identity_gives_fp16_rounding_including_special_values(nz, oracle):
     n = 96
     X = oracle.fill((n, n), 11, "uniform", -4.0, 4.0)
@@ -614,6 +623,7 @@ def test_config1_gemm_256_uniform(nz, oracle):
         assert np.max(np.abs(got - ref32)) <= 256 * 2.0 ** -23 * np.max(np.abs(truth))
 
 
+@pytest.mark.usefixtures("sliced")
 def test_config3_ragged_and_gemv(nz, oracle):
     A = oracle.fill((1000, 777), 3, "uniform", -1.0, 1.0)
     B = oracle.fill((777, 513), 1003, "uniform", -1.0, 1.0)
@@ -650,6 +660,7 @@ def test_config2_linear_bias_relu(nz, oracle):
 @pytest.mark.parametrize("sa,sb", [((2, 1, 2, 3), (1, 3, 3, 2)), ((3, 2, 5, 7), (3, 2, 7, 4)), ((1, 1, 9, 6), (4, 1, 6, 1)),
                                     ((2, 3, 4, 5), (1, 1, 5, 6)), ((1, 3, 4, 5), (2, 1, 5, 6)), ((5, 1, 1, 40), (1, 1, 40, 24)),
                                     ((4, 2, 130, 70), (1, 2, 70, 260)), ((1, 1, 33, 20), (3, 4, 20, 1))])
+@pytest.mark.usefixtures("sliced")
 def test_batched_broadcast_matches_oracle(nz, oracle, sa, sb):
     rng = np.random.default_rng(sum(sa) * 3 + sum(sb))
     A = rng.integers(-6, 7, size=sa).astype(np.float32)
@@ -671,6 +682,7 @@ def test_largest_batches(nz, sa, sb):
 @pytest.mark.parametrize("sa,sb", [((4, 1, 100, 1500), (1, 1, 1500, 130)),       # 4 members x 2 tiles, B shared
                                    ((3, 1, 130, 1100), (3, 1, 1100, 70)),        # both batched over n
                                    ((2, 1, 257, 4608), (1, 1, 4608, 250))])      # the column-matrix conv shape, small images
+@pytest.mark.usefixtures("sliced")
 def test_batched_products_with_few_tiles_split_the_contraction(nz, sa, sb):
     """Products batched over n whose tiles leave most CUs idle run their contraction in chunks (a
     workspace of partial sums per member, added in a fixed order): exact on integers."""
@@ -703,6 +715,7 @@ def test_thin_products_short_contraction_one_narrow_extent(nz, oracle, M, K, N, 
     assert np.array_equal(host(out), (P + bias).astype(np.float32))
 
 
+@pytest.mark.usefixtures("sliced")
 def test_bias_forms_and_relu_special_values(nz, oracle):
     M, K, N = 40, 24, 52
     rng = np.random.default_rng(1)

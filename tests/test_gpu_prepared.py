@@ -56,6 +56,7 @@ CONVS = [  # N, C, H, W, O, K, pad, w_batch: double-buffer resident kernel, sing
     (3, 24, 20, 20, 48, 1, 0, 1), (8, 16, 64, 64, 32, 3, 1, 8), (16, 16, 32, 32, 16, 5, 2, 1)]   # (1x1 below 32 channels: from there on it is a plain product without an image)
 
 
+@pytest.mark.usefixtures("conv_ways")
 @pytest.mark.parametrize("N,C,H,W,O,K,pad,wb", CONVS)
 def test_conv_forward_with_prepared_weights(nz, N, C, H, W, O, K, pad, wb):
     import torch
