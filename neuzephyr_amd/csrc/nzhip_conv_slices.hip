@@ -3,9 +3,9 @@
 // A small layer on channel-last copies is two launches, of which the first only rounds, and the column-matrix and strided 1x1 ways are two and
 // three; each launch is some 4 us of the host's time and 2 of the GPU's before any work. Here the waves gather fp32 themselves: about
 // 130 vector instructions and 32 requests for a chunk of 32 k, which is what bounds it (64 KB per CU in 0.5 us at best, the copies' kernels
-// take in half the bytes) and why larger layers stay with the others. us a call, host included, before and now: 16 x 4 x 10 x 10 -> 25 3x3 9.4 / 6.1,
-// 16 x 147 x 53 x 53 -> 16 1x1 at stride 2 15.1 / 6.5, 32 x 9 x 16 x 16 -> 16 7x7 at stride 2 14.3 / 7.9, 4 x 104 x 64 x 64 -> 19 3x3 15.4 / 9.3;
-// gradients 32 x 7 x 18 x 18 <- 93 1x1 17.7 / 5.8, 2 x 16 x 12 x 12 <- 48 3x3 8.7 / 5.7. Requests two or three chunks ahead changed nothing.
+// take in half the bytes) and why larger layers stay with the others. us a call, calls queued one behind the other, on the ways before and here:
+// 16 x 4 x 10 x 10 -> 25 3x3 7.3 / 4.0, 16 x 147 x 53 x 53 -> 16 1x1 at stride 2 15.3 / 5.3, 32 x 9 x 16 x 16 -> 16 7x7 at stride 2 10.8 / 8.1, 1 x 32 x 80 x 80 -> 11 5x5
+// 10.3 / 5.7; gradients 32 x 7 x 18 x 18 <- 93 1x1 14.2 / 4.1, 2 x 16 x 12 x 12 <- 48 3x3 8.2 / 4.9. Requests two or three chunks ahead changed nothing.
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>

@@ -66,7 +66,6 @@ __device__ __forceinline__ int phys_row(int r) {
 // per k tile finds the last one, whose missing k are zeroed, and one per tile the pieces that have to be turned back.
 // 16-byte accesses need no more than the 4-byte alignment of their elements: rows of 777 or 513 floats stream at the rate of
 // rows of 776 or 512 (1000 x 777 x 513: 14.9 us; element by element it was 33, through zero-padded copies of the operands 21).
-typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
 
 // How the accesses of an instance are kept inside the operands. INTERIOR: they are. PIECES: rows and 16-byte pieces are moved.
 // ELEMENTS: some contiguous extent is below 4, so pieces are made of single elements (an instance of its own: the choice made

@@ -3,10 +3,10 @@
 // Such a product is over in the time of a launch and a handful of requests to memory; what the other kernels spend is a chain of k steps with
 // a barrier each (the fused kernel), or a second launch (partial sums, rounded copies). Here every wave takes each 4th or 8th chunk of 32 k
 // of one tile, on its own: fp32 from memory to registers, fragments, MFMAs, no barrier and no data of another wave's until the sums meet in LDS
-// at the end. A product of 256^3 is 8 chunks, one per wave. In a workgroup's life of 2.9 us there 0.3 go by before the first request, 0.6 until it is
-// answered, 0.3 in the chunk, 0.3 in LDS, 1.0 in the sums and stores. With K = 2000 and 49 tiles a CU takes 100 GB/s in, what its vector memory path
-// returns to registers; that is what bounds it, so its tiles are 32 x 32 (more CUs) until there are enough of 64 x 64.
-// us before and now: 256^3 5.5 / 4.4, 300^3 8.0 / 4.9, 512^3 7.6 / 5.2, 100 x 1000 x 200 10.6 / 6.6, 33 x 512 x 33 9.9 / 4.9, 1024^3 13.8 / 11.9.
+// at the end. A product of 256^3 is 8 chunks, one per wave; half of a wave's cycles there are waits, and the launch is most of the rest. Longer sums are
+// bound by what the vector memory path returns to a CU's registers: a k of a 32 x 32 tile, 256 bytes, takes 2.2 to 2.3 ns (the estimate's fit below), 110 GB/s.
+// So tiles are 32 x 32 (more CUs) until there are enough of 64 x 64. us a call, calls queued one behind the other, on the kernels before and here:
+// 256^3 5.5 / 4.0, 300^3 8.0 / 4.4, 512^3 7.5 / 4.7, 100 x 1000 x 200 10.2 / 5.9, 33 x 512 x 33 9.8 / 4.4, 1024^3 12.7 / 11.5.
 #include <hip/hip_runtime.h>
 
 #include <cstdlib>
@@ -17,8 +17,6 @@
 #include "nzhip_slices.h"
 
 namespace nzhip {
-
-typedef float floatx2u __attribute__((ext_vector_type(2), aligned(4)));
 
 struct SliceArgs {
     const float* A;
