@@ -427,7 +427,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_f16mfma_kernel(const GemmKer
 
 // ---- host-side selection -------------------------------------------------------------------
 bool gemm_trace() {
-    static const char* env = getenv("NZHIP_TRACE");                  // 1: two lines per product on stderr (debugging only)
+    static const char* env = getenv("NZHIP_TRACE");                  // 1: lines per product and convolution on stderr (debugging only)
     return env && atoi(env);
 }
 
